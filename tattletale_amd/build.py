@@ -1,4 +1,4 @@
-"""Builds ``libttq_hip.so`` (gfx950 only) with hipcc.  ``python -m tattletale_amd.build``.
+"""Builds ``libttq_hip.so`` (gfx950 only) with hipcc and ``_ttq_torch.so`` with g++.  ``python -m tattletale_amd.build``.
 
 hipcc cross-compiles without a GPU, so this runs on any host with ROCm installed.  The
 library is written in-tree, next to this file.
@@ -14,6 +14,7 @@ from concurrent.futures import ThreadPoolExecutor
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libttq_hip.so")
+TORCH_EXT = os.path.join(HERE, "_ttq_torch.so")          # host half of the torch mirror (csrc/ttq_torch.cpp)
 LADDER_LIB = os.path.join(HERE, "libttq_ladder.so")      # bench.py's measurement ladders, built on demand
 
 SOURCES = [
@@ -128,6 +129,32 @@ def build_library(force: bool = True, verbose: bool = False) -> str:
     return LIB
 
 
+def build_torch_ext(force: bool = True, verbose: bool = False) -> str:
+    """Compile the native host half of qlinear.py (plain C++ against torch's headers; no device code)."""
+    import sysconfig
+
+    import torch
+    src = os.path.join(CSRC, "ttq_torch.cpp")
+    deps = [src, os.path.join(HERE, "..", "include", "ttq.h")]
+    if not force and os.path.exists(TORCH_EXT) and os.path.getmtime(TORCH_EXT) >= max(os.path.getmtime(d) for d in deps):
+        return TORCH_EXT
+    root = os.path.dirname(os.path.abspath(torch.__file__))
+    rocm = os.path.dirname(os.path.dirname(os.path.realpath(hipcc())))
+    include = [os.path.join(root, "include"), os.path.join(root, "include", "torch", "csrc", "api", "include"),
+               os.path.join(rocm, "include"), sysconfig.get_paths()["include"]]
+    cmd = [shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden",
+           "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch._C._GLIBCXX_USE_CXX11_ABI]
+    for d in include:
+        cmd += ["-isystem", d]
+    cmd += ["-o", TORCH_EXT, src, "-L" + os.path.join(root, "lib"), "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError("g++ failed for %s:\n%s\n%s" % (src, r.stdout, r.stderr))
+    if verbose:
+        print("built", TORCH_EXT)
+    return TORCH_EXT
+
+
 LADDER_SOURCES = ["ttq_ladder.hip", "ttq_ladder_gemm.hip"]
 
 
@@ -157,3 +184,4 @@ if __name__ == "__main__":
         build_ladder(force=True, verbose=True)
         sys.exit(0)
     build_library(force="--if-stale" not in sys.argv, verbose=True)
+    build_torch_ext(force="--if-stale" not in sys.argv, verbose=True)

@@ -21,7 +21,7 @@ from typing import Optional
 import torch
 
 from . import _lib
-from ._lib import BF16, F16, F32, QLinearStruct, TtqError, check
+from ._lib import BF16, F16, F32, QLinearStruct, TtqError, TtqLibraryError, check
 
 _DTYPE_CODE = {torch.float32: F32, torch.float16: F16, torch.bfloat16: BF16}
 
@@ -31,6 +31,34 @@ def _code(dt: torch.dtype) -> int:
         return _DTYPE_CODE[dt]
     except KeyError:
         raise TtqError(_lib.ERR_DTYPE, "dtype %s" % dt) from None
+
+
+_native_module = None
+
+
+def _native():
+    """The native host half (csrc/ttq_torch.cpp) with the library's entry points bound.  Its functions return the
+    output, a negative status, or 1 where the tensors are not what they take: the Python code behind each call then
+    finds and raises the error.  Raises if it is not built."""
+    global _native_module
+    if _native_module is None:
+        L = _lib.lib()
+        try:
+            from . import _ttq_torch as ext
+        except ImportError as e:
+            raise TtqLibraryError("tattletale_amd/_ttq_torch.so cannot be loaded (%s): build it with "
+                                  "`python -m tattletale_amd.build`" % e) from e
+        ext.bind(*(C.cast(fn, C.c_void_p).value for fn in (
+            L.ttq_linear_forward, L.ttq_linear_forward_ws, L.ttq_rmsnorm, L.ttq_silu_and_mul, L.ttq_gemv_q4_k_silu_mul,
+            L.ttq_gemm_q4_k_silu_mul)))
+        _native_module = ext
+    return _native_module
+
+
+def _native_status(r, where: str) -> None:
+    """Raises for a status of the library; returns for 1 (the caller goes on in Python)."""
+    if r != 1:
+        raise TtqError(r, where)
 
 
 def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
@@ -132,6 +160,12 @@ class QuantLinear:
         ``torch.float32`` for fp32 logits from 16-bit activations.  With ``workspace`` (a zero-filled
         uint8 tensor of at least ``workspace_bytes`` bytes) the call allocates nothing inside the
         library (``ttq_linear_forward_ws``)."""
+        r = (_native_module or _native()).linear_forward(
+            self.qweight, self.suh, self.svh, self.bias, self.format, self.in_features, self.out_features, self.bits,
+            self.codebook, self.precision, x, out_dtype, workspace)
+        if r.__class__ is not int:
+            return r
+        _native_status(r, "ttq_linear_forward" if workspace is None else "ttq_linear_forward_ws")
         if x.shape[-1] != self.in_features:
             raise TtqError(_lib.ERR_SHAPE, "QuantLinear.forward: last dim %d != in_features %d"
                            % (x.shape[-1], self.in_features))
@@ -324,6 +358,10 @@ def hadamard128_(v: torch.Tensor, pre: Optional[torch.Tensor] = None,
 def silu_and_mul(x: torch.Tensor) -> torch.Tensor:
     """(..., 2h) -> (..., h): silu(x[..., :h]) * x[..., h:]
     (workspace/transformers/src/kernels/activations.nim:14-38), through ``ttq_silu_and_mul``."""
+    r = (_native_module or _native()).silu_and_mul(x)
+    if r.__class__ is not int:
+        return r
+    _native_status(r, "ttq_silu_and_mul")
     dev = _require_device(x)
     if x.shape[-1] % 2:
         raise TtqError(_lib.ERR_SHAPE, "silu_and_mul: last dim must be even")
@@ -370,6 +408,10 @@ def rmsnorm(x: torch.Tensor, gamma: torch.Tensor, eps: float, residual: Optional
     """``RmsNorm.forward`` (residual None) / ``forward_with_residual``
     (workspace/transformers/src/layers/norm.nim:23-38) through ``ttq_rmsnorm``.
     Returns (normalized, new_residual or None)."""
+    r = (_native_module or _native()).rmsnorm(x, gamma, eps, residual)
+    if r.__class__ is not int:
+        return r
+    _native_status(r, "ttq_rmsnorm")
     dev = _require_device(x, gamma, residual)
     n = x.shape[-1]
     if gamma.numel() != n or gamma.dtype != x.dtype or (residual is not None and residual.shape != x.shape):
@@ -441,30 +483,38 @@ class QuantGatedMLP:
         ``FUSED_GEMM_MIN_ROWS`` rows the GEMM with silu_and_mul in its epilogue; everything else runs
         the projection, ``silu_and_mul`` and the down projection as three launches."""
         gu = self.gate_up_proj
-        n_ff = self.down_proj.in_features
-        m = x.numel() // gu.in_features
+        n_in, n_ff = gu.in_features, self.down_proj.in_features
         act = None
-        # one row, or two to four rows on the shapes whose fused kernel reads the weights once for all of them
-        # (rows of 2048 or 4096 values, 2 * n_ff from 4096 to 32768 weight rows)
-        few = 2 <= m <= 4 and gu.in_features in (2048, 4096) and n_ff % 8 == 0 and 2048 <= n_ff <= 16384
-        if gu.format == _lib.Q4_K and gu.bias is None and (m == 1 or few) and x.dtype in (torch.bfloat16, torch.float16):
-            try:
-                act = gemv_q4_k_silu_mul(gu.qweight, x.reshape(m, gu.in_features), n_ff, gu.in_features,
-                                         out_dtype=x.dtype).reshape(x.shape[:-1] + (n_ff,))
-            except TtqError as e:
-                if e.status != _lib.ERR_UNSUPPORTED:
-                    raise
-        elif (gu.format == _lib.Q4_K and gu.bias is None
-              and (m >= self.FUSED_GEMM_MIN_ROWS or self.FUSED_FEW_ROWS[0] <= m <= self.FUSED_FEW_ROWS[1])
-              and x.dtype == torch.bfloat16 and gu.in_features % 256 == 0):
-            try:
-                act = gemm_q4_k_silu_mul(gu.qweight, x.reshape(m, gu.in_features), n_ff,
-                                         gu.in_features).reshape(x.shape[:-1] + (n_ff,))
-            except TtqError as e:
-                if e.status != _lib.ERR_UNSUPPORTED:
-                    raise
+        if gu.format == _lib.Q4_K and gu.bias is None and x.dtype is not torch.float32 and x.shape[-1] == n_in:
+            m = x.numel() // n_in
+            # one row, or two to four rows on the shapes whose fused kernel reads the weights once for all of them
+            # (rows of 2048 or 4096 values, 2 * n_ff from 4096 to 32768 weight rows)
+            few = 2 <= m <= 4 and n_in in (2048, 4096) and n_ff % 8 == 0 and 2048 <= n_ff <= 16384
+            decode = m == 1 or few
+            if decode or (x.dtype is torch.bfloat16 and n_in % 256 == 0 and
+                          (m >= self.FUSED_GEMM_MIN_ROWS or self.FUSED_FEW_ROWS[0] <= m <= self.FUSED_FEW_ROWS[1])):
+                act = self._fused_activation(x, m, n_ff, n_in, not decode)
         if act is None:
             act = silu_and_mul(gu.forward(x))
         return self.down_proj.forward(act)
+
+    def _fused_activation(self, x: torch.Tensor, m: int, n_ff: int, n_in: int, gemm: bool) -> Optional[torch.Tensor]:
+        """silu(gate) * up in one launch; None where the shape has no fused kernel."""
+        qweight = self.gate_up_proj.qweight
+        r = (_native_module or _native()).q4_k_silu_mul(qweight, x, n_ff, n_in, gemm)
+        if r.__class__ is not int:
+            return r
+        if r == _lib.ERR_UNSUPPORTED:
+            return None
+        _native_status(r, "ttq_gemm_q4_k_silu_mul" if gemm else "ttq_gemv_q4_k_silu_mul")
+        try:                                     # tensors that the native half does not take
+            x2 = x.reshape(m, n_in)
+            act = (gemm_q4_k_silu_mul(qweight, x2, n_ff, n_in) if gemm else
+                   gemv_q4_k_silu_mul(qweight, x2, n_ff, n_in, out_dtype=x.dtype))
+        except TtqError as e:
+            if e.status != _lib.ERR_UNSUPPORTED:
+                raise
+            return None
+        return act.reshape(x.shape[:-1] + (n_ff,))
 
     __call__ = forward

@@ -1,0 +1,44 @@
+"""The native host half of qlinear.py (csrc/ttq_torch.cpp): what it hands back to Python, and that a call through it is
+the call through the C ABI."""
+import pytest
+import torch
+
+from tattletale_amd import QuantLinear, TtqError, _lib, formats as F, qlinear, quantize as Q
+
+
+def test_tensors_it_does_not_take_go_back_to_python():
+    n = qlinear._native()
+    x, g = torch.zeros(2, 256), torch.ones(256)
+    assert n.silu_and_mul(x) == 1 and n.rmsnorm(x, g, 1e-5, None) == 1          # not on a GPU
+    assert n.silu_and_mul(None) == 1 and n.linear_forward() == 1
+    layer = QuantLinear(torch.zeros(144, dtype=torch.uint8), F.Q4_K, 256, 1)
+    with pytest.raises(TtqError) as e:
+        layer.forward(x)
+    assert e.value.status == _lib.ERR_UNSUPPORTED
+
+
+@pytest.mark.gpu
+def test_forward_is_the_c_abi_call_and_errors_keep_their_status():
+    n_out, n_in = 48, 512
+    packed = torch.from_numpy(Q.quantize(F.Q4_K, Q.fill_normal(3, 0, 0.02, n_out * n_in).reshape(n_out, n_in))).cuda()
+    layer = QuantLinear.init(packed, F.Q4_K, n_in, n_out, bias=torch.ones(n_out, device="cuda"))
+    x = torch.randn(2, 3, n_in, device="cuda", dtype=torch.bfloat16)
+    y = layer.forward(x, out_dtype=torch.float32)
+    st, want = layer._struct(), torch.empty(6, n_out, device="cuda")
+    import ctypes as C
+    _lib.check(_lib.lib().ttq_linear_forward(C.byref(st), x.data_ptr(), F.BF16, 6, want.data_ptr(), F.F32,
+                                             torch.cuda.current_stream().cuda_stream), "abi")
+    assert y.shape == (2, 3, n_out) and torch.equal(y.view(6, n_out), want)
+    ws = torch.zeros(max(16, layer.workspace_bytes(6, x.dtype)), dtype=torch.uint8, device="cuda")
+    assert torch.equal(layer.forward(x, torch.float32, ws), y)
+    assert layer.forward(x[:0]).shape == (0, 3, n_out)
+    for bad, status in ((x[..., ::2], _lib.ERR_SHAPE), (x.transpose(0, 1), _lib.ERR_SHAPE), (x.cpu(), _lib.ERR_UNSUPPORTED),
+                        (x.double(), _lib.ERR_DTYPE)):
+        with pytest.raises(TtqError) as e:
+            layer.forward(bad)
+        assert e.value.status == status
+    with pytest.raises(TtqError) as e:                          # a status of the library itself
+        layer.forward(x, torch.float32, ws[1:])
+    assert e.value.status == _lib.ERR_WORKSPACE
+    out, res = qlinear.rmsnorm(x, torch.ones(n_in, device="cuda", dtype=x.dtype), 1e-5, x)
+    assert torch.equal(res, x + x) and out.shape == x.shape
