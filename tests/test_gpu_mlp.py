@@ -34,6 +34,17 @@ def test_silu_and_mul_elementwise(dt, ulp, tiny, m, h):
     assert np.all(np.abs(got - want) <= ulp * np.abs(want) + tiny)
 
 
+@pytest.mark.parametrize("dt,ulp,tiny", [("f32", 2.0 ** -22, 1e-37), ("bf16", 2.0 ** -8, 1e-37), ("f16", 2.0 ** -11, 2.0 ** -24)])
+@pytest.mark.parametrize("m,h", [(2, 1020), (2, 2056), (3, 2049), (32768 + 3, 8)])
+def test_silu_and_mul_edges_of_the_grid(dt, ulp, tiny, m, h):
+    """Rows one vector short of or beyond a workgroup's, rows of odd length (one element at a time), more rows than the
+    grid has: bounds as above."""
+    xd, xf = x_to_dev(Q.fill_normal(950 + h, 1, 2.5, m * 2 * h).reshape(m, 2 * h), dt)
+    got = QL.silu_and_mul(xd).float().cpu().numpy().astype(np.float64)
+    want = oracle.silu_and_mul_f64(xf.astype(np.float64))
+    assert np.all(np.abs(got - want) <= ulp * np.abs(want) + tiny)
+
+
 @pytest.mark.parametrize("xk", ["bf16", "f16"])
 @pytest.mark.parametrize("n_ff,n_in", [(16, 256), (100, 1024), (1000, 4096), (3000, 512), (20000, 256), (777, 8192), (520, 14336),
                                        (2048, 4096), (2100, 2048), (5000, 4096), (7177, 2048)])
