@@ -146,8 +146,8 @@ PyObject* rmsnorm(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (n != 4 || !p_rmsnorm) return answer(1);
   const at::Tensor *x = gpu_tensor(a[0]), *g = gpu_tensor(a[1]), *r = nullptr;
   if (!x || !g || x->dim() == 0 || g->device() != x->device() || g->scalar_type() != x->scalar_type()) return answer(1);
-  if (a[3] != Py_None &&
-      (!(r = gpu_tensor(a[3])) || r->device() != x->device() || r->sizes() != x->sizes()))
+  if (a[3] != Py_None && (!(r = gpu_tensor(a[3])) || r->device() != x->device() || r->sizes() != x->sizes() ||
+                          r->scalar_type() != x->scalar_type()))
     return answer(1);
   const double eps = PyFloat_AsDouble(a[2]);
   if (eps == -1.0 && PyErr_Occurred()) return nullptr;

@@ -414,7 +414,8 @@ def rmsnorm(x: torch.Tensor, gamma: torch.Tensor, eps: float, residual: Optional
     _native_status(r, "ttq_rmsnorm")
     dev = _require_device(x, gamma, residual)
     n = x.shape[-1]
-    if gamma.numel() != n or gamma.dtype != x.dtype or (residual is not None and residual.shape != x.shape):
+    if gamma.numel() != n or gamma.dtype != x.dtype or (residual is not None and
+                                                        (residual.shape != x.shape or residual.dtype != x.dtype)):
         raise TtqError(_lib.ERR_SHAPE, "rmsnorm: gamma / residual do not match x")
     normed = torch.empty_like(x)
     new_res = torch.empty_like(x) if residual is not None else None

@@ -42,3 +42,14 @@ def test_forward_is_the_c_abi_call_and_errors_keep_their_status():
     assert e.value.status == _lib.ERR_WORKSPACE
     out, res = qlinear.rmsnorm(x, torch.ones(n_in, device="cuda", dtype=x.dtype), 1e-5, x)
     assert torch.equal(res, x + x) and out.shape == x.shape
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("x_dtype,r_dtype", [(torch.float32, torch.bfloat16), (torch.float32, torch.float16),
+                                             (torch.bfloat16, torch.float32), (torch.bfloat16, torch.float16)])
+def test_rmsnorm_refuses_a_residual_of_another_type(x_dtype, r_dtype):
+    """The kernel reads the residual as x's type: one of half the size would be read beyond its end."""
+    x, gamma = torch.ones(3, 256, device="cuda", dtype=x_dtype), torch.ones(256, device="cuda", dtype=x_dtype)
+    with pytest.raises(TtqError) as e:
+        qlinear.rmsnorm(x, gamma, 1e-5, torch.ones(3, 256, device="cuda", dtype=r_dtype))
+    assert e.value.status == _lib.ERR_SHAPE
