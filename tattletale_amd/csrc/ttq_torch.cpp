@@ -66,19 +66,20 @@ const at::Tensor* gpu_tensor(PyObject* o) {
 
 // Binds the tensors' device and its current stream for one call.
 struct OnDevice {
-  explicit OnDevice(const at::Tensor& t)
-      : guard(t.device()), stream(c10::hip::getCurrentHIPStream(t.device().index()).stream()) {}
+  explicit OnDevice(c10::Device d) : guard(d), stream(c10::hip::getCurrentHIPStream(d.index()).stream()) {}
   c10::DeviceGuard guard;
   hipStream_t stream;
 };
 
+// The part of a call that other Python threads need not wait for: the output tensors, whose allocation may go to the
+// device or wait for another stream's block, and the library's call.  Back under the lock on an exception too.
 template <class Call>
 int released(Call call) {
-  int rc;
-  Py_BEGIN_ALLOW_THREADS
-  rc = call();
-  Py_END_ALLOW_THREADS
-  return rc;
+  struct Lock {
+    PyThreadState* state = PyEval_SaveThread();
+    ~Lock() { PyEval_RestoreThread(state); }
+  } lock;
+  return call();
 }
 
 bool as_int64(PyObject* o, int64_t& v) {
@@ -86,11 +87,16 @@ bool as_int64(PyObject* o, int64_t& v) {
   return !(v == -1 && PyErr_Occurred());
 }
 
-at::Tensor output(const at::Tensor& x, int64_t last, at::ScalarType type) {
-  c10::SmallVector<int64_t, 6> sizes(x.sizes().begin(), x.sizes().end());
-  sizes.back() = last;
-  return at::empty(sizes, x.options().dtype(type).requires_grad(false));
-}
+// An output with x's leading dimensions and device: described while x is read, made where the lock is released.
+struct Output {
+  Output(const at::Tensor& x, int64_t last, at::ScalarType type)
+      : sizes(x.sizes().begin(), x.sizes().end()), options(x.options().dtype(type).requires_grad(false)) {
+    sizes.back() = last;
+  }
+  at::Tensor make() const { return at::empty(sizes, options); }
+  c10::SmallVector<int64_t, 6> sizes;
+  at::TensorOptions options;
+};
 
 // (qweight, suh, svh, bias, format, n_in, n_out, bits, codebook, precision, x, out_dtype or None, workspace or None)
 PyObject* linear_forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
@@ -126,18 +132,18 @@ PyObject* linear_forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const int xd = dtype_code(x->scalar_type()), yd = dtype_code(yt);
   if (xd < 0 || yd < 0) return answer(1);
   const int64_t m = x->numel() / layer.n_in;
-  OnDevice on(*x);
-  at::Tensor y = output(*x, layer.n_out, yt);
   const void* xp = x->data_ptr();
-  void* yp = y.data_ptr();
-  int rc;
-  if (ws) {
-    void* wp = ws->data_ptr();
-    const int64_t bytes = (int64_t)ws->nbytes();
-    rc = released([&] { return p_linear_forward_ws(&layer, xp, xd, m, yp, yd, wp, bytes, on.stream); });
-  } else {
-    rc = released([&] { return p_linear_forward(&layer, xp, xd, m, yp, yd, on.stream); });
-  }
+  void* wp = ws ? ws->data_ptr() : nullptr;
+  const int64_t bytes = ws ? (int64_t)ws->nbytes() : 0;
+  const c10::Device device = x->device();
+  const Output out(*x, layer.n_out, yt);
+  at::Tensor y;
+  const int rc = released([&] {
+    const OnDevice on(device);
+    y = out.make();
+    return ws ? p_linear_forward_ws(&layer, xp, xd, m, y.data_ptr(), yd, wp, bytes, on.stream)
+              : p_linear_forward(&layer, xp, xd, m, y.data_ptr(), yd, on.stream);
+  });
   return rc == TTQ_OK ? THPVariable_Wrap(std::move(y)) : answer(rc);
 }
 
@@ -154,13 +160,17 @@ PyObject* rmsnorm(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const int64_t width = x->size(-1);
   const int xd = dtype_code(x->scalar_type());
   if (xd < 0 || width <= 0 || g->numel() != width) return answer(1);
-  OnDevice on(*x);
-  at::Tensor normed = output(*x, width, x->scalar_type()), sum;
-  if (r) sum = output(*x, width, x->scalar_type());
   const void *xp = x->data_ptr(), *rp = r ? r->data_ptr() : nullptr, *gp = g->data_ptr();
-  void *np = normed.data_ptr(), *sp = r ? sum.data_ptr() : nullptr;
   const int64_t m = x->numel() / width;
-  const int rc = released([&] { return p_rmsnorm(xp, rp, gp, (float)eps, xd, sp, np, m, width, on.stream); });
+  const c10::Device device = x->device();
+  const Output out(*x, width, x->scalar_type());
+  at::Tensor normed, sum;
+  const int rc = released([&] {
+    const OnDevice on(device);
+    normed = out.make();
+    if (rp) sum = out.make();
+    return p_rmsnorm(xp, rp, gp, (float)eps, xd, rp ? sum.data_ptr() : nullptr, normed.data_ptr(), m, width, on.stream);
+  });
   if (rc != TTQ_OK) return answer(rc);
   PyObject* pair = PyTuple_New(2);
   if (!pair) return nullptr;
@@ -182,12 +192,16 @@ PyObject* silu_and_mul(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const int xd = dtype_code(x->scalar_type());
   if (xd < 0) return answer(1);
   const int64_t h = x->size(-1) / 2;
-  OnDevice on(*x);
-  at::Tensor y = output(*x, h, x->scalar_type());
   const void* xp = x->data_ptr();
-  void* yp = y.data_ptr();
   const int64_t m = x->numel() / (2 * h);
-  const int rc = released([&] { return p_silu_and_mul(xp, yp, xd, m, h, on.stream); });
+  const c10::Device device = x->device();
+  const Output out(*x, h, x->scalar_type());
+  at::Tensor y;
+  const int rc = released([&] {
+    const OnDevice on(device);
+    y = out.make();
+    return p_silu_and_mul(xp, y.data_ptr(), xd, m, h, on.stream);
+  });
   return rc == TTQ_OK ? THPVariable_Wrap(std::move(y)) : answer(rc);
 }
 
@@ -204,12 +218,15 @@ PyObject* q4_k_silu_mul(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const bool gemm = a[4] == Py_True;
   const int xd = dtype_code(x->scalar_type());
   if (xd < 0 || (gemm && xd != TTQ_BF16)) return answer(1);
-  OnDevice on(*x);
-  at::Tensor y = output(*x, n_ff, x->scalar_type());
   const void *wp = q->data_ptr(), *xp = x->data_ptr();
-  void* yp = y.data_ptr();
   const int64_t m = x->numel() / n_in;
+  const c10::Device device = x->device();
+  const Output out(*x, n_ff, x->scalar_type());
+  at::Tensor y;
   const int rc = released([&] {
+    const OnDevice on(device);
+    y = out.make();
+    void* yp = y.data_ptr();
     return gemm ? p_gemm_q4_k_silu_mul(wp, static_cast<const uint16_t*>(xp), static_cast<uint16_t*>(yp), m, n_ff, n_in,
                                        on.stream)
                 : p_gemv_q4_k_silu_mul(wp, xp, xd, yp, xd, m, n_ff, n_in, on.stream);

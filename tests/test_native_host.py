@@ -1,5 +1,8 @@
 """The native host half of qlinear.py (csrc/ttq_torch.cpp): what it hands back to Python, and that a call through it is
 the call through the C ABI."""
+import threading
+import time
+
 import pytest
 import torch
 
@@ -53,3 +56,61 @@ def test_rmsnorm_refuses_a_residual_of_another_type(x_dtype, r_dtype):
     with pytest.raises(TtqError) as e:
         qlinear.rmsnorm(x, gamma, 1e-5, torch.ones(3, 256, device="cuda", dtype=r_dtype))
     assert e.value.status == _lib.ERR_SHAPE
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("call", ["linear", "rmsnorm", "silu_and_mul", "gate_up_silu"])
+def test_other_threads_run_while_an_output_is_allocated(call):
+    """An allocation that waits for the GPU (at the memory limit, for a block that another stream still uses) stops the
+    calling thread only: here for as long as 300 matrix products take, while a second thread ticks every half
+    millisecond.  Bound: no two ticks are half of the wait apart."""
+    x = torch.randn(32768, 1024, device="cuda").bfloat16()
+    packed = torch.from_numpy(Q.quantize(F.Q4_K, Q.fill_normal(3, 0, 0.02, 1024 * 1024).reshape(1024, 1024))).cuda()
+    layer = QuantLinear.init(packed, F.Q4_K, 1024, 1024)
+    gamma = torch.ones(1024, device="cuda", dtype=x.dtype)
+    run = {"linear": lambda: layer.forward(x), "silu_and_mul": lambda: qlinear.silu_and_mul(x),
+           "rmsnorm": lambda: qlinear.rmsnorm(x, gamma, 1e-5),
+           "gate_up_silu": lambda: qlinear._native().q4_k_silu_mul(packed, x, 512, 1024, True)}[call]
+    a = torch.ones(8192, 8192, device="cuda", dtype=torch.bfloat16)
+    b, side = torch.empty_like(a), torch.cuda.Stream()
+    run()                                                       # kernels loaded, workspaces made
+    torch.cuda.synchronize()
+    with torch.cuda.stream(side):
+        torch.mm(a, a, out=b)
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    reserved, fill = torch.cuda.memory_reserved(), []
+    while torch.cuda.memory_reserved() == reserved:             # until no free block is left that could hold the output
+        fill.append(torch.empty(32 << 20, dtype=torch.uint8, device="cuda"))
+    fill.pop()
+    torch.cuda.empty_cache()
+    held = torch.empty(1 << 30, dtype=torch.uint8, device="cuda")
+    gaps, stop = [], threading.Event()
+
+    def ticks():
+        last = time.perf_counter()
+        while not stop.is_set():
+            time.sleep(0.0005)
+            now = time.perf_counter()
+            gaps.append(now - last)
+            last = now
+
+    thread = threading.Thread(target=ticks)
+    thread.start()
+    total = torch.cuda.get_device_properties(0).total_memory
+    try:
+        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (8 << 20)) / total)
+        with torch.cuda.stream(side):
+            for _ in range(300):
+                torch.mm(a, a, out=b)
+        held.record_stream(side)
+        del held                                                # free again once the side stream is through
+        start = time.perf_counter()
+        run()
+        took = time.perf_counter() - start
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+        stop.set()
+        thread.join()
+    assert took > 0.05, "the allocation did not wait"
+    assert max(gaps) < took / 2
