@@ -239,6 +239,8 @@ func init*(_: type QuantRmsNorm, weight: TorchTensor, eps: float = 1e-6): QuantR
 
 proc forward_with_residual*(self: QuantRmsNorm, hidden_state, residual: TorchTensor): (TorchTensor, TorchTensor) =
   ## (normalized, new_residual), one kernel instead of an add and an rms_norm (the TODO of norm.nim:35).
+  if residual.scalarType() != hidden_state.scalarType():     # the kernel reads both as hidden_state's type
+    raise newException(QuantLinearError, "residual and hidden_state differ in type")
   let normalized = F.empty(hidden_state.sizes(), hidden_state.options())
   let new_residual = F.empty(hidden_state.sizes(), hidden_state.options())
   let rc = rmsnorm(hidden_state.data_ptr(byte), residual.data_ptr(byte), self.weight.data_ptr(byte),
@@ -251,6 +253,8 @@ proc forward_norm_gate_up*(norm: QuantRmsNorm, mlp: QuantGatedMLP,
                            hidden_state, residual: TorchTensor): (TorchTensor, TorchTensor) =
   ## Decode: add + RMSNorm + gate/up projection + silu_and_mul in ONE launch, then the down
   ## projection.  Returns (mlp output, new_residual).
+  if residual.scalarType() != hidden_state.scalarType():     # the kernel reads both as hidden_state's type
+    raise newException(QuantLinearError, "residual and hidden_state differ in type")
   let gu = mlp.gate_up_proj
   let nff = mlp.down_proj.in_features
   var shape = hidden_state.sizes().asNimView().toSeq()
