@@ -1,4 +1,4 @@
-"""Builds ``libttq_hip.so`` (gfx950 only) with hipcc and ``_ttq_torch.so`` with g++.  ``python -m tattletale_amd.build``.
+"""Builds ``libttq_hip.so`` (gfx950 only) with hipcc and the extension ``_ttq_torch`` with g++: ``python -m tattletale_amd.build``.
 
 hipcc cross-compiles without a GPU, so this runs on any host with ROCm installed.  The
 library is written in-tree, next to this file.
@@ -9,12 +9,15 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libttq_hip.so")
-TORCH_EXT = os.path.join(HERE, "_ttq_torch.so")          # host half of the torch mirror (csrc/ttq_torch.cpp)
+# host half of the torch mirror (csrc/ttq_torch.cpp), named for the Python it is built for, and what it was built with
+TORCH_EXT = os.path.join(HERE, "_ttq_torch" + sysconfig.get_config_var("EXT_SUFFIX"))
+TORCH_EXT_COMMAND = os.path.join(CSRC, "build", "ttq_torch.command")
 LADDER_LIB = os.path.join(HERE, "libttq_ladder.so")      # bench.py's measurement ladders, built on demand
 
 SOURCES = [
@@ -130,26 +133,32 @@ def build_library(force: bool = True, verbose: bool = False) -> str:
 
 
 def build_torch_ext(force: bool = True, verbose: bool = False) -> str:
-    """Compile the native host half of qlinear.py (plain C++ against torch's headers; no device code)."""
-    import sysconfig
-
+    """Compile the native host half of qlinear.py (plain C++ against torch's headers; no device code).  Without `force`
+    only where the sources are newer or it was built for another torch, Python or toolchain."""
     import torch
     src = os.path.join(CSRC, "ttq_torch.cpp")
     deps = [src, os.path.join(HERE, "..", "include", "ttq.h")]
-    if not force and os.path.exists(TORCH_EXT) and os.path.getmtime(TORCH_EXT) >= max(os.path.getmtime(d) for d in deps):
-        return TORCH_EXT
     root = os.path.dirname(os.path.abspath(torch.__file__))
     rocm = os.path.dirname(os.path.dirname(os.path.realpath(hipcc())))
     include = [os.path.join(root, "include"), os.path.join(root, "include", "torch", "csrc", "api", "include"),
                os.path.join(rocm, "include"), sysconfig.get_paths()["include"]]
     cmd = [shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden",
-           "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch._C._GLIBCXX_USE_CXX11_ABI]
+           "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch._C._GLIBCXX_USE_CXX11_ABI,
+           '-DTTQ_TORCH_VERSION="%s"' % torch.__version__]
     for d in include:
         cmd += ["-isystem", d]
     cmd += ["-o", TORCH_EXT, src, "-L" + os.path.join(root, "lib"), "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python"]
+    if not force and os.path.exists(TORCH_EXT) and os.path.exists(TORCH_EXT_COMMAND):
+        with open(TORCH_EXT_COMMAND) as f:
+            same = f.read() == "\n".join(cmd)
+        if same and os.path.getmtime(TORCH_EXT) >= max(os.path.getmtime(d) for d in deps):
+            return TORCH_EXT
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError("g++ failed for %s:\n%s\n%s" % (src, r.stdout, r.stderr))
+    os.makedirs(os.path.dirname(TORCH_EXT_COMMAND), exist_ok=True)
+    with open(TORCH_EXT_COMMAND, "w") as f:
+        f.write("\n".join(cmd))
     if verbose:
         print("built", TORCH_EXT)
     return TORCH_EXT

@@ -5,7 +5,8 @@
 //
 // Nothing is kept between calls: every call reads its tensors anew.  Each function returns the output tensor(s), a
 // negative ttq_status the library answered with, or 1 where the tensors do not meet the preconditions below: the
-// caller then takes its own path, which raises the error that names what is wrong.
+// caller then takes its own path, which raises the error that names what is wrong.  (That path makes the same call of
+// the library, and serves all of them where this extension is not built.)
 #include <torch/extension.h>
 #include <torch/csrc/Dtype.h>
 #include <torch/csrc/autograd/python_variable.h>
@@ -249,4 +250,8 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_ttq_torch", nullptr, -1, methods,
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__ttq_torch() { return PyModule_Create(&module); }
+PyMODINIT_FUNC PyInit__ttq_torch() {
+  PyObject* m = PyModule_Create(&module);
+  if (m && PyModule_AddStringConstant(m, "torch_version", TTQ_TORCH_VERSION) < 0) Py_CLEAR(m);
+  return m;
+}

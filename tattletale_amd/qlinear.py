@@ -15,13 +15,14 @@ the current stream and returns a tensor.  torch is used for device memory and st
 from __future__ import annotations
 
 import ctypes as C
+import warnings
 from dataclasses import dataclass
 from typing import Optional
 
 import torch
 
 from . import _lib
-from ._lib import BF16, F16, F32, QLinearStruct, TtqError, TtqLibraryError, check
+from ._lib import BF16, F16, F32, QLinearStruct, TtqError, check
 
 _DTYPE_CODE = {torch.float32: F32, torch.float16: F16, torch.bfloat16: BF16}
 
@@ -33,24 +34,44 @@ def _code(dt: torch.dtype) -> int:
         raise TtqError(_lib.ERR_DTYPE, "dtype %s" % dt) from None
 
 
+class _PythonHost:
+    """In place of the native host half where that is not built: no call is taken, the Python code behind each serves it."""
+
+    @staticmethod
+    def linear_forward(*args) -> int:
+        return 1
+
+    rmsnorm = silu_and_mul = q4_k_silu_mul = linear_forward
+
+
 _native_module = None
 
 
 def _native():
     """The native host half (csrc/ttq_torch.cpp) with the library's entry points bound.  Its functions return the
     output, a negative status, or 1 where the tensors are not what they take: the Python code behind each call then
-    finds and raises the error.  Raises if it is not built."""
+    finds and raises the error.  Not built, or built for another torch: that Python code makes the calls of the
+    library, the same kernels with some 5 us more host time each."""
     global _native_module
     if _native_module is None:
         L = _lib.lib()
+        why = ext = None
         try:
             from . import _ttq_torch as ext
         except ImportError as e:
-            raise TtqLibraryError("tattletale_amd/_ttq_torch.so cannot be loaded (%s): build it with "
-                                  "`python -m tattletale_amd.build`" % e) from e
-        ext.bind(*(C.cast(fn, C.c_void_p).value for fn in (
-            L.ttq_linear_forward, L.ttq_linear_forward_ws, L.ttq_rmsnorm, L.ttq_silu_and_mul, L.ttq_gemv_q4_k_silu_mul,
-            L.ttq_gemm_q4_k_silu_mul)))
+            why = str(e)
+        else:
+            built_for = getattr(ext, "torch_version", None)
+            if built_for != torch.__version__:
+                why = "built for torch %s, this is %s" % (built_for, torch.__version__)
+        if why is not None:
+            warnings.warn("tattletale_amd._ttq_torch is not used (%s): calls cost more host time.  Build it with "
+                          "`python -m tattletale_amd.build`" % why, RuntimeWarning, stacklevel=3)
+            ext = _PythonHost
+        else:
+            ext.bind(*(C.cast(fn, C.c_void_p).value for fn in (
+                L.ttq_linear_forward, L.ttq_linear_forward_ws, L.ttq_rmsnorm, L.ttq_silu_and_mul,
+                L.ttq_gemv_q4_k_silu_mul, L.ttq_gemm_q4_k_silu_mul)))
         _native_module = ext
     return _native_module
 

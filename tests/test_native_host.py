@@ -1,12 +1,22 @@
-"""The native host half of qlinear.py (csrc/ttq_torch.cpp): what it hands back to Python, and that a call through it is
-the call through the C ABI."""
+"""The native host half of qlinear.py (csrc/ttq_torch.cpp): what it hands back to Python, that a call through it is
+the call through the C ABI, and the Python code that serves the calls where it is not built."""
+import sys
 import threading
 import time
 
 import pytest
 import torch
 
-from tattletale_amd import QuantLinear, TtqError, _lib, formats as F, qlinear, quantize as Q
+import tattletale_amd
+from tattletale_amd import QuantGatedMLP, QuantLinear, TtqError, _lib, build, formats as F, qlinear, quantize as Q
+
+
+@pytest.fixture
+def python_host(monkeypatch):
+    """The program of a user who built libttq_hip.so only."""
+    monkeypatch.delattr(tattletale_amd, "_ttq_torch", raising=False)
+    monkeypatch.setitem(sys.modules, "tattletale_amd._ttq_torch", None)         # importing it raises ImportError
+    monkeypatch.setattr(qlinear, "_native_module", None)
 
 
 def test_tensors_it_does_not_take_go_back_to_python():
@@ -18,6 +28,78 @@ def test_tensors_it_does_not_take_go_back_to_python():
     with pytest.raises(TtqError) as e:
         layer.forward(x)
     assert e.value.status == _lib.ERR_UNSUPPORTED
+
+
+def test_calls_are_served_where_the_extension_is_not_built(python_host):
+    layer = QuantLinear(torch.zeros(144, dtype=torch.uint8), F.Q4_K, 256, 1)
+    with pytest.warns(RuntimeWarning, match="_ttq_torch is not used"):
+        with pytest.raises(TtqError) as e:                      # the operator's own answer to a CPU tensor
+            layer.forward(torch.zeros(2, 256))
+    assert e.value.status == _lib.ERR_UNSUPPORTED and qlinear._native() is qlinear._PythonHost
+
+
+def test_an_extension_of_another_torch_is_not_used(monkeypatch):
+    assert qlinear._native().torch_version == torch.__version__                 # it is built here
+    monkeypatch.setattr(qlinear, "_native_module", None)
+    monkeypatch.setattr(torch, "__version__", "0.0.0")
+    with pytest.warns(RuntimeWarning, match="this is 0.0.0"):
+        assert qlinear._native() is qlinear._PythonHost
+
+
+def test_the_extension_is_built_again_for_another_torch(monkeypatch, tmp_path):
+    runs = []
+
+    def gxx(cmd, **kw):
+        runs.append(cmd)
+        (tmp_path / "ext.so").write_bytes(b"")
+        return type("Done", (), {"returncode": 0, "stdout": "", "stderr": ""})
+    monkeypatch.setattr(build.subprocess, "run", gxx)
+    monkeypatch.setattr(build, "TORCH_EXT", str(tmp_path / "ext.so"))
+    monkeypatch.setattr(build, "TORCH_EXT_COMMAND", str(tmp_path / "build" / "ext.command"))
+    build.build_torch_ext(force=False)
+    build.build_torch_ext(force=False)
+    assert len(runs) == 1
+    monkeypatch.setattr(torch, "__version__", "0.0.0")
+    build.build_torch_ext(force=False)
+    assert len(runs) == 2
+
+
+def _every_call():
+    """Results of each entry point with a native half, by name."""
+    def packed(fmt, n_out, n_in, seed):
+        return torch.from_numpy(Q.quantize(fmt, Q.fill_normal(seed, 0, 0.02, n_out * n_in).reshape(n_out, n_in))).cuda()
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    n_in, n_ff, out = 2048, 2048, {}
+    gu = QuantLinear.init(packed(F.Q4_K, 2 * n_ff, n_in, 1), F.Q4_K, n_in, 2 * n_ff)
+    down = QuantLinear.init(packed(F.Q6_K, n_in, n_ff, 2), F.Q6_K, n_ff, n_in, bias=torch.ones(n_in, device="cuda"))
+    mlp = QuantGatedMLP.init(gu, down)
+    for dtype in (torch.float32, torch.float16, torch.bfloat16):
+        gamma = torch.randn(n_in, generator=gen, device="cuda").to(dtype)
+        for m in (1, 3, 20):
+            x = torch.randn(m, n_in, generator=gen, device="cuda").to(dtype)
+            ws = torch.zeros(max(16, down.workspace_bytes(m, dtype)), dtype=torch.uint8, device="cuda")
+            key = (m, dtype)
+            out["linear", key] = down.forward(x, out_dtype=torch.float32)
+            out["workspace", key] = down.forward(x, workspace=ws)
+            out["silu", key] = qlinear.silu_and_mul(x)
+            out["mlp", key] = mlp.forward(x.view(1, m, n_in))
+            out["norm", key], none = qlinear.rmsnorm(x, gamma, 1e-5)
+            out["norm + residual", key], out["residual", key] = qlinear.rmsnorm(x, gamma, 1e-5, x)
+            assert none is None
+    return out
+
+
+@pytest.mark.gpu
+def test_both_host_halves_give_the_same_results(request):
+    assert qlinear._native().torch_version == torch.__version__
+    native = _every_call()
+    request.getfixturevalue("python_host")
+    with pytest.warns(RuntimeWarning):
+        python = _every_call()
+    assert native.keys() == python.keys()
+    for k in native:
+        a, b = native[k], python[k]
+        assert a.shape == b.shape and a.dtype == b.dtype and torch.equal(a, b), k
 
 
 @pytest.mark.gpu
@@ -50,8 +132,10 @@ def test_forward_is_the_c_abi_call_and_errors_keep_their_status():
 @pytest.mark.gpu
 @pytest.mark.parametrize("x_dtype,r_dtype", [(torch.float32, torch.bfloat16), (torch.float32, torch.float16),
                                              (torch.bfloat16, torch.float32), (torch.bfloat16, torch.float16)])
-def test_rmsnorm_refuses_a_residual_of_another_type(x_dtype, r_dtype):
+@pytest.mark.parametrize("host", ["native", "python"])
+def test_rmsnorm_refuses_a_residual_of_another_type(x_dtype, r_dtype, host, monkeypatch):
     """The kernel reads the residual as x's type: one of half the size would be read beyond its end."""
+    monkeypatch.setattr(qlinear, "_native_module", qlinear._PythonHost if host == "python" else qlinear._native())
     x, gamma = torch.ones(3, 256, device="cuda", dtype=x_dtype), torch.ones(256, device="cuda", dtype=x_dtype)
     with pytest.raises(TtqError) as e:
         qlinear.rmsnorm(x, gamma, 1e-5, torch.ones(3, 256, device="cuda", dtype=r_dtype))
