@@ -54,41 +54,61 @@ template <> struct Pack16<f16_tag> {
   }
 };
 
-// V elements of a row per thread: 16 bytes or one element.  A row is gridDim.x workgroups wide and the rows lie along
-// gridDim.y: a flat index would take a 64-bit division per vector, as many instructions as the activation itself.
-// Bound by the launch up to a few MB (2.3 us), then by memory.  Against the flat index (fp32 one element at a time):
-// 2048 x 14336 bf16 36.0 -> 32.5 us (5.4 TB/s), fp16 37.3 -> 35.5; fp32 512 x 14336 18.0 -> 14.0, 2048 rows 72.8 -> 59.8.
+// V elements of a row per thread, 16 bytes or one element: thread i of a launch writes the i-th V elements of the
+// output.  Rows are packed into workgroups whatever their width.  The row that an index lies in (a row of the input has
+// 2h elements) comes from a multiplication with w's reciprocal, exact below 2^31: a 64-bit division takes as many
+// instructions as the activation itself, and workgroups of their own for each row idle on narrow rows.
+// Bound by the launch up to a few MB (2.4 us), then by memory and nearly as much by the exponentials and divisions.
+// us with a 64-bit division per thread / with workgroups to a row / now:
+//   bf16  2^20 x 8 11.0 / 482 / 10.6;  8192 x 2056 22.2 / 30.4 / 19.8;  2048 x 14336 36.1 / 33.3 / 32.5 (5.4 TB/s)
+//   fp16  2^20 x 8 11.8 / 520 / 11.0;  8192 x 2056 22.2 / 34.3 / 20.0;  333 x 13824 8.2 / 7.8 / 7.2
+//   fp32  2^20 x 8 25.3 / 238 / 19.1;  8192 x 2056 47.5 / 37.5 / 36.3;  512 x 14336 23.1 / 17.2 / 17.1
+// Eight activations to a thread make a wavefront long enough that four of them to a workgroup show as a last round
+// (333 x 13824 fp16 8.1 us, bf16 7.8 against 7.2 and 6.9); short wavefronts wait for workgroups to start instead
+// (in workgroups of 64 one element to a thread 4096 x 1023 takes 16.7 us against 8.9, fp32 43 x 18944 3.27 against 3.1).
+template <int V> constexpr uint32_t kSiluGroup = V == 8 ? 64 : 256;
+
 template <typename T, int V>
-__global__ void __launch_bounds__(256)
-silu_and_mul_kernel(const T* __restrict__ in, T* __restrict__ out, int64_t m, int64_t h) {
-  for (int64_t r = blockIdx.y; r < m; r += gridDim.y) {
-    for (int64_t c = ((int64_t)blockIdx.x * 256 + threadIdx.x) * V; c < h; c += (int64_t)gridDim.x * 256 * V) {
-      const int64_t gi = r * 2 * h + c, oi = r * h + c;
-      if constexpr (V == 1) {
-        YElem<T>::store(out, oi, silu_mul(XElem<T>::load(in, gi), XElem<T>::load(in, gi + h)));
-      } else {
-        constexpr int kE = Pack16<T>::kE;
-        static_assert(V == kE, "16 bytes");
-        const auto* ib = reinterpret_cast<const uint8_t*>(in);
-        auto* ob = reinterpret_cast<uint8_t*>(out);
-        constexpr int kBytes = 16 / kE;
-        float g[kE], u[kE], o[kE];
-        Pack16<T>::unpack(*reinterpret_cast<const uint4*>(ib + gi * kBytes), g);
-        Pack16<T>::unpack(*reinterpret_cast<const uint4*>(ib + (gi + h) * kBytes), u);
+__global__ void __launch_bounds__(kSiluGroup<V>)
+silu_and_mul_kernel(const T* __restrict__ in, T* __restrict__ out, int64_t up, uint32_t w, uint32_t total, uint32_t reciprocal,
+                    int shift) {
+  const uint32_t i = blockIdx.x * kSiluGroup<V> + threadIdx.x;
+  if (i >= total) return;
+  const uint32_t r = __umulhi(2 * i, reciprocal) >> shift;      // i / w
+  const int64_t g = i + r * w, u = g + up;
+  if constexpr (V == 1) {
+    YElem<T>::store(out, i, silu_mul(XElem<T>::load(in, g), XElem<T>::load(in, u)));
+  } else {
+    static_assert(V == Pack16<T>::kE, "16 bytes");
+    float gf[V], uf[V], o[V];
+    Pack16<T>::unpack(reinterpret_cast<const uint4*>(in)[g], gf);
+    Pack16<T>::unpack(reinterpret_cast<const uint4*>(in)[u], uf);
 #pragma unroll
-        for (int k = 0; k < V; k++) o[k] = silu_mul(g[k], u[k]);
-        *reinterpret_cast<uint4*>(ob + oi * kBytes) = Pack16<T>::pack(o);
-      }
-    }
+    for (int k = 0; k < V; k++) o[k] = silu_mul(gf[k], uf[k]);
+    reinterpret_cast<uint4*>(out)[i] = Pack16<T>::pack(o);
   }
 }
 
 template <typename T, int V>
 static void silu_and_mul_go(const void* in, void* out, int64_t m, int64_t h, hipStream_t s) {
-  const int64_t per = 256 * V;
-  const int64_t across = (h + per - 1) / per;
-  const dim3 grid((unsigned)(across < 65536 ? across : 65536), (unsigned)(m < 32768 ? m : 32768));
-  hipLaunchKernelGGL((silu_and_mul_kernel<T, V>), grid, dim3(256), 0, s, static_cast<const T*>(in), static_cast<T*>(out), m, h);
+  // A launch takes whole rows of 2^28 threads' work together (4 GiB of output: the launch is nothing beside it), or a
+  // part of one row that is longer.
+  constexpr int64_t kMost = 1 << 28;
+  constexpr uint32_t kGroup = kSiluGroup<V>;
+  const int64_t up = h / V;
+  const int64_t rows = up < kMost ? kMost / up : 1, across = up < kMost ? up : kMost;
+  for (int64_t r = 0; r < m; r += rows) {
+    for (int64_t c = 0; c < up; c += across) {
+      const uint32_t w = (uint32_t)(up - c < across ? up - c : across);
+      const uint32_t total = (uint32_t)(m - r < rows ? m - r : rows) * w;
+      int shift = 0;
+      while ((1u << shift) < w) shift++;
+      const uint32_t reciprocal = (uint32_t)((1ull << (31 + shift)) / w + 1);
+      hipLaunchKernelGGL((silu_and_mul_kernel<T, V>), dim3((total + kGroup - 1) / kGroup), dim3(kGroup), 0, s,
+                         static_cast<const T*>(in) + (r * 2 * up + c) * V, static_cast<T*>(out) + (r * up + c) * V, up, w,
+                         total, reciprocal, shift);
+    }
+  }
 }
 
 template <typename T>

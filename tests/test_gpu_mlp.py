@@ -35,14 +35,46 @@ def test_silu_and_mul_elementwise(dt, ulp, tiny, m, h):
 
 
 @pytest.mark.parametrize("dt,ulp,tiny", [("f32", 2.0 ** -22, 1e-37), ("bf16", 2.0 ** -8, 1e-37), ("f16", 2.0 ** -11, 2.0 ** -24)])
-@pytest.mark.parametrize("m,h", [(2, 1020), (2, 2056), (3, 2049), (32768 + 3, 8)])
+@pytest.mark.parametrize("m,h", [(2, 1020), (2, 1028), (2, 2040), (2, 2056), (3, 2049), (300, 1), (257, 3), (32768 + 3, 8)])
 def test_silu_and_mul_edges_of_the_grid(dt, ulp, tiny, m, h):
-    """Rows one vector short of or beyond a workgroup's, rows of odd length (one element at a time), more rows than the
-    grid has: bounds as above."""
+    """Rows one vector short of or beyond a workgroup's 256 (1020 and 1028 in fp32, 2040 and 2056 in the 16-bit types),
+    rows that are no whole vectors (one element at a time), rows of one to three elements, many narrow rows: bounds as
+    above."""
     xd, xf = x_to_dev(Q.fill_normal(950 + h, 1, 2.5, m * 2 * h).reshape(m, 2 * h), dt)
     got = QL.silu_and_mul(xd).float().cpu().numpy().astype(np.float64)
     want = oracle.silu_and_mul_f64(xf.astype(np.float64))
     assert np.all(np.abs(got - want) <= ulp * np.abs(want) + tiny)
+
+
+@pytest.mark.parametrize("m,h", [(2 ** 25 + 5, 64), (1, 2 ** 31 + 24)])
+def test_silu_and_mul_beyond_one_launch(m, h):
+    """More than the 2^28 vectors that a launch takes: whole rows per launch, and one row in parts.  Both ends with the
+    cut, and a sample in between, in bf16."""
+    x = torch.empty(m, 2 * h, device=DEV, dtype=torch.bfloat16).normal_()
+    y = QL.silu_and_mul(x)
+    y, g, u = (y, x[:, :h], x[:, h:]) if m > 1 else (y[0], x[0, :h], x[0, h:])
+    n = y.shape[0]
+    for part in (slice(0, 1000), slice(n - 1000, n), slice(0, n, 9973)):
+        want = torch.nn.functional.silu(g[part].double()) * u[part].double()
+        assert bool(((y[part].double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-37).all())
+
+
+def test_silu_and_mul_takes_narrow_rows_at_the_speed_of_wide_ones():
+    """The same number of elements as 2^20 rows of 8 and as 1024 rows of 8192 takes about the same time (bf16 10.7 and
+    10.8 us; 482 where each row had workgroups of its own).  Allowed: four times as long."""
+    def us(m, h):
+        x = torch.randn(m, 2 * h, device=DEV).bfloat16()
+        times = []
+        for _ in range(6):
+            a, b = torch.cuda.Event(True), torch.cuda.Event(True)
+            a.record()
+            for _ in range(10):
+                QL.silu_and_mul(x)
+            b.record()
+            b.synchronize()
+            times.append(a.elapsed_time(b) * 100)
+        return min(times)
+    assert us(2 ** 20, 8) <= 4 * us(1024, 8192)
 
 
 @pytest.mark.parametrize("xk", ["bf16", "f16"])
