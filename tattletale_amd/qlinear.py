@@ -187,9 +187,9 @@ class QuantLinear:
         if r.__class__ is not int:
             return r
         _native_status(r, "ttq_linear_forward" if workspace is None else "ttq_linear_forward_ws")
-        if x.shape[-1] != self.in_features:
-            raise TtqError(_lib.ERR_SHAPE, "QuantLinear.forward: last dim %d != in_features %d"
-                           % (x.shape[-1], self.in_features))
+        if x.dim() == 0 or x.shape[-1] != self.in_features:
+            raise TtqError(_lib.ERR_SHAPE, "QuantLinear.forward: x has shape %s, in_features is %d"
+                           % (tuple(x.shape), self.in_features))
         dev = _require_device(self.qweight, x)
         out_dtype = out_dtype or x.dtype
         m = x.numel() // self.in_features
@@ -384,8 +384,8 @@ def silu_and_mul(x: torch.Tensor) -> torch.Tensor:
         return r
     _native_status(r, "ttq_silu_and_mul")
     dev = _require_device(x)
-    if x.shape[-1] % 2:
-        raise TtqError(_lib.ERR_SHAPE, "silu_and_mul: last dim must be even")
+    if x.dim() == 0 or x.shape[-1] == 0 or x.shape[-1] % 2:
+        raise TtqError(_lib.ERR_SHAPE, "silu_and_mul: last dim must be even and not empty")
     h = x.shape[-1] // 2
     out = torch.empty(x.shape[:-1] + (h,), dtype=x.dtype, device=dev)
     with torch.cuda.device(dev):
@@ -434,10 +434,10 @@ def rmsnorm(x: torch.Tensor, gamma: torch.Tensor, eps: float, residual: Optional
         return r
     _native_status(r, "ttq_rmsnorm")
     dev = _require_device(x, gamma, residual)
-    n = x.shape[-1]
-    if gamma.numel() != n or gamma.dtype != x.dtype or (residual is not None and
-                                                        (residual.shape != x.shape or residual.dtype != x.dtype)):
-        raise TtqError(_lib.ERR_SHAPE, "rmsnorm: gamma / residual do not match x")
+    n = x.shape[-1] if x.dim() else 0
+    if n == 0 or gamma.numel() != n or gamma.dtype != x.dtype or (residual is not None and
+                                                                  (residual.shape != x.shape or residual.dtype != x.dtype)):
+        raise TtqError(_lib.ERR_SHAPE, "rmsnorm: x is empty, or gamma / residual do not match it")
     normed = torch.empty_like(x)
     new_res = torch.empty_like(x) if residual is not None else None
     with torch.cuda.device(dev):

@@ -25,9 +25,10 @@ def test_tensors_it_does_not_take_go_back_to_python():
     assert n.silu_and_mul(x) == 1 and n.rmsnorm(x, g, 1e-5, None) == 1          # not on a GPU
     assert n.silu_and_mul(None) == 1 and n.linear_forward() == 1
     layer = QuantLinear(torch.zeros(144, dtype=torch.uint8), F.Q4_K, 256, 1)
-    with pytest.raises(TtqError) as e:
-        layer.forward(x)
-    assert e.value.status == _lib.ERR_UNSUPPORTED
+    for bad, status in ((x, _lib.ERR_UNSUPPORTED), (x[0, 0], _lib.ERR_SHAPE), (x[:, 1:], _lib.ERR_SHAPE)):
+        with pytest.raises(TtqError) as e:
+            layer.forward(bad)
+        assert e.value.status == status
 
 
 def test_calls_are_served_where_the_extension_is_not_built(python_host):
@@ -140,6 +141,19 @@ def test_rmsnorm_refuses_a_residual_of_another_type(x_dtype, r_dtype, host, monk
     with pytest.raises(TtqError) as e:
         qlinear.rmsnorm(x, gamma, 1e-5, torch.ones(3, 256, device="cuda", dtype=r_dtype))
     assert e.value.status == _lib.ERR_SHAPE
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("host", ["native", "python"])
+@pytest.mark.parametrize("shape", [(), (3, 0), (0,)])
+def test_rows_of_no_elements_are_refused_as_a_shape(shape, host, monkeypatch):
+    monkeypatch.setattr(qlinear, "_native_module", qlinear._PythonHost if host == "python" else qlinear._native())
+    x, empty = torch.zeros(shape, device="cuda"), torch.zeros(0, device="cuda")
+    for call in (lambda: qlinear.silu_and_mul(x), lambda: qlinear.rmsnorm(x, empty, 1e-5), lambda: qlinear.rmsnorm(x, empty, 1e-5, x)):
+        with pytest.raises(TtqError) as e:
+            call()
+        assert e.value.status == _lib.ERR_SHAPE
+    assert qlinear.silu_and_mul(torch.zeros(0, 8, device="cuda")).shape == (0, 4)       # no rows: nothing to do
 
 
 @pytest.mark.gpu
