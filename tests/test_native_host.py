@@ -156,6 +156,69 @@ def test_rows_of_no_elements_are_refused_as_a_shape(shape, host, monkeypatch):
     assert qlinear.silu_and_mul(torch.zeros(0, 8, device="cuda")).shape == (0, 4)       # no rows: nothing to do
 
 
+def _calls(seed):
+    """Small inputs of their own, and the four calls on them in sequence."""
+    gen = torch.Generator(device="cuda").manual_seed(seed)
+    n_in, n_ff = 1024, 2048
+    gu, down = (QuantLinear.init(torch.from_numpy(Q.quantize(F.Q4_K, Q.fill_normal(seed, i, 0.03, a * b).reshape(a, b))).cuda(),
+                                 F.Q4_K, b, a) for i, (a, b) in enumerate(((2 * n_ff, n_in), (n_in, n_ff))))
+    mlp, gamma = QuantGatedMLP.init(gu, down), torch.ones(n_in, device="cuda", dtype=torch.bfloat16)
+
+    def run(x):
+        normed, residual = qlinear.rmsnorm(x, gamma, 1e-5, x)
+        return normed, residual, mlp.forward(normed), qlinear.silu_and_mul(gu.forward(normed))
+    return torch.randn(5, n_in, generator=gen, device="cuda").bfloat16(), run
+
+
+@pytest.mark.gpu
+def test_calls_run_on_the_callers_stream():
+    """The input is filled on a side stream, behind work that holds it up: a call on another stream would read it empty."""
+    x, run = _calls(1)
+    want = run(x)
+    a = torch.ones(8192, 8192, device="cuda", dtype=torch.bfloat16)
+    b, late, side = torch.mm(a, a), torch.zeros_like(x), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(side):
+        for _ in range(20):
+            torch.mm(a, a, out=b)
+        late.copy_(x)
+        got = run(late)
+    side.synchronize()
+    assert all(torch.equal(g, w) for g, w in zip(got, want))
+
+
+@pytest.mark.gpu
+def test_threads_on_streams_of_their_own():
+    work = [_calls(10 + i) for i in range(4)]
+    want = [run(x) for x, run in work]
+    torch.cuda.synchronize()
+    wrong = []
+
+    def go(i):
+        x, run = work[i]
+        try:
+            stream = torch.cuda.Stream()
+            with torch.cuda.stream(stream):
+                got = [run(x) for _ in range(25)]
+            stream.synchronize()
+            wrong.extend((i, k) for k, g in enumerate(got) if not all(torch.equal(p, q) for p, q in zip(g, want[i])))
+        except Exception as e:
+            wrong.append((i, e))
+    threads = [threading.Thread(target=go, args=(i,)) for i in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong
+
+
+@pytest.mark.gpu
+def test_an_input_that_requires_grad():
+    x, run = _calls(2)
+    got = run(x.clone().requires_grad_())
+    assert all(torch.equal(g, w) and not g.requires_grad for g, w in zip(got, run(x)))
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("call", ["linear", "rmsnorm", "silu_and_mul", "gate_up_silu"])
 def test_other_threads_run_while_an_output_is_allocated(call):
