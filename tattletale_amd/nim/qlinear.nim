@@ -167,7 +167,8 @@ proc forward*(self: QuantLinear, x: TorchTensor, workspace = none(TorchTensor)):
 # projection, silu_and_mul (workspace/transformers/src/kernels/activations.nim:14-38), down.
 
 const kTtqErrUnsupported = -6
-const kFusedGemmMinRows = 2048   # below it the plain GEMM (packed activations) + silu_and_mul are 4 to 6 % faster
+const kFusedGemmMinRows = 2048   # from it on gate and up reach silu in fp32 (error 2.9e-3 against 3.9e-3), at 6 to 11 % more
+                                 # time on layers of 3584 values and more; below it the separate launches, which are faster
 const kFusedFewRowsMin = 17     # 17..64 rows: the few-row kernel with silu_and_mul in its epilogue
 const kFusedFewRowsMax = 64
 
@@ -213,7 +214,7 @@ proc forward*(self: QuantGatedMLP, x: TorchTensor): TorchTensor =
       raise newException(QuantLinearError, "ttq_gemv_q4_k_silu_mul: " & $strerror(rc))
   elif gu.format == kQ4_K and gu.bias.isNone and x.scalarType() == kBfloat16 and
        (m >= kFusedGemmMinRows or (m >= kFusedFewRowsMin and m <= kFusedFewRowsMax)):
-    # prefill: silu_and_mul in the GEMM epilogue (breaks even at 512 rows, 15 % faster at 2048);
+    # prefill: silu_and_mul in the GEMM epilogue;
     # 17..64 rows: the same entry point runs the few-row kernel
     var shape = x.sizes().asNimView().toSeq()
     shape[^1] = nff

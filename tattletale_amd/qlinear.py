@@ -488,15 +488,20 @@ class QuantGatedMLP:
             raise TtqError(_lib.ERR_SHAPE, "QuantGatedMLP.init: hidden sizes differ")
         return cls(gate_up_proj, down_proj)
 
-    # The fused GEMM saves the (rows, 2 * intermediate) tensor and its round trip, but pays for the activation
-    # with quarter-rate exp2 / reciprocal in its epilogue and reads its activations through LDS, where the
-    # plain GEMM reads a packed copy: at 28672 x 4096 the three launches are 4 to 6 % faster from 512 to
-    # 1792 rows (128 against 136 us at 512, 340 against 356 at 1536), level at 2048 (452 / 454 us), and the fused
-    # GEMM is 4 % faster at 4096 (879 against 912 us), with 235 MB less to allocate.
+    # From here on silu_and_mul runs in the GEMM's epilogue, for what the result is rather than for speed: the activation
+    # gets its sums in fp32 where the separate launches round gate and up to bf16 first (distance from 64-bit
+    # arithmetic 2.9e-3 against 3.9e-3), and the (rows, 2 * intermediate) tensor is never made (235 MB at 4096 rows of
+    # 28672).  On wide layers that costs time, because the epilogue's exponentials and reciprocals are quarter rate and
+    # this GEMM reads its activations through LDS where the plain one reads a packed copy.  Fused / separate, us:
+    # 28672 x 4096 442 / 414 at 2048 rows, 885 / 823 at 4096, 1818 / 1670 at 8192; 27648 x 5120 and 37888 x 3584 6 to 11 %
+    # in the same direction; 6144 x 1024 43.8 / 47.6 and 77.8 / 77.9.  Fewer rows take the separate launches (28672 x 4096
+    # 125 / 118 at 512 rows, 416 / 371 at 1792): prompts of those lengths keep the faster form.
     FUSED_GEMM_MIN_ROWS = 2048
-    # 17..64 rows: the same entry point runs the few-row kernel with the activation in its epilogue (one
-    # launch and one (rows, 2 * intermediate) round trip less); up to 16 rows the few-row GEMV passes
-    # plus silu_and_mul are faster.
+    # 17 to 64 rows: the same entry point runs the few-row kernel with the activation in its epilogue, one launch and one
+    # (rows, 2 * intermediate) round trip less (28672 x 4096 at 32 rows 33.9 / 35.1 us, 6144 x 1024 5.8 / 8.1), and the same
+    # fp32 sums.  Below nine rows the decode kernels for several rows plus silu_and_mul are faster on wide layers
+    # (28672 x 4096 at 8 rows 26.8 / 23.0, 27648 x 5120 43.5 / 28.7); from 9 to 16 rows they are not (26.7 / 29.7 and
+    # 40.4 / 42.0 at 16) and are taken all the same.
     FUSED_FEW_ROWS = (17, 64)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
