@@ -169,8 +169,8 @@ PyObject* rmsnorm(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const int rc = released([&] {
     const OnDevice on(device);
     normed = out.make();
-    if (rp) sum = out.make();
-    return p_rmsnorm(xp, rp, gp, (float)eps, xd, rp ? sum.data_ptr() : nullptr, normed.data_ptr(), m, width, on.stream);
+    if (r) sum = out.make();                     // also for no rows, where rp is null
+    return p_rmsnorm(xp, rp, gp, (float)eps, xd, r ? sum.data_ptr() : nullptr, normed.data_ptr(), m, width, on.stream);
   });
   if (rc != TTQ_OK) return answer(rc);
   PyObject* pair = PyTuple_New(2);

@@ -145,6 +145,18 @@ def test_rmsnorm_refuses_a_residual_of_another_type(x_dtype, r_dtype, host, monk
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("host", ["native", "python"])
+def test_no_rows_give_outputs_of_no_rows(host, monkeypatch):
+    monkeypatch.setattr(qlinear, "_native_module", qlinear._PythonHost if host == "python" else qlinear._native())
+    x = torch.zeros(2, 0, 256, device="cuda", dtype=torch.bfloat16)
+    gamma = torch.ones(256, device="cuda", dtype=x.dtype)
+    layer = QuantLinear.init(torch.zeros(16 * 144, dtype=torch.uint8, device="cuda"), F.Q4_K, 256, 16)
+    normed, residual = qlinear.rmsnorm(x, gamma, 1e-5, x)
+    assert normed.shape == residual.shape == x.shape and qlinear.rmsnorm(x, gamma, 1e-5)[1] is None
+    assert layer.forward(x).shape == (2, 0, 16) and qlinear.silu_and_mul(x).shape == (2, 0, 128)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("host", ["native", "python"])
 @pytest.mark.parametrize("shape", [(), (3, 0), (0,)])
 def test_rows_of_no_elements_are_refused_as_a_shape(shape, host, monkeypatch):
     monkeypatch.setattr(qlinear, "_native_module", qlinear._PythonHost if host == "python" else qlinear._native())
@@ -153,7 +165,6 @@ def test_rows_of_no_elements_are_refused_as_a_shape(shape, host, monkeypatch):
         with pytest.raises(TtqError) as e:
             call()
         assert e.value.status == _lib.ERR_SHAPE
-    assert qlinear.silu_and_mul(torch.zeros(0, 8, device="cuda")).shape == (0, 4)       # no rows: nothing to do
 
 
 def _calls(seed):
