@@ -286,3 +286,21 @@ def test_other_threads_run_while_an_output_is_allocated(call):
         thread.join()
     assert took > 0.05, "the allocation did not wait"
     assert max(gaps) < took / 2
+
+
+@pytest.mark.gpu
+def test_an_output_that_does_not_fit_raises_and_leaves_the_program_usable():
+    """The exception leaves the stretch without the interpreter lock with the lock taken again."""
+    x = torch.randn(32768, 1024, device="cuda").bfloat16()
+    want = qlinear.silu_and_mul(x).clone()
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(0).total_memory
+    try:
+        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (1 << 30)) / total)
+        layer = QuantLinear.init(torch.zeros(65536 * 4 * 144, dtype=torch.uint8, device="cuda"), F.Q4_K, 1024, 65536)
+        with pytest.raises(torch.OutOfMemoryError):
+            layer.forward(x)                                    # 4 GiB
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    assert torch.equal(qlinear.silu_and_mul(x), want)
