@@ -32,6 +32,9 @@ typedef __attribute__((ext_vector_type(2))) _Float16 f16x2_t;
 struct OpsBF16 {
   static constexpr uint32_t kMagic = 0x43004300u;   // (128.0, 128.0)
   static constexpr float kOffset = 128.f;
+  static constexpr uint32_t kMagic6 = kMagic;       // six-bit quants: the same
+  static constexpr float kOffset6 = kOffset;
+  static constexpr int kShift6 = 0;
   static constexpr uint32_t kOnes = 0x3F803F80u;    // (1.0, 1.0)
   static __device__ __forceinline__ float dot2(uint32_t a, uint32_t b, float c) {
     bf16x2_t x, y;
@@ -43,6 +46,9 @@ struct OpsBF16 {
 struct OpsF16 {
   static constexpr uint32_t kMagic = 0x64006400u;   // (1024.0, 1024.0)
   static constexpr float kOffset = 1024.f;
+  static constexpr uint32_t kMagic6 = 0x5C005C00u;  // six-bit quants two bits up: 256 + q, a quarter of the offset in the sums
+  static constexpr float kOffset6 = 256.f;
+  static constexpr int kShift6 = 2;
   static constexpr uint32_t kOnes = 0x3C003C00u;
   static __device__ __forceinline__ float dot2(uint32_t a, uint32_t b, float c) {
     f16x2_t x, y;
@@ -119,6 +125,8 @@ __device__ __forceinline__ void make_pairs(const uint4& v, uint2& p0, uint2& p1)
 // high nibbles -> sub-block 2c+1.  Activation pairs of a unit, register 4i+kind for qs dword
 // i: kind 0 = (x[4i], x[4i+2]), 1 = (x[4i+1], x[4i+3]), 2/3 = the same 32 positions further.
 struct DotQ4K {
+  template <class Ops> static constexpr uint32_t kMagic = Ops::kMagic;
+  template <class Ops> static constexpr float kOffset = Ops::kOffset;
   static constexpr int kSums = 2;
   static __device__ __forceinline__ int64_t row_bytes(int n_in) { return (int64_t)(n_in >> 8) * 144; }
   static constexpr uint32_t kGroupBytes = 16 * 144;   // 64 units
@@ -222,8 +230,8 @@ struct DotQ4K {
 // (j = 1, 3) and 16 bytes of qh (2 bits per j).  Four bytes of each give one dword of four
 // 6-bit values per j; (Q & 0x00FF00FF) | magic and ((Q >> 8) & 0x00FF00FF) | magic turn it into
 // two float pairs.  Register 8j + 2d + parity holds (x[16j+4d+parity], x[16j+4d+parity+2]).
-// The weights are q - 32 and the magic adds 128 (bf16) or 1024 (fp16): the offset removed per j
-// is (kOffset + 32) * sum(x).
+// The weights are q - 32 and the magic adds 128 (bf16) or, with the quants two bits up, 256 (fp16; 1024 + q in the low
+// bits is 2.5e-6 from the float64 product, 256 + q 7e-7): the offset removed per j is (kOffset6 + 32) * sum(x).
 struct DotQ6K {
   static constexpr int kSums = 4;
   static __device__ __forceinline__ int64_t row_bytes(int n_in) { return (int64_t)(n_in >> 8) * 210; }
@@ -280,17 +288,19 @@ struct DotQ6K {
     const uint32_t A[4] = {r.a.x, r.a.y, r.a.z, r.a.w};
     const uint32_t B[4] = {r.b.x, r.b.y, r.b.z, r.b.w};
     const uint32_t H[4] = {r.h.x, r.h.y, r.h.z, r.h.w};
-    constexpr uint32_t N4 = 0x0F0F0F0Fu, H2 = 0x30303030u, M = 0x00FF00FFu;
+    constexpr int S = Ops::kShift6;            // the quants' place in their bytes
+    constexpr uint32_t N4 = 0x0F0F0F0Fu << S, H2 = 0x30303030u << S, M = 0x00FF00FFu;
+    auto up = [](uint32_t v, int n) { return n >= 0 ? v << n : v >> -n; };
     float acc[4][2];
 #pragma unroll
     for (int j = 0; j < 4; j++) acc[j][0] = acc[j][1] = 0.f;
 #pragma unroll
     for (int d = 0; d < 4; d++) {
       uint32_t Q[4];
-      Q[0] = (A[d] & N4) | ((H[d] << 4) & H2);
-      Q[1] = (B[d] & N4) | ((H[d] << 2) & H2);
-      Q[2] = ((A[d] >> 4) & N4) | (H[d] & H2);
-      Q[3] = ((B[d] >> 4) & N4) | ((H[d] >> 2) & H2);
+      Q[0] = (up(A[d], S) & N4) | (up(H[d], S + 4) & H2);
+      Q[1] = (up(B[d], S) & N4) | (up(H[d], S + 2) & H2);
+      Q[2] = (up(A[d], S - 4) & N4) | (up(H[d], S) & H2);
+      Q[3] = (up(B[d], S - 4) & N4) | (up(H[d], S - 2) & H2);
 #pragma unroll
       for (int j = 0; j < 4; j++) {
         acc[j][0] = Ops::dot2(and_or(Q[j], M, magic), xr[8 * j + 2 * d], acc[j][0]);
@@ -309,11 +319,9 @@ struct DotQ6K {
     const float t3 = (dd * c3) * ((acc[3][0] + acc[3][1]) - off[3]);
     return (t0 + t1) + (t2 + t3);
   }
-  static constexpr float kExtraOffset = 32.f;
+  template <class Ops> static constexpr uint32_t kMagic = Ops::kMagic6;
+  template <class Ops> static constexpr float kOffset = Ops::kOffset6 + 32.f;
 };
-
-template <class F> struct ExtraOffset { static constexpr float value = 0.f; };
-template <> struct ExtraOffset<DotQ6K> { static constexpr float value = 32.f; };
 
 __device__ __forceinline__ void load_x_regs(const uint32_t* xs, int it, int lane, uint32_t (&xr)[32]) {
   const uint4* xs4 = reinterpret_cast<const uint4*>(xs);
@@ -405,8 +413,8 @@ gemv_dot2_kernel(const uint8_t* __restrict__ w, const uint16_t* __restrict__ x, 
   TTQ_TRACE_POINT(gw, 1);
   // wavefronts without rows fall through: their loads are clamped and their stores masked
 
-  const uint32_t magic = opaque_vgpr(Ops::kMagic);
-  constexpr float kOff = Ops::kOffset + ExtraOffset<F>::value;
+  const uint32_t magic = opaque_vgpr(F::template kMagic<Ops>);
+  constexpr float kOff = F::template kOffset<Ops>;
   auto store_rows = [&](auto& acc, int base) {
     constexpr int kN = (int)(sizeof(acc) / sizeof(float));
 #pragma unroll
@@ -592,8 +600,8 @@ gemv_dot2_multi_kernel(const uint8_t* __restrict__ w, const uint16_t* __restrict
   }
   __syncthreads();
 
-  const uint32_t magic = opaque_vgpr(Ops::kMagic);
-  constexpr float kOff = Ops::kOffset + ExtraOffset<F>::value;
+  const uint32_t magic = opaque_vgpr(F::template kMagic<Ops>);
+  constexpr float kOff = F::template kOffset<Ops>;
   auto store = [&](int row, int t, float v) {
     v = wave_sum_to_lane63(v);
     if (lane == 63 && row < row_end && t0 + t < m)
