@@ -560,6 +560,7 @@ const char* ttq_route_name(int route) {
     case TTQ_ROUTE_GEMV_DOT2_MULTI: return "gemv_dot2_multi";
     case TTQ_ROUTE_GEMV_GENERIC: return "gemv_generic";
     case TTQ_ROUTE_GEMV_LONG: return "gemv_long";
+    case TTQ_ROUTE_GEMV_TILE: return "gemv_tile";
     case TTQ_ROUTE_GEMM_SKINNY_F32_SCALED_F16: return "gemm_skinny_f32_scaled_f16";
     case TTQ_ROUTE_GEMM_PC: return "gemm_pc";
     case TTQ_ROUTE_GEMM_PC_SPLIT_K: return "gemm_pc_split_k";

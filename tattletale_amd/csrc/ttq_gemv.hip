@@ -468,6 +468,8 @@ hipError_t launch_gemv(int format, const void* w, const void* x, int x_dtype, vo
       default: return hipErrorInvalidValue;
     }
   }
+  if (gemv_tile_preferred(format, x_dtype, m, n_out, n_in))
+    TTQ_ROUTE(kRouteGemvTile, launch_gemv_tile(format, w, x, x_dtype, y, y_dtype, bias, bias_dtype, m, n_out, n_in, s));
   // a few rows at once: four per pass for up to four rows and for rows too long for the 8- and
   // 16-token tables, else eight or sixteen per pass
   if (gemv_q4k_stream4_supported(format, x_dtype, m, n_out, n_in))
@@ -527,6 +529,7 @@ float gemv_estimate_us(int format, int x_dtype, int64_t m, int64_t n_out, int64_
   const float mb = (float)(n_out * (n_in / per) * blk) * 1e-6f;
   // rows of any length: a pass over the weights per activation row (72 MB in 24.6 us, 155 MB in 51 us, 463 MB in 122 us)
   if (gemv_row_is_long(format, x_dtype, n_in)) return (float)m * (mb / 3.5f + 3.f);
+  if (gemv_tile_preferred(format, x_dtype, m, n_out, n_in)) return gemv_tile_estimate_us(m, n_out, n_in);
   const bool b4 = gemv_q4k_batch4_supported(format, x_dtype, m, n_out, n_in);
   if (b4 && m <= 4) return mb / 2.75f + 2.f;
   if (gemv_q4k_batch_supported(format, x_dtype, m, n_out, n_in)) {

@@ -32,6 +32,7 @@ enum : int {
   kRouteGemvDot2Multi = 13,
   kRouteGemvGeneric = 14,
   kRouteGemvLong = 15,
+  kRouteGemvTile = 16,
   kRouteGemmSkinnyF32ScaledF16 = 19,
   kRouteGemmPc = 20,
   kRouteGemmPcSplitK = 21,
@@ -157,6 +158,13 @@ bool gemv_q6k_stream4_supported(int format, int x_dtype, int64_t m, int64_t n_ou
 hipError_t launch_gemv_q6k_stream4(const void* w, const void* x, int x_dtype, void* y, int y_dtype,
                                    const void* bias, int bias_dtype, int64_t m, int64_t n_out, int64_t n_in,
                                    hipStream_t s);
+
+// Q6_K as integers on the 16-bit matrix cores, one to eight activation rows (one of fp32), any shape (ttq_gemv_tile.hip).
+bool gemv_tile_supported(int format, int x_dtype, int64_t m, int64_t n_out, int64_t n_in);
+bool gemv_tile_preferred(int format, int x_dtype, int64_t m, int64_t n_out, int64_t n_in);
+float gemv_tile_estimate_us(int64_t m, int64_t n_out, int64_t n_in);
+hipError_t launch_gemv_tile(int format, const void* w, const void* x, int x_dtype, void* y, int y_dtype,
+                            const void* bias, int bias_dtype, int64_t m, int64_t n_out, int64_t n_in, hipStream_t s);
 
 // int8 matrix-core path for Q8_0, any activation dtype (ttq_gemv_q8_mfma.hip).
 // Q8_0 through the matrix cores, rows read as aligned 64-byte windows (ttq_gemv_q8_win.hip).

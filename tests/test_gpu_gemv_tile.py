@@ -1,0 +1,88 @@
+"""The Q6_K decode kernel for one to eight rows of any length (route ``gemv_tile``): edges of its tiles (4, 8 and 16 weight
+rows by 4, 2 and 1 blocks), of the workgroups' shares, of the rows' ends and of the matrix's end.
+
+The float64 product over the library's own dense copy of the weights (bit-exact against the oracle, test_gpu_dequant.py) is
+the reference.  Bound: products are exact, a sum over a sub-block of 16 in fp32 carries the offset 256 + 63 of the quants beside
+weights of up to 32 in magnitude, so its rounding is 2^-24 * 320 / 32 per addition at worst, 6e-7 of the largest term; over
+random signs and many sub-blocks the relative 2-norm stays below 2e-6 (3e-7 measured)."""
+import numpy as np
+import pytest
+import torch
+
+from tattletale_amd import QuantLinear, formats as F
+from tattletale_amd import qlinear as QL
+
+from util import DEV, packed_to_dev, random_blocks
+
+pytestmark = pytest.mark.gpu
+DT = {"f32": torch.float32, "f16": torch.float16, "bf16": torch.bfloat16}
+
+
+def layer(n_out, n_in, bias=None):
+    w = packed_to_dev(random_blocks(F.Q6_K, n_out * (n_in // 256), seed=n_out + n_in))
+    return QuantLinear.init(w, F.Q6_K, n_in, n_out, bias=bias, precision=F.PRECISION_F32_SCALES)
+
+
+def dense(lay):
+    return QL.dequantize(F.Q6_K, lay.qweight, lay.out_features, lay.in_features).double()
+
+
+# rows of 1, 2, 3, 5, 9 and 27 blocks (an odd and an even number of blocks in all: where the matrix ends inside a dword),
+# row counts that are and are not whole tiles
+SHAPES = [(33337, 256), (33344, 256), (66700, 512), (11115, 768), (45003, 768), (6671, 1280), (30006, 1280), (3709, 2304), (1237, 6912),
+          (2451, 6912), (48001, 1024)]
+
+
+@pytest.mark.parametrize("n_out,n_in", SHAPES)
+@pytest.mark.parametrize("xk,m", [("f32", 1), ("bf16", 1), ("f16", 1), ("bf16", 2), ("f16", 2), ("f16", 3), ("bf16", 4), ("f16", 5),
+                                  ("bf16", 8)])
+def test_tile_edges(n_out, n_in, xk, m):
+    gen = torch.Generator(DEV).manual_seed(n_out)
+    bias = torch.randn(n_out, device=DEV, generator=gen).to(DT[xk])
+    lay = layer(n_out, n_in, bias)
+    if lay.route(m, DT[xk], torch.float32) != "gemv_tile":
+        pytest.skip("another kernel is the faster one for this size")
+    x = torch.randn(m, n_in, device=DEV, generator=gen).to(DT[xk])
+    wd = dense(lay)
+    ref = x.double() @ wd.T + bias.double()
+    y = lay.forward(x, out_dtype=torch.float32)
+    assert ((y.double() - ref).norm(dim=-1) / ref.norm(dim=-1)).max().item() <= 2e-6
+    if xk != "f32":      # 16-bit outputs are the same sums, rounded once
+        assert torch.equal(lay.forward(x), y.to(DT[xk]))
+    # unit vectors: the dequantized columns, bit for bit (without the bias)
+    lay = QuantLinear.init(lay.qweight, F.Q6_K, n_in, n_out, precision=F.PRECISION_F32_SCALES)
+    cols = [0, n_in - 1, 15, 16, 127, 128, n_in - 256, n_in - 17][:m] if m > 1 else [n_in - 1]
+    e = torch.zeros(m, n_in, device=DEV, dtype=DT[xk])
+    e[torch.arange(m), torch.tensor(cols)] = 1.0
+    assert torch.equal(lay.forward(e, out_dtype=torch.float32), wd[:, cols].T.float() + 0.0)
+
+
+def test_every_size_of_route_is_reached():
+    """The cases above are not all skipped: each of the kernel's five forms runs at least on these."""
+    for n_out, n_in, m, dt in [(33337, 256, 1, "f32"), (1237, 6912, 1, "bf16"), (2451, 6912, 1, "bf16"), (66700, 512, 2, "f16"),
+                               (33337, 256, 4, "bf16"), (6671, 1280, 8, "bf16")]:
+        if (n_out, n_in, m) != (1237, 6912, 1):
+            assert layer(n_out, n_in).route(m, DT[dt], torch.float32) == "gemv_tile", (n_out, n_in, m, dt)
+
+
+@pytest.mark.parametrize("xk,m", [("f32", 1), ("bf16", 1), ("f16", 2), ("bf16", 4), ("f16", 8)])
+def test_non_finite_rows_and_large_values(xk, m):
+    n_out, n_in = 30006, 1280
+    lay = layer(n_out, n_in)
+    assert lay.route(m, DT[xk], torch.float32) == "gemv_tile"
+    x = torch.randn(m, n_in, device=DEV, generator=torch.Generator(DEV).manual_seed(3)).to(DT[xk])
+    want = lay.forward(x, out_dtype=torch.float32)
+    for bad in (float("inf"), float("nan")):
+        z = x.clone()
+        z[m - 1, 700] = bad
+        y = lay.forward(z, out_dtype=torch.float32)
+        assert not torch.isfinite(y[m - 1]).any()
+        assert torch.equal(y[: m - 1], want[: m - 1])
+    if xk == "f32":      # one value near the top of the range: its products with quants of up to 63 stay finite
+        z = torch.zeros_like(x)
+        z[0, 700] = 5e36
+        ref = z.double() @ dense(lay).T
+        fits = ref.abs() < 3e38
+        y = lay.forward(z)
+        assert fits.float().mean() > 0.5 and torch.isfinite(y[fits]).all()
+        assert ((y.double() - ref)[fits].norm() / ref[fits].norm()).item() <= 1e-6
