@@ -41,6 +41,7 @@ SOURCES = [
     "ttq_gemm_pc.hip",
     "ttq_gemm_pcd.hip",
     "ttq_gemm_skinny.hip",
+    "ttq_gemm_rows.hip",
     "ttq_exl3.hip",
     "ttq_exl3_mfma.hip",
     "ttq_exl3_prefill.hip",

@@ -446,9 +446,19 @@ int ttq_linear_forward(const ttq_qlinear* layer, const void* x, int x_dtype, int
   // TTQ_FORWARD_ROUTE (developer builds, A/B measurements): 1 = always the decode kernels, 2 = the GEMM whenever it exists
   static const int knob = ttq::dev_knob("TTQ_FORWARD_ROUTE", 0);
   const int route = layer->precision == TTQ_PRECISION_F32_SCALES ? 1 : knob;
+  // Which calls may have their weights rounded is decided by the kernels that round them in registers or tiles and the decode
+  // kernels of fixed-point or packed-dot arithmetic; faster kernels of either kind since then (the streamed few-row form, the
+  // integer kernels) compete inside of it, and a call that decodes exactly is not moved to rounded weights by them.
+  const auto few_us = [&](int64_t rows) { return ttq::gemm_skinny_registers_estimate_us(layer->format, rows, n_out, n_in); };
   if (gemm_ok && m >= 5 && route != 1) {
+    float us_rounding = m <= 64 ? few_us(m) : 1e30f;
+    if (us_rounding < 1e29f || layer->format == TTQ_Q4_K || ttq::gemm_pc_supported(layer->format, m, n_out, n_in, 112)) {
+      const float us = ttq::gemm_pc_estimate_us(layer->format, m, n_out, n_in);
+      us_rounding = us < us_rounding ? us : us_rounding;
+    }
     if (route == 2 ||
-        ttq::gemm_estimate_us(layer->format, m, n_out, n_in) < ttq::gemv_estimate_us(layer->format, x_dtype, m, n_out, n_in))
+        (us_rounding < ttq::gemv_estimate_us(layer->format, x_dtype, m, n_out, n_in, false) &&
+         ttq::gemm_estimate_us(layer->format, m, n_out, n_in) < ttq::gemv_estimate_us(layer->format, x_dtype, m, n_out, n_in)))
       return hip_status(ttq::launch_gemm(layer->format, layer->qweight, static_cast<const uint16_t*>(x), y, y_dtype,
                                          layer->bias, layer->bias_dtype, m, n_out, n_in, s));
   }
@@ -458,21 +468,24 @@ int ttq_linear_forward(const ttq_qlinear* layer, const void* x, int x_dtype, int
   // by the few-row kernel (64 rows per launch) or, from where it is cheaper, by the prefill GEMM over a packed fp16
   // copy of the activations -- unless passes of the decode kernels are cheaper still.
   if (x_dtype == TTQ_F16 && block_fmt && m >= 5 && route != 1) {
-    float us_few = 1e30f, us_gemm = 1e30f;
+    float us_few = 1e30f, us_gemm = 1e30f, us_rounding = 1e30f;
     if (ttq::gemm_skinny_supported(layer->format, m < 64 ? m : 64, n_out, n_in)) {
       const int64_t full = m / 64, rest = m % 64;
       us_few = (float)full * ttq::gemm_skinny_estimate_us(layer->format, 64, n_out, n_in);
       if (rest) us_few += ttq::gemm_skinny_estimate_us(layer->format, rest, n_out, n_in);
+      us_rounding = (full ? (float)full * few_us(64) : 0.f) + (rest ? few_us(rest) : 0.f);
     }
     if (m > 64 && ttq::gemm_pc_supported(layer->format, m < 8192 ? m : 8192, n_out, n_in, 112))
       us_gemm = ttq::gemm_pc_estimate_us(layer->format, m, n_out, n_in) + 2.5f + (float)(m * n_in * 4) / 3.0e6f;
+    us_rounding = us_gemm < us_rounding ? us_gemm : us_rounding;
+    const bool rounds = route == 2 || us_rounding < ttq::gemv_estimate_us(layer->format, x_dtype, m, n_out, n_in, false);
     const float us_gemv = ttq::gemv_estimate_us(layer->format, x_dtype, m, n_out, n_in);
     // (several launches of the few-row kernel against one short round of the tiled kernel: the margin of the bf16
     // chooser, whose estimate for the tiled kernel is fitted to full rounds and about a third too high for a short one)
-    if (us_gemm < (m > 64 ? us_few / 0.65f : us_few) && (route == 2 || us_gemm < us_gemv))
+    if (rounds && us_gemm < (m > 64 ? us_few / 0.65f : us_few) && (route == 2 || us_gemm < us_gemv))
       return hip_status(ttq::launch_gemm_pc_x(layer->format, layer->qweight, x, x_dtype, y, y_dtype, layer->bias,
                                               layer->bias_dtype, m, n_out, n_in, s, true));
-    if (us_few < 1e29f && (route == 2 || us_few < us_gemv)) {
+    if (rounds && us_few < 1e29f && (route == 2 || us_few < us_gemv)) {
       if (ttq::route_probe(ttq::kRouteGemmSkinnyChunked)) return TTQ_OK;
       return hip_status(ttq::launch_gemm_skinny_chunked(layer->format, layer->qweight, static_cast<const uint16_t*>(x),
                                                         x_dtype, y, y_dtype, layer->bias, layer->bias_dtype, m, n_out,
@@ -498,23 +511,30 @@ int ttq_linear_forward(const ttq_qlinear* layer, const void* x, int x_dtype, int
   // that also beats passes of the decode kernels where those have no kernel of several rows for fp32 activations
   // (Q6_K 14336 x 4096 at four rows: 20 us against 49; the 128256 x 4096 head 149 against 408).
   if (x_dtype == TTQ_F32 && block_fmt && m >= 2 && route != 1) {
-    float us_few = 1e30f, us_gemm = 1e30f;
+    float us_few = 1e30f, us_gemm = 1e30f, us_rounding = 1e30f;
     // (up to 8192 rows: the scaled copy of all rows sits in the workspace at once)
     if (m <= 8192 && ttq::gemm_skinny_supported(layer->format, m < 64 ? m : 64, n_out, n_in)) {
       // (the scaling pass: a workgroup per row walks it twice -- 3 us on rows of 4096 values, 4.3 us on 14336)
       const int64_t full = m / 64, rest = m % 64;
       us_few = (float)full * ttq::gemm_skinny_estimate_us(layer->format, 64, n_out, n_in) + 2.5f + (float)n_in * 0.13e-3f;
       if (rest) us_few += ttq::gemm_skinny_estimate_us(layer->format, rest, n_out, n_in);
+      us_rounding = (full ? (float)full * few_us(64) : 0.f) + (rest ? few_us(rest) : 0.f) + 2.5f + (float)n_in * 0.13e-3f;
     }
     if (m >= 5 && ttq::gemm_pc_supported(layer->format, m < 8192 ? m : 8192, n_out, n_in, 112))
       us_gemm = ttq::gemm_pc_estimate_us(layer->format, m, n_out, n_in) + 5.f + (float)(m * n_in * 10) / 3.0e6f;
-    const float us_gemv = ttq::gemv_estimate_us(layer->format, x_dtype, m, n_out, n_in);
-    if ((m > 64 ? us_few / 0.65f : us_few) < us_gemm && (route == 2 || us_few < us_gemv)) {
+    us_rounding = us_gemm < us_rounding ? us_gemm : us_rounding;
+    const bool rounds = route == 2 || us_rounding < ttq::gemv_estimate_us(layer->format, x_dtype, m, n_out, n_in, false);
+    // (the integer kernel takes two rows of Q6_K to a pass: us of it / of the few-row kernel 14336 x 4096 19.3 / 22.5, 28672 x 4096
+    // 27.0 / 30.5, 43008 x 4096 38.3 / 38.9, 128256 x 4096 88 / 91 -- and of four rows 34 / 22, 49 / 30, 68 / 38, 160 / 91.  The small
+    // matrices, where the two agree to 3 us, stay with the kernel that takes any number of rows.)
+    const bool integer_passes = (int64_t)n_out * n_in >= (int64_t)120 << 20;
+    const float us_gemv = ttq::gemv_estimate_us(layer->format, x_dtype, m, n_out, n_in, integer_passes);
+    if (rounds && (m > 64 ? us_few / 0.65f : us_few) < us_gemm && (route == 2 || us_few < us_gemv)) {
       if (ttq::route_probe(ttq::kRouteGemmSkinnyF32ScaledF16)) return TTQ_OK;
       return hip_status(ttq::launch_gemm_skinny_f32(layer->format, layer->qweight, static_cast<const float*>(x), y, y_dtype,
                                                     layer->bias, layer->bias_dtype, m, n_out, n_in, s));
     }
-    if (us_gemm < 1e29f && (route == 2 || us_gemm < us_gemv))
+    if (rounds && us_gemm < 1e29f && (route == 2 || us_gemm < us_gemv))
       return hip_status(ttq::launch_gemm_pc_x(layer->format, layer->qweight, x, x_dtype, y, y_dtype, layer->bias,
                                               layer->bias_dtype, m, n_out, n_in, s, true));
   }
@@ -560,6 +580,7 @@ const char* ttq_route_name(int route) {
     case TTQ_ROUTE_GEMV_DOT2_MULTI: return "gemv_dot2_multi";
     case TTQ_ROUTE_GEMV_GENERIC: return "gemv_generic";
     case TTQ_ROUTE_GEMV_LONG: return "gemv_long";
+    case TTQ_ROUTE_GEMM_ROWS_EXACT: return "gemm_rows_exact";
     case TTQ_ROUTE_GEMV_TILE: return "gemv_tile";
     case TTQ_ROUTE_GEMM_SKINNY_F32_SCALED_F16: return "gemm_skinny_f32_scaled_f16";
     case TTQ_ROUTE_GEMM_PC: return "gemm_pc";

@@ -623,7 +623,8 @@ hipError_t launch_skinny_fmt(int format, const uint8_t* wb, const uint16_t* x_bf
 
 }  // namespace
 
-bool gemm_skinny_supported(int format, int64_t m, int64_t n_out, int64_t n_in) {
+// this file's kernel
+static bool skinny_registers_supported(int format, int64_t m, int64_t n_out, int64_t n_in) {
   static const int disabled = dev_knob("TTQ_GEMM_NO_SKINNY", 0);
   const int64_t block_bytes = format == kQ4_K ? 144 : (format == kQ6_K ? 210 : 272);
   // weight byte offsets and activation element offsets are 32-bit in the kernel; outputs are stored
@@ -633,13 +634,29 @@ bool gemm_skinny_supported(int format, int64_t m, int64_t n_out, int64_t n_in) {
          m * n_in < ((int64_t)1 << 31);
 }
 
+// The form that streams the weights through LDS (ttq_gemm_rows.hip): many weight rows, and outputs that are not whole groups of
+// eight.
+static bool use_rows(int format, int64_t m, int64_t n_out, int64_t n_in) {
+  return gemm_rows_supported(format, m, n_out, n_in) &&
+         (gemm_rows_preferred(n_out) || !skinny_registers_supported(format, m, n_out, n_in));
+}
+
+bool gemm_skinny_supported(int format, int64_t m, int64_t n_out, int64_t n_in) {
+  return skinny_registers_supported(format, m, n_out, n_in) || gemm_rows_supported(format, m, n_out, n_in);
+}
+
+float gemm_skinny_registers_estimate_us(int format, int64_t m, int64_t n_out, int64_t n_in) {
+  return skinny_registers_supported(format, m, n_out, n_in) ? skinny_choose(format, m, n_out, n_in, false).cost_us : 1e30f;
+}
+
 float gemm_skinny_estimate_us(int format, int64_t m, int64_t n_out, int64_t n_in) {
+  if (use_rows(format, m, n_out, n_in)) return gemm_rows_estimate_us(format, m, n_out, n_in);
   return skinny_choose(format, m, n_out, n_in, false).cost_us;
 }
 
 // The fused gate||up + silu_and_mul form: n_ff outputs from 2 * n_ff weight rows (Q4_K).
 bool gemm_skinny_silu_mul_supported(int64_t m, int64_t n_ff, int64_t n_in) {
-  return gemm_skinny_supported(kQ4_K, m, 2 * n_ff, n_in) && n_ff % 8 == 0;
+  return skinny_registers_supported(kQ4_K, m, 2 * n_ff, n_in) && n_ff % 8 == 0;
 }
 
 float gemm_skinny_silu_mul_estimate_us(int64_t m, int64_t n_ff, int64_t n_in) {
@@ -660,6 +677,8 @@ hipError_t launch_gemm_skinny(int format, const void* w, const uint16_t* x, int 
   if (m == 0 || n_out == 0) return hipSuccess;
   if (y_dtype != kBF16 && y_dtype != kF32 && y_dtype != kF16) return hipErrorInvalidValue;
   const uint8_t* wb = static_cast<const uint8_t*>(w);
+  if ((x_dtype == kF16 || (x_dtype == kBF16 && !row_scale)) && use_rows(format, m, n_out, n_in))
+    return launch_gemm_rows(format, w, x, x_dtype, y, y_dtype, bias, bias_dtype, m, n_out, n_in, s, row_scale);
   if (x_dtype == kBF16) {
     if (row_scale) return hipErrorInvalidValue;      // (row factors come with the scaled fp16 copy of fp32 activations)
     switch (format) {

@@ -456,6 +456,24 @@ bool gemv_row_is_long(int format, int x_dtype, int64_t n_in) {
   return n_in > (dot2 ? kMaxGemvIn16 : kMaxGemvInF32);
 }
 
+// Passes of eight fp16 rows, or the exact form of the kernel for up to 64: 32003 x 5120 at 9 / 16 / 43 / 64 rows
+// 42 / 41 / 53 / 61 us in one launch, 34 us a pass (with passes of four rows in packed dots 272 / 354 / 918 / 1322).
+static float rows_exact_us(int64_t m, int64_t n_out, int64_t n_in) {
+  const int64_t full = m / 64, rest = m % 64;
+  float us = full ? (float)full * 1.2f * gemm_rows_estimate_us(kQ6_K, 64, n_out, n_in) : 0.f;
+  if (rest) us += 1.2f * gemm_rows_estimate_us(kQ6_K, rest, n_out, n_in);
+  return us;
+}
+static float tile_passes_us(int x_dtype, int64_t m, int64_t n_out, int64_t n_in) {
+  const int64_t per = gemv_tile_rows(x_dtype), rest = m % per;
+  return (float)(m / per) * gemv_tile_estimate_us(x_dtype, per, n_out, n_in) +
+         (rest ? gemv_tile_estimate_us(x_dtype, rest, n_out, n_in) : 0.f);
+}
+static bool rows_exact_preferred(int x_dtype, int64_t m, int64_t n_out, int64_t n_in) {
+  return x_dtype == kF16 && m > 8 && gemm_rows_supported(kQ6_K, m < 64 ? m : 64, n_out, n_in) &&
+         rows_exact_us(m, n_out, n_in) < tile_passes_us(x_dtype, m, n_out, n_in);
+}
+
 hipError_t launch_gemv(int format, const void* w, const void* x, int x_dtype, void* y, int y_dtype,
                        const void* bias, int bias_dtype, int64_t m, int64_t n_out, int64_t n_in,
                        hipStream_t s) {
@@ -467,6 +485,23 @@ hipError_t launch_gemv(int format, const void* w, const void* x, int x_dtype, vo
       case kQ6_K: TTQ_ROUTE(kRouteGemvLong, launch_long_xy<FmtQ6_K>(w, x, x_dtype, y, y_dtype, bias, bias_dtype, m, n_out, n_in, s));
       default: return hipErrorInvalidValue;
     }
+  }
+  // Q6_K, more rows than a pass of the integer kernel takes: in fp16 the form for many rows (64 to a launch), else passes
+  const int64_t per_pass = gemv_tile_rows(x_dtype);
+  if (m > per_pass && gemv_tile_preferred(format, x_dtype, per_pass, n_out, n_in)) {
+    const bool rows = rows_exact_preferred(x_dtype, m, n_out, n_in);
+    if (route_probe(rows ? kRouteGemmRowsExact : kRouteGemvTile)) return hipSuccess;
+    const int64_t step = rows ? 64 : per_pass, xsize = x_dtype == kF32 ? 4 : 2, ysize = y_dtype == kF32 ? 4 : 2;
+    for (int64_t r = 0; r < m; r += step) {
+      const int64_t n = m - r < step ? m - r : step;
+      const void* xr = static_cast<const char*>(x) + r * n_in * xsize;
+      void* yr = static_cast<char*>(y) + r * n_out * ysize;
+      const hipError_t e = rows && n > per_pass
+          ? launch_gemm_rows_exact(w, static_cast<const uint16_t*>(xr), yr, y_dtype, bias, bias_dtype, n, n_out, n_in, s)
+          : launch_gemv_tile(format, w, xr, x_dtype, yr, y_dtype, bias, bias_dtype, n, n_out, n_in, s);
+      if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
   }
   if (gemv_tile_preferred(format, x_dtype, m, n_out, n_in))
     TTQ_ROUTE(kRouteGemvTile, launch_gemv_tile(format, w, x, x_dtype, y, y_dtype, bias, bias_dtype, m, n_out, n_in, s));
@@ -524,12 +559,17 @@ hipError_t launch_gemv(int format, const void* w, const void* x, int x_dtype, vo
 // Rough time (microseconds) of launch_gemv for m >= 2 activation rows, following the dispatch
 // above: passes over the weights x (packed megabytes / measured rate of the kernel that runs
 // + a fixed cost).  ttq_linear_forward weighs it against the prefill GEMM.
-float gemv_estimate_us(int format, int x_dtype, int64_t m, int64_t n_out, int64_t n_in) {
+float gemv_estimate_us(int format, int x_dtype, int64_t m, int64_t n_out, int64_t n_in, bool integer_kernels) {
   const int64_t per = format == kQ8_0 ? 32 : 256, blk = format == kQ8_0 ? 34 : (format == kQ4_K ? 144 : 210);
   const float mb = (float)(n_out * (n_in / per) * blk) * 1e-6f;
   // rows of any length: a pass over the weights per activation row (72 MB in 24.6 us, 155 MB in 51 us, 463 MB in 122 us)
   if (gemv_row_is_long(format, x_dtype, n_in)) return (float)m * (mb / 3.5f + 3.f);
-  if (gemv_tile_preferred(format, x_dtype, m, n_out, n_in)) return gemv_tile_estimate_us(m, n_out, n_in);
+  if (integer_kernels) {
+    const int64_t per = gemv_tile_rows(x_dtype);
+    if (m > per && gemv_tile_preferred(format, x_dtype, per, n_out, n_in))
+      return rows_exact_preferred(x_dtype, m, n_out, n_in) ? rows_exact_us(m, n_out, n_in) : tile_passes_us(x_dtype, m, n_out, n_in);
+    if (gemv_tile_preferred(format, x_dtype, m, n_out, n_in)) return gemv_tile_estimate_us(x_dtype, m, n_out, n_in);
+  }
   const bool b4 = gemv_q4k_batch4_supported(format, x_dtype, m, n_out, n_in);
   if (b4 && m <= 4) return mb / 2.75f + 2.f;
   if (gemv_q4k_batch_supported(format, x_dtype, m, n_out, n_in)) {

@@ -32,10 +32,8 @@
 // kernel, passes of the several-row int8 kernel), us: 32003 x 5120 fp16 one row 43.7 -> 30, two 55.7 -> 29.9, four 101.6 -> 30.5,
 // eight 189 -> 34; fp32 one row 55.9 -> 31.3; 5120 x 5120 fp16 12.2 -> 9.4, four rows 19.6 -> 12; 5120 x 13824 19.8 -> 16.9;
 // 128256 x 4096 bf16 at eight rows 152.7 -> 95, fp32 117 -> 87.
-#include <type_traits>
-
 #include "ttq_internal.h"
-#include "ttq_stream_common.h"
+#include "ttq_tile_common.h"
 
 namespace ttq {
 namespace {
@@ -46,172 +44,19 @@ constexpr int kTlDepth = 2;                // tiles in a wavefront's ring: one m
 constexpr int kTlXBlock = 528;             // 256 activations in LDS: the four lanes of a product's k-set on different banks
 constexpr int kTlZeroBytes = 512;          // what the lanes off the block diagonal read
 
-// four bytes -> two dwords of 16-bit halves (byte | hi << 8)
-__device__ __forceinline__ void spread_bytes(uint32_t u, uint32_t hi, uint32_t& a, uint32_t& b) {
-  a = __builtin_amdgcn_perm(hi, u, 0x04010400u);
-  b = __builtin_amdgcn_perm(hi, u, 0x04030402u);
-}
 template <class XT> __device__ __forceinline__ float half_pair_sum(uint32_t v) {
   if constexpr (std::is_same<XT, f16_tag>::value) return f16_bits_to_f32((uint16_t)(v & 0xFFFFu)) + f16_bits_to_f32((uint16_t)(v >> 16));
   else return __uint_as_float(v << 16) + __uint_as_float(v & 0xFFFF0000u);
 }
-template <class XT>
-__device__ __forceinline__ f32x4_t tile_mfma(const uint4& x, const uint32_t (&w)[4], f32x4_t c) {
-  if constexpr (std::is_same<XT, f16_tag>::value) {
-    f16x8_t a, b;
-    __builtin_memcpy(&a, &x, 16);
-    __builtin_memcpy(&b, w, 16);
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
-  } else {
-    bf16x8_t a, b;
-    __builtin_memcpy(&a, &x, 16);
-    __builtin_memcpy(&b, w, 16);
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
-  }
-}
-
-// One request: 64 lanes fetch 16 bytes each from base + off into 1 KiB of LDS.  In assembly, so that the compiler, which
-// cannot tell these asynchronous writes from its own LDS accesses, does not wait for every one of them.  STREAM: lines that
-// no other request shares leave the caches early.
-template <bool STREAM>
-__device__ __forceinline__ void tile_request(uint32_t lds, const uint8_t* base, uint32_t off) {
-  if constexpr (STREAM)
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt" ::"s"(lds), "v"(off), "s"(base) : "memory");
-  else
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base) : "memory");
-}
-
-struct TlQ6K {
-  static constexpr int kSub = 16;            // weights per scale
-  static constexpr int kChains = 4;          // matrix products per tile, each over four sub-blocks of every block
-  static constexpr int kSteps = kSub / 8;
-  static constexpr int kChunks = 14;         // 16-byte pieces of a block in LDS
-  static constexpr int kSlot = 16 * kChunks * 16;
-  static constexpr int kRequests = 4;
-  // chain 2h + p: sub-blocks 8h + 4p + g, g = lane / 16
-  static __device__ __forceinline__ constexpr int lane_k(int g) { return 16 * g; }
-  static __device__ __forceinline__ constexpr int chain_k(int c) { return 64 * c; }
-  static __device__ __forceinline__ void sub_of(int sub, int& c, int& g) { c = sub >> 2; g = sub & 3; }
-
-  struct Lane {
-    uint32_t src[kRequests], odd2[kRequests];                   // request addresses
-    uint32_t over, fix;                                          // bit i: request i is past the row's end / reads the last block
-    uint32_t ql[2], qlx[2], qh[2], qhx[2], sc, dd;              // operand addresses in a slot
-    uint32_t qh_shift, sc_shift, odd, d_mask, d_fix;
-    // rows: of a group; kq_last: the last block of a row's last tile
-    template <int KQ> __device__ __forceinline__ void init(int lane, int nsb, int rows, int kq_last, bool odd_total) {
-      const int n = lane & 15, g = lane >> 4;
-      over = fix = 0;
-#pragma unroll
-      for (int i = 0; i < kRequests; i++) {
-        const int p = min(64 * i + lane, 16 * kChunks - 1);
-        const int pb = p / kChunks, pos = p - pb * kChunks, c = (pos + 2 * kChunks - pb) % kChunks;
-        const int r = min(pb / KQ, rows - 1), kq = pb % KQ;
-        const uint32_t blk = (uint32_t)(r * nsb + kq);
-        src[i] = blk * 210u + (c < 13 ? 16u * c : 196u);
-        odd2[i] = 2u * (blk & 1u);
-        if (kq > kq_last) over |= 1u << i;
-        if (odd_total && r == rows - 1 && kq == kq_last && c == 13) fix |= 1u << i;
-      }
-      auto at = [&](int c) { return (uint32_t)(16 * (n * kChunks + (c + n) % kChunks)); };
-#pragma unroll
-      for (int h = 0; h < 2; h++) {
-        ql[h] = at(4 * h + g);
-        qlx[h] = at(4 * h + g + 1);
-        qh[h] = at(8 + 2 * h + (g & 1));
-        qhx[h] = at(8 + 2 * h + (g & 1) + 1);
-      }
-      sc = at(12);
-      dd = at(13) + 12;
-      qh_shift = 2u * (g >> 1);
-      sc_shift = 8u * g;
-      const int r = min(n / KQ, rows - 1), kq = n % KQ;
-      odd = (uint32_t)(r * nsb + kq) & 1u;
-      d_mask = kq > kq_last ? 0u : 0xFFFFu;
-      d_fix = (odd_total && r == rows - 1 && kq == kq_last) ? 16u : 0u;
-    }
-  };
-  // block: index of the tile's first block in the matrix; tail: a row's last tile; last: the matrix's last tile
-  template <bool STREAM>
-  static __device__ __forceinline__ void request(const Lane& L, int lane, uint32_t lds, const uint8_t* w, int64_t block, bool tail, bool last) {
-    const bool odd = block & 1;
-    const uint8_t* base = w + block * 210 - (odd ? 2 : 0);
-    uint32_t off[kRequests];
-#pragma unroll
-    for (int i = 0; i < kRequests; i++) off[i] = L.src[i] + (odd ? L.odd2[i] : 0u - L.odd2[i]);
-    if (tail) {
-#pragma unroll
-      for (int i = 0; i < kRequests; i++) {
-        if ((L.over >> i) & 1u) off[i] = 0u;
-        if (last && ((L.fix >> i) & 1u)) off[i] -= 2u;
-      }
-    }
-#pragma unroll
-    for (int i = 0; i < kRequests; i++)
-      if (i < kRequests - 1 || lane < 32) tile_request<STREAM>(lds + 1024 * i, base, off[i]);
-  }
-  struct Raw { uint32_t ql[2][4], qh[2][4], sc[4], d; };
-  static __device__ __forceinline__ void read(Raw& r, const uint8_t* slot, const Lane& L, int64_t block, bool tail, bool last) {
-    const uint32_t sh = (((uint32_t)block + L.odd) & 1u) * 16u;
-#pragma unroll
-    for (int h = 0; h < 2; h++) {
-      const uint4 a = *reinterpret_cast<const uint4*>(slot + L.ql[h]);
-      const uint32_t ax = *reinterpret_cast<const uint32_t*>(slot + L.qlx[h]);
-      const uint4 b = *reinterpret_cast<const uint4*>(slot + L.qh[h]);
-      const uint32_t bx = *reinterpret_cast<const uint32_t*>(slot + L.qhx[h]);
-      r.ql[h][0] = __builtin_amdgcn_alignbit(a.y, a.x, sh);
-      r.ql[h][1] = __builtin_amdgcn_alignbit(a.z, a.y, sh);
-      r.ql[h][2] = __builtin_amdgcn_alignbit(a.w, a.z, sh);
-      r.ql[h][3] = __builtin_amdgcn_alignbit(ax, a.w, sh);
-      r.qh[h][0] = __builtin_amdgcn_alignbit(b.y, b.x, sh + L.qh_shift);
-      r.qh[h][1] = __builtin_amdgcn_alignbit(b.z, b.y, sh + L.qh_shift);
-      r.qh[h][2] = __builtin_amdgcn_alignbit(b.w, b.z, sh + L.qh_shift);
-      r.qh[h][3] = __builtin_amdgcn_alignbit(bx, b.w, sh + L.qh_shift);
-    }
-    const uint4 s = *reinterpret_cast<const uint4*>(slot + L.sc);
-    const uint32_t e = *reinterpret_cast<const uint32_t*>(slot + L.dd);
-    r.sc[0] = __builtin_amdgcn_alignbit(s.y, s.x, sh);
-    r.sc[1] = __builtin_amdgcn_alignbit(s.z, s.y, sh);
-    r.sc[2] = __builtin_amdgcn_alignbit(s.w, s.z, sh);
-    r.sc[3] = __builtin_amdgcn_alignbit(e, s.w, sh);
-    // (the last block of the matrix, at an even place: its last piece was fetched two bytes early; blocks past the end of
-    // the row: no scale)
-    r.d = (e >> (last ? (sh | L.d_fix) : sh)) & (tail ? L.d_mask : 0xFFFFu);
-  }
-  struct Prep { float s[4]; };
-  static __device__ __forceinline__ void prepare(const Raw& r, const Lane& L, Prep& P) {
-    const float d = f16_bits_to_f32((uint16_t)r.d);
-#pragma unroll
-    for (int c = 0; c < 4; c++) P.s[c] = d * (float)(int)__builtin_amdgcn_sbfe((int)r.sc[c], L.sc_shift, 8);
-  }
-  // The integer q (0 .. 63) as a 16-bit float with an offset that costs no instruction: bf16 0x4300 | q = 128 + q, fp16
-  // 0x5C00 | q << 2 = 256 + q.  The sums are started at -(offset + 32) * sum(x).
-  template <class XT> static constexpr float kStart = std::is_same<XT, f16_tag>::value ? -288.f : -160.f;
-  template <class XT>
-  static __device__ __forceinline__ void weights(const Raw& r, int c, int t, uint32_t (&w)[4]) {
-    constexpr bool H = std::is_same<XT, f16_tag>::value;
-    constexpr uint32_t N = H ? 0x3C3C3C3Cu : 0x0F0F0F0Fu, Q = H ? 0xC0C0C0C0u : 0x30303030u;
-    const int h = c >> 1, p = c & 1;
-#pragma unroll
-    for (int k = 0; k < 2; k++) {
-      const uint32_t l = r.ql[h][2 * t + k], q = r.qh[h][2 * t + k];
-      // (the bit pairs of the low nibbles are bits 0-1 of the bytes of q, those of the high nibbles bits 4-5)
-      const uint32_t lo = H ? (p ? l >> 2 : l << 2) : (p ? l >> 4 : l), hi = H ? (p ? q << 2 : q << 6) : (p ? q : q << 4);
-      const uint32_t u = (lo & N) | (hi & Q);
-      spread_bytes(u, H ? 0x5C5C5C5Cu : 0x43434343u, w[2 * k], w[2 * k + 1]);
-    }
-  }
-};
-
-// J: activation rows as the matrix cores see them (an fp32 row is three bf16 ones).  KQ: blocks along K of a tile, of
+// J: activation rows as the matrix cores see them, PARTS to an activation row (three for fp32).  KQ: blocks along K of a tile, of
 // 16 / KQ weight rows.
-template <class F, class XT, int J, int KQ>
+template <class F, class XT, int J, int KQ, int PARTS>
 __global__ void __launch_bounds__(kTlThreads)
 gemv_tile_kernel(const uint8_t* __restrict__ w, const void* __restrict__ x, int n_out, int n_in, int depth, int m, int x_dtype,
                  int y_dtype, void* __restrict__ y, const void* __restrict__ bias, int bias_dtype) {
   extern __shared__ __attribute__((aligned(1024))) uint8_t tl_lds[];
   constexpr int JB = (J * KQ + 3) / 4, JI = J * KQ < 4 ? J * KQ : 4, R = 16 / KQ;
-  constexpr int SB = F::kSub;
+  constexpr int SB = F::kSub, M = J / PARTS;                    // activation rows at most
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n = lane & 15, g = lane >> 4;
@@ -223,22 +68,22 @@ gemv_tile_kernel(const uint8_t* __restrict__ w, const void* __restrict__ x, int 
   float* sums = reinterpret_cast<float*>(zero + kTlZeroBytes);                  // [tile][chain][jb][4 g + pseudo row % 4]
   uint8_t* xs = reinterpret_cast<uint8_t*>(sums + tpr * F::kChains * JB * 16);
   const uint32_t kpad = (uint32_t)tpr * KQ * 256u, xstride = (uint32_t)tpr * KQ * kTlXBlock;
-  float* part = reinterpret_cast<float*>(xs + J * xstride);                     // [wave][first, last][J][R]
+  float* part = reinterpret_cast<float*>(xs + J * xstride);                     // [wave][first, last][M][R]
   const uint32_t ring_lds = (uint32_t)__builtin_amdgcn_readfirstlane((int)sm_lds(ring)), xs_lds = sm_lds(xs);
 
-  const bool f32x = x_dtype == kF32;
   // ---- 16-bit activations: requests straight to their place
-  if (!f32x) {
+  if constexpr (PARTS == 1) {
     for (int row = 0; row < m; row++)
       for (int b = wave; b < nsb; b += kTlWaves)
         if (lane < 32)
           tile_request<false>((uint32_t)__builtin_amdgcn_readfirstlane((int)(xs_lds + row * xstride + kTlXBlock * b)),
                             static_cast<const uint8_t*>(x) + ((int64_t)row * n_in + 256 * b) * 2, 16u * (uint32_t)lane);
-  } else if constexpr (J == 3) {
-    for (int v8 = tid; v8 < n_in / 8; v8 += kTlThreads) {
+  } else {
+    for (int e = tid; e < m * (n_in / 8); e += kTlThreads) {
+      const int row = e / (n_in / 8), v8 = e - row * (n_in / 8);
       // three bf16 terms that add up to the fp32 value: every term is the rest cut to its upper 16 bits.  Times 2^-8, undone on
       // the sums: 128 + q then overflows no earlier than the value itself.
-      const float4* src = reinterpret_cast<const float4*>(static_cast<const float*>(x) + 8 * v8);
+      const float4* src = reinterpret_cast<const float4*>(static_cast<const float*>(x) + (int64_t)row * n_in + 8 * v8);
       const float4 f0 = src[0], f1 = src[1];
       float f[8] = {f0.x, f0.y, f0.z, f0.w, f1.x, f1.y, f1.z, f1.w};
 #pragma unroll
@@ -253,7 +98,7 @@ gemv_tile_kernel(const uint8_t* __restrict__ w, const void* __restrict__ x, int 
           f[2 * i] -= __uint_as_float(lo);
           f[2 * i + 1] -= __uint_as_float(hi);
         }
-        *reinterpret_cast<uint4*>(xs + p * xstride + kTlXBlock * (v8 >> 5) + 16 * (v8 & 31)) = make_uint4(o[0], o[1], o[2], o[3]);
+        *reinterpret_cast<uint4*>(xs + (3 * row + p) * xstride + kTlXBlock * (v8 >> 5) + 16 * (v8 & 31)) = make_uint4(o[0], o[1], o[2], o[3]);
       }
     }
   }
@@ -297,7 +142,7 @@ gemv_tile_kernel(const uint8_t* __restrict__ w, const void* __restrict__ x, int 
     else if (later == 1) sm_wait_vmcnt<F::kRequests>();
     else sm_wait_vmcnt<0>();
   };
-  if (!f32x) {
+  if constexpr (PARTS == 1) {
     const int out = min(t1 - t0, depth);
     if (out >= 4) sm_wait_vmcnt<4 * F::kRequests>();
     else wait_later(out);
@@ -387,9 +232,11 @@ gemv_tile_kernel(const uint8_t* __restrict__ w, const void* __restrict__ x, int 
   // the wavefront has done its tiles of group q: whole rows are outputs, else the sums wait for the other wavefronts'
   auto finish = [&](int q, bool whole, int which) {
     const int kq = n % KQ, r = n / KQ, col = first_row(q) + r;
-    float tot[(J + 3) / 4 * 4];
+    float tot[(M + 3) / 4 * 4];
 #pragma unroll
-    for (int j = 0; j < J; j++) {
+    for (int j = 0; j < (M + 3) / 4 * 4; j++) tot[j] = 0.f;
+#pragma unroll
+    for (int j = J - 1; j >= 0; j--) {        // (an fp32 row's small terms first)
       // the lane's own block among the pseudo rows of row j
       float v = acc[(j * KQ) >> 2][(j * KQ) & 3];
 #pragma unroll
@@ -397,19 +244,18 @@ gemv_tile_kernel(const uint8_t* __restrict__ w, const void* __restrict__ x, int 
       v = add_xor32(add_xor16(v));
       if constexpr (KQ >= 2) v += lane_xor<1>(v, lane);
       if constexpr (KQ >= 4) v += lane_xor<2>(v, lane);
-      tot[j] = v;
+      tot[j / PARTS] += v;
+    }
+    if constexpr (PARTS > 1) {
+#pragma unroll
+      for (int j = 0; j < M; j++) tot[j] *= 0x1p8f;
     }
 #pragma unroll
-    for (int j = J; j < (J + 3) / 4 * 4; j++) tot[j] = 0.f;
-    if constexpr (J == 3) {
-      if (f32x) tot[0] = (tot[0] + (tot[1] + tot[2])) * 0x1p8f;
-    }
-#pragma unroll
-    for (int jb = 0; jb < (J + 3) / 4; jb++) {
+    for (int jb = 0; jb < (M + 3) / 4; jb++) {
       const int j = 4 * jb + g;
       const float v = g == 0 ? tot[4 * jb] : (g == 1 ? tot[4 * jb + 1] : (g == 2 ? tot[4 * jb + 2] : tot[4 * jb + 3]));
       if (kq == 0 && j < m) {
-        if (!whole) part[((wave * 2 + which) * J + j) * R + r] = v;
+        if (!whole) part[((wave * 2 + which) * M + j) * R + r] = v;
         else if (col >= R * (g0 + q) && col < n_out) put(j, col, v);
       }
     }
@@ -443,9 +289,9 @@ gemv_tile_kernel(const uint8_t* __restrict__ w, const void* __restrict__ x, int 
     if (run_start(wave - 1) <= qa * tpr) {
       for (int e = lane; e < m * R; e += 64) {
         const int r = e % R, j = e / R;
-        float v = part[((2 * (wave - 1) + (run_start(wave - 1) == qa * tpr ? 0 : 1)) * J + j) * R + r];
+        float v = part[((2 * (wave - 1) + (run_start(wave - 1) == qa * tpr ? 0 : 1)) * M + j) * R + r];
         for (int u = wave; u < kTlWaves && run_start(u) < (qa + 1) * tpr; u++)
-          if (run_start(u + 1) > run_start(u)) v += part[(2 * u * J + j) * R + r];
+          if (run_start(u + 1) > run_start(u)) v += part[(2 * u * M + j) * R + r];
         const int col = first_row(qa) + r;
         if (col >= R * (g0 + qa) && col < n_out) put(j, col, v);
       }
@@ -469,11 +315,11 @@ size_t tile_lds_bytes(int j, int kq, int64_t n_in, int depth) {
          (size_t)2 * kTlWaves * j * (16 / kq) * 4;
 }
 
-template <class F, class XT, int J, int KQ>
+template <class F, class XT, int J, int KQ, int PARTS = 1>
 hipError_t launch_tile_j(const TlArgs& a, hipStream_t s) {
   constexpr int depth = kTlDepth;
   const size_t lds = tile_lds_bytes<F>(J, KQ, a.n_in, depth);
-  auto kernel = gemv_tile_kernel<F, XT, J, KQ>;
+  auto kernel = gemv_tile_kernel<F, XT, J, KQ, PARTS>;
   static LargeLds configured;
   if (lds > 64 * 1024) {
     const hipError_t e = allow_large_lds(reinterpret_cast<const void*>(kernel), configured);
@@ -499,12 +345,15 @@ hipError_t launch_tile_x(const TlArgs& a, hipStream_t s) {
 
 }  // namespace
 
+int gemv_tile_rows(int x_dtype) { return x_dtype == kF32 ? 2 : 8; }
+
 // Whether the kernel takes the shape: all activations of a pass are in LDS at once, beside the ring.
 bool gemv_tile_supported(int format, int x_dtype, int64_t m, int64_t n_out, int64_t n_in) {
   static const int disabled = dev_knob("TTQ_NO_TILE", 0);
   if (disabled || format != kQ6_K || n_in % 256 != 0 || m < 1 || m > 8 || n_out > 0x3FFFFFFF || n_in > (1 << 22)) return false;
-  if (x_dtype == kF32 && m > 1) return false;
-  const int j = x_dtype == kF32 ? 3 : (m <= 2 ? (int)m : (m <= 4 ? 4 : 8)), kq = m > 2 ? 1 : (m == 2 || x_dtype == kF32 ? 2 : 4);
+  const bool f32 = x_dtype == kF32;
+  if (m > gemv_tile_rows(x_dtype)) return false;
+  const int j = f32 ? 3 * (int)m : (m <= 2 ? (int)m : (m <= 4 ? 4 : 8)), kq = f32 ? (m == 1 ? 2 : 1) : (m == 1 ? 4 : (m == 2 ? 2 : 1));
   return tile_lds_bytes<TlQ6K>(j, kq, n_in, kTlDepth) <= kTlLds;
 }
 
@@ -524,16 +373,17 @@ bool gemv_tile_preferred(int format, int x_dtype, int64_t m, int64_t n_out, int6
   if (!gemv_tile_supported(format, x_dtype, m, n_out, n_in)) return false;
   if (always) return true;
   const float mb = (float)(n_out * (n_in >> 8) * 210) * 1e-6f;
-  if (x_dtype == kF32) return mb >= 7.f;
+  if (x_dtype == kF32) return mb >= (m == 1 ? 7.f : 5.f);
   if (m == 1) return !gemv_q6k_stream_supported(format, x_dtype, n_out, n_in) && mb >= (n_in > 4096 ? 12.f : 27.f);
   if (mb < 5.f) return false;
   return !gemv_q6k_stream4_supported(format, x_dtype, m, n_out, n_in) || (m > 4 && mb >= 100.f);
 }
 
 // Several rows, us: 21.5 / 134 / 431 MB 10.2 / 28.9 / 84 for two rows, 11.8 / 30 / 87 for four, 15.1 / 33.4 / 98 for eight.
-float gemv_tile_estimate_us(int64_t m, int64_t n_out, int64_t n_in) {
+// (an fp32 row is three.)
+float gemv_tile_estimate_us(int x_dtype, int64_t m, int64_t n_out, int64_t n_in) {
   const float mb = (float)(n_out * (n_in >> 8) * 210) * 1e-6f;
-  return m <= 4 ? 5.f + mb / 5.2f : 8.3f + mb / 4.8f;
+  return (x_dtype == kF32 ? 3 * m : m) <= 4 ? 5.f + mb / 5.2f : 8.3f + mb / 4.8f;
 }
 
 hipError_t launch_gemv_tile(int format, const void* w, const void* x, int x_dtype, void* y, int y_dtype, const void* bias,
@@ -541,7 +391,7 @@ hipError_t launch_gemv_tile(int format, const void* w, const void* x, int x_dtyp
   if (m == 0 || n_out == 0) return hipSuccess;
   if (format != kQ6_K) return hipErrorInvalidValue;
   const TlArgs a{static_cast<const uint8_t*>(w), x, y, bias, (int)m, (int)n_out, (int)n_in, x_dtype, y_dtype, bias_dtype};
-  if (x_dtype == kF32) return launch_tile_j<TlQ6K, bf16_tag, 3, 2>(a, s);
+  if (x_dtype == kF32) return m == 1 ? launch_tile_j<TlQ6K, bf16_tag, 3, 2, 3>(a, s) : launch_tile_j<TlQ6K, bf16_tag, 6, 1, 3>(a, s);
   if (x_dtype == kF16) return launch_tile_x<TlQ6K, f16_tag>(a, s);
   return launch_tile_x<TlQ6K, bf16_tag>(a, s);
 }

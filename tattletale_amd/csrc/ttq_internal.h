@@ -33,6 +33,7 @@ enum : int {
   kRouteGemvGeneric = 14,
   kRouteGemvLong = 15,
   kRouteGemvTile = 16,
+  kRouteGemmRowsExact = 17,
   kRouteGemmSkinnyF32ScaledF16 = 19,
   kRouteGemmPc = 20,
   kRouteGemmPcSplitK = 21,
@@ -159,10 +160,11 @@ hipError_t launch_gemv_q6k_stream4(const void* w, const void* x, int x_dtype, vo
                                    const void* bias, int bias_dtype, int64_t m, int64_t n_out, int64_t n_in,
                                    hipStream_t s);
 
-// Q6_K as integers on the 16-bit matrix cores, one to eight activation rows (one of fp32), any shape (ttq_gemv_tile.hip).
+// Q6_K as integers on the 16-bit matrix cores, one to eight activation rows (two of fp32), any shape (ttq_gemv_tile.hip).
+int gemv_tile_rows(int x_dtype);      // rows of a pass at most
 bool gemv_tile_supported(int format, int x_dtype, int64_t m, int64_t n_out, int64_t n_in);
 bool gemv_tile_preferred(int format, int x_dtype, int64_t m, int64_t n_out, int64_t n_in);
-float gemv_tile_estimate_us(int64_t m, int64_t n_out, int64_t n_in);
+float gemv_tile_estimate_us(int x_dtype, int64_t m, int64_t n_out, int64_t n_in);
 hipError_t launch_gemv_tile(int format, const void* w, const void* x, int x_dtype, void* y, int y_dtype,
                             const void* bias, int bias_dtype, int64_t m, int64_t n_out, int64_t n_in, hipStream_t s);
 
@@ -215,7 +217,8 @@ hipError_t launch_gemv_q4k_batch4(const void* w, const void* x, int x_dtype, voi
                                   int64_t n_in, hipStream_t s);
 
 // Rough times (microseconds) of the two ways to run a few activation rows.
-float gemv_estimate_us(int format, int x_dtype, int64_t m, int64_t n_out, int64_t n_in);
+// integer_kernels: with the kernels of ttq_gemv_tile.hip and the exact form of ttq_gemm_rows.hip among the decode kernels
+float gemv_estimate_us(int format, int x_dtype, int64_t m, int64_t n_out, int64_t n_in, bool integer_kernels = true);
 float gemm_pc_estimate_us(int format, int64_t m, int64_t n_out, int64_t n_in);
 int gemv_q4k_batch_tokens(int64_t m, int64_t n_in);
 
@@ -232,11 +235,22 @@ hipError_t allow_large_lds(const void* kernel, LargeLds& state);
 // registers (ttq_gemm_skinny.hip).
 bool gemm_skinny_supported(int format, int64_t m, int64_t n_out, int64_t n_in);
 float gemm_skinny_estimate_us(int format, int64_t m, int64_t n_out, int64_t n_in);
+// of the register kernel alone; 1e30 for shapes it does not take
+float gemm_skinny_registers_estimate_us(int format, int64_t m, int64_t n_out, int64_t n_in);
 // x: bf16 or fp16 activations (the weights are rounded once to the same type); y: bf16, fp16 or fp32.
 // row_scale (fp16 activations only): a factor per row on the sums, before the bias.
 hipError_t launch_gemm_skinny(int format, const void* w, const uint16_t* x, int x_dtype, void* y, int y_dtype,
                               const void* bias, int bias_dtype, int64_t m, int64_t n_out, int64_t n_in,
                               hipStream_t s, const float* row_scale = nullptr);
+// The form for many weight rows, any number of them (ttq_gemm_rows.hip): Q4_K, Q6_K.
+bool gemm_rows_supported(int format, int64_t m, int64_t n_out, int64_t n_in);
+bool gemm_rows_preferred(int64_t n_out);
+float gemm_rows_estimate_us(int format, int64_t m, int64_t n_out, int64_t n_in);
+hipError_t launch_gemm_rows(int format, const void* w, const uint16_t* x, int x_dtype, void* y, int y_dtype, const void* bias,
+                            int bias_dtype, int64_t m, int64_t n_out, int64_t n_in, hipStream_t s, const float* row_scale);
+// Q6_K and fp16 activations with nothing rounded before the sums: a decode kernel for 9 to 64 rows.
+hipError_t launch_gemm_rows_exact(const void* w, const uint16_t* x_f16, void* y, int y_dtype, const void* bias, int bias_dtype, int64_t m,
+                                  int64_t n_out, int64_t n_in, hipStream_t s);
 // Any number of rows, 64 per launch.
 hipError_t launch_gemm_skinny_chunked(int format, const void* w, const uint16_t* x, int x_dtype, void* y, int y_dtype,
                                       const void* bias, int bias_dtype, int64_t m, int64_t n_out, int64_t n_in,
