@@ -32,12 +32,9 @@ struct Codebook {
 // (lower index gets a+b, upper a-b), so the results do not depend on how it is laid out.
 template <int D, int N>
 __device__ __forceinline__ void fwht_lane_stage(float (&v)[N], int lane) {
-  const bool upper = (lane & D) != 0;
+  const float sign = (lane & D) != 0 ? -1.f : 1.f;      // (the sum and the difference by one instruction, rounded once as they are)
 #pragma unroll
-  for (int i = 0; i < N; i++) {
-    const float o = lane_xor<D>(v[i], lane);
-    v[i] = upper ? (o - v[i]) : (v[i] + o);
-  }
+  for (int i = 0; i < N; i++) v[i] = fmaf_(sign, v[i], lane_xor<D>(v[i], lane));
 }
 __device__ __forceinline__ void fwht128_quad(float (&v)[4], int lane) {
   float t;
@@ -76,22 +73,12 @@ __device__ __forceinline__ void load_x4(const bf16_tag* p, float (&v)[4]) {
 typedef _Float16 f16x4_t __attribute__((ext_vector_type(4)));
 typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
 
-// 16 wavefronts: a wavefront issues one vector instruction about every five clocks however many others
-// share its SIMD, so the decode rate of a compute unit grows with the number of resident wavefronts.
-constexpr int kXmThreads = 1024;
-constexpr int kXmKSplit = kXmThreads / kWave / 8; // wavefronts per tile column; each takes 8 / kXmKSplit k-tiles of a group
-constexpr int kXmTilesPerWave = 8 / kXmKSplit;
-constexpr int kXmTok = 8;                         // activation rows per workgroup (two B columns each)
-constexpr int kXmChunkTiles = 32;                 // k-tiles per LDS pass
-constexpr int kXmChunkK = kXmChunkTiles * 16;
-constexpr int kXmColStride = kXmChunkK + 8;       // halfs; 16 bytes of padding: the 16 columns' 8-byte B reads fall on all 64 banks
-
-// Codebook value of the trellis state in bits OFF .. OFF+15 of `w`, written as an fp16 number into half
-// HALF of `dst` (the other half is kept when HALF is 1): the sum of the two fp16 numbers that the masked
-// hash holds, added by one instruction that picks both halves of its operand itself.
-template <int CB, int OFF, int HALF, bool LAST = false>
-__device__ __forceinline__ void xm_code(uint32_t w, uint32_t& dst) {
-  uint32_t u = __builtin_amdgcn_ubfe(w, OFF, 16) * Codebook<CB>::kMul;
+// Codebook value of a 16-bit trellis state, written as an fp16 number into half HALF of `dst` (the other half is kept
+// when HALF is 1): the sum of the two fp16 numbers that the masked hash holds, added by one instruction that picks both
+// halves of its operand itself.
+template <int CB, int HALF, bool LAST = false>
+__device__ __forceinline__ void xm_code(uint32_t state, uint32_t& dst) {
+  uint32_t u = state * Codebook<CB>::kMul;
   if constexpr (CB == 0) u += 64248484u;
   u = (u & 0x8FFF8FFFu) ^ 0x3B603B60u;
   if constexpr (HALF == 0)
@@ -147,65 +134,58 @@ template <> struct XmRaw<bf16_tag> {
   }
 };
 
-// Where a lane's windows lie inside a tile's dword string.
+// Where a lane's windows lie inside a packed tile, as it is in memory: a cyclic string of 16-bit words, most significant bit
+// first.  The four bytes that a window starts in lie in two consecutive dwords; one byte permutation brings them into
+// string order (byte s of the string is byte s ^ 1 in memory), and a weight's state is a bit field of the result: the
+// first starts 0..7 bits below the top, which depends on the lane only where the number of bits per weight is odd.
+// (Two funnel-shift operands with their halves swapped first, as this was before, take two more instructions per window.)
 template <int BITS>
 struct XmLane {
-  static constexpr int kWin = BITS <= 5 ? 1 : 2;     // funnel shifts per four weights
-  int dw[kWin];                                      // first dword to read, relative to the tile (may be -1)
-  uint32_t sh[kWin];                                 // funnel shift
+  static constexpr int kWin = BITS <= 4 ? 1 : 2;     // windows per four weights
+  static constexpr int kPer = 4 / kWin;
+  uint32_t at[kWin][2];                              // byte offsets of the two dwords in the tile
+  uint32_t sel[kWin];                                // byte selector
+  uint32_t down;                                     // 4 if the lane's windows start four bits lower, else 0
   __device__ __forceinline__ void init(int lane) {
     const int j = lane & 15, q = lane >> 4;
+    down = (BITS & 1) ? 4u * (q & 1) : 0u;
 #pragma unroll
     for (int w = 0; w < kWin; w++) {
       const int bit = (16 * j + 4 * q + 2 * w) * BITS;
-      const int o = bit & 31, d = bit >> 5;
-      // alignbit(hi, lo, s) = low 32 bits of (hi:lo) >> s, s < 32: a window that starts on a dword
-      // boundary takes the pair one dword earlier and shifts by nothing
-      dw[w] = d - (o == 0);
-      sh[w] = (32 - o) & 31;
-    }
-  }
-  // the dwords of one tile that hold this lane's windows
-  __device__ __forceinline__ void fetch(const uint32_t* tile, uint32_t (&c)[kWin][2]) const {
+      const int b = bit >> 3, d = b >> 2;
+      at[w][0] = 4u * d;
+      at[w][1] = 4u * ((d + 1) % (8 * BITS));
+      sel[w] = 0;
 #pragma unroll
-    for (int w = 0; w < kWin; w++) {
-      c[w][0] = tile[dw[w]];
-      c[w][1] = tile[dw[w] + 1];
+      for (int i = 0; i < 4; i++) sel[w] |= (uint32_t)((b + 3 - i - 4 * d) ^ 1) << (8 * i);
     }
   }
-  // the four weights as the matrix cores' A fragment (two registers of two fp16 each)
+  // The four weights as half of an A fragment (two registers of two fp16 each).  (The bits that a window of two weights
+  // starts below its byte: 2 w BITS + 4 q BITS modulo 8; the first part is a constant, the second is `down`, and
+  // where the sum passes 8 it starts in the byte after.)
+  template <int CB, int W, int E, int HALF, bool LAST = false>
+  __device__ __forceinline__ void code(uint32_t w, uint32_t& dst) const {
+    constexpr int kTop = (2 * W * BITS) & 7;
+    if constexpr (BITS & 1) xm_code<CB, HALF, LAST>(__builtin_amdgcn_ubfe(w, field(W, E), 16), dst);
+    else xm_code<CB, HALF, LAST>(__builtin_amdgcn_ubfe(w, 16 - kTop - E * BITS, 16), dst);
+  }
+  __device__ __forceinline__ uint32_t field(int w, int e) const { return 16u - (((uint32_t)(2 * w * BITS) + down) & 7u) - (uint32_t)(e * BITS); }
   template <int CB>
-  __device__ __forceinline__ f16x4_t decode(const uint32_t (&c)[kWin][2]) const {
-    uint32_t r[2];
+  __device__ __forceinline__ void decode(const uint32_t (&c)[kWin][2], uint32_t (&r)[2]) const {
+    const uint32_t w0 = __builtin_amdgcn_perm(c[0][1], c[0][0], sel[0]);
     if constexpr (kWin == 1) {
-      const uint32_t w = __builtin_amdgcn_alignbit(c[0][0], c[0][1], sh[0]);
-      xm_code<CB, 16, 0>(w, r[0]);
-      xm_code<CB, 16 - BITS, 1>(w, r[0]);
-      xm_code<CB, 16 - 2 * BITS, 0>(w, r[1]);
-      xm_code<CB, 16 - 3 * BITS, 1, true>(w, r[1]);
+      code<CB, 0, 0, 0>(w0, r[0]);
+      code<CB, 0, 1, 1>(w0, r[0]);
+      code<CB, 0, 2, 0>(w0, r[1]);
+      code<CB, 0, 3, 1, true>(w0, r[1]);
     } else {
-#pragma unroll
-      for (int p = 0; p < 2; p++) {
-        const uint32_t w = __builtin_amdgcn_alignbit(c[p][0], c[p][1], sh[p]);
-        xm_code<CB, 16, 0>(w, r[p]);
-        if (p == 0) xm_code<CB, 16 - BITS, 1>(w, r[p]);
-        else xm_code<CB, 16 - BITS, 1, true>(w, r[p]);
-      }
+      const uint32_t w1 = __builtin_amdgcn_perm(c[kWin - 1][1], c[kWin - 1][0], sel[kWin - 1]);
+      code<CB, 0, 0, 0>(w0, r[0]);
+      code<CB, 0, 1, 1>(w0, r[0]);
+      code<CB, 1, 0, 0>(w1, r[1]);
+      code<CB, 1, 1, 1, true>(w1, r[1]);
     }
-    f16x4_t a;
-    __builtin_memcpy(&a, r, 8);
-    return a;
   }
-};
-
-template <int BITS>
-struct XmGeom {
-  static constexpr int kTileDw = 8 * BITS;
-  static constexpr int kTileStride = kTileDw + 1;                       // + the wrap dword
-  static constexpr int kSlabDw = 1 + kXmChunkTiles * 8 * kTileStride;   // one dword in front for dw == -1
-  static constexpr int kRunPieces = 16 * BITS;                          // 16-byte pieces of one k-tile's run
-  static constexpr int kPieces = kXmChunkTiles * kRunPieces;            // of a full pass
-  static constexpr int kSets = (kPieces + kXmThreads - 1) / kXmThreads; // pieces per thread
 };
 
 }  // namespace ttq

@@ -3,214 +3,318 @@
 //   y = svh o H( T * H(suh o x) ) + bias
 //
 // Work split.  A workgroup owns one Hadamard group of 128 output channels (8 tiles across) and one
-// slice of the reduction dimension; its 8 wavefronts take one 16-channel tile column each.  The
+// slice of the reduction dimension; two of its 16 wavefronts take a 16-channel tile column, half of every
+// group's eight k-tiles each.  The
 // slices of a group hand their sums to the group's last slice through tagged words in a workspace (one
 // store and one load each); the last slice adds them in a fixed order, rotates the 128 sums of
 // each row and writes y.  With one slice there is no workspace traffic.
 //
-// Weights.  For one k-tile the 8 tiles of the group are contiguous in trellis[k_tile][n_tile][16*bits],
-// so the workgroup copies whole runs of 256*bits bytes, 16 bytes per lane, into LDS: up to 32 k-tiles per
-// pass, requested one pass ahead.  On the way in every dword's halves are swapped, which turns the
-// string of 16-bit words (most significant bit first) into a string of big-endian dwords; every tile
-// is followed by a copy of its first dword, because the string is cyclic.
+// Activations.  They are rotated into LDS before the wavefronts part, as much of the slice as fits (all of it for a
+// few rows): x o suh, the 128-group butterfly in registers, then a power-of-two scale per (row, group) that brings the
+// group's largest magnitude to 2^14, and a split into two fp16 terms (value and remainder), which together carry 22
+// bits.  The B operand holds up to 8 activation rows as 16 columns (term 0, term 1 of each); the two columns are added
+// at the end, and each group's matrix-core sum is scaled back in fp32 before it joins the running sum.
 //
-// Decode.  v_mfma_f32_16x16x16_f16 wants from lane (j = lane % 16, q = lane / 16) the four weights
-// k = 4q .. 4q+3 of channel j: the windows that start at bit (16j + 4q + e) * bits, e = 0..3.  The
-// lane reads the two dwords that hold them, one funnel shift aligns the first window to bit 31, and
-// the others are bit fields at constant offsets below it (two funnel shifts for 6..8 bits per weight).
-// Per weight: one bit-field extract, one 32-bit multiply, one three-input bit operation, one fp16 add
-// that writes its half of the A fragment directly.
+// Weights.  A wavefront copies the tiles that it decodes into a ring of its own by LDS DMA, packed as they are in
+// memory, 16 tiles to a stage, and waits for nobody: there is no barrier until its tiles are done.  (With passes of 32 k-tiles
+// that all wavefronts staged together, every pass waited twice for the slowest one, and for the two that rotated its
+// activations.  us, one row, passes / rings: 28672 x 4096 3 bits 33.4 / 27.6, 6 bits 43.4 / 32.3; 14336 x 4096 5 bits 24.6 /
+// 19.9; 4096 x 14336 3 bits 18.7 / 17.7, eight rows 28.6 / 21.8; 4096 x 4096 2 .. 6 bits 9.1 / 8.9 / 10.0 / 10.0 / 12.4 and 8.3 / 8.95 / 9.3 / 10.3 /
+// 11.0, where the launch, the rotation and the hand-off are most of it.)
 //
-// Activations.  Each slice rotates its own part of x: x o suh, the 128-group butterfly in registers,
-// then a power-of-two scale per (row, group) that brings the group's largest magnitude to 2^14, and a
-// split into two fp16 terms (value and remainder), which together carry 22 bits.  The B operand holds
-// up to 8 activation rows as 16 columns (term 0, term 1 of each); the two columns are added at the end,
-// and each group's matrix-core sum is scaled back in fp32 before it joins the running sum.
+// Decode.  The matrix cores want from lane (j = lane % 16, q = lane / 16) the four weights k = 4q .. 4q+3 of channel j
+// of a tile: the windows that start at bit (16j + 4q + e) * bits, e = 0..3.  The lane reads the two dwords that hold
+// them, a byte permutation lines them up, and per weight there are a bit-field extract, a 32-bit multiply, one
+// three-input bit operation and one fp16 add that writes its half of the A fragment directly, 17 instructions of
+// the 19 that a tile costs a wavefront (the vector units are busy 85 % of the time at 28672 x 4096; 224 of 256 compute units).
 #include "ttq_exl3_common.h"
+#include "ttq_stream_common.h"
 
 #include <mutex>
 #include <unordered_map>
 
 namespace ttq {
 
+constexpr int kXmThreads = 1024;                      // 16 wavefronts: the decode is a chain of instructions, which four to a SIMD hide
+constexpr int kXmTok = 8;                             // activation rows per workgroup (two B columns each)
+constexpr int kXmKSplit = kXmThreads / kWave / 8;     // wavefronts per tile column; each takes 8 / kXmKSplit k-tiles of a group
+constexpr int kXmTilesPerWave = 8 / kXmKSplit;
+constexpr int kXmStageGroups = 4;                     // Hadamard groups (128 k) to a stage of the ring
+constexpr int kXmLds = 160 * 1024;
+
+// A stage is kXmStageGroups * kXmTilesPerWave packed tiles of 32 * BITS bytes.  Two stages in flight behind the one that is
+// decoded are 6 KiB * BITS a workgroup for up to 4 bits; above that one is as much.
+template <int BITS>
+struct XmGeom {
+  static constexpr int kTileBytes = 32 * BITS;
+  static constexpr int kTiles = kXmStageGroups * kXmTilesPerWave;
+  static constexpr int kPieces = kTiles * 2 * BITS;                       // of 16 bytes
+  static constexpr int kReq = (kPieces + 63) / 64;                        // requests per stage
+  static constexpr int kSlotBytes = kReq * 1024;
+  static constexpr int kDepth = BITS <= 4 ? 3 : 2;
+  static constexpr int kRingBytes = (kXmThreads / kWave) * kDepth * kSlotBytes;
+};
+template <typename T>
+__device__ __forceinline__ T lds_at(uint32_t a) {
+  return *(const __attribute__((address_space(3))) T*)(size_t)a;
+}
+constexpr int kXmColPad = 8;                          // halfs: the 16 columns of a B read fall on different banks
+// LDS for `groups` Hadamard groups of activations of `cols` columns: the terms and their scales
+constexpr int xm_x_bytes(int cols, int groups) { return cols * (groups * 128 + kXmColPad) * 2 + cols * groups * 4; }
+
+// The first activations (16 bytes a lane in fp32, else 8) and their signs, then the N requests of a stage at lds and the 1 KiB
+// places after it, and a wait for the activations alone.  In one statement: the compiler, which knows nothing of the
+// requests, would wait for them too.
+#define TTQ_XM_REQUEST(I) "s_add_u32 m0, %[lds], " #I "*1024\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %[a" #I "], off\n\t"
+#define TTQ_XM_FIRST(X, REQUESTS, N, ...)                                                                                  \
+  asm volatile("global_load_dwordx2 %[s], %[sp], off\n\tglobal_load_" X " %[x], %[xp], off\n\t" REQUESTS "s_waitcnt vmcnt(" #N ")" \
+               : [s] "=&v"(s), [x] "=&v"(v)                                                                                \
+               : [sp] "v"(sp), [xp] "v"(xp), [lds] "s"(lds), __VA_ARGS__                                                  \
+               : "memory", "scc")
+#define TTQ_XM_FIRST_N(X)                                                                                                  \
+  if constexpr (N == 1) TTQ_XM_FIRST(X, TTQ_XM_REQUEST(0), 1, [a0] "v"(a[0]));                                            \
+  else if constexpr (N == 2) TTQ_XM_FIRST(X, TTQ_XM_REQUEST(0) TTQ_XM_REQUEST(1), 2, [a0] "v"(a[0]), [a1] "v"(a[1]));      \
+  else if constexpr (N == 3)                                                                                               \
+    TTQ_XM_FIRST(X, TTQ_XM_REQUEST(0) TTQ_XM_REQUEST(1) TTQ_XM_REQUEST(2), 3, [a0] "v"(a[0]), [a1] "v"(a[1]), [a2] "v"(a[2])); \
+  else                                                                                                                     \
+    TTQ_XM_FIRST(X, TTQ_XM_REQUEST(0) TTQ_XM_REQUEST(1) TTQ_XM_REQUEST(2) TTQ_XM_REQUEST(3), 4, [a0] "v"(a[0]),            \
+                 [a1] "v"(a[1]), [a2] "v"(a[2]), [a3] "v"(a[3]))
+typedef uint32_t xm_u32x2 __attribute__((ext_vector_type(2)));
+template <int N, typename XT>
+__device__ __forceinline__ void xm_first_loads(XmRaw<XT>& xv, uint2& sv, const XT* xp, const uint16_t* sp, uint32_t lds,
+                                               const uint8_t* const (&a)[N]) {
+  static_assert(N >= 1 && N <= 4);
+  xm_u32x2 s;
+  if constexpr (sizeof(xv) == 16) {
+    sm_u32x4 v;
+    TTQ_XM_FIRST_N("dwordx4");
+    __builtin_memcpy(&xv, &v, 16);
+  } else {
+    xm_u32x2 v;
+    TTQ_XM_FIRST_N("dwordx2");
+    __builtin_memcpy(&xv, &v, 8);
+  }
+  __builtin_memcpy(&sv, &s, 8);
+}
+#undef TTQ_XM_FIRST_N
+#undef TTQ_XM_FIRST
+#undef TTQ_XM_REQUEST
+
 template <int BITS, int CB, typename XT>
 __global__ void __launch_bounds__(kXmThreads)
 gemv_exl3_mfma_kernel(const uint16_t* __restrict__ trellis, const uint16_t* __restrict__ suh,
                       const uint16_t* __restrict__ svh, const XT* __restrict__ x, void* __restrict__ y, int y_dtype,
                       const void* __restrict__ bias, int bias_dtype, int m, int n_out, int n_in, int slice_tiles,
-                      unsigned long long* __restrict__ accum, int poll_limit) {
+                      int chunk_groups, unsigned long long* __restrict__ accum, int poll_limit) {
   using G = XmGeom<BITS>;
-  __shared__ uint32_t slab[G::kSlabDw];
-  __shared__ __attribute__((aligned(16))) _Float16 xs[2 * kXmTok * kXmColStride];
-  __shared__ float inv_s[kXmChunkTiles / 8][2 * kXmTok];
-  __shared__ __attribute__((aligned(16))) float yp[kXmTok * 128];
-  __shared__ __attribute__((aligned(16))) float yq[(kXmKSplit - 1) * kXmTok * 128 + 4];   // the other wavefronts of a tile column
+  extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
+  _Float16* xs = reinterpret_cast<_Float16*>(lds + G::kRingBytes);
+  float* yp = reinterpret_cast<float*>(lds);                      // (after the last tile: the rings are done with)
+  float* yq = yp + kXmTok * 128;                                  // the other wavefronts of a tile column
 
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int grp = blockIdx.x, slice = blockIdx.y, nslices = gridDim.y;
   const int t0 = blockIdx.z * kXmTok;
-  const int ntok = min(kXmTok, m - t0);
+  const int ntok = min(kXmTok, m - t0), cols = 2 * ntok;
   const int nt_n = n_out >> 4, kt_n = n_in >> 4;
   const int kt_begin = slice * slice_tiles;
-  const int kt_end = min(kt_n, kt_begin + slice_tiles);
+  const int groups = (min(kt_n, kt_begin + slice_tiles) - kt_begin) >> 3;        // Hadamard groups of this slice
   const int col = lane & 15, q = lane >> 4;
+  const int xstride = chunk_groups * 128 + kXmColPad;
+  float* inv_s = reinterpret_cast<float*>(xs + cols * xstride);                  // [group of the chunk][column]
+  const int tcol = wave & 7, kpart = wave >> 3;          // tile column, and which k-tiles of every group
 
   XmLane<BITS> ln;
   ln.init(lane);
 
   // The tag of this launch's hand-off words: the workspace's generation count + 1 (read now, needed at the end).
   // accum[0] holds the generation, accum[1] the number of groups that have finished, the words start at accum + 8.
-  uint32_t tag = 0;
-  if (nslices > 1)
-    tag = __hip_atomic_load(reinterpret_cast<const uint32_t*>(accum), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u;
+  // (Without a branch around the load, which would be waited for where the branch ends; a launch that is not sliced reads
+  // any dword.)
+  const uint32_t generation =
+      __hip_atomic_load(nslices > 1 ? reinterpret_cast<const uint32_t*>(accum) : reinterpret_cast<const uint32_t*>(trellis),
+                        __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 
-  // ---- weights: global -> registers, one pass ahead
-  const char* wbase = reinterpret_cast<const char*>(trellis) + (int64_t)grp * 8 * (32 * BITS);
-  const int64_t row_bytes = (int64_t)nt_n * (32 * BITS);
-  uint4 pre[G::kSets];
-  // (a thread whose piece lies past the end of a short pass re-reads the last k-tile: no branch around the load)
-  auto request = [&](int kt_first, int cnt) {
+  // ---- weights: stage s holds this wavefront's tiles of the groups 4s .. 4s+3 of the slice (past its end the last group's again)
+  const int64_t row_bytes = (int64_t)nt_n * G::kTileBytes;
+  const uint8_t* wbase = reinterpret_cast<const uint8_t*>(trellis) + ((int64_t)grp * 8 + tcol) * G::kTileBytes +
+                         (int64_t)(kt_begin + kpart * kXmTilesPerWave) * row_bytes;
+  const uint32_t ring = sm_lds(lds) + (uint32_t)(wave * G::kDepth * G::kSlotBytes);
+  const int stages = (groups + kXmStageGroups - 1) / kXmStageGroups;
+  int64_t src[G::kReq];
+  auto place = [&](int left) {                           // left: groups from the stage's first on
 #pragma unroll
-    for (int i = 0; i < G::kSets; i++) {
-      const int p = tid + i * kXmThreads;
-      const int ktl = p / G::kRunPieces, r = p - ktl * G::kRunPieces;
-      pre[i] = *reinterpret_cast<const uint4*>(wbase + (int64_t)(kt_first + min(ktl, cnt - 1)) * row_bytes + r * 16);
+    for (int r = 0; r < G::kReq; r++) {
+      const int p = min(64 * r + lane, G::kPieces - 1), t = p / (2 * BITS), c = p - t * (2 * BITS);
+      const int gl = min(t / kXmTilesPerWave, left - 1);
+      src[r] = (int64_t)(gl * 8 + t % kXmTilesPerWave) * row_bytes + 16 * c;
     }
   };
-  // piece set i of a pass (the i-th 16 bytes of every thread) into LDS
-  auto stage = [&](int i, int cnt) {
-    const int p = tid + i * kXmThreads;
-    const int ktl = p / G::kRunPieces, r = p - ktl * G::kRunPieces;
-    if (ktl < cnt) {
-      const int nt = r / (2 * BITS), ci = r - nt * (2 * BITS);
-      uint32_t* dst = slab + 1 + (ktl * 8 + nt) * G::kTileStride + 4 * ci;
-      const uint32_t c0 = __builtin_amdgcn_alignbit(pre[i].x, pre[i].x, 16);
-      dst[0] = c0;
-      dst[1] = __builtin_amdgcn_alignbit(pre[i].y, pre[i].y, 16);
-      dst[2] = __builtin_amdgcn_alignbit(pre[i].z, pre[i].z, 16);
-      dst[3] = __builtin_amdgcn_alignbit(pre[i].w, pre[i].w, 16);
-      if (ci == 0) dst[G::kTileDw] = c0;
+  place(groups);
+  int asked = 0, ask_slot = 0;
+  auto request = [&]() {
+    const int left = groups - asked * kXmStageGroups;
+    if (left < kXmStageGroups) place(left);
+    const uint8_t* base = wbase + (int64_t)asked * (kXmStageGroups * 8) * row_bytes;
+    const uint32_t dst = ring + (uint32_t)(ask_slot * G::kSlotBytes);
+#pragma unroll
+    for (int r = 0; r < G::kReq; r++) {
+      const uint8_t* a = base + src[r];
+      // (in assembly: the compiler would wait for all of them before any LDS read that follows)
+      asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(dst + r * 1024), "v"(a) : "memory");
     }
+    asked++;
+    ask_slot = ask_slot == G::kDepth - 1 ? 0 : ask_slot + 1;
   };
 
-  // ---- activations of a pass: (row, group) items of 32 lanes; an item's four values per lane are requested
-  // early (before the weights of the first pass, one pass ahead after that) and rotated when the pass begins
+  // ---- activations of a chunk: (row, group) items of 32 lanes, four values each; the next item's are requested before
+  // one is rotated (and the first one's before the weights')
   const int hw = tid >> 5, l32 = tid & 31;
-  constexpr int kItemsPerThread = (kXmTok * 4 + kXmThreads / 32 - 1) / (kXmThreads / 32);
-  XmRaw<XT> xv[kItemsPerThread];
-  uint2 sv[kItemsPerThread];
-  auto x_request = [&](int kt_first, int ngl) {
-#pragma unroll
-    for (int it = 0; it < kItemsPerThread; it++) {
-      const int item = hw + it * (kXmThreads / 32), t = min(item >> 2, ntok - 1), gl = min(item & 3, ngl - 1);
-      const int64_t k = (int64_t)kt_first * 16 + gl * 128 + 4 * l32;
-      __builtin_memcpy(&sv[it], __builtin_assume_aligned(suh + k, 8), 8);
-      xv[it].load(x + (int64_t)(t0 + t) * n_in + k);
-    }
+  XmRaw<XT> xv;
+  uint2 sv;
+  const uint16_t* sp;
+  const XT* xp;
+  auto x_place = [&](int g0, int ng, int item) {
+    const int it = min(item, ntok * ng - 1), t = ntok == 1 ? 0 : it / ng, gl = it - t * ng;
+    const int64_t k = (int64_t)kt_begin * 16 + (int64_t)(g0 + gl) * 128 + 4 * l32;
+    sp = suh + k;
+    xp = x + (int64_t)(t0 + t) * n_in + k;
   };
-  auto x_stage = [&](int ngl) {
+  auto x_request = [&](int g0, int ng, int item) {
+    x_place(g0, ng, item);
+    __builtin_memcpy(&sv, __builtin_assume_aligned(sp, 8), 8);
+    xv.load(xp);
+  };
+  auto x_stage = [&](int g0, int ng) {
+    for (int item = hw; item < ntok * ng; item += kXmThreads / 32) {
+      const int t = ntok == 1 ? 0 : item / ng, gl = item - t * ng;
+      float v[4];
+      xv.get(v);
+      v[0] *= f16_bits_to_f32((uint16_t)sv.x);
+      v[1] *= f16_bits_to_f32((uint16_t)(sv.x >> 16));
+      v[2] *= f16_bits_to_f32((uint16_t)sv.y);
+      v[3] *= f16_bits_to_f32((uint16_t)(sv.y >> 16));
+      if (item + kXmThreads / 32 < ntok * ng) x_request(g0, ng, item + kXmThreads / 32);
+      fwht128_quad(v, lane);
+      float amax = fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3])));
+      amax = fmaxf(amax, lane_xor<1>(amax, lane));
+      amax = fmaxf(amax, lane_xor<2>(amax, lane));
+      amax = fmaxf(amax, lane_xor<4>(amax, lane));
+      amax = fmaxf(amax, lane_xor<8>(amax, lane));
+      amax = fmaxf(amax, lane_xor<16>(amax, lane));
+      // scale 2^(14 - exponent of amax); all-zero groups get the largest scale, which changes nothing
+      int se = 268 - (int)((__float_as_uint(amax) >> 23) & 0xFF);
+      se = se > 254 ? 254 : se;
+      const float sc = __uint_as_float((uint32_t)se << 23);
+      f16x4_t hi, lo;
 #pragma unroll
-    for (int it = 0; it < kItemsPerThread; it++) {
-      const int item = hw + it * (kXmThreads / 32), t = item >> 2, gl = item & 3;
-      if (item < kXmTok * 4 && t < ntok && gl < ngl) {
-        float v[4];
-        xv[it].get(v);
-        v[0] *= f16_bits_to_f32((uint16_t)sv[it].x);
-        v[1] *= f16_bits_to_f32((uint16_t)(sv[it].x >> 16));
-        v[2] *= f16_bits_to_f32((uint16_t)sv[it].y);
-        v[3] *= f16_bits_to_f32((uint16_t)(sv[it].y >> 16));
-        fwht128_quad(v, lane);
-        float amax = fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3])));
-        amax = fmaxf(amax, lane_xor<1>(amax, lane));
-        amax = fmaxf(amax, lane_xor<2>(amax, lane));
-        amax = fmaxf(amax, lane_xor<4>(amax, lane));
-        amax = fmaxf(amax, lane_xor<8>(amax, lane));
-        amax = fmaxf(amax, lane_xor<16>(amax, lane));
-        // scale 2^(14 - exponent of amax); all-zero groups get the largest scale, which changes nothing
-        int se = 268 - (int)((__float_as_uint(amax) >> 23) & 0xFF);
-        se = se > 254 ? 254 : se;
-        const float sc = __uint_as_float((uint32_t)se << 23);
-        f16x4_t hi, lo;
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-          const float s = v[i] * sc;
-          hi[i] = (_Float16)s;
-          lo[i] = (_Float16)(s - (float)hi[i]);
-        }
-        const int kl = gl * 128 + 4 * l32;
-        *reinterpret_cast<f16x4_t*>(xs + (2 * t) * kXmColStride + kl) = hi;
-        *reinterpret_cast<f16x4_t*>(xs + (2 * t + 1) * kXmColStride + kl) = lo;
-        if (l32 == 0) {
-          // 1/sqrt(128) of the input rotation over the scale
-          const float inv = 0.08838834764831845f * __uint_as_float((uint32_t)(254 - se) << 23);
-          inv_s[gl][2 * t] = inv;
-          inv_s[gl][2 * t + 1] = inv;
-        }
+      for (int i = 0; i < 4; i++) {
+        const float s = v[i] * sc;
+        hi[i] = (_Float16)s;
+        lo[i] = (_Float16)(s - (float)hi[i]);
+      }
+      // (a B operand of 32 k is 16 consecutive bytes: four k of one k-tile, the same four of the next)
+      const int kl = gl * 128 + (l32 >> 3) * 32 + (l32 & 3) * 8 + (l32 >> 2 & 1) * 4;
+      *reinterpret_cast<f16x4_t*>(xs + (2 * t) * xstride + kl) = hi;
+      *reinterpret_cast<f16x4_t*>(xs + (2 * t + 1) * xstride + kl) = lo;
+      if (l32 == 0) {
+        // 1/sqrt(128) of the input rotation over the scale
+        const float inv = 0.08838834764831845f * __uint_as_float((uint32_t)(254 - se) << 23);
+        inv_s[gl * cols + 2 * t] = inv;
+        inv_s[gl * cols + 2 * t + 1] = inv;
       }
     }
   };
 
+  // (half-wavefronts split unevenly over the items: the lanes of one wavefront may leave x_stage's loop at different times, which
+  // lane_xor within 32 lanes does not mind)
   {
-    const int cnt0 = min(kXmChunkTiles, kt_end - kt_begin);
-    x_request(kt_begin, cnt0 >> 3);
-    __builtin_amdgcn_sched_barrier(0);     // the small loads stay in front of the weights: they are waited for first
-    request(kt_begin, cnt0);
+    x_place(0, min(chunk_groups, groups), hw);
+    const uint8_t* first[G::kReq];
+#pragma unroll
+    for (int r = 0; r < G::kReq; r++) first[r] = wbase + src[r];
+    xm_first_loads<G::kReq>(xv, sv, xp, sp, ring, first);
+    asked = ask_slot = 1;
   }
 
   f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
-  for (int kt0 = kt_begin; kt0 < kt_end; kt0 += kXmChunkTiles) {
-    const int cnt = min(kXmChunkTiles, kt_end - kt0);       // a multiple of 8
-    const int ngl = cnt >> 3;
-    if (kt0 != kt_begin) __syncthreads();                   // the previous pass has been read
-    x_stage(ngl);
-    // ---- decode and multiply: this wavefront's tile column and its share of every group's 8 k-tiles (one
-    // Hadamard group per scale); the LDS reads of a group are issued while the group before it is decoded
-    // (decoding a pass's first groups before its last pieces had landed was tried and gained nothing)
-    const _Float16* xcol = xs + col * kXmColStride + 4 * q;
-    const int tcol = wave & 7, kpart = wave >> 3;          // tile column, and which k-tiles of every group
-    const uint32_t* wcol = slab + 1 + (kpart * kXmTilesPerWave * 8 + tcol) * G::kTileStride;
-    const _Float16* xpart = xcol + kpart * kXmTilesPerWave * 16;
-    constexpr int kWin = XmLane<BITS>::kWin;
-    uint32_t cw[2][kXmTilesPerWave][kWin][2];
-    f16x4_t bx[2][kXmTilesPerWave];
-    float inv[2];
-    auto fetch_group = [&](int gl, int buf) {
-#pragma unroll
-      for (int i = 0; i < kXmTilesPerWave; i++) {
-        const int ktl = gl * 8 + i;
-        ln.fetch(wcol + ktl * 8 * G::kTileStride, cw[buf][i]);
-        bx[buf][i] = *reinterpret_cast<const f16x4_t*>(xpart + ktl * 16);
-      }
-      inv[buf] = inv_s[gl][col];
-    };
-    auto compute_group = [&](int buf) {
-      f32x4_t d = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int i = 0; i < kXmTilesPerWave; i++)
-        d = __builtin_amdgcn_mfma_f32_16x16x16f16(ln.template decode<CB>(cw[buf][i]), bx[buf][i], d, 0, 0, 0);
-#pragma unroll
-      for (int r = 0; r < 4; r++) acc[r] = fmaf_(d[r], inv[buf], acc[r]);
-    };
-#pragma unroll
-    for (int i = 0; i < G::kSets; i++) stage(i, cnt);
-    if (kt0 + kXmChunkTiles < kt_end) {
-      const int cnt1 = min(kXmChunkTiles, kt_end - kt0 - kXmChunkTiles);
-      x_request(kt0 + kXmChunkTiles, cnt1 >> 3);
-      __builtin_amdgcn_sched_barrier(0);
-      request(kt0 + kXmChunkTiles, cnt1);
+  const int xcol = col < cols ? col : 0;                 // (columns past the last row's: their sums are not looked at)
+  int slot = 0, done = 0;
+  for (int g0 = 0; g0 < groups; g0 += chunk_groups) {    // a chunk is a whole number of stages, or the slice
+    const int ng = min(chunk_groups, groups - g0);
+    if (g0 > 0) {
+      sm_barrier();                                      // the chunk before has been read
+      x_request(g0, ng, hw);
     }
-    __syncthreads();
-    fetch_group(0, 0);
-    for (int gl = 0; gl < ngl; gl += 2) {
-      if (gl + 1 < ngl) fetch_group(gl + 1, 1);
-      compute_group(0);
-      if (gl + 1 < ngl) {
-        if (gl + 2 < ngl) fetch_group(gl + 2, 0);
-        compute_group(1);
+    x_stage(g0, ng);
+    while (asked < min(stages, done + G::kDepth)) request();
+    sm_barrier();
+    // LDS addresses in registers, so that the reads of a stage differ in their constant offsets only
+    uint32_t xa = sm_lds(xs + xcol * xstride + kpart * kXmTilesPerWave * 16 + 8 * q), ia = sm_lds(inv_s + xcol);
+    for (int left = ng; left > 0; left -= kXmStageGroups) {
+      // requests complete in order: all but those of the stages after this one have landed
+      switch (asked - done - 1) {
+        case 0: sm_wait_vmcnt<0>(); break;
+        case 1: sm_wait_vmcnt<G::kReq>(); break;
+        default: sm_wait_vmcnt<2 * G::kReq>(); break;
       }
+      constexpr int kWin = XmLane<BITS>::kWin;
+      uint32_t cw[2][kXmTilesPerWave][kWin][2];
+      f16x8_t bx[2][kXmTilesPerWave / 2];
+      float inv[2];
+      uint32_t wa[kWin][2];
+#pragma unroll
+      for (int w = 0; w < kWin; w++)
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+          wa[w][h] = ring + (uint32_t)(slot * G::kSlotBytes) + ln.at[w][h];
+          asm("" : "+v"(wa[w][h]));
+        }
+      asm("" : "+v"(xa), "+v"(ia));
+      auto fetch_group = [&](int gl, int buf) {
+#pragma unroll
+        for (int i = 0; i < kXmTilesPerWave; i++) {
+#pragma unroll
+          for (int w = 0; w < kWin; w++)
+#pragma unroll
+            for (int h = 0; h < 2; h++)
+              cw[buf][i][w][h] = lds_at<uint32_t>(wa[w][h] + (gl * kXmTilesPerWave + i) * G::kTileBytes);
+          if (i % 2 == 0) bx[buf][i / 2] = lds_at<f16x8_t>(xa + (gl * 128 + i * 16) * 2);
+        }
+        inv[buf] = lds_at<float>(ia + gl * 4 * cols);
+      };
+      auto compute_group = [&](int buf) {
+        f32x4_t d = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < kXmTilesPerWave; i += 2) {
+          uint32_t r[4];
+          ln.template decode<CB>(cw[buf][i], reinterpret_cast<uint32_t(&)[2]>(r[0]));
+          ln.template decode<CB>(cw[buf][i + 1], reinterpret_cast<uint32_t(&)[2]>(r[2]));
+          f16x8_t a;
+          __builtin_memcpy(&a, r, 16);
+          d = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, bx[buf][i / 2], d, 0, 0, 0);
+        }
+#pragma unroll
+        for (int r = 0; r < 4; r++) acc[r] = fmaf_(d[r], inv[buf], acc[r]);
+      };
+      // the LDS reads of a group are issued while the group before it is decoded
+      fetch_group(0, 0);
+#pragma unroll
+      for (int gl = 0; gl < kXmStageGroups; gl++) {
+        if (gl < left) {
+          if (gl + 1 < kXmStageGroups && gl + 1 < left) fetch_group(gl + 1, (gl + 1) & 1);
+          compute_group(gl & 1);
+        }
+      }
+      // (the slot is free for a later stage: its reads have returned)
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      done++;
+      slot = slot == G::kDepth - 1 ? 0 : slot + 1;
+      if (asked < stages) request();
+      xa += kXmStageGroups * 256;
+      ia += kXmStageGroups * 4 * cols;
     }
   }
-
   // ---- the two terms of each row.  Then, in a sliced launch, every slice but the last hands its sums
   // to the last one straight from the registers, through tagged 64-bit words (the launch's tag in the high
   // half, the float in the low half) written and read with agent-scope accesses, which are coherent across
@@ -224,9 +328,9 @@ gemv_exl3_mfma_kernel(const uint16_t* __restrict__ trellis, const uint16_t* __re
   // will; that takes a wavefront dispatch held back for poll_limit polls (tens of milliseconds by default).
 #pragma unroll
   for (int r = 0; r < 4; r++) acc[r] += lane_xor<1>(acc[r], lane);
-  const int tcol = wave & 7, kpart = wave >> 3;
   const bool owner = (col & 1) == 0 && (col >> 1) < ntok;      // this lane holds 4 channel sums of row col / 2
   constexpr int kPartWords = kXmTok * 128;                        // words per (slice, k part)
+  const uint32_t tag = generation + 1u;
   unsigned long long* words = nullptr;
   if (nslices > 1) {
     words = accum + 8 + (((int64_t)blockIdx.z * gridDim.x + grp) * nslices) * (kXmKSplit * kPartWords);
@@ -241,50 +345,73 @@ gemv_exl3_mfma_kernel(const uint16_t* __restrict__ trellis, const uint16_t* __re
       return;
     }
   }
+  sm_barrier();                                          // all tiles have been read: the rings' place is free
   {
     float* dst = kpart == 0 ? yp : yq + (kpart - 1) * kPartWords;
     if (owner) *reinterpret_cast<float4*>(dst + (col >> 1) * 128 + tcol * 16 + 4 * q) = make_float4(acc[0], acc[1], acc[2], acc[3]);
   }
   __syncthreads();
-  constexpr int kHandoffBatch = 16;
-  for (int e = tid; e < ntok * 128; e += kXmThreads) {
-    // the other slices' words for this output (sixteen loads in flight before the first is looked at: the fourteen
-    // words of a launch in eight slices in one round trip to the memory side),
-    // then this workgroup's own sums
-    float s = 0.f;
-    bool late = false;
-    const int nparts = (nslices - 1) * kXmKSplit;
+  // The other slices' words, sixteen loads in flight before the first is looked at, and dealt out over several threads to a sum
+  // where there are more: a round trip to the memory side is most of what this costs, and with one thread to a sum the 62
+  // words of 32 slices took four of them (1024 x 4096, one row: 8.95 -> 7.4 us).  Sixteen words are a batch, batch b is
+  // added to part b % 8, the parts to each other: the same order for any number of rows.
+  constexpr int kHandoffBatch = 16, kHandoffParts = 8;
+  float* red = yq + (kXmKSplit - 1) * kPartWords;              // [part][sum]
+  const int nwords = (nslices - 1) * kXmKSplit, sums = ntok * 128;
+  const int batches = (nwords + kHandoffBatch - 1) / kHandoffBatch, parts = min(batches, kHandoffParts);
+  int deal = 1;                                                // threads to a sum (scalar shifts and compares: an integer division here is 0.4 us)
+  while (deal < parts && sums * deal * 2 <= kXmThreads) deal *= 2;
+  float handed = 0.f;
+  if (nwords > 0) {
     // The slices of a group finish their decode within a fraction of a microsecond of each other, and a word asked for
     // before it has reached the memory side costs a second round trip (about 0.9 us); 256 clocks of patience before
-    // the first look make the first look the only one (4096 x 4096, one row: 9.1 -> 8.8 us; two to six units of 64
-    // clocks measure the same).
-    if (nparts > 0) __builtin_amdgcn_s_sleep(4);
-    for (int p0 = 0; p0 < nparts; p0 += kHandoffBatch) {
-      unsigned long long w[kHandoffBatch];
+    // the first look make the first look the only one (one to six units of 64 clocks measure the same).
+    __builtin_amdgcn_s_sleep(4);
+    int d = 0;
+    for (int r = wave >> 1; r >= ntok; r -= ntok) d++;
+    const int e = tid - d * sums;
+    if (d < deal) {
+      for (int part = d; part < parts; part += deal) {
+        float c = 0.f;
+        bool late = false;
+        for (int b = part; b < batches; b += kHandoffParts) {
+          const int p0 = b * kHandoffBatch;
+          unsigned long long w[kHandoffBatch];
 #pragma unroll
-      for (int i = 0; i < kHandoffBatch; i++)
-        w[i] = __hip_atomic_load(words + (int64_t)min(p0 + i, nparts - 1) * kPartWords + e, __ATOMIC_RELAXED,
-                                 __HIP_MEMORY_SCOPE_AGENT);
+          for (int i = 0; i < kHandoffBatch; i++)
+            w[i] = __hip_atomic_load(words + (int64_t)min(p0 + i, nwords - 1) * kPartWords + e, __ATOMIC_RELAXED,
+                                     __HIP_MEMORY_SCOPE_AGENT);
 #pragma unroll
-      for (int i = 0; i < kHandoffBatch; i++) {
-        if (p0 + i < nparts) {
-          unsigned long long* wp = words + (int64_t)(p0 + i) * kPartWords + e;
-          for (int polls = 0; (uint32_t)(w[i] >> 32) != tag && polls < poll_limit; polls++) {
-            __builtin_amdgcn_s_sleep(2);
-            w[i] = __hip_atomic_load(wp, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          for (int i = 0; i < kHandoffBatch; i++) {
+            if (p0 + i < nwords) {
+              unsigned long long* wp = words + (int64_t)(p0 + i) * kPartWords + e;
+              for (int polls = 0; (uint32_t)(w[i] >> 32) != tag && polls < poll_limit; polls++) {
+                __builtin_amdgcn_s_sleep(2);
+                w[i] = __hip_atomic_load(wp, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+              }
+              late |= (uint32_t)(w[i] >> 32) != tag;
+              c += __uint_as_float((uint32_t)w[i]);
+            }
           }
-          late |= (uint32_t)(w[i] >> 32) != tag;
-          s += __uint_as_float((uint32_t)w[i]);
         }
+        if (late) c = __uint_as_float(0x7FC00000u);
+        if (deal > 1) red[part * sums + e] = c;
+        else handed += c;
       }
     }
-    s += yp[e];
-#pragma unroll
-    for (int k = 1; k < kXmKSplit; k++) s += yq[(k - 1) * kPartWords + e];
-    yp[e] = late ? __uint_as_float(0x7FC00000u) : s;
+    if (deal > 1) __syncthreads();
   }
-  // Thread 0 has now seen (or given up on) a word of every other slice of its group, so each of them has read
-  // the generation count.  It counts its group in here and looks at the answer after the output phase: the group
+  if (tid < sums) {
+    if (deal > 1)
+      for (int part = 0; part < parts; part++) handed += red[part * sums + tid];
+    float s = handed;
+    s += yp[tid];
+#pragma unroll
+    for (int k = 1; k < kXmKSplit; k++) s += yq[(k - 1) * kPartWords + tid];
+    yp[tid] = s;
+  }
+  // The workgroup has now seen (or given up on) a word of every other slice of its group, so each of them has read
+  // the generation count.  Thread 0 counts its group in here and looks at the answer after the output phase: the group
   // that is counted last advances the generation.
   uint32_t counted = 0;
   if (nslices > 1 && tid == 0)
@@ -346,9 +473,21 @@ static hipError_t xm_launch(const Exl3Plan& p, const uint16_t* trellis, const ui
                             const void* x, void* y, int y_dtype, const void* bias, int bias_dtype, int64_t m,
                             int64_t n_out, int64_t n_in, unsigned long long* accum, hipStream_t s) {
   const dim3 grid((unsigned)p.groups, (unsigned)p.slices, (unsigned)p.row_groups), block(kXmThreads);
-  hipLaunchKernelGGL((gemv_exl3_mfma_kernel<BITS, CB, XT>), grid, block, 0, s, trellis, suh, svh,
+  // activations in LDS: the whole slice, or as many whole stages of the ring as fit
+  const int cols = 2 * (int)(m < kXmTok ? m : kXmTok), room = kXmLds - XmGeom<BITS>::kRingBytes;
+  int chunk = p.slice_tiles / 8;
+  if (xm_x_bytes(cols, chunk) > room) {
+    chunk = (room - xm_x_bytes(cols, 0)) / (xm_x_bytes(cols, 1) - xm_x_bytes(cols, 0));
+    chunk = chunk / kXmStageGroups * kXmStageGroups;
+  }
+  const size_t lds = (size_t)XmGeom<BITS>::kRingBytes + xm_x_bytes(cols, chunk);
+  auto kernel = gemv_exl3_mfma_kernel<BITS, CB, XT>;
+  static LargeLds configured;
+  const hipError_t e = allow_large_lds(reinterpret_cast<const void*>(kernel), configured);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(kernel, grid, block, lds, s, trellis, suh, svh,
                      static_cast<const XT*>(x), y, y_dtype, bias, bias_dtype, (int)m, (int)n_out, (int)n_in, p.slice_tiles,
-                     accum, g_exl3_poll_limit.load(std::memory_order_relaxed));
+                     chunk, accum, g_exl3_poll_limit.load(std::memory_order_relaxed));
   return hipGetLastError();
 }
 

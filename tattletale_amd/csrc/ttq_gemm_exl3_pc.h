@@ -11,9 +11,8 @@
 //       the matrix cores, one does not).  Wavefront p decodes k-tile 4 s + p % 4 of step s for four of the tile's
 //       eight column blocks.  The 4 x 32 x bits bytes of those tiles are consecutive in trellis[k_tile][n_tile]; they
 //       come by LDS DMA into a ring of eight steps private to the wavefront (3 us ahead of their use, no registers
-//       held), a lane reads the two dwords that hold its four windows, swaps their halves (MSB-first 16-bit words -> a
-//       big-endian bit string), decodes four weights as in the decode GEMV (XmLane) and stores them as half of a B
-//       fragment unit.  A decoded tile thus serves every row of the tile (64 * MB) instead of 64.  (Tiles of 256 rows:
+//       held), a lane reads the two dwords that hold its four windows, decodes four weights as in the decode GEMV (XmLane) and
+//       stores them as half of a B fragment unit.  A decoded tile thus serves every row of the tile (64 * MB) instead of 64.  (Tiles of 256 rows:
 //       four producers with eight column blocks each, see xg_producers.)
 //   epilogue: after the copies of a launch split along K have met, a consumer rotates the 128 sums of each of its
 //       rows in registers (butterflies over the column blocks in place, over the columns of a block by DPP moves),
@@ -92,14 +91,6 @@ gemm_exl3_pc_kernel(const uint8_t* __restrict__ trellis, const uint16_t* __restr
     XmLane<BITS> ln;
     ln.init(lane);
     constexpr int kWin = XmLane<BITS>::kWin;
-    constexpr int kTileDw = 8 * BITS;
-    // byte offsets, inside a tile, of the two dwords of each window (the bit string of a tile is cyclic)
-    uint32_t woff[kWin][2];
-#pragma unroll
-    for (int w = 0; w < kWin; w++) {
-      woff[w][0] = (uint32_t)(((ln.dw[w] + kTileDw) % kTileDw) * 4);
-      woff[w][1] = (uint32_t)(((ln.dw[w] + 1) % kTileDw) * 4);
-    }
     const int nt_n = n_out >> 4;
     const int64_t kt_bytes = (int64_t)nt_n * (32 * BITS);             // one k-tile of the whole matrix
     const uint8_t* run0 = trellis + (int64_t)((n0 >> 4) + nt0) * (32 * BITS);  // this wavefront's column blocks, k-tile 0
@@ -131,7 +122,7 @@ gemm_exl3_pc_kernel(const uint8_t* __restrict__ trellis, const uint16_t* __restr
       for (int t = 0; t < 4; t++)
 #pragma unroll
         for (int w = 0; w < kWin; w++) {
-          const uint32_t a0 = slot + woff[w][0], a1 = slot + woff[w][1];
+          const uint32_t a0 = slot + ln.at[w][0], a1 = slot + ln.at[w][1];
           asm volatile("ds_read_b32 %0, %2 offset:%4\n\tds_read_b32 %1, %3 offset:%4"
                        : "=&v"(r.v[t][w][0]), "=&v"(r.v[t][w][1])
                        : "v"(a0), "v"(a1), "n"((NT0 + t) * 32 * BITS)
@@ -159,15 +150,9 @@ gemm_exl3_pc_kernel(const uint8_t* __restrict__ trellis, const uint16_t* __restr
       constexpr int NT0 = decltype(ntc)::value;
 #pragma unroll
       for (int t = 0; t < 4; t++) {
-        uint32_t c[kWin][2];
-#pragma unroll
-        for (int w = 0; w < kWin; w++) {
-          c[w][0] = __builtin_amdgcn_alignbit(r.v[t][w][0], r.v[t][w][0], 16);
-          c[w][1] = __builtin_amdgcn_alignbit(r.v[t][w][1], r.v[t][w][1], 16);
-        }
-        const f16x4_t v = ln.template decode<CB>(c);
-        uint64_t bits64;
-        __builtin_memcpy(&bits64, &v, 8);
+        uint32_t v[2];
+        ln.template decode<CB>(r.v[t], v);
+        const uint64_t bits64 = (uint64_t)v[1] << 32 | v[0];
         asm volatile("ds_write_b64 %0, %1 offset:%2" : : "v"(dst), "v"(bits64), "n"((NT0 + t) * 1024) : "memory");
       }
     };

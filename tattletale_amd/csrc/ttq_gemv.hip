@@ -488,7 +488,7 @@ hipError_t launch_gemv(int format, const void* w, const void* x, int x_dtype, vo
   }
   // Q6_K, more rows than a pass of the integer kernel takes: in fp16 the form for many rows (64 to a launch), else passes
   const int64_t per_pass = gemv_tile_rows(x_dtype);
-  if (m > per_pass && gemv_tile_preferred(format, x_dtype, per_pass, n_out, n_in)) {
+  if (format == kQ6_K && m > per_pass && gemv_tile_preferred(format, x_dtype, per_pass, n_out, n_in)) {
     const bool rows = rows_exact_preferred(x_dtype, m, n_out, n_in);
     if (route_probe(rows ? kRouteGemmRowsExact : kRouteGemvTile)) return hipSuccess;
     const int64_t step = rows ? 64 : per_pass, xsize = x_dtype == kF32 ? 4 : 2, ysize = y_dtype == kF32 ? 4 : 2;
@@ -503,7 +503,7 @@ hipError_t launch_gemv(int format, const void* w, const void* x, int x_dtype, vo
     }
     return hipSuccess;
   }
-  if (gemv_tile_preferred(format, x_dtype, m, n_out, n_in))
+  if (format == kQ6_K && gemv_tile_preferred(format, x_dtype, m, n_out, n_in))
     TTQ_ROUTE(kRouteGemvTile, launch_gemv_tile(format, w, x, x_dtype, y, y_dtype, bias, bias_dtype, m, n_out, n_in, s));
   // a few rows at once: four per pass for up to four rows and for rows too long for the 8- and
   // 16-token tables, else eight or sixteen per pass

@@ -370,12 +370,12 @@ bool gemv_tile_supported(int format, int x_dtype, int64_t m, int64_t n_out, int6
 //     int8 stream computes, to 2e-6, and up to 100 MB, where a second pass costs little, that agreement is kept.
 bool gemv_tile_preferred(int format, int x_dtype, int64_t m, int64_t n_out, int64_t n_in) {
   static const int always = dev_knob("TTQ_TILE_FIRST", 0);
+  const float mb = (float)(n_out * (n_in >> 8) * 210) * 1e-6f;
+  if (format != kQ6_K || (mb < 5.f && !always)) return false;      // (first: small calls are where the host's time counts)
   if (!gemv_tile_supported(format, x_dtype, m, n_out, n_in)) return false;
   if (always) return true;
-  const float mb = (float)(n_out * (n_in >> 8) * 210) * 1e-6f;
   if (x_dtype == kF32) return mb >= (m == 1 ? 7.f : 5.f);
   if (m == 1) return !gemv_q6k_stream_supported(format, x_dtype, n_out, n_in) && mb >= (n_in > 4096 ? 12.f : 27.f);
-  if (mb < 5.f) return false;
   return !gemv_q6k_stream4_supported(format, x_dtype, m, n_out, n_in) || (m > 4 && mb >= 100.f);
 }
 

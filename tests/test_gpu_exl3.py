@@ -121,6 +121,27 @@ def test_exl3_rows_beyond_16384_values(n_out, n_in, m):
         assert np.array_equal(yd.cpu().numpy(), y)
 
 
+@pytest.mark.parametrize("bits,n_out,n_in,m", [
+    (3, 256, 4096 + 128, 8), (1, 128, 20 * 1024, 3),           # more slices than one batch of hand-off words
+    (8, 4096, 13 * 128, 62), (5, 2048, 17 * 128, 128),         # whole slices whose activations take several chunks of LDS
+    (7, 33024, 3 * 128, 1),                                    # whole slices that are not a whole stage of the rings
+])
+def test_exl3_gemv_rings_and_hand_off(bits, n_out, n_in, m):
+    """The stages of a wavefront's ring, the chunks of activations, the batches of hand-off words; every row is the same bits
+    as on its own as long as the launch is divided alike (up to eight rows)."""
+    rng = np.random.default_rng(bits)
+    tr = rng.integers(0, 65536, (n_in // 16, n_out // 16, 16 * bits), dtype=np.uint16)
+    suh, svh = (Q.f32_to_f16(rng.choice([-1.0, 1.0], n).astype(np.float32)) for n in (n_in, n_out))
+    T = oracle.exl3_decode(tr, n_out, n_in, bits, F.CB_MCG)
+    x = Q.f32_to_f16(Q.fill_normal(630, 1, 1.0, m * n_in).reshape(m, n_in))
+    dev = [packed_to_dev(tr)] + [bits_to_dev(v, "f16") for v in (suh, svh, x)]
+    y = QL.gemv_exl3(*dev, n_out, n_in, bits, F.CB_MCG)
+    for i in sorted({0, m // 2, m - 1}):
+        assert rel_l2(y[i].cpu().numpy(), oracle.exl3_gemv_f64(T, suh, svh, x[i])) <= TOL
+        if m <= 8:
+            assert torch.equal(QL.gemv_exl3(*dev[:3], dev[3][i:i + 1], n_out, n_in, bits, F.CB_MCG)[0], y[i])
+
+
 def test_exl3_many_rows_take_whole_slices():
     """Enough (output group, row group) units to fill the GPU: no slicing, eight LDS passes per workgroup."""
     n_out, n_in, bits, m = 1024, 4096, 2, 8 * 33 + 5
