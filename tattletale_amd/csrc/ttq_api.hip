@@ -450,14 +450,21 @@ int ttq_linear_forward(const ttq_qlinear* layer, const void* x, int x_dtype, int
   // kernels of fixed-point or packed-dot arithmetic; faster kernels of either kind since then (the streamed few-row form, the
   // integer kernels) compete inside of it, and a call that decodes exactly is not moved to rounded weights by them.
   const auto few_us = [&](int64_t rows) { return ttq::gemm_skinny_registers_estimate_us(layer->format, rows, n_out, n_in); };
+  // (asked first whether any of them takes the shape: small calls wait for the host, and the estimates twice are 0.8 us)
+  const bool streamed = m >= 2 && (layer->format == TTQ_Q4_K || layer->format == TTQ_Q6_K) &&
+                        (ttq::gemm_rows_preferred(n_out) || few_us(m < 64 ? m : 64) > 1e29f);
+  const bool newer = streamed || (layer->format == TTQ_Q6_K && (int64_t)n_out * n_in >= 6000000);
   if (gemm_ok && m >= 5 && route != 1) {
-    float us_rounding = m <= 64 ? few_us(m) : 1e30f;
-    if (us_rounding < 1e29f || layer->format == TTQ_Q4_K || ttq::gemm_pc_supported(layer->format, m, n_out, n_in, 112)) {
-      const float us = ttq::gemm_pc_estimate_us(layer->format, m, n_out, n_in);
-      us_rounding = us < us_rounding ? us : us_rounding;
+    float us_rounding = 0.f;
+    if (newer) {
+      us_rounding = m <= 64 ? few_us(m) : 1e30f;
+      if (us_rounding < 1e29f || layer->format == TTQ_Q4_K || ttq::gemm_pc_supported(layer->format, m, n_out, n_in, 112)) {
+        const float us = ttq::gemm_pc_estimate_us(layer->format, m, n_out, n_in);
+        us_rounding = us < us_rounding ? us : us_rounding;
+      }
     }
     if (route == 2 ||
-        (us_rounding < ttq::gemv_estimate_us(layer->format, x_dtype, m, n_out, n_in, false) &&
+        ((!newer || us_rounding < ttq::gemv_estimate_us(layer->format, x_dtype, m, n_out, n_in, false)) &&
          ttq::gemm_estimate_us(layer->format, m, n_out, n_in) < ttq::gemv_estimate_us(layer->format, x_dtype, m, n_out, n_in)))
       return hip_status(ttq::launch_gemm(layer->format, layer->qweight, static_cast<const uint16_t*>(x), y, y_dtype,
                                          layer->bias, layer->bias_dtype, m, n_out, n_in, s));
@@ -473,12 +480,12 @@ int ttq_linear_forward(const ttq_qlinear* layer, const void* x, int x_dtype, int
       const int64_t full = m / 64, rest = m % 64;
       us_few = (float)full * ttq::gemm_skinny_estimate_us(layer->format, 64, n_out, n_in);
       if (rest) us_few += ttq::gemm_skinny_estimate_us(layer->format, rest, n_out, n_in);
-      us_rounding = (full ? (float)full * few_us(64) : 0.f) + (rest ? few_us(rest) : 0.f);
+      if (newer) us_rounding = (full ? (float)full * few_us(64) : 0.f) + (rest ? few_us(rest) : 0.f);
     }
     if (m > 64 && ttq::gemm_pc_supported(layer->format, m < 8192 ? m : 8192, n_out, n_in, 112))
       us_gemm = ttq::gemm_pc_estimate_us(layer->format, m, n_out, n_in) + 2.5f + (float)(m * n_in * 4) / 3.0e6f;
     us_rounding = us_gemm < us_rounding ? us_gemm : us_rounding;
-    const bool rounds = route == 2 || us_rounding < ttq::gemv_estimate_us(layer->format, x_dtype, m, n_out, n_in, false);
+    const bool rounds = route == 2 || !newer || us_rounding < ttq::gemv_estimate_us(layer->format, x_dtype, m, n_out, n_in, false);
     const float us_gemv = ttq::gemv_estimate_us(layer->format, x_dtype, m, n_out, n_in);
     // (several launches of the few-row kernel against one short round of the tiled kernel: the margin of the bf16
     // chooser, whose estimate for the tiled kernel is fitted to full rounds and about a third too high for a short one)
@@ -518,12 +525,12 @@ int ttq_linear_forward(const ttq_qlinear* layer, const void* x, int x_dtype, int
       const int64_t full = m / 64, rest = m % 64;
       us_few = (float)full * ttq::gemm_skinny_estimate_us(layer->format, 64, n_out, n_in) + 2.5f + (float)n_in * 0.13e-3f;
       if (rest) us_few += ttq::gemm_skinny_estimate_us(layer->format, rest, n_out, n_in);
-      us_rounding = (full ? (float)full * few_us(64) : 0.f) + (rest ? few_us(rest) : 0.f) + 2.5f + (float)n_in * 0.13e-3f;
+      if (newer) us_rounding = (full ? (float)full * few_us(64) : 0.f) + (rest ? few_us(rest) : 0.f) + 2.5f + (float)n_in * 0.13e-3f;
     }
     if (m >= 5 && ttq::gemm_pc_supported(layer->format, m < 8192 ? m : 8192, n_out, n_in, 112))
       us_gemm = ttq::gemm_pc_estimate_us(layer->format, m, n_out, n_in) + 5.f + (float)(m * n_in * 10) / 3.0e6f;
     us_rounding = us_gemm < us_rounding ? us_gemm : us_rounding;
-    const bool rounds = route == 2 || us_rounding < ttq::gemv_estimate_us(layer->format, x_dtype, m, n_out, n_in, false);
+    const bool rounds = route == 2 || !newer || us_rounding < ttq::gemv_estimate_us(layer->format, x_dtype, m, n_out, n_in, false);
     // (the integer kernel takes two rows of Q6_K to a pass: us of it / of the few-row kernel 14336 x 4096 19.3 / 22.5, 28672 x 4096
     // 27.0 / 30.5, 43008 x 4096 38.3 / 38.9, 128256 x 4096 88 / 91 -- and of four rows 34 / 22, 49 / 30, 68 / 38, 160 / 91.  The small
     // matrices, where the two agree to 3 us, stay with the kernel that takes any number of rows.)
