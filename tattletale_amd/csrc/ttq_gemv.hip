@@ -490,7 +490,7 @@ hipError_t launch_gemv(int format, const void* w, const void* x, int x_dtype, vo
   const int64_t per_pass = gemv_tile_rows(x_dtype);
   if (format == kQ6_K && m > per_pass && gemv_tile_preferred(format, x_dtype, per_pass, n_out, n_in)) {
     const bool rows = rows_exact_preferred(x_dtype, m, n_out, n_in);
-    if (route_probe(rows ? kRouteGemmRowsExact : kRouteGemvTile)) return hipSuccess;
+    if (rows && route_probe(kRouteGemmRowsExact)) return hipSuccess;
     const int64_t step = rows ? 64 : per_pass, xsize = x_dtype == kF32 ? 4 : 2, ysize = y_dtype == kF32 ? 4 : 2;
     for (int64_t r = 0; r < m; r += step) {
       const int64_t n = m - r < step ? m - r : step;
@@ -499,12 +499,12 @@ hipError_t launch_gemv(int format, const void* w, const void* x, int x_dtype, vo
       const hipError_t e = rows && n > per_pass
           ? launch_gemm_rows_exact(w, static_cast<const uint16_t*>(xr), yr, y_dtype, bias, bias_dtype, n, n_out, n_in, s)
           : launch_gemv_tile(format, w, xr, x_dtype, yr, y_dtype, bias, bias_dtype, n, n_out, n_in, s);
-      if (e != hipSuccess) return e;
+      if (e != hipSuccess || t_route_probe) return e;
     }
     return hipSuccess;
   }
   if (format == kQ6_K && gemv_tile_preferred(format, x_dtype, m, n_out, n_in))
-    TTQ_ROUTE(kRouteGemvTile, launch_gemv_tile(format, w, x, x_dtype, y, y_dtype, bias, bias_dtype, m, n_out, n_in, s));
+    return launch_gemv_tile(format, w, x, x_dtype, y, y_dtype, bias, bias_dtype, m, n_out, n_in, s);
   // a few rows at once: four per pass for up to four rows and for rows too long for the 8- and
   // 16-token tables, else eight or sixteen per pass
   if (gemv_q4k_stream4_supported(format, x_dtype, m, n_out, n_in))

@@ -319,6 +319,8 @@ template <class F, class XT, int J, int KQ, int PARTS = 1>
 hipError_t launch_tile_j(const TlArgs& a, hipStream_t s) {
   constexpr int depth = kTlDepth;
   const size_t lds = tile_lds_bytes<F>(J, KQ, a.n_in, depth);
+  if (lds > kTlLds) return hipErrorInvalidValue;
+  if (route_probe(kRouteGemvTile)) return hipSuccess;      // (here, so that the query answers for the form that would run)
   auto kernel = gemv_tile_kernel<F, XT, J, KQ, PARTS>;
   static LargeLds configured;
   if (lds > 64 * 1024) {
@@ -331,15 +333,22 @@ hipError_t launch_tile_j(const TlArgs& a, hipStream_t s) {
   return hipGetLastError();
 }
 
-// One row: four blocks to a tile, except where the last tile of long matrices' rows would be half empty (32003 x 2560 21.3 us
-// with four, 17.9 with two; 7168 x 3584 9.7 / 9.9).
-bool tile_wide(int64_t n_out, int64_t n_in) { return (n_in >> 8) % 4 == 0 || n_out * (n_in >> 8) * 210 < (24 << 20); }
+// The form of a call: activation rows as the matrix cores see them, blocks along K of a tile.
+struct TlForm { int j, kq; };
+TlForm tile_form(int x_dtype, int64_t m, int64_t n_out, int64_t n_in) {
+  if (x_dtype == kF32) return m == 1 ? TlForm{3, 2} : TlForm{6, 1};
+  if (m > 1) return m == 2 ? TlForm{2, 2} : TlForm{m <= 4 ? 4 : 8, 1};
+  // One row: four blocks to a tile, except where the last tile of long matrices' rows would be half empty (32003 x 2560 21.3 us
+  // with four, 17.9 with two; 7168 x 3584 9.7 / 9.9).  Two take more LDS, and end at rows of 41216 values.
+  const bool wide = (n_in >> 8) % 4 == 0 || n_out * (n_in >> 8) * 210 < (24 << 20);
+  return TlForm{1, wide || tile_lds_bytes<TlQ6K>(1, 2, n_in, kTlDepth) > kTlLds ? 4 : 2};
+}
 
 template <class F, class XT>
-hipError_t launch_tile_x(const TlArgs& a, hipStream_t s) {
-  if (a.m == 1) return tile_wide(a.n_out, a.n_in) ? launch_tile_j<F, XT, 1, 4>(a, s) : launch_tile_j<F, XT, 1, 2>(a, s);
-  if (a.m == 2) return launch_tile_j<F, XT, 2, 2>(a, s);
-  if (a.m <= 4) return launch_tile_j<F, XT, 4, 1>(a, s);
+hipError_t launch_tile_x(const TlArgs& a, const TlForm& f, hipStream_t s) {
+  if (f.j == 1) return f.kq == 4 ? launch_tile_j<F, XT, 1, 4>(a, s) : launch_tile_j<F, XT, 1, 2>(a, s);
+  if (f.j == 2) return launch_tile_j<F, XT, 2, 2>(a, s);
+  if (f.j == 4) return launch_tile_j<F, XT, 4, 1>(a, s);
   return launch_tile_j<F, XT, 8, 1>(a, s);
 }
 
@@ -351,10 +360,9 @@ int gemv_tile_rows(int x_dtype) { return x_dtype == kF32 ? 2 : 8; }
 bool gemv_tile_supported(int format, int x_dtype, int64_t m, int64_t n_out, int64_t n_in) {
   static const int disabled = dev_knob("TTQ_NO_TILE", 0);
   if (disabled || format != kQ6_K || n_in % 256 != 0 || m < 1 || m > 8 || n_out > 0x3FFFFFFF || n_in > (1 << 22)) return false;
-  const bool f32 = x_dtype == kF32;
   if (m > gemv_tile_rows(x_dtype)) return false;
-  const int j = f32 ? 3 * (int)m : (m <= 2 ? (int)m : (m <= 4 ? 4 : 8)), kq = f32 ? (m == 1 ? 2 : 1) : (m == 1 ? 4 : (m == 2 ? 2 : 1));
-  return tile_lds_bytes<TlQ6K>(j, kq, n_in, kTlDepth) <= kTlLds;
+  const TlForm f = tile_form(x_dtype, m, n_out, n_in);
+  return tile_lds_bytes<TlQ6K>(f.j, f.kq, n_in, kTlDepth) <= kTlLds;
 }
 
 // Whether it is the faster one among the decode kernels.  Startup (the activations' sums, a barrier, one tile's chain) is some
@@ -391,9 +399,10 @@ hipError_t launch_gemv_tile(int format, const void* w, const void* x, int x_dtyp
   if (m == 0 || n_out == 0) return hipSuccess;
   if (format != kQ6_K) return hipErrorInvalidValue;
   const TlArgs a{static_cast<const uint8_t*>(w), x, y, bias, (int)m, (int)n_out, (int)n_in, x_dtype, y_dtype, bias_dtype};
-  if (x_dtype == kF32) return m == 1 ? launch_tile_j<TlQ6K, bf16_tag, 3, 2, 3>(a, s) : launch_tile_j<TlQ6K, bf16_tag, 6, 1, 3>(a, s);
-  if (x_dtype == kF16) return launch_tile_x<TlQ6K, f16_tag>(a, s);
-  return launch_tile_x<TlQ6K, bf16_tag>(a, s);
+  const TlForm f = tile_form(x_dtype, m, n_out, n_in);
+  if (x_dtype == kF32) return f.j == 3 ? launch_tile_j<TlQ6K, bf16_tag, 3, 2, 3>(a, s) : launch_tile_j<TlQ6K, bf16_tag, 6, 1, 3>(a, s);
+  if (x_dtype == kF16) return launch_tile_x<TlQ6K, f16_tag>(a, f, s);
+  return launch_tile_x<TlQ6K, bf16_tag>(a, f, s);
 }
 
 }  // namespace ttq

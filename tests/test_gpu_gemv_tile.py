@@ -57,6 +57,18 @@ def test_tile_edges(n_out, n_in, xk, m):
     assert torch.equal(lay.forward(e, out_dtype=torch.float32), wd[:, cols].T.float() + 0.0)
 
 
+@pytest.mark.parametrize("n_out,n_in,xk", [(1024, 40960, "bf16"), (1024, 41216, "f16"), (1027, 41472, "bf16"), (777, 44800, "f16")])
+def test_rows_that_leave_little_lds(n_out, n_in, xk):
+    """Rows on both sides of the length where a tile of two blocks along K no longer fits beside the activations.  Bound: the sums
+    of 2^-24 * 320 / 32 per addition of the module's docstring, over more sub-blocks: the same 2e-6."""
+    lay = layer(n_out, n_in)
+    assert lay.route(1, DT[xk], torch.float32) == "gemv_tile"
+    x = torch.randn(1, n_in, device=DEV, generator=torch.Generator(DEV).manual_seed(n_out)).to(DT[xk])
+    ref = x.double() @ dense(lay).T
+    y = lay.forward(x, out_dtype=torch.float32)
+    assert ((y.double() - ref).norm() / ref.norm()).item() <= 2e-6
+
+
 def test_every_size_of_route_is_reached():
     """The cases above are not all skipped: each of the kernel's five forms runs at least on these."""
     for n_out, n_in, m, dt in [(33337, 256, 1, "f32"), (1237, 6912, 1, "bf16"), (2451, 6912, 1, "bf16"), (66700, 512, 2, "f16"),

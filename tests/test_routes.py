@@ -92,6 +92,23 @@ def test_the_single_role_gemm_serves_only_activations_beyond_4_gib():
     assert route(Q4_K, 48, 256, (1 << 32) // 512, BF16, BF16) == "gemm_q4k_tiles"
 
 
+def test_every_form_of_the_tile_kernel_that_is_chosen_fits_a_compute_unit():
+    """The form of a call (blocks along K to a tile) decides how much LDS it takes; the route query fails for a form that needs more
+    than a compute unit has.  Every row length the staged kernels take, matrices on both sides of the forms' rule."""
+    L = _lib.lib()
+    tile = 0
+    for x_dtype, longest in ((F32, 64), (F16, 256), (BF16, 256)):
+        for blocks in range(1, longest + 1):
+            for n_out in (745, 2600, 8192, 32003):
+                for m in (1, 2, 3, 5, 8, 17):
+                    st = QLinearStruct(format=Q6_K, n_out=n_out, n_in=256 * blocks, precision=_lib.PRECISION_F32_SCALES)
+                    r = L.ttq_route(C.byref(st), m, x_dtype, F32)
+                    assert r > 0, (x_dtype, n_out, 256 * blocks, m, r)
+                    tile += r == _lib.ROUTE["gemv_tile"]
+    assert tile > 1000
+    assert route(Q6_K, 1024, 41472, 1, BF16, F32) == route(Q6_K, 8192, 44800, 1, F16, F32) == "gemv_tile"
+
+
 def test_route_is_a_pure_query():
     L = _lib.lib()
     st = QLinearStruct(format=Q4_K, n_out=14336, n_in=4096)
