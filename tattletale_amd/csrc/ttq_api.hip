@@ -531,9 +531,9 @@ int ttq_linear_forward(const ttq_qlinear* layer, const void* x, int x_dtype, int
       us_gemm = ttq::gemm_pc_estimate_us(layer->format, m, n_out, n_in) + 5.f + (float)(m * n_in * 10) / 3.0e6f;
     us_rounding = us_gemm < us_rounding ? us_gemm : us_rounding;
     const bool rounds = route == 2 || !newer || us_rounding < ttq::gemv_estimate_us(layer->format, x_dtype, m, n_out, n_in, false);
-    // (the integer kernel takes two rows of Q6_K to a pass: us of it / of the few-row kernel 14336 x 4096 19.3 / 22.5, 28672 x 4096
-    // 27.0 / 30.5, 43008 x 4096 38.3 / 38.9, 128256 x 4096 88 / 91 -- and of four rows 34 / 22, 49 / 30, 68 / 38, 160 / 91.  The small
-    // matrices, where the two agree to 3 us, stay with the kernel that takes any number of rows.)
+    // (the integer kernel takes two rows of Q6_K to a pass: us of it / of the few-row kernel 14336 x 4096 18.1 / 21.1, 28672 x 4096
+    // 27.0 / 28.9, 32000 x 5120 33.8 / 34.5, 43008 x 4096 38.2 / 36.4, 128256 x 4096 106 / 92 -- and of four rows twice that / the
+    // same.  The small matrices, where the two agree to 3 us, stay with the kernel that takes any number of rows.)
     const bool integer_passes = (int64_t)n_out * n_in >= (int64_t)120 << 20;
     const float us_gemv = ttq::gemv_estimate_us(layer->format, x_dtype, m, n_out, n_in, integer_passes);
     if (rounds && (m > 64 ? us_few / 0.65f : us_few) < us_gemm && (route == 2 || us_few < us_gemv)) {

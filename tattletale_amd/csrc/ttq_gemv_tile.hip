@@ -5,11 +5,14 @@
 // { u8 ql[128]; u8 qh[64]; i8 scales[16]; f16 d } of 256 weights, w = d * scale[e / 16] * (q6[e] - 32).
 //
 // Arithmetic.  A quant of six bits is exact in 16-bit floating point, and so is its product with a bf16 or fp16 activation in
-// the fp32 sums of v_mfma_f32_16x16x32: nothing is rounded before the block scales meet the sum over a sub-block (1e-7 to
-// 3e-7 from the float64 product; the int8 kernels that read activations as 15-bit block fixed point are at 1e-5 to 3e-5).  An
-// fp32 activation is three bf16 terms that add up to it, taken as three rows.  Two bytes become two 16-bit floats with one
-// v_perm: 0x43 over q is the bf16 number 128 + q, 0x5C over 4 q the fp16 number 256 + q.  The offset is not subtracted (one
-// instruction for two weights) but summed with the activations beforehand: every sum starts at -(offset + 32) * sum(x).
+// the fp32 sums of v_mfma_f32_16x16x32: nothing is rounded before the block scales meet the sum over a sub-block.  Two bytes
+// become two 16-bit floats with one v_perm: 0x43 over q is the bf16 number 128 + q, 0x5C over 4 q the fp16 number 256 + q.  The
+// offset is not subtracted (one instruction for two weights) but summed with the activations beforehand: every sum starts at
+// -(offset + 32) * sum(x).  An fp32 activation is three bf16 terms that add up to it, taken as three rows, and meets q - 32 itself
+// (five instructions for four weights more, 128256 x 4096 91 -> 105 us).  From the float64 product, activations of mean zero /
+// of mean one and deviation one: fp32 0.8e-7 to 1.0e-7 either way (the generic kernel 1.1e-7), bf16 0.9e-7 to 1.3e-7 / 1.3e-7 to
+// 2.0e-7 (packed dots 1.3e-7 to 1.7e-7 / 3.4e-7 to 3.9e-7), fp16 2.8e-7 to 5.8e-7 / 6e-7 to 1.3e-6 (packed dots 3e-6 / 8e-6 to
+// 9e-6); the int8 kernels that read activations as 15-bit block fixed point are at 1e-5 to 3e-5.
 //
 // Matrix layout.  Weights are the operand with one weight per column, and lane (n, g), n = lane % 16, g = lane / 16, holds
 // sub-blocks 4 c + g of its block, eight weights of a different sub-block in every lane group.  The other operand is
@@ -30,8 +33,8 @@
 // start at any dword of LDS, where pairs of dwords take three times as long as 16 bytes on their own boundary: 85.  A third
 // ring slot, sixteen wavefronts, operands of four tiles in registers: no gain.  Measured (before: packed-dot or generic
 // kernel, passes of the several-row int8 kernel), us: 32003 x 5120 fp16 one row 43.7 -> 30, two 55.7 -> 29.9, four 101.6 -> 30.5,
-// eight 189 -> 34; fp32 one row 55.9 -> 31.3; 5120 x 5120 fp16 12.2 -> 9.4, four rows 19.6 -> 12; 5120 x 13824 19.8 -> 16.9;
-// 128256 x 4096 bf16 at eight rows 152.7 -> 95, fp32 117 -> 87.
+// eight 189 -> 34; fp32 one row 52.0 -> 33.6; 5120 x 5120 fp16 12.2 -> 9.4, four rows 19.6 -> 12; 5120 x 13824 19.8 -> 16.9;
+// 128256 x 4096 bf16 at eight rows 152.7 -> 98, fp32 one row 122 -> 105; 1024 x 41472 bf16 19.1 -> 13.1.
 #include "ttq_internal.h"
 #include "ttq_tile_common.h"
 
@@ -57,6 +60,7 @@ gemv_tile_kernel(const uint8_t* __restrict__ w, const void* __restrict__ x, int 
   extern __shared__ __attribute__((aligned(1024))) uint8_t tl_lds[];
   constexpr int JB = (J * KQ + 3) / 4, JI = J * KQ < 4 ? J * KQ : 4, R = 16 / KQ;
   constexpr int SB = F::kSub, M = J / PARTS;                    // activation rows at most
+  constexpr bool kSigned = PARTS > 1;                           // weights without an offset: the sums start at zero
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n = lane & 15, g = lane >> 4;
@@ -66,7 +70,7 @@ gemv_tile_kernel(const uint8_t* __restrict__ w, const void* __restrict__ x, int 
   uint8_t* ring = tl_lds + wave * depth * F::kSlot;
   uint8_t* zero = tl_lds + kTlWaves * depth * F::kSlot;
   float* sums = reinterpret_cast<float*>(zero + kTlZeroBytes);                  // [tile][chain][jb][4 g + pseudo row % 4]
-  uint8_t* xs = reinterpret_cast<uint8_t*>(sums + tpr * F::kChains * JB * 16);
+  uint8_t* xs = reinterpret_cast<uint8_t*>(sums + (kSigned ? 0 : tpr * F::kChains * JB * 16));
   const uint32_t kpad = (uint32_t)tpr * KQ * 256u, xstride = (uint32_t)tpr * KQ * kTlXBlock;
   float* part = reinterpret_cast<float*>(xs + J * xstride);                     // [wave][first, last][M][R]
   const uint32_t ring_lds = (uint32_t)__builtin_amdgcn_readfirstlane((int)sm_lds(ring)), xs_lds = sm_lds(xs);
@@ -81,13 +85,13 @@ gemv_tile_kernel(const uint8_t* __restrict__ w, const void* __restrict__ x, int 
   } else {
     for (int e = tid; e < m * (n_in / 8); e += kTlThreads) {
       const int row = e / (n_in / 8), v8 = e - row * (n_in / 8);
-      // three bf16 terms that add up to the fp32 value: every term is the rest cut to its upper 16 bits.  Times 2^-8, undone on
-      // the sums: 128 + q then overflows no earlier than the value itself.
+      // three bf16 terms that add up to the fp32 value: every term is the rest cut to its upper 16 bits, and what is left of an
+      // infinite value is nothing.  A quarter of it: the weights are four times themselves.
       const float4* src = reinterpret_cast<const float4*>(static_cast<const float*>(x) + (int64_t)row * n_in + 8 * v8);
       const float4 f0 = src[0], f1 = src[1];
       float f[8] = {f0.x, f0.y, f0.z, f0.w, f1.x, f1.y, f1.z, f1.w};
 #pragma unroll
-      for (int i = 0; i < 8; i++) f[i] *= 0x1p-8f;
+      for (int i = 0; i < 8; i++) f[i] *= 0.25f;
 #pragma unroll
       for (int p = 0; p < 3; p++) {
         uint32_t o[4];
@@ -95,8 +99,8 @@ gemv_tile_kernel(const uint8_t* __restrict__ w, const void* __restrict__ x, int 
         for (int i = 0; i < 4; i++) {
           const uint32_t lo = __float_as_uint(f[2 * i]) & 0xFFFF0000u, hi = __float_as_uint(f[2 * i + 1]) & 0xFFFF0000u;
           o[i] = (lo >> 16) | hi;
-          f[2 * i] -= __uint_as_float(lo);
-          f[2 * i + 1] -= __uint_as_float(hi);
+          f[2 * i] = f[2 * i] == __uint_as_float(lo) ? 0.f : f[2 * i] - __uint_as_float(lo);
+          f[2 * i + 1] = f[2 * i + 1] == __uint_as_float(hi) ? 0.f : f[2 * i + 1] - __uint_as_float(hi);
         }
         *reinterpret_cast<uint4*>(xs + (3 * row + p) * xstride + kTlXBlock * (v8 >> 5) + 16 * (v8 & 31)) = make_uint4(o[0], o[1], o[2], o[3]);
       }
@@ -149,7 +153,7 @@ gemv_tile_kernel(const uint8_t* __restrict__ w, const void* __restrict__ x, int 
   }
   sm_barrier();
   // ---- sums of the activations over sub-blocks, times what the sums of products start at
-  {
+  if constexpr (!kSigned) {
     const int subs = (int)kpad / SB;
     for (int row = 0; row < J; row++)
       for (int sub = tid; sub < subs; sub += kTlThreads) {
@@ -166,8 +170,8 @@ gemv_tile_kernel(const uint8_t* __restrict__ w, const void* __restrict__ x, int 
         }
         sums[((t * F::kChains + c) * JB + (P >> 2)) * 16 + 4 * gg + (P & 3)] = F::template kStart<XT> * v;
       }
+    sm_barrier();
   }
-  sm_barrier();
 
   // operand lane (i = n, g): pseudo row i % 4 of the block diagonal i / 4 == g; pseudo row P = KQ * row + block
   uint32_t xbase[JB], xmask[JB];
@@ -186,14 +190,14 @@ gemv_tile_kernel(const uint8_t* __restrict__ w, const void* __restrict__ x, int 
   };
   clear();
   // a tile's activations and the values its sums start at
-  struct Acts { uint4 x[JB][F::kChains][F::kSteps]; f32x4_t s[F::kChains][JB]; };
+  struct Acts { uint4 x[JB][F::kChains][F::kSteps]; f32x4_t s[kSigned ? 1 : F::kChains][JB]; };
   auto load_acts = [&](Acts& t, int k) {
 #pragma unroll
     for (int c = 0; c < F::kChains; c++)
 #pragma unroll
       for (int jb = 0; jb < JB; jb++) {
         const uint32_t xa = xbase[jb] + (xmask[jb] & (uint32_t)(kTlXBlock * KQ * k));
-        t.s[c][jb] = *reinterpret_cast<const f32x4_t*>(sums + ((k * F::kChains + c) * JB + jb) * 16 + 4 * g);
+        if constexpr (!kSigned) t.s[c][jb] = *reinterpret_cast<const f32x4_t*>(sums + ((k * F::kChains + c) * JB + jb) * 16 + 4 * g);
 #pragma unroll
         for (int i = 0; i < F::kSteps; i++) t.x[jb][c][i] = *reinterpret_cast<const uint4*>(tl_lds + xa + 2 * F::chain_k(c) + 16 * i);
       }
@@ -205,21 +209,26 @@ gemv_tile_kernel(const uint8_t* __restrict__ w, const void* __restrict__ x, int 
 #pragma unroll
     for (int c = 0; c < F::kChains; c++) {
 #pragma unroll
-      for (int jb = 0; jb < JB; jb++) d[c][jb] = a.s[c][jb];
+      for (int jb = 0; jb < JB; jb++) d[c][jb] = kSigned ? f32x4_t{0.f, 0.f, 0.f, 0.f} : a.s[kSigned ? 0 : c][jb];
 #pragma unroll
       for (int i = 0; i < F::kSteps; i++) {
         uint32_t wv[4];
-        F::template weights<XT>(r, c, i, wv);
+        if constexpr (kSigned) F::signed_weights(r, c, i, wv);
+        else F::template weights<XT>(r, c, i, wv);
 #pragma unroll
         for (int jb = 0; jb < JB; jb++) d[c][jb] = tile_mfma<XT>(a.x[jb][c][i], wv, d[c][jb]);
       }
     }
+    // (a tile's four products among themselves first: the running sum, the largest of them, is rounded once a tile)
 #pragma unroll
-    for (int c = 0; c < F::kChains; c++)
+    for (int jb = 0; jb < JB; jb++)
 #pragma unroll
-      for (int jb = 0; jb < JB; jb++)
+      for (int i = 0; i < JI; i++) {
+        float t = P.s[0] * d[0][jb][i];
 #pragma unroll
-        for (int i = 0; i < JI; i++) acc[jb][i] = fmaf_(P.s[c], d[c][jb][i], acc[jb][i]);
+        for (int c = 1; c < F::kChains; c++) t = fmaf_(P.s[c], d[c][jb][i], t);
+        acc[jb][i] += t;
+      }
   };
 
   auto put = [&](int row, int col, float v) {
@@ -245,10 +254,6 @@ gemv_tile_kernel(const uint8_t* __restrict__ w, const void* __restrict__ x, int 
       if constexpr (KQ >= 2) v += lane_xor<1>(v, lane);
       if constexpr (KQ >= 4) v += lane_xor<2>(v, lane);
       tot[j / PARTS] += v;
-    }
-    if constexpr (PARTS > 1) {
-#pragma unroll
-      for (int j = 0; j < M; j++) tot[j] *= 0x1p8f;
     }
 #pragma unroll
     for (int jb = 0; jb < (M + 3) / 4; jb++) {
@@ -309,16 +314,16 @@ struct TlArgs {
 
 constexpr size_t kTlLds = 160 * 1024;
 template <class F>
-size_t tile_lds_bytes(int j, int kq, int64_t n_in, int depth) {
+size_t tile_lds_bytes(int j, int kq, int parts, int64_t n_in, int depth) {
   const size_t jb = (j * kq + 3) / 4, tpr = ((n_in >> 8) + kq - 1) / kq;
-  return (size_t)kTlWaves * depth * F::kSlot + kTlZeroBytes + tpr * F::kChains * jb * 64 + (size_t)j * (kTlXBlock * kq * tpr) +
+  return (size_t)kTlWaves * depth * F::kSlot + kTlZeroBytes + (parts > 1 ? 0 : tpr * F::kChains * jb * 64) + (size_t)j * (kTlXBlock * kq * tpr) +
          (size_t)2 * kTlWaves * j * (16 / kq) * 4;
 }
 
 template <class F, class XT, int J, int KQ, int PARTS = 1>
 hipError_t launch_tile_j(const TlArgs& a, hipStream_t s) {
   constexpr int depth = kTlDepth;
-  const size_t lds = tile_lds_bytes<F>(J, KQ, a.n_in, depth);
+  const size_t lds = tile_lds_bytes<F>(J, KQ, PARTS, a.n_in, depth);
   if (lds > kTlLds) return hipErrorInvalidValue;
   if (route_probe(kRouteGemvTile)) return hipSuccess;      // (here, so that the query answers for the form that would run)
   auto kernel = gemv_tile_kernel<F, XT, J, KQ, PARTS>;
@@ -341,7 +346,7 @@ TlForm tile_form(int x_dtype, int64_t m, int64_t n_out, int64_t n_in) {
   // One row: four blocks to a tile, except where the last tile of long matrices' rows would be half empty (32003 x 2560 21.3 us
   // with four, 17.9 with two; 7168 x 3584 9.7 / 9.9).  Two take more LDS, and end at rows of 41216 values.
   const bool wide = (n_in >> 8) % 4 == 0 || n_out * (n_in >> 8) * 210 < (24 << 20);
-  return TlForm{1, wide || tile_lds_bytes<TlQ6K>(1, 2, n_in, kTlDepth) > kTlLds ? 4 : 2};
+  return TlForm{1, wide || tile_lds_bytes<TlQ6K>(1, 2, 1, n_in, kTlDepth) > kTlLds ? 4 : 2};
 }
 
 template <class F, class XT>
@@ -362,7 +367,7 @@ bool gemv_tile_supported(int format, int x_dtype, int64_t m, int64_t n_out, int6
   if (disabled || format != kQ6_K || n_in % 256 != 0 || m < 1 || m > 8 || n_out > 0x3FFFFFFF || n_in > (1 << 22)) return false;
   if (m > gemv_tile_rows(x_dtype)) return false;
   const TlForm f = tile_form(x_dtype, m, n_out, n_in);
-  return tile_lds_bytes<TlQ6K>(f.j, f.kq, n_in, kTlDepth) <= kTlLds;
+  return tile_lds_bytes<TlQ6K>(f.j, f.kq, x_dtype == kF32 ? 3 : 1, n_in, kTlDepth) <= kTlLds;
 }
 
 // Whether it is the faster one among the decode kernels.  Startup (the activations' sums, a barrier, one tile's chain) is some
@@ -388,7 +393,8 @@ bool gemv_tile_preferred(int format, int x_dtype, int64_t m, int64_t n_out, int6
 }
 
 // Several rows, us: 21.5 / 134 / 431 MB 10.2 / 28.9 / 84 for two rows, 11.8 / 30 / 87 for four, 15.1 / 33.4 / 98 for eight.
-// (an fp32 row is three.)
+// (an fp32 row is three; its signed weights add a tenth, which is left out: where the few-row kernel over rounded weights is faster
+// by no more than that, the call keeps its precision.)
 float gemv_tile_estimate_us(int x_dtype, int64_t m, int64_t n_out, int64_t n_in) {
   const float mb = (float)(n_out * (n_in >> 8) * 210) * 1e-6f;
   return (x_dtype == kF32 ? 3 * m : m) <= 4 ? 5.f + mb / 5.2f : 8.3f + mb / 4.8f;

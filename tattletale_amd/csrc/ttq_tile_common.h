@@ -146,6 +146,23 @@ struct TlQ6K {
 #pragma unroll
     for (int c = 0; c < 4; c++) P.s[c] = d * (float)(int)__builtin_amdgcn_sbfe((int)r.sc[c], L.sc_shift, 8);
   }
+  // q - 32 itself as bf16, for fp32 activations in three terms: with an offset in the sums, activations whose mean is not zero
+  // leave a rounding that the fp32 kernel does not have (1.5e-7 to 2.0e-7 from the float64 product instead of 1.1e-7), and an
+  // infinite one makes a NaN of every output.  4 q with its top bit turned is the signed byte 4 (q - 32), one conversion to
+  // fp32 each, whose upper half is exact: times 4, which the caller takes out of the activations.
+  static __device__ __forceinline__ void signed_weights(const Raw& r, int c, int t, uint32_t (&w)[4]) {
+    const int h = c >> 1, p = c & 1;
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+      const uint32_t l = r.ql[h][2 * t + k], q = r.qh[h][2 * t + k];
+      const uint32_t u = (((p ? l >> 2 : l << 2) & 0x3C3C3C3Cu) | ((p ? q << 2 : q << 6) & 0xC0C0C0C0u)) ^ 0x80808080u;
+      uint32_t f[4];
+#pragma unroll
+      for (int i = 0; i < 4; i++) f[i] = __float_as_uint((float)(int)(int8_t)(u >> (8 * i)));
+      w[2 * k] = __builtin_amdgcn_perm(f[1], f[0], 0x07060302u);
+      w[2 * k + 1] = __builtin_amdgcn_perm(f[3], f[2], 0x07060302u);
+    }
+  }
   // The integer q (0 .. 63) as a 16-bit float with an offset that costs no instruction: bf16 0x4300 | q = 128 + q, fp16
   // 0x5C00 | q << 2 = 256 + q.  The sums are started at -(offset + 32) * sum(x).
   template <class XT> static constexpr float kStart = std::is_same<XT, f16_tag>::value ? -288.f : -160.f;

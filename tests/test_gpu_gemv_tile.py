@@ -69,6 +69,34 @@ def test_rows_that_leave_little_lds(n_out, n_in, xk):
     assert ((y.double() - ref).norm() / ref.norm()).item() <= 2e-6
 
 
+@pytest.mark.parametrize("n_out,n_in", [(30006, 1280), (5120, 5120), (4096, 7680)])
+@pytest.mark.parametrize("m", [1, 2])
+def test_fp32_rows_whose_mean_is_not_zero(n_out, n_in, m):
+    """fp32 activations meet q - 32 itself, so their mean leaves nothing behind.  Bound: a product's first terms are whole
+    multiples of a common power of two and their sums exact, what is rounded are the running sums, once a tile and lane: at
+    most 40 additions of a growing sum (in the square mean a third of its end), each off by 0.29 ulp, 0.29 * 2^-23 * sqrt(40 / 3) =
+    1.3e-7 (with an offset in the sums: 1.5e-7 to 2.0e-7)."""
+    lay = layer(n_out, n_in)
+    assert lay.route(m, torch.float32, torch.float32) == "gemv_tile"
+    x = torch.randn(m, n_in, device=DEV, generator=torch.Generator(DEV).manual_seed(n_in)) + 1
+    ref = x.double() @ dense(lay).T
+    y = lay.forward(x)
+    assert ((y.double() - ref).norm(dim=-1) / ref.norm(dim=-1)).max().item() <= 1.3e-7
+
+
+def test_an_infinite_fp32_value_gives_infinities():
+    n_out, n_in = 30006, 1280
+    lay = layer(n_out, n_in)
+    wd = dense(lay)
+    x = torch.randn(2, n_in, device=DEV, generator=torch.Generator(DEV).manual_seed(7))
+    x[0, 300], x[1, 1279] = float("inf"), float("-inf")
+    assert lay.route(2, torch.float32, torch.float32) == "gemv_tile"
+    for y, z in ((lay.forward(x), x), (lay.forward(x[:1]), x[:1])):
+        want = (z.double() @ wd.T).float()                     # infinite times zero: not a number
+        assert torch.equal(torch.nan_to_num(y, nan=0.0, posinf=1.0, neginf=-1.0), torch.nan_to_num(want, nan=0.0, posinf=1.0, neginf=-1.0))
+        assert torch.equal(y.isnan(), want.isnan()) and want.isinf().float().mean() > 0.9
+
+
 def test_every_size_of_route_is_reached():
     """The cases above are not all skipped: each of the kernel's five forms runs at least on these."""
     for n_out, n_in, m, dt in [(33337, 256, 1, "f32"), (1237, 6912, 1, "bf16"), (2451, 6912, 1, "bf16"), (66700, 512, 2, "f16"),
