@@ -6,12 +6,12 @@
 //
 // Arithmetic.  A quant of six bits is exact in 16-bit floating point, and so is its product with a bf16 or fp16 activation in
 // the fp32 sums of v_mfma_f32_16x16x32: nothing is rounded before the block scales meet the sum over a sub-block.  Two bytes
-// become two 16-bit floats with one v_perm: 0x43 over q is the bf16 number 128 + q, 0x5C over 4 q the fp16 number 256 + q.  The
+// become two 16-bit floats with one v_perm: 0x3D over q is the bf16 number (128 + q) / 4096, 0x5C over 4 q the fp16 number 256 + q.  The
 // offset is not subtracted (one instruction for two weights) but summed with the activations beforehand: every sum starts at
 // -(offset + 32) * sum(x).  An fp32 activation is three bf16 terms that add up to it, taken as three rows, and meets q - 32 itself
 // (five instructions for four weights more, 128256 x 4096 91 -> 105 us).  From the float64 product, activations of mean zero /
 // of mean one and deviation one: fp32 0.8e-7 to 1.0e-7 either way (the generic kernel 1.1e-7), bf16 0.9e-7 to 1.3e-7 / 1.3e-7 to
-// 2.0e-7 (packed dots 1.3e-7 to 1.7e-7 / 3.4e-7 to 3.9e-7), fp16 2.8e-7 to 5.8e-7 / 6e-7 to 1.3e-6 (packed dots 3e-6 / 8e-6 to
+// 2.0e-7 (packed dots 1.3e-7 to 1.7e-7 / 3.4e-7 to 3.9e-7), fp16 2.8e-7 to 3.5e-7 / 6e-7 to 9e-7 (packed dots 3e-6 / 8e-6 to
 // 9e-6); the int8 kernels that read activations as 15-bit block fixed point are at 1e-5 to 3e-5.
 //
 // Matrix layout.  Weights are the operand with one weight per column, and lane (n, g), n = lane % 16, g = lane / 16, holds
@@ -47,9 +47,10 @@ constexpr int kTlDepth = 2;                // tiles in a wavefront's ring: one m
 constexpr int kTlXBlock = 528;             // 256 activations in LDS: the four lanes of a product's k-set on different banks
 constexpr int kTlZeroBytes = 512;          // what the lanes off the block diagonal read
 
-template <class XT> __device__ __forceinline__ float half_pair_sum(uint32_t v) {
-  if constexpr (std::is_same<XT, f16_tag>::value) return f16_bits_to_f32((uint16_t)(v & 0xFFFFu)) + f16_bits_to_f32((uint16_t)(v >> 16));
-  else return __uint_as_float(v << 16) + __uint_as_float(v & 0xFFFF0000u);
+// sum + k * both halves of v
+template <class XT> __device__ __forceinline__ float add_halves(float k, uint32_t v, float sum) {
+  if constexpr (std::is_same<XT, f16_tag>::value) return fmaf_(k, f16_bits_to_f32((uint16_t)(v & 0xFFFFu)), fmaf_(k, f16_bits_to_f32((uint16_t)(v >> 16)), sum));
+  else return fmaf_(k, __uint_as_float(v << 16), fmaf_(k, __uint_as_float(v & 0xFFFF0000u), sum));
 }
 // J: activation rows as the matrix cores see them, PARTS to an activation row (three for fp32).  KQ: blocks along K of a tile, of
 // 16 / KQ weight rows.
@@ -166,9 +167,9 @@ gemv_tile_kernel(const uint8_t* __restrict__ w, const void* __restrict__ x, int 
           const uint4 q = reinterpret_cast<const uint4*>(xs + row * xstride + kTlXBlock * blk + 2 * SB * (sub & (256 / SB - 1)))[k];
           const uint32_t d4[4] = {q.x, q.y, q.z, q.w};
 #pragma unroll
-          for (int i = 0; i < 4; i++) v += half_pair_sum<XT>(d4[i]);
+          for (int i = 0; i < 4; i++) v = add_halves<XT>(F::template kStart<XT>, d4[i], v);
         }
-        sums[((t * F::kChains + c) * JB + (P >> 2)) * 16 + 4 * gg + (P & 3)] = F::template kStart<XT> * v;
+        sums[((t * F::kChains + c) * JB + (P >> 2)) * 16 + 4 * gg + (P & 3)] = v;
       }
     sm_barrier();
   }
@@ -254,6 +255,10 @@ gemv_tile_kernel(const uint8_t* __restrict__ w, const void* __restrict__ x, int 
       if constexpr (KQ >= 2) v += lane_xor<1>(v, lane);
       if constexpr (KQ >= 4) v += lane_xor<2>(v, lane);
       tot[j / PARTS] += v;
+    }
+    if constexpr (!kSigned) {
+#pragma unroll
+      for (int j = 0; j < M; j++) tot[j] *= F::template kUnscale<XT>;
     }
 #pragma unroll
     for (int jb = 0; jb < (M + 3) / 4; jb++) {

@@ -163,9 +163,11 @@ struct TlQ6K {
       w[2 * k + 1] = __builtin_amdgcn_perm(f[3], f[2], 0x07060302u);
     }
   }
-  // The integer q (0 .. 63) as a 16-bit float with an offset that costs no instruction: bf16 0x4300 | q = 128 + q, fp16
-  // 0x5C00 | q << 2 = 256 + q.  The sums are started at -(offset + 32) * sum(x).
-  template <class XT> static constexpr float kStart = std::is_same<XT, f16_tag>::value ? -288.f : -160.f;
+  // The integer q (0 .. 63) as a 16-bit float with an offset that costs no instruction: bf16 0x3D00 | q = (128 + q) / 4096, fp16
+  // 0x5C00 | q << 2 = 256 + q.  The sums are started at -(offset + 32) * sum(x).  (The 4096, taken out of the finished sum by
+  // kUnscale, keeps the sums of a sub-block finite for every finite bf16 activation.)
+  template <class XT> static constexpr float kStart = std::is_same<XT, f16_tag>::value ? -288.f : -160.f / 4096.f;
+  template <class XT> static constexpr float kUnscale = std::is_same<XT, f16_tag>::value ? 1.f : 4096.f;
   template <class XT>
   static __device__ __forceinline__ void weights(const Raw& r, int c, int t, uint32_t (&w)[4]) {
     constexpr bool H = std::is_same<XT, f16_tag>::value;
@@ -177,7 +179,7 @@ struct TlQ6K {
       // (the bit pairs of the low nibbles are bits 0-1 of the bytes of q, those of the high nibbles bits 4-5)
       const uint32_t lo = H ? (p ? l >> 2 : l << 2) : (p ? l >> 4 : l), hi = H ? (p ? q << 2 : q << 6) : (p ? q : q << 4);
       const uint32_t u = (lo & N) | (hi & Q);
-      spread_bytes(u, H ? 0x5C5C5C5Cu : 0x43434343u, w[2 * k], w[2 * k + 1]);
+      spread_bytes(u, H ? 0x5C5C5C5Cu : 0x3D3D3D3Du, w[2 * k], w[2 * k + 1]);
     }
   }
 };

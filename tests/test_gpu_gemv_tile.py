@@ -97,6 +97,26 @@ def test_an_infinite_fp32_value_gives_infinities():
         assert torch.equal(y.isnan(), want.isnan()) and want.isinf().float().mean() > 0.9
 
 
+@pytest.mark.parametrize("m", [1, 2, 4, 8])
+@pytest.mark.parametrize("size", [3e38, 1e36, 1e-34])
+def test_bf16_activations_at_both_ends_of_the_range(m, size):
+    """Whole rows of activations of one magnitude, signs at random: finite results, as exact as others.  The block scales are
+    turned down (up for small ones), so that the results lie inside of the type.  Bound: the module's; for 1e-34 the products,
+    divided by 4096, end at 2^-149 and are 2^-126 and larger: 23 bits."""
+    n_out, n_in = 30006, 1280
+    raw = random_blocks(F.Q6_K, n_out * (n_in // 256), seed=1).reshape(-1, 210)
+    raw[:, 208:210] = np.frombuffer(np.float16(1e-6 if size > 1 else 1e3).tobytes(), np.uint8)
+    lay = QuantLinear.init(packed_to_dev(raw.reshape(-1)), F.Q6_K, n_in, n_out, precision=F.PRECISION_F32_SCALES)
+    assert lay.route(m, torch.bfloat16, torch.float32) == "gemv_tile"
+    sign = torch.randint(0, 2, (m, n_in), device=DEV, generator=torch.Generator(DEV).manual_seed(m)) * 2.0 - 1
+    x = (sign * size).to(torch.bfloat16)
+    x[0] = x[0].abs()
+    ref = x.double() @ dense(lay).T
+    y = lay.forward(x, out_dtype=torch.float32)
+    assert torch.isfinite(ref.float()).all() and torch.isfinite(y).all()
+    assert ((y.double() - ref).norm(dim=-1) / ref.norm(dim=-1)).max().item() <= 2e-6
+
+
 def test_every_size_of_route_is_reached():
     """The cases above are not all skipped: each of the kernel's five forms runs at least on these."""
     for n_out, n_in, m, dt in [(33337, 256, 1, "f32"), (1237, 6912, 1, "bf16"), (2451, 6912, 1, "bf16"), (66700, 512, 2, "f16"),
