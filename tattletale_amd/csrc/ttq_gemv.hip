@@ -456,8 +456,11 @@ bool gemv_row_is_long(int format, int x_dtype, int64_t n_in) {
   return n_in > (dot2 ? kMaxGemvIn16 : kMaxGemvInF32);
 }
 
-// Passes of eight fp16 rows, or the exact form of the kernel for up to 64: 32003 x 5120 at 9 / 16 / 43 / 64 rows
-// 42 / 41 / 53 / 61 us in one launch, 34 us a pass (with passes of four rows in packed dots 272 / 354 / 918 / 1322).
+// More rows of Q6_K than a pass of the integer kernel takes: passes of it, in fp16 also the exact form of the kernel for up to 64
+// (32003 x 5120 at 9 / 16 / 43 / 64 rows 42 / 41 / 53 / 61 us in one launch, 34 us a pass), or all of them in one launch of packed dots
+// (four rows a pass; 272 / 354 / 918 / 1322) or of the generic kernel, which on small matrices overlap their passes: fp32
+// 1024 x 6144 at eight rows 22 us there and 38 in passes of two, 2560 x 4096 at 64 177 and 246 (4096 x 4096 275 and 254);
+// bf16 1536 x 4096 at 32 rows 28 and 39 (3072 x 4096 44 and 40).
 static float rows_exact_us(int64_t m, int64_t n_out, int64_t n_in) {
   const int64_t full = m / 64, rest = m % 64;
   float us = full ? (float)full * 1.2f * gemm_rows_estimate_us(kQ6_K, 64, n_out, n_in) : 0.f;
@@ -469,9 +472,23 @@ static float tile_passes_us(int x_dtype, int64_t m, int64_t n_out, int64_t n_in)
   return (float)(m / per) * gemv_tile_estimate_us(x_dtype, per, n_out, n_in) +
          (rest ? gemv_tile_estimate_us(x_dtype, rest, n_out, n_in) : 0.f);
 }
-static bool rows_exact_preferred(int x_dtype, int64_t m, int64_t n_out, int64_t n_in) {
-  return x_dtype == kF16 && m > 8 && gemm_rows_supported(kQ6_K, m < 64 ? m : 64, n_out, n_in) &&
-         rows_exact_us(m, n_out, n_in) < tile_passes_us(x_dtype, m, n_out, n_in);
+// Within a tenth of 512 .. 8192 rows of 256 .. 5120 (fp32 6912) values at 8 to 64 activation rows.
+static float overlapped_passes_us(int x_dtype, int64_t m, int64_t n_out, int64_t n_in) {
+  const float rows = (float)n_out * 1e-3f;
+  if (x_dtype == kF32) return 5.5f + (float)m * (float)((n_in + 4095) / 4096) * (n_out > 6144 ? 0.8f : 1.f) * rows;
+  return (n_out > 2048 ? 6.5f : 2.f) + (float)((m + 3) / 4) * (n_in > 4096 ? 1.65f : 1.f) * (n_out > 2048 ? 1.5f : 2.f) * rows;
+}
+enum class ManyRows { kOther, kPasses, kRowsExact };
+static ManyRows many_rows(int format, int x_dtype, int64_t m, int64_t n_out, int64_t n_in) {
+  const int64_t per = gemv_tile_rows(x_dtype);
+  if (format != kQ6_K || m <= per || !gemv_tile_competes(format, x_dtype, per, n_out, n_in)) return ManyRows::kOther;
+  const float us_tile = tile_passes_us(x_dtype, m, n_out, n_in);
+  const bool rows = x_dtype == kF16 && gemm_rows_supported(kQ6_K, m < 64 ? m : 64, n_out, n_in) && rows_exact_us(m, n_out, n_in) < us_tile;
+  const float us = rows ? rows_exact_us(m, n_out, n_in) : us_tile;
+  // (a matrix that the int8 kernel of several rows takes comes here only where that is known to be slower)
+  if (!gemv_q6k_stream4_supported(format, x_dtype, per, n_out, n_in) && overlapped_passes_us(x_dtype, m, n_out, n_in) <= us)
+    return ManyRows::kOther;
+  return rows ? ManyRows::kRowsExact : ManyRows::kPasses;
 }
 
 hipError_t launch_gemv(int format, const void* w, const void* x, int x_dtype, void* y, int y_dtype,
@@ -486,10 +503,10 @@ hipError_t launch_gemv(int format, const void* w, const void* x, int x_dtype, vo
       default: return hipErrorInvalidValue;
     }
   }
-  // Q6_K, more rows than a pass of the integer kernel takes: in fp16 the form for many rows (64 to a launch), else passes
-  const int64_t per_pass = gemv_tile_rows(x_dtype);
-  if (format == kQ6_K && m > per_pass && gemv_tile_preferred(format, x_dtype, per_pass, n_out, n_in)) {
-    const bool rows = rows_exact_preferred(x_dtype, m, n_out, n_in);
+  const ManyRows many = many_rows(format, x_dtype, m, n_out, n_in);
+  if (many != ManyRows::kOther) {
+    const int64_t per_pass = gemv_tile_rows(x_dtype);
+    const bool rows = many == ManyRows::kRowsExact;
     if (rows && route_probe(kRouteGemmRowsExact)) return hipSuccess;
     const int64_t step = rows ? 64 : per_pass, xsize = x_dtype == kF32 ? 4 : 2, ysize = y_dtype == kF32 ? 4 : 2;
     for (int64_t r = 0; r < m; r += step) {
@@ -503,7 +520,7 @@ hipError_t launch_gemv(int format, const void* w, const void* x, int x_dtype, vo
     }
     return hipSuccess;
   }
-  if (format == kQ6_K && gemv_tile_preferred(format, x_dtype, m, n_out, n_in))
+  if (gemv_tile_preferred(format, x_dtype, m, n_out, n_in))
     return launch_gemv_tile(format, w, x, x_dtype, y, y_dtype, bias, bias_dtype, m, n_out, n_in, s);
   // a few rows at once: four per pass for up to four rows and for rows too long for the 8- and
   // 16-token tables, else eight or sixteen per pass
@@ -565,9 +582,9 @@ float gemv_estimate_us(int format, int x_dtype, int64_t m, int64_t n_out, int64_
   // rows of any length: a pass over the weights per activation row (72 MB in 24.6 us, 155 MB in 51 us, 463 MB in 122 us)
   if (gemv_row_is_long(format, x_dtype, n_in)) return (float)m * (mb / 3.5f + 3.f);
   if (integer_kernels) {
-    const int64_t per = gemv_tile_rows(x_dtype);
-    if (m > per && gemv_tile_preferred(format, x_dtype, per, n_out, n_in))
-      return rows_exact_preferred(x_dtype, m, n_out, n_in) ? rows_exact_us(m, n_out, n_in) : tile_passes_us(x_dtype, m, n_out, n_in);
+    const ManyRows many = many_rows(format, x_dtype, m, n_out, n_in);
+    if (many == ManyRows::kRowsExact) return rows_exact_us(m, n_out, n_in);
+    if (many == ManyRows::kPasses) return tile_passes_us(x_dtype, m, n_out, n_in);
     if (gemv_tile_preferred(format, x_dtype, m, n_out, n_in)) return gemv_tile_estimate_us(x_dtype, m, n_out, n_in);
   }
   const bool b4 = gemv_q4k_batch4_supported(format, x_dtype, m, n_out, n_in);

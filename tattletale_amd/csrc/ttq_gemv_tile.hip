@@ -375,34 +375,60 @@ bool gemv_tile_supported(int format, int x_dtype, int64_t m, int64_t n_out, int6
   return tile_lds_bytes<TlQ6K>(f.j, f.kq, x_dtype == kF32 ? 3 : 1, n_in, kTlDepth) <= kTlLds;
 }
 
-// Whether it is the faster one among the decode kernels.  Startup (the activations' sums, a barrier, one tile's chain) is some
-// 4 us, so small matrices stay where they are.  Measured, us, this kernel / the other:
-//   one row, 16-bit, against packed dots: 2560 x 6912 (14.5 MB) 8.2 / 9.7, 4096 x 5120 8.2 / 9.1, 5120 x 5120 9.4 / 12.2; rows of up
-//     to 4096 values, which packed dots hold in registers: 7168 x 3584 (21 MB) 9.7 / 8.4, 13824 x 2560 (29 MB) 10.7 / 11.0,
-//     32003 x 2560 17.9 / 21.1, 100001 x 3584 59.9 / 66; the int8 stream, where it takes the shape, is faster (8192 x 8192 14.7 / 13.4)
-//   one fp32 row, against the generic kernel: 2560 x 2560 (5.4 MB) 6.8 / 6.8, 3328 x 3328 (9 MB) 7.6 / 8.7, 1024 x 4096 6.1 / 4.2
-//   two rows, against packed dots: 2048 x 2048 (3.4 MB) 5.5 / 4.0, 2560 x 2560 6.3 / 7.0, 5120 x 5120 10.2 / 14.5
-//   four rows, against packed dots: 2048 x 2048 6.0 / 5.4, 2560 x 2560 6.9 / 8.7, 32003 x 5120 30 / 101
-//   the several-row int8 kernel, where it takes the shape: two rows of 28672 x 8192 40.2 / 36.8, four of 128256 x 4096 84.7 / 78,
-//     eight of 128256 x 4096 95 / 152.7, of 151936 x 1024 35.7 / 55.3 (one pass against two).  It computes what the single-row
-//     int8 stream computes, to 2e-6, and up to 100 MB, where a second pass costs little, that agreement is kept.
-bool gemv_tile_preferred(int format, int x_dtype, int64_t m, int64_t n_out, int64_t n_in) {
-  static const int always = dev_knob("TTQ_TILE_FIRST", 0);
+// Whether it competes with the other decode kernels at all: startup (the activations' sums, a barrier, one tile's chain) is some
+// 4 us, so small matrices stay where they are, and 16-bit calls that the int8 stream takes stay there (8192 x 8192 one row 14.7 us
+// here, 13.4 there), except for more rows than that kernel takes at once: it computes what the single-row stream computes, to
+// 2e-6, and up to 100 MB, where a second pass costs little, that agreement is kept (128256 x 4096 at eight rows 95 / 152.7,
+// 151936 x 1024 35.7 / 55.3; four rows of 128256 x 4096 84.7 / 78).
+bool gemv_tile_competes(int format, int x_dtype, int64_t m, int64_t n_out, int64_t n_in) {
   const float mb = (float)(n_out * (n_in >> 8) * 210) * 1e-6f;
-  if (format != kQ6_K || (mb < 5.f && !always)) return false;      // (first: small calls are where the host's time counts)
+  if (format != kQ6_K || mb < 5.f) return false;      // (first: small calls are where the host's time counts)
   if (!gemv_tile_supported(format, x_dtype, m, n_out, n_in)) return false;
-  if (always) return true;
-  if (x_dtype == kF32) return mb >= (m == 1 ? 7.f : 5.f);
-  if (m == 1) return !gemv_q6k_stream_supported(format, x_dtype, n_out, n_in) && mb >= (n_in > 4096 ? 12.f : 27.f);
-  return !gemv_q6k_stream4_supported(format, x_dtype, m, n_out, n_in) || (m > 4 && mb >= 100.f);
+  if (x_dtype == kF32) return true;
+  return m == 1 ? !gemv_q6k_stream_supported(format, x_dtype, n_out, n_in)
+                : !gemv_q6k_stream4_supported(format, x_dtype, m, n_out, n_in) || (m > 4 && mb >= 100.f);
 }
 
-// Several rows, us: 21.5 / 134 / 431 MB 10.2 / 28.9 / 84 for two rows, 11.8 / 30 / 87 for four, 15.1 / 33.4 / 98 for eight.
-// (an fp32 row is three; its signed weights add a tenth, which is left out: where the few-row kernel over rounded weights is faster
-// by no more than that, the call keeps its precision.)
+// Whether it is the faster one, for as many rows as a pass takes.  A workgroup has 4, 8 or 16 weight rows at least and all of K: where
+// that leaves compute units idle, the kernels that give a wavefront a row of its own win as long as they hold a row's activations
+// in registers (up to 4096 values) or their rounds are whole.  Measured, us, this kernel / the other:
+//   one row, 16-bit, against packed dots: rows of more than 4096 values from 12 MB on, 2560 x 6912 8.2 / 9.7, 1000 x 16128 8.0 / 8.7,
+//     but for 1025 to 2048 of them, a whole round there: 2048 x 8192 7.3 / 7.1, 1536 x 11008 8.5 / 7.9, 2048 x 16128 10.5 / 10.1
+//     (2048 x 22528 12.6 / 13.8); rows of up to 4096 values 7168 x 3584 (21 MB) 9.7 / 8.4, 13824 x 2560 (29 MB) 10.7 / 11.0,
+//     32003 x 2560 17.9 / 21.1
+//   one fp32 row, against the generic kernel: up to 4096 values 3072 x 4096 8.3 / 7.3, 3328 x 3328 7.5 / 8.5, 4096 x 4096 8.6 / 9.1;
+//     longer 1024 x 9216 9.3 / 8.4, 1152 x 9216 9.6 / 12.7, 568 x 16384 11.5 / 10.3, 768 x 16384 11.7 / 11.8; 2560 x 2560 6.8 / 6.8
+//   two rows, against packed dots: 2048 x 4096 6.1 / 4.8, 2560 x 4096 7.4 / 7.5, 2048 x 8192 8.4 / 7.8, 2048 x 14336 11.0 / 11.9,
+//     768 x 22528 12.3 / 13.9
+//   three and four: 2048 x 11008 12.8 / 12.2, 2560 x 4096 8.0 / 9.1, 32003 x 5120 30 / 101
+//   five to eight: 1536 x 4096 10.1 / 9.7, 2048 x 3072 9.4 / 10.0, 1536 x 5120 11.4 / 14.8
+//   two fp32 rows, against the generic kernel: 1536 x 4096 7.9 / 6.5, 2048 x 4096 8.1 / 8.1, 1024 x 7936 11.0 / 8.6, 1536 x 6912 11.1 / 11.6
+bool gemv_tile_preferred(int format, int x_dtype, int64_t m, int64_t n_out, int64_t n_in) {
+  static const int always = dev_knob("TTQ_TILE_FIRST", 0);
+  if (!gemv_tile_competes(format, x_dtype, m, n_out, n_in)) return false;
+  if (always) return true;
+  const float mb = (float)(n_out * (n_in >> 8) * 210) * 1e-6f;
+  const bool shorter = n_in <= 4096;
+  if (x_dtype == kF32) {
+    if (m > 1) return n_out > (shorter ? 1536 : 1024);
+    return mb >= 7.f && (shorter ? n_out > 3072 : n_out > 1024 || (n_out >= 768 && n_in >= 14336));
+  }
+  if (m == 1) return shorter ? mb >= 27.f : mb >= 12.f && !(n_out > 1024 && n_out <= 2048 && n_in <= 16384);
+  if (m == 2) return n_out > 2048 || mb >= 18.f || n_in > 16384;
+  return m <= 4 ? n_out > 2048 : !shorter || n_out > 1792;
+}
+
+// Several rows, us: 21.5 / 134 / 431 MB 10.2 / 28.9 / 84 for two rows, 11.8 / 30 / 87 for four, 15.1 / 33.4 / 98 for eight.  fp32 rows,
+// which are three each: small matrices by the tiles that a wavefront has one after the other, one row 2048 x 4096 (one) 6.1,
+// 512 x 16128 (four) 11.5, two rows 4096 x 4096 (two) 7.9, 1024 x 6144 (three) 9.7.  The signed weights add a tenth to large ones, which
+// is left out: where the few-row kernel over rounded weights is faster by no more than that, the call keeps its precision.
 float gemv_tile_estimate_us(int x_dtype, int64_t m, int64_t n_out, int64_t n_in) {
   const float mb = (float)(n_out * (n_in >> 8) * 210) * 1e-6f;
-  return (x_dtype == kF32 ? 3 * m : m) <= 4 ? 5.f + mb / 5.2f : 8.3f + mb / 4.8f;
+  const float us = (x_dtype == kF32 ? 3 * m : m) <= 4 ? 5.f + mb / 5.2f : 8.3f + mb / 4.8f;
+  if (x_dtype != kF32) return us;
+  const int rows = m == 1 ? 2048 : 4096;             // a group of them for every compute unit
+  const float steps = (float)(n_in >> 8) * (m == 1 ? 1.f / 16 : 1.f / 8) * (float)((n_out + rows - 1) / rows);
+  return us < 4.2f + 1.9f * steps ? us : 4.2f + 1.9f * steps;
 }
 
 hipError_t launch_gemv_tile(int format, const void* w, const void* x, int x_dtype, void* y, int y_dtype, const void* bias,
