@@ -470,6 +470,7 @@ int ttq_linear_forward(const ttq_qlinear* layer, const void* x, int x_dtype, int
                                          layer->bias, layer->bias_dtype, m, n_out, n_in, s));
   }
   const bool block_fmt = layer->format == TTQ_Q4_K || layer->format == TTQ_Q6_K || layer->format == TTQ_Q8_0;
+  const auto few_margin = [&]() { return ttq::few_row_margin(layer->format, x_dtype, m, n_out, n_in); };
   // fp16 activations, five rows or more: the operator computes in the type of x, so the weights are rounded to fp16
   // (11 bits: the result stays in the 1e-3 class of the decode kernels) and multiplied on the fp16 matrix cores --
   // by the few-row kernel (64 rows per launch) or, from where it is cheaper, by the prefill GEMM over a packed fp16
@@ -487,9 +488,7 @@ int ttq_linear_forward(const ttq_qlinear* layer, const void* x, int x_dtype, int
     us_rounding = us_gemm < us_rounding ? us_gemm : us_rounding;
     const bool rounds = route == 2 || !newer || us_rounding < ttq::gemv_estimate_us(layer->format, x_dtype, m, n_out, n_in, false);
     const float us_gemv = ttq::gemv_estimate_us(layer->format, x_dtype, m, n_out, n_in);
-    // (several launches of the few-row kernel against one short round of the tiled kernel: the margin of the bf16
-    // chooser, whose estimate for the tiled kernel is fitted to full rounds and about a third too high for a short one)
-    if (rounds && us_gemm < (m > 64 ? us_few / 0.65f : us_few) && (route == 2 || us_gemm < us_gemv))
+    if (rounds && us_gemm < 1e29f && us_gemm < us_few / few_margin() && (route == 2 || us_gemm < us_gemv || us_few < us_gemv))
       return hip_status(ttq::launch_gemm_pc_x(layer->format, layer->qweight, x, x_dtype, y, y_dtype, layer->bias,
                                               layer->bias_dtype, m, n_out, n_in, s, true));
     if (rounds && us_few < 1e29f && (route == 2 || us_few < us_gemv)) {
@@ -536,7 +535,7 @@ int ttq_linear_forward(const ttq_qlinear* layer, const void* x, int x_dtype, int
     // same.  The small matrices, where the two agree to 3 us, stay with the kernel that takes any number of rows.)
     const bool integer_passes = (int64_t)n_out * n_in >= (int64_t)120 << 20;
     const float us_gemv = ttq::gemv_estimate_us(layer->format, x_dtype, m, n_out, n_in, integer_passes);
-    if (rounds && (m > 64 ? us_few / 0.65f : us_few) < us_gemm && (route == 2 || us_few < us_gemv)) {
+    if (rounds && us_few / few_margin() < us_gemm && (route == 2 || us_few < us_gemv)) {
       if (ttq::route_probe(ttq::kRouteGemmSkinnyF32ScaledF16)) return TTQ_OK;
       return hip_status(ttq::launch_gemm_skinny_f32(layer->format, layer->qweight, static_cast<const float*>(x), y, y_dtype,
                                                     layer->bias, layer->bias_dtype, m, n_out, n_in, s));

@@ -96,6 +96,9 @@ float gemm_pc_estimate_us(int format, int64_t m, int64_t n_out, int64_t n_in) {
   return c * (format == kQ8_0 ? 1.9f : (format == kQ6_K ? 1.4f : 1.f)) + 2.f;
 }
 
+// Whether a launch for this shape is divided along K.
+bool gemm_pc_splits_k(int64_t m, int64_t n_out, int64_t n_in) { return pc_choose(m, n_out, n_in, false).splits > 1; }
+
 // Launches of 256-row tiles read the activations from a copy in fragment order (ttq_gemm_pcd.h), made by one pass
 // over X into a workspace: with no X traffic through LDS their K loop is 6 % (64-column tiles) to 15 % (112-column
 // tiles) shorter, which pays for the pass (2.5 us + the bytes at about 7 TB/s, they come out of the caches) on every

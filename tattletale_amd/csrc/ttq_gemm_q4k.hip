@@ -400,19 +400,30 @@ static hipError_t launch_nj(const uint8_t* wb, const uint16_t* x, void* y, int y
   return hipErrorInvalidValue;
 }
 
-// The few-row kernel (ttq_gemm_skinny.hip: up to 64 rows, weights dequantized in registers, no tile
-// of W in LDS) where it exists for the shape and is estimated to be faster than the tiled kernel.
+// The few-row kernel (ttq_gemm_skinny.hip: up to 64 rows, weights dequantized in registers, no tile of W in LDS) is taken where it
+// exists for the shape and its estimate lies below this share of the tiled kernel's, whose own is fitted to full rounds and
+// about a third too high for a single short one.
+//   Several launches of it (65 rows and more): that third.  The streamed form, whose own estimate is the closer one, more: us in
+//     chunks / tiled, fp16 41488 x 1024 at 128 rows 38.5 / 34.4, 81808 x 768 at 100 49 / 41, 83312 x 2560 at 80 112 / 95, bf16 118848 x 768 at 128 71 / 63.
+//   One launch of the streamed form, which gives a wavefront all of K, where the tiled kernel would split K (few rows of weights; its
+//     estimate is up to twice too high there): bf16 27 x 3072 at 64 rows 18.6 / 11.8, Q4_K 1145 x 4096 at 37 19.4 / 14.2, fp32
+//     415 x 15360 at 40 71 / 47 (given up with it: 8538 x 15360 at 12 60 / 70).
+float few_row_margin(int format, int x_dtype, int64_t m, int64_t n_out, int64_t n_in) {
+  if (!gemm_skinny_streams(format, m < 64 ? m : 64, n_out, n_in)) return m > 64 ? 0.65f : 1.f;
+  if (m > 64) return x_dtype == kF32 ? 0.6f : 0.45f;
+  return gemm_pc_splits_k(m, n_out, n_in) ? 0.6f : 1.f;
+}
 static bool prefer_skinny(int format, int64_t m, int64_t n_out, int64_t n_in) {
-  return gemm_skinny_supported(format, m, n_out, n_in) &&
-         (!gemm_pc_supported(format, m, n_out, n_in, 112) ||
-          gemm_skinny_estimate_us(format, m, n_out, n_in) < gemm_pc_estimate_us(format, m, n_out, n_in));
+  if (!gemm_skinny_supported(format, m, n_out, n_in)) return false;
+  if (!gemm_pc_supported(format, m, n_out, n_in, 112)) return true;
+  const float us_few = gemm_skinny_estimate_us(format, m, n_out, n_in), us_pc = gemm_pc_estimate_us(format, m, n_out, n_in);
+  return us_few < us_pc && us_few < few_row_margin(format, kBF16, m, n_out, n_in) * us_pc;
 }
 
 // 65 .. 256 rows on a matrix with few columns (attention output, down projection: 4096 columns are 37 tiles of
 // 112 for 256 compute units) leave the tiled kernel one short round whose length is the latency of its K loop.
 // It then splits K over copies of the grid (ttq_gemm_pc.hip); where the rows are too short for that, two or
-// three launches of the few-row kernel, 64 rows each, can still be faster.  The margin covers the tiled
-// kernel's estimate, which is fitted to full rounds and is about a third too high for a single short one.
+// three launches of the few-row kernel, 64 rows each, can still be faster.
 static float skinny_chunks_estimate_us(int format, int64_t m, int64_t n_out, int64_t n_in) {
   const int64_t full = m / 64, rest = m % 64;
   float us = (float)full * gemm_skinny_estimate_us(format, 64, n_out, n_in);
@@ -422,7 +433,8 @@ static float skinny_chunks_estimate_us(int format, int64_t m, int64_t n_out, int
 static bool prefer_skinny_chunks(int format, int64_t m, int64_t n_out, int64_t n_in) {
   if (m <= 64 || m > 256 || !gemm_skinny_supported(format, 64, n_out, n_in)) return false;
   if (!gemm_pc_supported(format, m, n_out, n_in, 112)) return false;
-  return skinny_chunks_estimate_us(format, m, n_out, n_in) < 0.65f * gemm_pc_estimate_us(format, m, n_out, n_in);
+  return skinny_chunks_estimate_us(format, m, n_out, n_in) <
+         few_row_margin(format, kBF16, m, n_out, n_in) * gemm_pc_estimate_us(format, m, n_out, n_in);
 }
 
 bool gemm_supported(int format, int64_t m, int64_t n_out, int64_t n_in) {

@@ -636,7 +636,7 @@ static bool skinny_registers_supported(int format, int64_t m, int64_t n_out, int
 
 // The form that streams the weights through LDS (ttq_gemm_rows.hip): many weight rows, and outputs that are not whole groups of
 // eight.
-static bool use_rows(int format, int64_t m, int64_t n_out, int64_t n_in) {
+bool gemm_skinny_streams(int format, int64_t m, int64_t n_out, int64_t n_in) {
   return gemm_rows_supported(format, m, n_out, n_in) &&
          (gemm_rows_preferred(n_out) || !skinny_registers_supported(format, m, n_out, n_in));
 }
@@ -650,7 +650,7 @@ float gemm_skinny_registers_estimate_us(int format, int64_t m, int64_t n_out, in
 }
 
 float gemm_skinny_estimate_us(int format, int64_t m, int64_t n_out, int64_t n_in) {
-  if (use_rows(format, m, n_out, n_in)) return gemm_rows_estimate_us(format, m, n_out, n_in);
+  if (gemm_skinny_streams(format, m, n_out, n_in)) return gemm_rows_estimate_us(format, m, n_out, n_in);
   return skinny_choose(format, m, n_out, n_in, false).cost_us;
 }
 
@@ -677,7 +677,7 @@ hipError_t launch_gemm_skinny(int format, const void* w, const uint16_t* x, int 
   if (m == 0 || n_out == 0) return hipSuccess;
   if (y_dtype != kBF16 && y_dtype != kF32 && y_dtype != kF16) return hipErrorInvalidValue;
   const uint8_t* wb = static_cast<const uint8_t*>(w);
-  if ((x_dtype == kF16 || (x_dtype == kBF16 && !row_scale)) && use_rows(format, m, n_out, n_in))
+  if ((x_dtype == kF16 || (x_dtype == kBF16 && !row_scale)) && gemm_skinny_streams(format, m, n_out, n_in))
     return launch_gemm_rows(format, w, x, x_dtype, y, y_dtype, bias, bias_dtype, m, n_out, n_in, s, row_scale);
   if (x_dtype == kBF16) {
     if (row_scale) return hipErrorInvalidValue;      // (row factors come with the scaled fp16 copy of fp32 activations)

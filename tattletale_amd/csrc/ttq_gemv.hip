@@ -463,8 +463,8 @@ bool gemv_row_is_long(int format, int x_dtype, int64_t n_in) {
 // bf16 1536 x 4096 at 32 rows 28 and 39 (3072 x 4096 44 and 40).
 static float rows_exact_us(int64_t m, int64_t n_out, int64_t n_in) {
   const int64_t full = m / 64, rest = m % 64;
-  float us = full ? (float)full * 1.2f * gemm_rows_estimate_us(kQ6_K, 64, n_out, n_in) : 0.f;
-  if (rest) us += 1.2f * gemm_rows_estimate_us(kQ6_K, rest, n_out, n_in);
+  float us = full ? (float)full * 1.12f * gemm_rows_estimate_us(kQ6_K, 64, n_out, n_in) : 0.f;
+  if (rest) us += 1.12f * gemm_rows_estimate_us(kQ6_K, rest, n_out, n_in);
   return us;
 }
 static float tile_passes_us(int x_dtype, int64_t m, int64_t n_out, int64_t n_in) {

@@ -221,6 +221,7 @@ hipError_t launch_gemv_q4k_batch4(const void* w, const void* x, int x_dtype, voi
 // integer_kernels: with the kernels of ttq_gemv_tile.hip and the exact form of ttq_gemm_rows.hip among the decode kernels
 float gemv_estimate_us(int format, int x_dtype, int64_t m, int64_t n_out, int64_t n_in, bool integer_kernels = true);
 float gemm_pc_estimate_us(int format, int64_t m, int64_t n_out, int64_t n_in);
+bool gemm_pc_splits_k(int64_t m, int64_t n_out, int64_t n_in);
 int gemv_q4k_batch_tokens(int64_t m, int64_t n_in);
 
 // Compute units of the current device (256 when the query fails); cached per device ordinal.
@@ -236,6 +237,10 @@ hipError_t allow_large_lds(const void* kernel, LargeLds& state);
 // registers (ttq_gemm_skinny.hip).
 bool gemm_skinny_supported(int format, int64_t m, int64_t n_out, int64_t n_in);
 float gemm_skinny_estimate_us(int format, int64_t m, int64_t n_out, int64_t n_in);
+// whether a launch of the few-row kernel is its streamed form (ttq_gemm_rows.hip)
+bool gemm_skinny_streams(int format, int64_t m, int64_t n_out, int64_t n_in);
+// the few-row kernel is taken below this share of the tiled kernel's estimate
+float few_row_margin(int format, int x_dtype, int64_t m, int64_t n_out, int64_t n_in);
 // of the register kernel alone; 1e30 for shapes it does not take
 float gemm_skinny_registers_estimate_us(int format, int64_t m, int64_t n_out, int64_t n_in);
 // x: bf16 or fp16 activations (the weights are rounded once to the same type); y: bf16, fp16 or fp32.
