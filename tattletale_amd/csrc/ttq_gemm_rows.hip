@@ -328,10 +328,9 @@ bool gemm_rows_supported(int format, int64_t m, int64_t n_out, int64_t n_in) {
 // blocks leave wavefronts idle.  Measured at 16 rows, us, here / the register kernel, which splits K over its wavefronts: Q4_K
 // 28672 x 4096 (seven blocks) 22.7 / 26.2, 14336 x 4096 (three and a half) 16.6 / 14.4; Q6_K fp16 28672 x 8192 48 / 67,
 // 13824 x 5120 23.2 / 23.4, 5120 x 13824 48 / 30.
-// (the compute units are asked for once: the query of the current device is 0.1 us, and a call comes here several times)
 bool gemm_rows_preferred(int64_t n_out) {
-  static const int64_t cus = device_num_cus();
-  return (n_out + 15) / 16 >= 5 * cus;
+  const int64_t blocks = (n_out + 15) / 16;
+  return blocks >= 5 && blocks >= 5 * (int64_t)device_num_cus();      // (asked per device, as everywhere)
 }
 
 // A launch + passes x steps along K x (a step's chain of waits and reads + its tiles) + the outputs, fitted to 95 shapes of 31 to
