@@ -138,17 +138,27 @@ template <> struct XmRaw<bf16_tag> {
 // first.  The four bytes that a window starts in lie in two consecutive dwords; one byte permutation brings them into
 // string order (byte s of the string is byte s ^ 1 in memory), and a weight's state is a bit field of the result: the
 // first starts 0..7 bits below the top, which depends on the lane only where the number of bits per weight is odd.
-// (Two funnel-shift operands with their halves swapped first, as this was before, take two more instructions per window.)
+// (Two funnel-shift operands with their halves swapped first take two more instructions per window.)  With five bits, four
+// weights are 31 bits, more than what is left of 32 from the byte they start in, but not from the bit: there one funnel shift, and
+// one window, against two permutations, two windows and twice the reads: 4096 x 4096 one row 10.2 -> 9.7 us, 512 rows 50.7 -> 46.6.
 template <int BITS>
 struct XmLane {
-  static constexpr int kWin = BITS <= 4 ? 1 : 2;     // windows per four weights
-  static constexpr int kPer = 4 / kWin;
+  static constexpr bool kFunnel = BITS == 5;
+  static constexpr int kWin = BITS <= 5 ? 1 : 2;     // windows per four weights
   uint32_t at[kWin][2];                              // byte offsets of the two dwords in the tile
-  uint32_t sel[kWin];                                // byte selector
+  uint32_t sel[kWin];                                // byte selector (funnel: shift)
   uint32_t down;                                     // 4 if the lane's windows start four bits lower, else 0
   __device__ __forceinline__ void init(int lane) {
     const int j = lane & 15, q = lane >> 4;
     down = (BITS & 1) ? 4u * (q & 1) : 0u;
+    if constexpr (kFunnel) {
+      // (a window that starts on a dword boundary takes the pair one dword earlier and shifts by nothing)
+      const int bit = (16 * j + 4 * q) * BITS, o = bit & 31, d = (bit >> 5) - (o == 0);
+      at[0][0] = 4u * ((d + 8 * BITS) % (8 * BITS));
+      at[0][1] = 4u * ((d + 1) % (8 * BITS));
+      sel[0] = (32 - o) & 31;
+      return;
+    }
 #pragma unroll
     for (int w = 0; w < kWin; w++) {
       const int bit = (16 * j + 4 * q + 2 * w) * BITS;
@@ -166,13 +176,17 @@ struct XmLane {
   template <int CB, int W, int E, int HALF, bool LAST = false>
   __device__ __forceinline__ void code(uint32_t w, uint32_t& dst) const {
     constexpr int kTop = (2 * W * BITS) & 7;
-    if constexpr (BITS & 1) xm_code<CB, HALF, LAST>(__builtin_amdgcn_ubfe(w, field(W, E), 16), dst);
+    if constexpr ((BITS & 1) && !kFunnel) xm_code<CB, HALF, LAST>(__builtin_amdgcn_ubfe(w, field(W, E), 16), dst);
     else xm_code<CB, HALF, LAST>(__builtin_amdgcn_ubfe(w, 16 - kTop - E * BITS, 16), dst);
   }
   __device__ __forceinline__ uint32_t field(int w, int e) const { return 16u - (((uint32_t)(2 * w * BITS) + down) & 7u) - (uint32_t)(e * BITS); }
   template <int CB>
   __device__ __forceinline__ void decode(const uint32_t (&c)[kWin][2], uint32_t (&r)[2]) const {
-    const uint32_t w0 = __builtin_amdgcn_perm(c[0][1], c[0][0], sel[0]);
+    uint32_t w0;
+    if constexpr (kFunnel)
+      w0 = __builtin_amdgcn_alignbit(__builtin_amdgcn_alignbit(c[0][0], c[0][0], 16), __builtin_amdgcn_alignbit(c[0][1], c[0][1], 16), sel[0]);
+    else
+      w0 = __builtin_amdgcn_perm(c[0][1], c[0][0], sel[0]);
     if constexpr (kWin == 1) {
       code<CB, 0, 0, 0>(w0, r[0]);
       code<CB, 0, 1, 1>(w0, r[0]);

@@ -18,9 +18,11 @@
 // Weights.  A wavefront copies the tiles that it decodes into a ring of its own by LDS DMA, packed as they are in
 // memory, 16 tiles to a stage, and waits for nobody: there is no barrier until its tiles are done.  (With passes of 32 k-tiles
 // that all wavefronts staged together, every pass waited twice for the slowest one, and for the two that rotated its
-// activations.  us, one row, passes / rings: 28672 x 4096 3 bits 33.4 / 27.6, 6 bits 43.4 / 32.3; 14336 x 4096 5 bits 24.6 /
-// 19.9; 4096 x 14336 3 bits 18.7 / 17.7, eight rows 28.6 / 21.8; 4096 x 4096 2 .. 6 bits 9.1 / 8.9 / 10.0 / 10.0 / 12.4 and 8.3 / 8.95 / 9.3 / 10.3 /
-// 11.0, where the launch, the rotation and the hand-off are most of it.)
+// activations.  us, one row, passes / rings: 28672 x 4096 3 bits 30.7 / 24.9, 5 bits 35.8 / 27.3, 7 bits 43.9 / 30.5; 4096 x 14336 3 bits
+// 18.9 / 16.8, 6 bits 26.6 / 19.1; 4096 x 4096 1 .. 8 bits 8.0 / 8.65 / 8.5 / 9.7 / 9.7 / 12.1 / 11.2 / 12.6 and 8.2 / 8.0 / 8.5 / 8.7 / 9.7 /
+// 10.7 / 10.8 / 11.1; 2048 x 1024, where a slice is one group, 2 bits 5.7 / 6.0, 4 bits 6.0 / 6.2, 6 bits 6.8 / 6.7: there the passes were
+// 0.1 to 0.3 faster,
+// where the launch, the rotation and the hand-off are most of it.)
 //
 // Decode.  The matrix cores want from lane (j = lane % 16, q = lane / 16) the four weights k = 4q .. 4q+3 of channel j
 // of a tile: the windows that start at bit (16j + 4q + e) * bits, e = 0..3.  The lane reads the two dwords that hold
@@ -135,7 +137,7 @@ gemv_exl3_mfma_kernel(const uint16_t* __restrict__ trellis, const uint16_t* __re
       __hip_atomic_load(nslices > 1 ? reinterpret_cast<const uint32_t*>(accum) : reinterpret_cast<const uint32_t*>(trellis),
                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 
-  // ---- weights: stage s holds this wavefront's tiles of the groups 4s .. 4s+3 of the slice (past its end the last group's again)
+  // ---- weights: stage s holds this wavefront's tiles of the groups 4s .. 4s+3 of the slice (past its end what it has, again)
   const int64_t row_bytes = (int64_t)nt_n * G::kTileBytes;
   const uint8_t* wbase = reinterpret_cast<const uint8_t*>(trellis) + ((int64_t)grp * 8 + tcol) * G::kTileBytes +
                          (int64_t)(kt_begin + kpart * kXmTilesPerWave) * row_bytes;
@@ -143,10 +145,14 @@ gemv_exl3_mfma_kernel(const uint16_t* __restrict__ trellis, const uint16_t* __re
   const int stages = (groups + kXmStageGroups - 1) / kXmStageGroups;
   int64_t src[G::kReq];
   auto place = [&](int left) {                           // left: groups from the stage's first on
+    // (where the lanes past the last piece are more than none, they and those of absent groups repeat the last one: 2304 x 768, seven
+    // bits, 8.7 -> 7.0 us; whole requests repeat the last group: 3072 x 1024, eight bits, 6.7 against 7.0)
+    constexpr bool kWhole = G::kPieces % 64 == 0;
+    const int last = kWhole ? G::kPieces - 1 : min(left, kXmStageGroups) * (kXmTilesPerWave * 2 * BITS) - 1;
 #pragma unroll
     for (int r = 0; r < G::kReq; r++) {
-      const int p = min(64 * r + lane, G::kPieces - 1), t = p / (2 * BITS), c = p - t * (2 * BITS);
-      const int gl = min(t / kXmTilesPerWave, left - 1);
+      const int p = min(64 * r + lane, last), t = p / (2 * BITS), c = p - t * (2 * BITS);
+      const int gl = kWhole ? min(t / kXmTilesPerWave, left - 1) : t / kXmTilesPerWave;
       src[r] = (int64_t)(gl * 8 + t % kXmTilesPerWave) * row_bytes + 16 * c;
     }
   };
@@ -364,9 +370,12 @@ gemv_exl3_mfma_kernel(const uint16_t* __restrict__ trellis, const uint16_t* __re
   float handed = 0.f;
   if (nwords > 0) {
     // The slices of a group finish their decode within a fraction of a microsecond of each other, and a word asked for
-    // before it has reached the memory side costs a second round trip (about 0.9 us); 256 clocks of patience before
-    // the first look make the first look the only one (one to six units of 64 clocks measure the same).
-    __builtin_amdgcn_s_sleep(4);
+    // before it has reached the memory side costs a second round trip (about 0.9 us): 256 clocks of patience before
+    // the first look make it the only one.  64 are enough for slices of a few groups with a look at sixteen words, and up to three
+    // bits, where the decode is short.  us with 64 / 256 clocks: 2048 x 1024 two bits 6.05 / 6.19, four 6.22 / 6.35, 4096 x 4096 three
+    // 8.46 / 8.65, four 8.99 / 8.83, six 11.2 / 11.0, 1536 x 1536 (22 words) four 6.87 / 6.68.
+    if (BITS <= 3 || (groups < kXmStageGroups && nwords <= kHandoffBatch)) __builtin_amdgcn_s_sleep(1);
+    else __builtin_amdgcn_s_sleep(4);
     int d = 0;
     for (int r = wave >> 1; r >= ntok; r -= ntok) d++;
     const int e = tid - d * sums;
