@@ -187,8 +187,8 @@ typedef enum {
   TTQ_ROUTE_GEMV_DOT2_MULTI = 13,
   TTQ_ROUTE_GEMV_GENERIC = 14,
   TTQ_ROUTE_GEMV_LONG = 15,          /* rows longer than the staged kernels take: nothing staged in LDS */
-  TTQ_ROUTE_GEMM_ROWS_EXACT = 17,    /* the same arithmetic for 9-64 rows of fp16 activations */
-  TTQ_ROUTE_GEMV_TILE = 16,          /* Q6_K as integers on the 16-bit matrix cores, 1-8 rows */
+  TTQ_ROUTE_GEMV_TILE = 16,          /* Q6_K as integers on the 16-bit matrix cores, 1-8 rows to a pass (2 of fp32) */
+  TTQ_ROUTE_GEMM_ROWS_EXACT = 17,    /* the same arithmetic for 9-64 rows of fp16 activations to a launch */
   TTQ_ROUTE_GEMM_SKINNY_F32_SCALED_F16 = 19, /* fp32 activations, few rows: the few-row kernel in fp16 over a copy scaled row by row */
   TTQ_ROUTE_GEMM_PC = 20,            /* producer / consumer prefill GEMM */
   TTQ_ROUTE_GEMM_PC_SPLIT_K = 21,    /* ... in several copies along K (takes a workspace) */

@@ -1,5 +1,7 @@
-// Decode GEMV for Q6_K weights and one to eight activation rows on gfx950, any number of weight rows of any length: the
-// quants as small integers on the 16-bit matrix cores.
+// Decode GEMV for Q6_K weights and one to eight activation rows (one or two of fp32) on gfx950, any number of weight rows: the
+// quants as small integers on the 16-bit matrix cores.  All activations of a pass are in LDS, which bounds the rows' length:
+// 45056 values for one 16-bit row, 22528 for two, 11008 for three and four, 5120 for five to eight; 16384 for one fp32 row (the
+// decode kernels' own bound), 7936 for two.
 //
 // Operator: F.linear with a few activation rows (workspace/libtorch/src/abi/neural_nets.nim:64-81) over GGUF Q6_K blocks
 // { u8 ql[128]; u8 qh[64]; i8 scales[16]; f16 d } of 256 weights, w = d * scale[e / 16] * (q6[e] - 32).
@@ -42,7 +44,9 @@ namespace ttq {
 namespace {
 
 constexpr int kTlWaves = 8, kTlThreads = 64 * kTlWaves;
-constexpr int kTlDepth = 2;                // tiles in a wavefront's ring: one multiplied, one in flight (54 KiB a compute unit)
+constexpr int kTlDepth = 2;                // tiles in a wavefront's ring: one multiplied, one in flight (56 KiB a compute unit)
+
+static_assert(kTlDepth == 2, "slots and waits alternate");
 
 constexpr int kTlXBlock = 528;             // 256 activations in LDS: the four lanes of a product's k-set on different banks
 constexpr int kTlZeroBytes = 512;          // what the lanes off the block diagonal read
@@ -54,10 +58,11 @@ template <class XT> __device__ __forceinline__ float add_halves(float k, uint32_
 }
 // J: activation rows as the matrix cores see them, PARTS to an activation row (three for fp32).  KQ: blocks along K of a tile, of
 // 16 / KQ weight rows.
-template <class F, class XT, int J, int KQ, int PARTS>
+template <class XT, int J, int KQ, int PARTS>
 __global__ void __launch_bounds__(kTlThreads)
-gemv_tile_kernel(const uint8_t* __restrict__ w, const void* __restrict__ x, int n_out, int n_in, int depth, int m, int x_dtype,
-                 int y_dtype, void* __restrict__ y, const void* __restrict__ bias, int bias_dtype) {
+gemv_tile_kernel(const uint8_t* __restrict__ w, const void* __restrict__ x, int n_out, int n_in, int m, int y_dtype,
+                 void* __restrict__ y, const void* __restrict__ bias, int bias_dtype) {
+  using F = TlQ6K;
   extern __shared__ __attribute__((aligned(1024))) uint8_t tl_lds[];
   constexpr int JB = (J * KQ + 3) / 4, JI = J * KQ < 4 ? J * KQ : 4, R = 16 / KQ;
   constexpr int SB = F::kSub, M = J / PARTS;                    // activation rows at most
@@ -68,8 +73,8 @@ gemv_tile_kernel(const uint8_t* __restrict__ w, const void* __restrict__ x, int 
   const int nsb = n_in >> 8, tpr = (nsb + KQ - 1) / KQ;       // blocks and tiles of a row
   const int groups = (n_out + R - 1) / R;                      // of R rows
 
-  uint8_t* ring = tl_lds + wave * depth * F::kSlot;
-  uint8_t* zero = tl_lds + kTlWaves * depth * F::kSlot;
+  uint8_t* ring = tl_lds + wave * kTlDepth * F::kSlot;
+  uint8_t* zero = tl_lds + kTlWaves * kTlDepth * F::kSlot;
   float* sums = reinterpret_cast<float*>(zero + kTlZeroBytes);                  // [tile][chain][jb][4 g + pseudo row % 4]
   uint8_t* xs = reinterpret_cast<uint8_t*>(sums + (kSigned ? 0 : tpr * F::kChains * JB * 16));
   const uint32_t kpad = (uint32_t)tpr * KQ * 256u, xstride = (uint32_t)tpr * KQ * kTlXBlock;
@@ -126,14 +131,14 @@ gemv_tile_kernel(const uint8_t* __restrict__ w, const void* __restrict__ x, int 
     r_left--;
     const bool tail = r_k == tpr - 1;
     F::template request<KQ == 4>(L, lane, ring_lds + r_slot * F::kSlot, w, (int64_t)r_row * nsb + r_k * KQ, tail, tail && r_row == last_row0);
-    r_slot = r_slot == depth - 1 ? 0 : r_slot + 1;
+    r_slot ^= 1;
     r_k++;
     if (tail) {
       r_k = 0;
       r_row = first_row(++r_q);
     }
   };
-  for (int d = 0; d < depth; d++) request_next();
+  for (int d = 0; d < kTlDepth; d++) request_next();
 
   // ---- zeros: for the lanes off the block diagonal, and behind the rows
   if (tid < kTlZeroBytes / 16) reinterpret_cast<uint4*>(zero)[tid] = make_uint4(0, 0, 0, 0);
@@ -141,16 +146,11 @@ gemv_tile_kernel(const uint8_t* __restrict__ w, const void* __restrict__ x, int 
     const int blk = e >> 5, row = blk / (KQ > 1 ? KQ - 1 : 1), b = nsb + blk % (KQ > 1 ? KQ - 1 : 1);
     if (row < J && b < tpr * KQ) *reinterpret_cast<uint4*>(xs + row * xstride + kTlXBlock * b + 16 * (e & 31)) = make_uint4(0, 0, 0, 0);
   }
-  auto wait_later = [&](int later) {
-    if (later >= 3) sm_wait_vmcnt<3 * F::kRequests>();
-    else if (later == 2) sm_wait_vmcnt<2 * F::kRequests>();
-    else if (later == 1) sm_wait_vmcnt<F::kRequests>();
+  // (requests complete in order)
+  if constexpr (PARTS == 1) {                                   // the activations have landed: all but the first tiles
+    if (t1 - t0 >= 2) sm_wait_vmcnt<2 * F::kRequests>();
+    else if (t1 - t0 == 1) sm_wait_vmcnt<F::kRequests>();
     else sm_wait_vmcnt<0>();
-  };
-  if constexpr (PARTS == 1) {
-    const int out = min(t1 - t0, depth);
-    if (out >= 4) sm_wait_vmcnt<4 * F::kRequests>();
-    else wait_later(out);
   }
   sm_barrier();
   // ---- sums of the activations over sub-blocks, times what the sums of products start at
@@ -277,14 +277,15 @@ gemv_tile_kernel(const uint8_t* __restrict__ w, const void* __restrict__ x, int 
     Acts acts;
     load_acts(acts, k);
     const bool tail = k == tpr - 1;
-    wait_later(min(t1 - 1 - t, depth - 1));
+    if (t < t1 - 1) sm_wait_vmcnt<F::kRequests>();                // all but the next tile
+    else sm_wait_vmcnt<0>();
     typename F::Raw r;
     F::read(r, ring + slot * F::kSlot, L, (int64_t)row * nsb + k * KQ, tail, tail && row == last_row0);
     // (the slot is free for a later tile once the reads have returned)
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     request_next();
     multiply(r, acts);
-    slot = slot == depth - 1 ? 0 : slot + 1;
+    slot ^= 1;
     k++;
     if (tail || t == t1 - 1) {
       finish(q, tail && begun == 0, q == qa ? 0 : 1);
@@ -314,24 +315,23 @@ struct TlArgs {
   const void* x;
   void* y;
   const void* bias;
-  int m, n_out, n_in, x_dtype, y_dtype, bias_dtype;
+  int m, n_out, n_in, y_dtype, bias_dtype;
 };
 
 constexpr size_t kTlLds = 160 * 1024;
-template <class F>
-size_t tile_lds_bytes(int j, int kq, int parts, int64_t n_in, int depth) {
+size_t tile_lds_bytes(int j, int kq, int parts, int64_t n_in) {
+  using F = TlQ6K;
   const size_t jb = (j * kq + 3) / 4, tpr = ((n_in >> 8) + kq - 1) / kq;
-  return (size_t)kTlWaves * depth * F::kSlot + kTlZeroBytes + (parts > 1 ? 0 : tpr * F::kChains * jb * 64) + (size_t)j * (kTlXBlock * kq * tpr) +
+  return (size_t)kTlWaves * kTlDepth * F::kSlot + kTlZeroBytes + (parts > 1 ? 0 : tpr * F::kChains * jb * 64) + (size_t)j * (kTlXBlock * kq * tpr) +
          (size_t)2 * kTlWaves * j * (16 / kq) * 4;
 }
 
-template <class F, class XT, int J, int KQ, int PARTS = 1>
+template <class XT, int J, int KQ, int PARTS = 1>
 hipError_t launch_tile_j(const TlArgs& a, hipStream_t s) {
-  constexpr int depth = kTlDepth;
-  const size_t lds = tile_lds_bytes<F>(J, KQ, PARTS, a.n_in, depth);
+  const size_t lds = tile_lds_bytes(J, KQ, PARTS, a.n_in);
   if (lds > kTlLds) return hipErrorInvalidValue;
   if (route_probe(kRouteGemvTile)) return hipSuccess;      // (here, so that the query answers for the form that would run)
-  auto kernel = gemv_tile_kernel<F, XT, J, KQ, PARTS>;
+  auto kernel = gemv_tile_kernel<XT, J, KQ, PARTS>;
   static LargeLds configured;
   if (lds > 64 * 1024) {
     const hipError_t e = allow_large_lds(reinterpret_cast<const void*>(kernel), configured);
@@ -339,7 +339,7 @@ hipError_t launch_tile_j(const TlArgs& a, hipStream_t s) {
   }
   const int64_t groups = ((int64_t)a.n_out + 16 / KQ - 1) / (16 / KQ), cus = device_num_cus();
   hipLaunchKernelGGL(kernel, dim3((unsigned)(groups < cus ? groups : cus)), dim3(kTlThreads), lds, s, a.w, a.x, a.n_out, a.n_in,
-                     depth, a.m, a.x_dtype, a.y_dtype, a.y, a.bias, a.bias_dtype);
+                     a.m, a.y_dtype, a.y, a.bias, a.bias_dtype);
   return hipGetLastError();
 }
 
@@ -351,15 +351,15 @@ TlForm tile_form(int x_dtype, int64_t m, int64_t n_out, int64_t n_in) {
   // One row: four blocks to a tile, except where the last tile of long matrices' rows would be half empty (32003 x 2560 21.3 us
   // with four, 17.9 with two; 7168 x 3584 9.7 / 9.9).  Two take more LDS, and end at rows of 41216 values.
   const bool wide = (n_in >> 8) % 4 == 0 || n_out * (n_in >> 8) * 210 < (24 << 20);
-  return TlForm{1, wide || tile_lds_bytes<TlQ6K>(1, 2, 1, n_in, kTlDepth) > kTlLds ? 4 : 2};
+  return TlForm{1, wide || tile_lds_bytes(1, 2, 1, n_in) > kTlLds ? 4 : 2};
 }
 
-template <class F, class XT>
+template <class XT>
 hipError_t launch_tile_x(const TlArgs& a, const TlForm& f, hipStream_t s) {
-  if (f.j == 1) return f.kq == 4 ? launch_tile_j<F, XT, 1, 4>(a, s) : launch_tile_j<F, XT, 1, 2>(a, s);
-  if (f.j == 2) return launch_tile_j<F, XT, 2, 2>(a, s);
-  if (f.j == 4) return launch_tile_j<F, XT, 4, 1>(a, s);
-  return launch_tile_j<F, XT, 8, 1>(a, s);
+  if (f.j == 1) return f.kq == 4 ? launch_tile_j<XT, 1, 4>(a, s) : launch_tile_j<XT, 1, 2>(a, s);
+  if (f.j == 2) return launch_tile_j<XT, 2, 2>(a, s);
+  if (f.j == 4) return launch_tile_j<XT, 4, 1>(a, s);
+  return launch_tile_j<XT, 8, 1>(a, s);
 }
 
 }  // namespace
@@ -372,7 +372,7 @@ bool gemv_tile_supported(int format, int x_dtype, int64_t m, int64_t n_out, int6
   if (disabled || format != kQ6_K || n_in % 256 != 0 || m < 1 || m > 8 || n_out > 0x3FFFFFFF || n_in > (1 << 22)) return false;
   if (m > gemv_tile_rows(x_dtype)) return false;
   const TlForm f = tile_form(x_dtype, m, n_out, n_in);
-  return tile_lds_bytes<TlQ6K>(f.j, f.kq, x_dtype == kF32 ? 3 : 1, n_in, kTlDepth) <= kTlLds;
+  return tile_lds_bytes(f.j, f.kq, x_dtype == kF32 ? 3 : 1, n_in) <= kTlLds;
 }
 
 // Whether it competes with the other decode kernels at all: startup (the activations' sums, a barrier, one tile's chain) is some
@@ -435,11 +435,11 @@ hipError_t launch_gemv_tile(int format, const void* w, const void* x, int x_dtyp
                             int bias_dtype, int64_t m, int64_t n_out, int64_t n_in, hipStream_t s) {
   if (m == 0 || n_out == 0) return hipSuccess;
   if (format != kQ6_K) return hipErrorInvalidValue;
-  const TlArgs a{static_cast<const uint8_t*>(w), x, y, bias, (int)m, (int)n_out, (int)n_in, x_dtype, y_dtype, bias_dtype};
+  const TlArgs a{static_cast<const uint8_t*>(w), x, y, bias, (int)m, (int)n_out, (int)n_in, y_dtype, bias_dtype};
   const TlForm f = tile_form(x_dtype, m, n_out, n_in);
-  if (x_dtype == kF32) return f.j == 3 ? launch_tile_j<TlQ6K, bf16_tag, 3, 2, 3>(a, s) : launch_tile_j<TlQ6K, bf16_tag, 6, 1, 3>(a, s);
-  if (x_dtype == kF16) return launch_tile_x<TlQ6K, f16_tag>(a, f, s);
-  return launch_tile_x<TlQ6K, bf16_tag>(a, f, s);
+  if (x_dtype == kF32) return f.j == 3 ? launch_tile_j<bf16_tag, 3, 2, 3>(a, s) : launch_tile_j<bf16_tag, 6, 1, 3>(a, s);
+  if (x_dtype == kF16) return launch_tile_x<f16_tag>(a, f, s);
+  return launch_tile_x<bf16_tag>(a, f, s);
 }
 
 }  // namespace ttq

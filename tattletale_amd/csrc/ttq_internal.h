@@ -160,7 +160,8 @@ hipError_t launch_gemv_q6k_stream4(const void* w, const void* x, int x_dtype, vo
                                    const void* bias, int bias_dtype, int64_t m, int64_t n_out, int64_t n_in,
                                    hipStream_t s);
 
-// Q6_K as integers on the 16-bit matrix cores, one to eight activation rows (two of fp32), any shape (ttq_gemv_tile.hip).
+// Q6_K as integers on the 16-bit matrix cores, one to eight activation rows (two of fp32), any number of weight rows
+// (ttq_gemv_tile.hip).
 int gemv_tile_rows(int x_dtype);      // rows of a pass at most
 bool gemv_tile_supported(int format, int x_dtype, int64_t m, int64_t n_out, int64_t n_in);
 bool gemv_tile_competes(int format, int x_dtype, int64_t m, int64_t n_out, int64_t n_in);
