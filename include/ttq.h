@@ -189,11 +189,12 @@ typedef enum {
   TTQ_ROUTE_GEMV_LONG = 15,          /* rows longer than the staged kernels take: nothing staged in LDS */
   TTQ_ROUTE_GEMV_TILE = 16,          /* Q6_K as integers on the 16-bit matrix cores, 1-8 rows to a pass (2 of fp32) */
   TTQ_ROUTE_GEMM_ROWS_EXACT = 17,    /* the same arithmetic for 9-64 rows of fp16 activations to a launch */
+  TTQ_ROUTE_GEMM_ROWS = 18,          /* up to 64 rows, 16-bit: the few-row kernel's form that streams the weights through LDS */
   TTQ_ROUTE_GEMM_SKINNY_F32_SCALED_F16 = 19, /* fp32 activations, few rows: the few-row kernel in fp16 over a copy scaled row by row */
   TTQ_ROUTE_GEMM_PC = 20,            /* producer / consumer prefill GEMM */
   TTQ_ROUTE_GEMM_PC_SPLIT_K = 21,    /* ... in several copies along K (takes a workspace) */
   TTQ_ROUTE_GEMM_SKINNY = 22,        /* 17-64 rows */
-  TTQ_ROUTE_GEMM_SKINNY_CHUNKED = 23,
+  TTQ_ROUTE_GEMM_SKINNY_CHUNKED = 23, /* fp16 activations, or 64 rows a launch (of either form of the kernel) */
   TTQ_ROUTE_GEMM_Q4K_TILES = 24,     /* single-role tiled kernel: more than 4 GiB of activations */
   TTQ_ROUTE_GEMM_PC_BF16_COPY = 25,  /* TTQ_PRECISION_BF16_OK: fp32 activations rounded to bf16 by the packing pass */
   TTQ_ROUTE_GEMM_PC_PACKED = 26,     /* long launches: activations packed in fragment order first (takes a workspace) */

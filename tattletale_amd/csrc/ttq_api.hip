@@ -492,7 +492,9 @@ int ttq_linear_forward(const ttq_qlinear* layer, const void* x, int x_dtype, int
       return hip_status(ttq::launch_gemm_pc_x(layer->format, layer->qweight, x, x_dtype, y, y_dtype, layer->bias,
                                               layer->bias_dtype, m, n_out, n_in, s, true));
     if (rounds && us_few < 1e29f && (route == 2 || us_few < us_gemv)) {
-      if (ttq::route_probe(ttq::kRouteGemmSkinnyChunked)) return TTQ_OK;
+      if (ttq::route_probe(ttq::t_route_probe && m <= 64 && ttq::gemm_skinny_streams(layer->format, m, n_out, n_in)
+                               ? ttq::kRouteGemmRows : ttq::kRouteGemmSkinnyChunked))
+        return TTQ_OK;
       return hip_status(ttq::launch_gemm_skinny_chunked(layer->format, layer->qweight, static_cast<const uint16_t*>(x),
                                                         x_dtype, y, y_dtype, layer->bias, layer->bias_dtype, m, n_out,
                                                         n_in, s));
@@ -588,6 +590,7 @@ const char* ttq_route_name(int route) {
     case TTQ_ROUTE_GEMV_LONG: return "gemv_long";
     case TTQ_ROUTE_GEMM_ROWS_EXACT: return "gemm_rows_exact";
     case TTQ_ROUTE_GEMV_TILE: return "gemv_tile";
+    case TTQ_ROUTE_GEMM_ROWS: return "gemm_rows";
     case TTQ_ROUTE_GEMM_SKINNY_F32_SCALED_F16: return "gemm_skinny_f32_scaled_f16";
     case TTQ_ROUTE_GEMM_PC: return "gemm_pc";
     case TTQ_ROUTE_GEMM_PC_SPLIT_K: return "gemm_pc_split_k";

@@ -453,7 +453,8 @@ hipError_t launch_gemm(int format, const void* w, const uint16_t* x_bf16, void* 
                        int bias_dtype, int64_t m, int64_t n_out, int64_t n_in, hipStream_t s) {
   if (m == 0 || n_out == 0) return hipSuccess;
   if (prefer_skinny(format, m, n_out, n_in))
-    TTQ_ROUTE(kRouteGemmSkinny, launch_gemm_skinny(format, w, x_bf16, kBF16, y, y_dtype, bias, bias_dtype, m, n_out, n_in, s));
+    TTQ_ROUTE((t_route_probe && gemm_skinny_streams(format, m, n_out, n_in) ? kRouteGemmRows : kRouteGemmSkinny),
+              launch_gemm_skinny(format, w, x_bf16, kBF16, y, y_dtype, bias, bias_dtype, m, n_out, n_in, s));
   if (prefer_skinny_chunks(format, m, n_out, n_in))
     TTQ_ROUTE(kRouteGemmSkinnyChunked,
               launch_gemm_skinny_chunked(format, w, x_bf16, kBF16, y, y_dtype, bias, bias_dtype, m, n_out, n_in, s));

@@ -34,6 +34,7 @@ enum : int {
   kRouteGemvLong = 15,
   kRouteGemvTile = 16,
   kRouteGemmRowsExact = 17,
+  kRouteGemmRows = 18,
   kRouteGemmSkinnyF32ScaledF16 = 19,
   kRouteGemmPc = 20,
   kRouteGemmPcSplitK = 21,

@@ -18,11 +18,13 @@ DT = {"f32": torch.float32, "f16": torch.float16, "bf16": torch.bfloat16}
 TOL = {"bf16": 3 * 2.0 ** -8, "f16": 3 * 2.0 ** -11, "f32": 4.2 * 2.0 ** -11}
 
 
-def run(fmt, n_out, n_in, m, xk, bias=True):
+def run(fmt, n_out, n_in, m, xk, bias=True, route=None):
     gen = torch.Generator(DEV).manual_seed(n_out + m)
     w = packed_to_dev(random_blocks(fmt, n_out * (n_in // 256), seed=n_out + n_in))
     b = torch.randn(n_out, device=DEV, generator=gen).to(DT[xk]) if bias else None
     lay = QuantLinear.init(w, fmt, n_in, n_out, bias=b)
+    if route is not None:
+        assert lay.route(m, DT[xk], torch.float32) == route
     x = torch.randn(m, n_in, device=DEV, generator=gen).to(DT[xk])
     wd = QL.dequantize(fmt, w, n_out, n_in).double()
     ref = x.double() @ wd.T + (b.double() if bias else 0)
@@ -35,28 +37,56 @@ def run(fmt, n_out, n_in, m, xk, bias=True):
     return lay, x, y
 
 
-@pytest.mark.parametrize("fmt", [F.Q4_K, F.Q6_K])
-@pytest.mark.parametrize("n_out,n_in", [(20480, 256), (20487, 768), (65537, 512), (33000, 1280), (20481, 2304)])
-@pytest.mark.parametrize("m,xk", [(9, "f16"), (16, "bf16"), (17, "f16"), (33, "bf16"), (48, "f16"), (49, "bf16"), (64, "f16"), (64, "bf16"),
-                                  (12, "f32"), (50, "f32")])
+# (fp32 activations: the kernel runs on their scaled fp16 copy wherever the matrix has five blocks of rows to a compute unit, or an
+# odd number of them; the route names the copy)
+ROUTE = {"bf16": "gemm_rows", "f16": "gemm_rows", "f32": "gemm_skinny_f32_scaled_f16"}
+ROWS = [(9, "f16"), (16, "bf16"), (17, "f16"), (33, "bf16"), (48, "f16"), (49, "bf16"), (64, "f16"), (64, "bf16"), (12, "f32"), (50, "f32")]
+LARGE = [(20480, 256), (20488, 768), (65544, 512), (33000, 1280), (20488, 2304)]
+
+
+def decodes(fmt, n_out, n_in, m, xk):
+    """Calls of the lists above that passes of the decode kernels serve faster."""
+    if fmt == F.Q4_K:
+        return xk != "f32" and (m <= 16 or (n_out == 65544 and xk == "f16" and m < 64))
+    return (n_out, n_in, m) == (20480, 256, 9)
+
+
+@pytest.mark.parametrize("fmt,n_out,n_in,m,xk", [(f, o, i, m, x) for f in (F.Q4_K, F.Q6_K) for o, i in LARGE for m, x in ROWS
+                                                 if not decodes(f, o, i, m, x)])
 def test_many_weight_rows(fmt, n_out, n_in, m, xk):
-    run(fmt, n_out, n_in, m, xk)
+    run(fmt, n_out, n_in, m, xk, route=ROUTE[xk])
+
+
+@pytest.mark.parametrize("fmt,n_out,n_in,m", [(F.Q6_K, o, i, m) for o, i in [(20487, 768), (65537, 512), (20481, 2304)] for m in (9, 17, 33, 64)] +
+                         [(F.Q4_K, o, i, m) for o, i in [(20487, 768), (65537, 512), (20481, 2304)] for m in (33, 64)] +
+                         [(f, o, i, m) for o in (1, 3, 15, 17, 100, 255, 1003, 4097) for f, i, m in
+                          [(F.Q4_K, 256, 17), (F.Q4_K, 768, 40), (F.Q4_K, 1024, 64), (F.Q6_K, 256, 32), (F.Q6_K, 768, 48), (F.Q6_K, 1024, 64)]])
+def test_any_number_of_outputs(fmt, n_out, n_in, m):
+    run(fmt, n_out, n_in, m, "bf16", route="gemm_rows")
+
+
+@pytest.mark.parametrize("fmt,n_out,m", [(F.Q4_K, 15, 64), (F.Q4_K, 1003, 64), (F.Q4_K, 4097, 31), (F.Q6_K, 1003, 64), (F.Q6_K, 4097, 31)])
+def test_any_number_of_outputs_fp32(fmt, n_out, m):
+    run(fmt, n_out, 1024, m, "f32", route=ROUTE["f32"])
 
 
 @pytest.mark.parametrize("fmt", [F.Q4_K, F.Q6_K])
 @pytest.mark.parametrize("n_out", [1, 3, 15, 17, 100, 255, 1003, 4097])
 @pytest.mark.parametrize("m,xk", [(5, "f16"), (16, "f16"), (31, "f32"), (64, "f16"), (7, "bf16"), (40, "bf16")])
 def test_outputs_that_are_not_whole_groups_of_eight(fmt, n_out, m, xk):
+    """The same bounds for the calls around them, most of which the decode kernels take: fp16 ones with such a number of outputs
+    decode at every row count."""
     run(fmt, n_out, 1024, m, xk)
 
 
 @pytest.mark.parametrize("fmt", [F.Q4_K, F.Q6_K])
 def test_non_finite_rows_stay_alone_and_rows_do_not_depend_on_their_neighbours(fmt):
-    lay, x, y = run(fmt, 20487, 1280, 21, "f16", bias=False)
+    lay, x, y = run(fmt, 20488, 1280, 21, "f16", bias=False, route="gemm_rows")
     z = x.clone()
     z[20, 1279] = float("inf")
     got = lay.forward(z, out_dtype=torch.float32)
     assert not torch.isfinite(got[20]).any() and torch.equal(got[:20], y[:20])
+    assert lay.route(18, torch.float16, torch.float32) == "gemm_rows"
     assert torch.equal(lay.forward(x[:18], out_dtype=torch.float32), y[:18])
 
 
@@ -71,7 +101,7 @@ def test_exact_form(n_out, n_in, m):
     raw = random_blocks(F.Q6_K, n_out * (n_in // 256), seed=n_out)
     w = packed_to_dev(raw)
     lay = QuantLinear.init(w, F.Q6_K, n_in, n_out, precision=F.PRECISION_F32_SCALES)
-    assert lay.route(m, torch.float16, torch.float32) in ("gemm_rows_exact", "gemv_tile")
+    assert lay.route(m, torch.float16, torch.float32) == ("gemv_tile" if (n_out, m) == (3001, 9) else "gemm_rows_exact")
     x = torch.randn(m, n_in, device=DEV, generator=gen).half()
     wd = QL.dequantize(F.Q6_K, w, n_out, n_in).double()
     blk = w.view(-1, 210)

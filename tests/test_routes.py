@@ -48,12 +48,36 @@ PINNED = [
     ("down projection of a 53248-wide MLP, decode", Q4_K, 16384, 53248, 1, BF16, F32, 0, "gemv_dot2"),
     ("rows beyond 65536 values", Q4_K, 4096, 65536 + 256, 1, BF16, F32, 0, "gemv_long"),
     ("fp32 activations beyond 16384 values", Q8_0, 4096, 16384 + 32, 1, F32, F32, 0, "gemv_long"),
+    ("6-bit projection 5120x5120, decode", Q6_K, 5120, 5120, 1, F16, F16, 0, "gemv_tile"),
+    ("LM head of an odd vocabulary, decode", Q6_K, 32003, 5120, 1, F16, F32, 0, "gemv_tile"),
+    ("LM head, eight rows", Q6_K, 128256, 4096, 8, BF16, F32, 0, "gemv_tile"),
+    ("6-bit projection, one fp32 row", Q6_K, 5120, 5120, 1, F32, F32, 0, "gemv_tile"),
+    ("LM head of an odd vocabulary, 43 fp16 rows", Q6_K, 32003, 5120, 43, F16, F32, 0, "gemm_rows_exact"),
+    ("LM head, 43 fp16 rows", Q6_K, 152064, 3584, 43, F16, F32, 0, "gemm_rows"),
+    ("gate||up of a wide MLP, 43 fp16 rows", Q4_K, 37888, 3584, 43, F16, F16, 0, "gemm_rows"),
+    ("LM head of an odd vocabulary, 33 bf16 rows", Q6_K, 32003, 5120, 33, BF16, F32, 0, "gemm_rows"),
+    # few rows of weights: the kernels that give a wavefront a row of its own, or the tiled one
+    ("short 6-bit matrix, four rows", Q6_K, 1536, 4096, 4, BF16, BF16, 0, "gemv_dot2_multi"),
+    ("short 6-bit matrix, two rows", Q6_K, 758, 8192, 2, F16, F16, 0, "gemv_dot2_multi"),
+    ("short 6-bit matrix, long rows, decode", Q6_K, 1280, 13568, 1, BF16, BF16, 0, "gemv_dot2"),
+    ("6-bit projection 3072x4096, one fp32 row", Q6_K, 3072, 4096, 1, F32, F32, 0, "gemv_generic"),
+    ("odd number of outputs, 37 rows", Q4_K, 1145, 4096, 37, BF16, BF16, 0, "gemm_pc_split_k"),
+    ("odd number of outputs, 100 rows", Q6_K, 638, 768, 100, BF16, BF16, 0, "gemm_pc"),
+    ("many rows of weights, 278 fp16 rows", Q6_K, 26816, 256, 278, F16, F16, 0, "gemm_pc_f16"),
 ]
 
 
 @pytest.mark.parametrize("what,fmt,n_out,n_in,m,xd,yd,bits,want", PINNED, ids=[p[0] for p in PINNED])
 def test_benchmark_and_model_shapes_reach_their_kernels(what, fmt, n_out, n_in, m, xd, yd, bits, want):
     assert route(fmt, n_out, n_in, m, xd, yd, bits) == want
+
+
+def test_many_exact_rows_of_a_small_matrix_take_one_launch():
+    for n_out, n_in, m, xd in ((960, 6656, 267, F32), (1024, 6144, 8, F32), (2560, 4096, 64, F32), (1024, 6144, 2, F32)):
+        assert route(Q6_K, n_out, n_in, m, xd, F32, precision=_lib.PRECISION_F32_SCALES) == "gemv_generic"
+    assert route(Q6_K, 1536, 4096, 32, BF16, BF16, precision=_lib.PRECISION_F32_SCALES) == "gemv_dot2_multi"
+    for n_out, n_in, m, xd in ((131071, 512, 221, F32), (5120, 5120, 64, F32), (5120, 5120, 64, BF16), (3072, 4096, 32, BF16)):
+        assert route(Q6_K, n_out, n_in, m, xd, F32, precision=_lib.PRECISION_F32_SCALES) == "gemv_tile"
 
 
 def test_precision_flags_steer_the_route():
