@@ -106,8 +106,8 @@ template <int BITS, int CB, typename XT>
 __global__ void __launch_bounds__(kXmThreads)
 gemv_exl3_mfma_kernel(const uint16_t* __restrict__ trellis, const uint16_t* __restrict__ suh,
                       const uint16_t* __restrict__ svh, const XT* __restrict__ x, void* __restrict__ y, int y_dtype,
-                      const void* __restrict__ bias, int bias_dtype, int m, int n_out, int n_in, int slice_tiles,
-                      int chunk_groups, unsigned long long* __restrict__ accum, int poll_limit) {
+                      const void* __restrict__ bias, int bias_dtype, int m, int n_out, int n_in, int slice_groups,
+                      int short_slices, int chunk_groups, unsigned long long* __restrict__ accum, int poll_limit) {
   using G = XmGeom<BITS>;
   extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
   _Float16* xs = reinterpret_cast<_Float16*>(lds + G::kRingBytes);
@@ -118,9 +118,11 @@ gemv_exl3_mfma_kernel(const uint16_t* __restrict__ trellis, const uint16_t* __re
   const int grp = blockIdx.x, slice = blockIdx.y, nslices = gridDim.y;
   const int t0 = blockIdx.z * kXmTok;
   const int ntok = min(kXmTok, m - t0), cols = 2 * ntok;
-  const int nt_n = n_out >> 4, kt_n = n_in >> 4;
-  const int kt_begin = slice * slice_tiles;
-  const int groups = (min(kt_n, kt_begin + slice_tiles) - kt_begin) >> 3;        // Hadamard groups of this slice
+  const int nt_n = n_out >> 4;
+  // Hadamard groups of this slice: slice_groups, and one more from short_slices on
+  const int longer = slice - short_slices;
+  const int kt_begin = 8 * (slice * slice_groups + max(longer, 0));
+  const int groups = slice_groups + (longer >= 0 ? 1 : 0);
   const int col = lane & 15, q = lane >> 4;
   const int xstride = chunk_groups * 128 + kXmColPad;
   float* inv_s = reinterpret_cast<float*>(xs + cols * xstride);                  // [group of the chunk][column]
@@ -458,16 +460,21 @@ Exl3Plan exl3_mfma_plan(int64_t m, int64_t n_out, int64_t n_in) {
   Exl3Plan p;
   p.groups = (int)(n_out / 128);
   p.row_groups = (int)((m + kXmTok - 1) / kXmTok);
-  const int kt_n = (int)(n_in / 16);
   const int64_t units = (int64_t)p.groups * p.row_groups;
   const int cus = device_num_cus();
-  // enough slices to put a workgroup on every compute unit, each a whole number of Hadamard groups
+  // Enough slices to put a workgroup on every compute unit, each a whole number of Hadamard groups, as few as leave the longest as
+  // long as it is, and no two more than one group apart.  The longest are the last ones: a last slice that is done before the
+  // others asks again and again for words that they have yet to write, which holds up the writers (us, all but the last slice
+  // equally long and the last what is left / the extra groups in the first slices / in the last ones: 7168 x 1792, 14 groups in
+  // four slices, one row of six bits 14.0 / 10.1 / 10.0, eight rows 22.4 / 14.2 / 12.1; 5120 x 5120 eight rows of two bits
+  // 18.7 / 15.4 / 13.2; the one shape of 30 that loses, 9984 x 2816 with 22 groups in three, 13.4 / 13.3 / 14.1).
   int64_t want = units >= cus ? 1 : cus / units;
-  if (want > kt_n / 8) want = kt_n / 8;
-  int tiles = (int)((kt_n + want - 1) / want);
-  tiles = (tiles + 7) / 8 * 8;
-  p.slice_tiles = tiles;
-  p.slices = (kt_n + tiles - 1) / tiles;
+  const int k_groups = (int)(n_in / 128);
+  if (want > k_groups) want = k_groups;
+  const int longest = (int)((k_groups + want - 1) / want);
+  p.slices = (k_groups + longest - 1) / longest;
+  p.slice_groups = k_groups / p.slices;
+  p.short_slices = p.slices - k_groups % p.slices;
   p.accum_words = p.slices > 1 ? 8 + units * p.slices * kXmKSplit * kXmTok * 128 : 0;   // 8 control words in front
   return p;
 }
@@ -484,7 +491,7 @@ static hipError_t xm_launch(const Exl3Plan& p, const uint16_t* trellis, const ui
   const dim3 grid((unsigned)p.groups, (unsigned)p.slices, (unsigned)p.row_groups), block(kXmThreads);
   // activations in LDS: the whole slice, or as many whole stages of the ring as fit
   const int cols = 2 * (int)(m < kXmTok ? m : kXmTok), room = kXmLds - XmGeom<BITS>::kRingBytes;
-  int chunk = p.slice_tiles / 8;
+  int chunk = p.slice_groups + (p.short_slices < p.slices ? 1 : 0);
   if (xm_x_bytes(cols, chunk) > room) {
     chunk = (room - xm_x_bytes(cols, 0)) / (xm_x_bytes(cols, 1) - xm_x_bytes(cols, 0));
     chunk = chunk / kXmStageGroups * kXmStageGroups;
@@ -495,8 +502,8 @@ static hipError_t xm_launch(const Exl3Plan& p, const uint16_t* trellis, const ui
   const hipError_t e = allow_large_lds(reinterpret_cast<const void*>(kernel), configured);
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(kernel, grid, block, lds, s, trellis, suh, svh,
-                     static_cast<const XT*>(x), y, y_dtype, bias, bias_dtype, (int)m, (int)n_out, (int)n_in, p.slice_tiles,
-                     chunk, accum, g_exl3_poll_limit.load(std::memory_order_relaxed));
+                     static_cast<const XT*>(x), y, y_dtype, bias, bias_dtype, (int)m, (int)n_out, (int)n_in, p.slice_groups,
+                     p.short_slices, chunk, accum, g_exl3_poll_limit.load(std::memory_order_relaxed));
   return hipGetLastError();
 }
 

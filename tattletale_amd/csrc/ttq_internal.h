@@ -362,7 +362,8 @@ hipError_t launch_gemm_exl3(const uint16_t* trellis, const uint16_t* suh, const 
 // dimension is sliced and how many 64-bit accumulator words a sliced launch needs (zero before and
 // after every launch).
 struct Exl3Plan {
-  int groups, row_groups, slices, slice_tiles;
+  int groups, row_groups, slices;
+  int slice_groups, short_slices;      // Hadamard groups of a slice, one more of those from short_slices on
   int64_t accum_words;
 };
 Exl3Plan exl3_mfma_plan(int64_t m, int64_t n_out, int64_t n_in);

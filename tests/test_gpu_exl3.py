@@ -285,3 +285,26 @@ def test_exl3_prefill_full_shape_4096x4096_m512_sampled_rows():
     assert np.all(np.isfinite(y))
     for i in (0, 63, 64, 255, 448, 511):
         assert rel_l2(y[i], oracle.exl3_gemv_f64(T, suh, svh, x[i])) <= 2e-2, i
+
+
+@pytest.mark.parametrize("n_out,n_in", [(7168, 1792), (4352, 3328), (5120, 1280), (10240, 1792), (2560, 6912), (384, 1408), (16384, 3840)])
+@pytest.mark.parametrize("bits,m", [(2, 1), (3, 8), (6, 7), (5, 3)])
+def test_slices_of_unequal_length(n_out, n_in, bits, m):
+    """Hadamard groups along K that are no multiple of the slices (14, 26, 10, 14, 54, 11 and 30 of them).  Activations carry 22 bits
+    and sums are fp32 over up to 6912 values: 2^-22 + 2^-24 sqrt(6912) of the result's size at most in the square mean, 5e-6."""
+    gen = torch.Generator(DEV).manual_seed(n_out + m)
+    tr = torch.randint(0, 256, (n_out * n_in * bits // 8,), dtype=torch.uint8, device=DEV, generator=gen)
+    suh, svh = (((torch.rand(n, device=DEV, generator=gen) + 0.5) * (torch.randint(0, 2, (n,), device=DEV, generator=gen) * 2 - 1)).half()
+                for n in (n_in, n_out))
+    x = torch.randn(m, n_in, device=DEV, generator=gen).half()
+    h = torch.ones(1, 1, dtype=torch.float64, device=DEV)
+    for _ in range(7):
+        h = torch.cat([torch.cat([h, h], 1), torch.cat([h, -h], 1)], 0) / 2 ** 0.5
+    T = QL.dequantize_exl3(tr, n_out, n_in, bits).double()
+    xr = ((x.double() * suh.double()).view(-1, 128) @ h).view(m, n_in)
+    want = ((xr @ T.T).reshape(-1, 128) @ h).view(m, n_out) * svh.double()
+    lay = QuantLinear.init(tr, F.EXL3, n_in, n_out, suh=suh, svh=svh, bits=bits)
+    assert lay.route(m, torch.float16, torch.float32) == "exl3_gemv_sliced"
+    y = lay.forward(x, out_dtype=torch.float32)
+    assert ((y.double() - want).norm(dim=-1) / want.norm(dim=-1)).max().item() <= 5e-6
+    assert torch.equal(y[:1], lay.forward(x[:1], out_dtype=torch.float32))
