@@ -397,7 +397,8 @@ bool gemv_tile_competes(int format, int x_dtype, int64_t m, int64_t n_out, int64
 //     (2048 x 22528 12.6 / 13.8); rows of up to 4096 values 7168 x 3584 (21 MB) 9.7 / 8.4, 13824 x 2560 (29 MB) 10.7 / 11.0,
 //     32003 x 2560 17.9 / 21.1
 //   one fp32 row, against the generic kernel: up to 4096 values 3072 x 4096 8.3 / 7.3, 3328 x 3328 7.5 / 8.5, 4096 x 4096 8.6 / 9.1;
-//     longer 1024 x 9216 9.3 / 8.4, 1152 x 9216 9.6 / 12.7, 568 x 16384 11.5 / 10.3, 768 x 16384 11.7 / 11.8; 2560 x 2560 6.8 / 6.8
+//     longer 1024 x 9216 9.3 / 8.4, 1152 x 9216 9.6 / 12.7, 768 x 15104 11.2 / 10.5,
+//     896 x 14336 11.0 / 10.7, 1024 x 14336 11.2 / 11.8; 2560 x 2560 6.8 / 6.8
 //   two rows, against packed dots: 2048 x 4096 6.1 / 4.8, 2560 x 4096 7.4 / 7.5, 2048 x 8192 8.4 / 7.8, 2048 x 14336 11.0 / 11.9,
 //     768 x 22528 12.3 / 13.9
 //   three and four: 2048 x 11008 12.8 / 12.2, 2560 x 4096 8.0 / 9.1, 32003 x 5120 30 / 101
@@ -411,7 +412,7 @@ bool gemv_tile_preferred(int format, int x_dtype, int64_t m, int64_t n_out, int6
   const bool shorter = n_in <= 4096;
   if (x_dtype == kF32) {
     if (m > 1) return n_out > (shorter ? 1536 : 1024);
-    return mb >= 7.f && (shorter ? n_out > 3072 : n_out > 1024 || (n_out >= 768 && n_in >= 14336));
+    return mb >= 7.f && (shorter ? n_out > 3072 : n_out >= (n_in >= 14336 ? 1024 : 1025));
   }
   if (m == 1) return shorter ? mb >= 27.f : mb >= 12.f && !(n_out > 1024 && n_out <= 2048 && n_in <= 16384);
   if (m == 2) return n_out > 2048 || mb >= 18.f || n_in > 16384;

@@ -60,6 +60,8 @@ PINNED = [
     ("short 6-bit matrix, four rows", Q6_K, 1536, 4096, 4, BF16, BF16, 0, "gemv_dot2_multi"),
     ("short 6-bit matrix, two rows", Q6_K, 758, 8192, 2, F16, F16, 0, "gemv_dot2_multi"),
     ("short 6-bit matrix, long rows, decode", Q6_K, 1280, 13568, 1, BF16, BF16, 0, "gemv_dot2"),
+    ("short 6-bit matrix, long rows, one fp32 row", Q6_K, 896, 14336, 1, F32, F32, 0, "gemv_generic"),
+    ("short 6-bit matrix, three fp32 rows", Q6_K, 2560, 2560, 3, F32, F32, 0, "gemv_generic"),
     ("6-bit projection 3072x4096, one fp32 row", Q6_K, 3072, 4096, 1, F32, F32, 0, "gemv_generic"),
     ("odd number of outputs, 37 rows", Q4_K, 1145, 4096, 37, BF16, BF16, 0, "gemm_pc_split_k"),
     ("odd number of outputs, 100 rows", Q6_K, 638, 768, 100, BF16, BF16, 0, "gemm_pc"),
