@@ -363,7 +363,7 @@ hipError_t launch_gemm_exl3(const uint16_t* trellis, const uint16_t* suh, const 
 // after every launch).
 struct Exl3Plan {
   int groups, row_groups, slices;
-  int slice_groups, short_slices;      // Hadamard groups of a slice, one more of those from short_slices on
+  int slice_groups;                    // Hadamard groups of the shortest slice
   int64_t accum_words;
 };
 Exl3Plan exl3_mfma_plan(int64_t m, int64_t n_out, int64_t n_in);
