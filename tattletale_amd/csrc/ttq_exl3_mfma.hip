@@ -20,9 +20,8 @@
 // that all wavefronts staged together, every pass waited twice for the slowest one, and for the two that rotated its
 // activations.  us, one row, passes / rings: 28672 x 4096 3 bits 30.7 / 24.9, 5 bits 35.8 / 27.3, 7 bits 43.9 / 30.5; 4096 x 14336 3 bits
 // 18.9 / 16.8, 6 bits 26.6 / 19.1; 4096 x 4096 1 .. 8 bits 8.0 / 8.65 / 8.5 / 9.7 / 9.7 / 12.1 / 11.2 / 12.6 and 8.2 / 8.0 / 8.5 / 8.7 / 9.7 /
-// 10.7 / 10.8 / 11.1; 2048 x 1024, where a slice is one group, 2 bits 5.7 / 6.0, 4 bits 6.0 / 6.2, 6 bits 6.8 / 6.7: there the passes were
-// 0.1 to 0.3 faster,
-// where the launch, the rotation and the hand-off are most of it.)
+// 10.5 / 10.7 / 11.1; 2048 x 1024, where a slice is one group, 2 bits 5.86 / 6.09, 4 bits 6.04 / 6.26, 6 bits 6.7 / 6.5: there the passes
+// were 0.2 faster up to five bits, and the launch, the rotation and the hand-off are most of it.)
 //
 // Decode.  The matrix cores want from lane (j = lane % 16, q = lane / 16) the four weights k = 4q .. 4q+3 of channel j
 // of a tile: the windows that start at bit (16j + 4q + e) * bits, e = 0..3.  The lane reads the two dwords that hold
@@ -151,12 +150,12 @@ gemv_exl3_mfma_kernel(const uint16_t* __restrict__ trellis, const uint16_t* __re
     // (where the lanes past the last piece are more than none, they and those of absent groups repeat the last one: 2304 x 768, seven
     // bits, 8.7 -> 7.0 us; whole requests repeat the last group: 3072 x 1024, eight bits, 6.7 against 7.0)
     constexpr bool kWhole = G::kPieces % 64 == 0;
-    const int last = kWhole ? G::kPieces - 1 : min(left, kXmStageGroups) * (kXmTilesPerWave * 2 * BITS) - 1;
+    const uint32_t last = kWhole ? G::kPieces - 1 : (uint32_t)min(left, kXmStageGroups) * (kXmTilesPerWave * 2 * BITS) - 1;
 #pragma unroll
     for (int r = 0; r < G::kReq; r++) {
-      const int p = min(64 * r + lane, last), t = p / (2 * BITS), c = p - t * (2 * BITS);
-      const int gl = kWhole ? min(t / kXmTilesPerWave, left - 1) : t / kXmTilesPerWave;
-      src[r] = (int64_t)(gl * 8 + t % kXmTilesPerWave) * row_bytes + 16 * c;
+      const uint32_t p = min(64u * r + (uint32_t)lane, last), t = p / (2u * BITS), c = p - t * (2u * BITS);
+      const uint32_t gl = kWhole ? min(t / kXmTilesPerWave, (uint32_t)left - 1u) : t / kXmTilesPerWave;
+      src[r] = (int64_t)((uint64_t)(gl * 8 + t % kXmTilesPerWave) * (uint64_t)row_bytes) + 16u * c;
     }
   };
   place(groups);
@@ -183,8 +182,11 @@ gemv_exl3_mfma_kernel(const uint16_t* __restrict__ trellis, const uint16_t* __re
   uint2 sv;
   const uint16_t* sp;
   const XT* xp;
+  // (item / ng by a reciprocal, an integer division being 0.15 to 0.3 us of a launch of several rows: a quotient below 8 is off by
+  // 8 * 2^-22 at most and 0.5 / ng from the next whole number, with ng below 320 for what LDS holds)
+  auto row_of = [&](int item, int ng) { return (int)(((float)item + 0.5f) * __builtin_amdgcn_rcpf((float)ng)); };
   auto x_place = [&](int g0, int ng, int item) {
-    const int it = min(item, ntok * ng - 1), t = ntok == 1 ? 0 : it / ng, gl = it - t * ng;
+    const int it = min(item, ntok * ng - 1), t = row_of(it, ng), gl = it - t * ng;
     const int64_t k = (int64_t)kt_begin * 16 + (int64_t)(g0 + gl) * 128 + 4 * l32;
     sp = suh + k;
     xp = x + (int64_t)(t0 + t) * n_in + k;
@@ -196,7 +198,7 @@ gemv_exl3_mfma_kernel(const uint16_t* __restrict__ trellis, const uint16_t* __re
   };
   auto x_stage = [&](int g0, int ng) {
     for (int item = hw; item < ntok * ng; item += kXmThreads / 32) {
-      const int t = ntok == 1 ? 0 : item / ng, gl = item - t * ng;
+      const int t = row_of(item, ng), gl = item - t * ng;
       float v[4];
       xv.get(v);
       v[0] *= f16_bits_to_f32((uint16_t)sv.x);
