@@ -21,9 +21,10 @@
 // rounding beyond), the block's d in fp32 on the sums: 1.4e-4 from the float64 product where rounded weights are at 2.0e-4,
 // and one instruction for two weights instead of five.
 //
-// Measured (before: the register kernel; from 32 bf16 rows the tiled GEMM), us: Q6_K fp16 152064 x 3584 at 16 / 43 / 64 rows
-// 179 / 191 / 222 -> 101 / 127 / 157, 128256 x 4096 at 16 rows 156 -> 91; Q4_K 37888 x 3584 34 / 50 / 63 -> 26 / 33 / 38; bf16 32003 x
-// 5120 at 16 rows 100 -> 36.  Exact, 128257 x 4096 fp16 at 43 rows 2417 -> 155 (passes of four rows in packed dots).
+// Measured (before: the register kernel; on odd numbers of outputs the tiled GEMM), us: Q6_K fp16 152064 x 3584 at 16 / 43 / 64 rows
+// 179 / 194 / 224 -> 99 / 125 / 153, 128256 x 4096 at 16 / 43 158 / 170 -> 92 / 117, bf16 157 / 167 -> 96 / 122; Q4_K fp16 37888 x 3584 at
+// 43 / 64 50 / 64 -> 33 / 36; bf16 32003 x 5120 at 16 rows 100 -> 35.  Exact, 128257 x 4096 fp16 at 43 rows 2412 -> 161 (passes of four
+// rows in packed dots).
 #include "ttq_internal.h"
 #include "ttq_tile_common.h"
 

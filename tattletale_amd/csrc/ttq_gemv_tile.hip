@@ -32,11 +32,12 @@
 //
 // What bounds it: the requests.  They alone take 69 us for 128256 x 4096 (431 MB) in runs of 840 bytes and 80 in runs of 210
 // (KQ = 1), the arithmetic alone 52 to 61, both together 81 (5.3 TB/s); whole-line requests would take 64, but operands then
-// start at any dword of LDS, where pairs of dwords take three times as long as 16 bytes on their own boundary: 85.  A third
+// start at any dword of LDS, where pairs of dwords take three times as long as 16 bytes on their own boundary: 85.  (Parts switched
+// off in forms that are not kept.  Counters at eight rows: LDS busy 76 % of the time, 42 % in conflicts, vector units 56 %, matrix cores 17 %.)  A third
 // ring slot, sixteen wavefronts, operands of four tiles in registers: no gain.  Measured (before: packed-dot or generic
-// kernel, passes of the several-row int8 kernel), us: 32003 x 5120 fp16 one row 43.7 -> 30, two 55.7 -> 29.9, four 101.6 -> 30.5,
-// eight 189 -> 34; fp32 one row 52.0 -> 33.6; 5120 x 5120 fp16 12.2 -> 9.4, four rows 19.6 -> 12; 5120 x 13824 19.8 -> 16.9;
-// 128256 x 4096 bf16 at eight rows 152.7 -> 98, fp32 one row 122 -> 105; 1024 x 41472 bf16 19.1 -> 13.1.
+// kernel, passes of the several-row int8 kernel), us: 32003 x 5120 fp16 one row 45.3 -> 27.5, two 56.9 -> 28.4, four 101.8 -> 29.3,
+// eight 188 -> 32.1; fp32 one row 56.9 -> 34.1; 5120 x 5120 fp16 12.0 -> 8.8, four rows 19.5 -> 11.2; 5120 x 13824 19.6 -> 16.3;
+// 128256 x 4096 bf16 at eight rows 152 -> 96, fp32 one row 120 -> 102; 1024 x 41472 bf16 18.2 -> 12.3.
 #include "ttq_internal.h"
 #include "ttq_tile_common.h"
 

@@ -498,10 +498,14 @@ class QuantGatedMLP:
     # 125 / 118 at 512 rows, 416 / 371 at 1792): prompts of those lengths keep the faster form.
     FUSED_GEMM_MIN_ROWS = 2048
     # 17 to 64 rows: the same entry point runs the few-row kernel with the activation in its epilogue, one launch and one
-    # (rows, 2 * intermediate) round trip less (28672 x 4096 at 32 rows 33.9 / 35.1 us, 6144 x 1024 5.8 / 8.1), and the same
-    # fp32 sums.  Below nine rows the decode kernels for several rows plus silu_and_mul are faster on wide layers
-    # (28672 x 4096 at 8 rows 26.8 / 23.0, 27648 x 5120 43.5 / 28.7); from 9 to 16 rows they are not (26.7 / 29.7 and
-    # 40.4 / 42.0 at 16) and are taken all the same.
+    # (rows, 2 * intermediate) round trip less, and the same fp32 sums.  It is faster where the separate GEMM would be the
+    # same kernel (fused / separate, us, at 32 rows 6144 x 1024 6.0 / 8.3, 12288 x 2048 10.1 / 12.4, 17920 x 1536 17.1 / 19.4);
+    # wide layers (20480 weight rows and more) have a plain GEMM that streams its weights through LDS and no fused form of
+    # it, and the fused launch is taken for its sums although it costs time (28672 x 4096 at 32 rows 35.1 / 28.7, at 64
+    # 35.1 / 34.2, 27648 x 5120 40.3 / 32.9, 37888 x 3584 46.2 / 30.3).  Below nine rows the decode kernels for several rows
+    # plus silu_and_mul are faster on wide layers (28672 x 4096 at 8 rows 27.4 / 24.0, 27648 x 5120 44.4 / 27.8).  From 9 to
+    # 16 rows either is (at 16 28672 x 4096 27.0 / 29.4, 37888 x 3584 35.2 / 40.8, 27648 x 5120 40.3 / 29.0); the separate
+    # launches are taken.
     FUSED_FEW_ROWS = (17, 64)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:

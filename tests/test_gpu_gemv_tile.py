@@ -1,4 +1,4 @@
-"""The Q6_K decode kernel for one to eight rows of any length (route ``gemv_tile``): edges of its tiles (4, 8 and 16 weight
+"""The Q6_K decode kernel for one to eight rows (route ``gemv_tile``): edges of its tiles (4, 8 and 16 weight
 rows by 4, 2 and 1 blocks), of the workgroups' shares, of the rows' ends and of the matrix's end.
 
 The float64 product over the library's own dense copy of the weights (bit-exact against the oracle, test_gpu_dequant.py) is
