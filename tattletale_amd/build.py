@@ -35,6 +35,7 @@ SOURCES = [
     "ttq_gemv_q8_mfma.hip",
     "ttq_gemv_q8_win.hip",
     "ttq_gemv_tile.hip",
+    "ttq_gemv_short.hip",
     "ttq_gemv_q4k_batch.hip",
     "ttq_gemv_q4k_batch4.hip",
     "ttq_gemm_q4k.hip",

@@ -493,6 +493,22 @@ static ManyRows many_rows(int format, int x_dtype, int64_t m, int64_t n_out, int
   return rows ? ManyRows::kRowsExact : ManyRows::kPasses;
 }
 
+// Small matrices take the kernel that reads everything at once, but for calls of Q6_K that the tile kernel has: one or two
+// fp32 rows, and any of 8 million weights and more.
+bool gemv_short_first(int format, int x_dtype, int64_t m, int64_t n_out, int64_t n_in) {
+  if (!gemv_short_preferred(format, x_dtype, m, n_out, n_in)) return false;
+  const bool large = n_out * n_in >= 8000000;
+  if (format != kQ6_K || !(large || (x_dtype == kF32 && m <= 2))) return true;
+  return !gemv_tile_preferred(format, x_dtype, m, n_out, n_in) && !(large && many_rows(format, x_dtype, m, n_out, n_in) != ManyRows::kOther);
+}
+
+// (reported as the family whose calls it takes: fp32 arithmetic, or 16-bit activations of the K formats)
+hipError_t launch_gemv_short_routed(int format, const void* w, const void* x, int x_dtype, void* y, int y_dtype, const void* bias,
+                                    int bias_dtype, int64_t m, int64_t n_out, int64_t n_in, hipStream_t s) {
+  const int id = format == kQ8_0 || x_dtype == kF32 ? kRouteGemvGeneric : (m == 1 ? kRouteGemvDot2 : kRouteGemvDot2Multi);
+  TTQ_ROUTE(id, launch_gemv_short(format, w, x, x_dtype, y, y_dtype, bias, bias_dtype, m, n_out, n_in, s));
+}
+
 hipError_t launch_gemv(int format, const void* w, const void* x, int x_dtype, void* y, int y_dtype,
                        const void* bias, int bias_dtype, int64_t m, int64_t n_out, int64_t n_in,
                        hipStream_t s) {
@@ -505,6 +521,10 @@ hipError_t launch_gemv(int format, const void* w, const void* x, int x_dtype, vo
       default: return hipErrorInvalidValue;
     }
   }
+  // (16-bit rows of Q4_K: the operator alone, calls of the GEMV itself with one row and with several stay within
+  // 2e-6 of each other there, as the kernels below do)
+  if (!(format == kQ4_K && x_dtype != kF32) && gemv_short_first(format, x_dtype, m, n_out, n_in))
+    return launch_gemv_short_routed(format, w, x, x_dtype, y, y_dtype, bias, bias_dtype, m, n_out, n_in, s);
   const ManyRows many = many_rows(format, x_dtype, m, n_out, n_in);
   if (many != ManyRows::kOther) {
     const int64_t per_pass = gemv_tile_rows(x_dtype);
@@ -584,6 +604,12 @@ float gemv_estimate_us(int format, int x_dtype, int64_t m, int64_t n_out, int64_
   // rows of any length: a pass over the weights per activation row (72 MB in 24.6 us, 155 MB in 51 us, 463 MB in 122 us)
   if (gemv_row_is_long(format, x_dtype, n_in)) return (float)m * (mb / 3.5f + 3.f);
   if (integer_kernels) {
+    // (never more than the estimate without it: no call that decoded is moved to rounded weights by the better guess; five rows of 16 bits
+    // and more keep the rounding kernels that they have, 2432 x 1024 Q8_0 fp16 at six rows 4.4 there and 4.9)
+    if ((x_dtype == kF32 || m <= 4) && gemv_short_first(format, x_dtype, m, n_out, n_in)) {
+      const float us = gemv_short_estimate_us(format, x_dtype, m, n_out, n_in), old = gemv_estimate_us(format, x_dtype, m, n_out, n_in, false);
+      return us < old ? us : old;
+    }
     const ManyRows many = many_rows(format, x_dtype, m, n_out, n_in);
     if (many == ManyRows::kRowsExact) return rows_exact_us(m, n_out, n_in);
     if (many == ManyRows::kPasses) return tile_passes_us(x_dtype, m, n_out, n_in);
