@@ -638,12 +638,12 @@ int64_t ttq_workspace_bytes(const ttq_qlinear* layer, int64_t m, int x_dtype) {
   // (fp16 activations beyond 64 rows may take the prefill GEMM over a packed fp16 copy; fp32 ones over a scaled
   // fp16 copy, or a bf16 copy where the layer allows it)
   const int copy_dtype = (x_dtype == TTQ_F16 && m > 64) || x_dtype == TTQ_F32 ? x_dtype : TTQ_BF16;
-  int64_t scratch = ((int64_t)ttq::gemm_pc_packed_bytes(m, n_out, n_in, copy_dtype) + 255) & ~(int64_t)255;
+  int64_t scratch = ((int64_t)ttq::gemm_pc_packed_bytes(layer->format, m, n_out, n_in, copy_dtype) + 255) & ~(int64_t)255;
   int64_t partials = (int64_t)ttq::device_num_cus() * (16 * 4 * (16 * 4 + 1) * 4);
   const int64_t rows[3] = {m, block_rows, m % kGemmRows};
   for (int64_t r : rows) {
     if (r <= 0) continue;
-    const int64_t p = (int64_t)ttq::gemm_pc_partials_bytes(r, n_out, n_in);
+    const int64_t p = (int64_t)ttq::gemm_pc_partials_bytes(layer->format, copy_dtype, r, n_out, n_in);
     if (p > partials) partials = p;
   }
   return header + scratch + ((partials + 255) & ~(int64_t)255);

@@ -527,8 +527,8 @@ __device__ __forceinline__ void pc_epilogue(f32x4_t (&acc)[MB][NJ], const PcEpi&
 
 // 64 k of a producer thread's row (chunk C of the 256 k in `r`), dequantized, rounded to bf16 and stored as B
 // fragments into W stage `buf` of the tile at LDS address sw_addr.  whalf / wj / wn: the thread's half of every
-// 32-byte chunk, its column block and its column inside the block.
-template <int NJ, int FMT, int ABL, int C, class XT = bf16_tag>
+// 32-byte chunk, its column block and its column inside the block.  PART: only `lo` (0), only `hi` (1), both (2).
+template <int NJ, int FMT, int ABL, int C, class XT = bf16_tag, int PART = 2>
 __device__ __forceinline__ void pc_dequant_to_lds(const typename WFmt<FMT>::Raw& r, int buf, int whalf, int wj, int wn,
                                                   uint32_t sw_addr) {
   using WF = WFmt<FMT>;
@@ -553,34 +553,39 @@ __device__ __forceinline__ void pc_dequant_to_lds(const typename WFmt<FMT>::Raw&
   } else if constexpr (WF::kWholeKsub) {
     // k = 32*half + e -> ksub `half`, groups 0..3
     const uint32_t base = sw_addr + (uint32_t)(buf * kWUnits + whalf * (NJ * 64) + wj * 64 + wn) * 16u;
-    lds_store16(base, lo[0], lo[1], lo[2], lo[3]);
-    lds_store16(base + 256u, lo[4], lo[5], lo[6], lo[7]);
-    lds_store16(base + 512u, hi[0], hi[1], hi[2], hi[3]);
-    lds_store16(base + 768u, hi[4], hi[5], hi[6], hi[7]);
+    if constexpr (PART != 1) {
+      lds_store16(base, lo[0], lo[1], lo[2], lo[3]);
+      lds_store16(base + 256u, lo[4], lo[5], lo[6], lo[7]);
+    }
+    if constexpr (PART != 0) {
+      lds_store16(base + 512u, hi[0], hi[1], hi[2], hi[3]);
+      lds_store16(base + 768u, hi[4], hi[5], hi[6], hi[7]);
+    }
   } else {
     // k = 16*half + e  -> ksub 0, groups 2*half and 2*half+1; k = 32 + 16*half + e: ksub 1
     const uint32_t base = sw_addr + (uint32_t)(buf * kWUnits + (wj * 4 + 2 * whalf) * 16 + wn) * 16u;
-    lds_store16(base, lo[0], lo[1], lo[2], lo[3]);
-    lds_store16(base + 256u, lo[4], lo[5], lo[6], lo[7]);
-    lds_store16(base + NJ * 1024u, hi[0], hi[1], hi[2], hi[3]);
-    lds_store16(base + NJ * 1024u + 256u, hi[4], hi[5], hi[6], hi[7]);
+    if constexpr (PART != 1) {
+      lds_store16(base, lo[0], lo[1], lo[2], lo[3]);
+      lds_store16(base + 256u, lo[4], lo[5], lo[6], lo[7]);
+    }
+    if constexpr (PART != 0) {
+      lds_store16(base + NJ * 1024u, hi[0], hi[1], hi[2], hi[3]);
+      lds_store16(base + NJ * 1024u + 256u, hi[4], hi[5], hi[6], hi[7]);
+    }
   }
 }
 
 // The W producer role (wavefronts 4-7 of either kernel): thread pt (0..255) owns one row of the tile and half of
 // every 32-byte chunk; it loads the packed blocks, dequantizes 64 k per step and writes the B fragments into the
 // double-buffered W tile at LDS address sw_addr, keeping the step barrier `bar`.
-template <int NJ, int FMT, bool FUSE, int ABL, class XT = bf16_tag, typename Bar>
-__device__ __forceinline__ void pc_produce_w(const uint8_t* __restrict__ w, int pt, int n0, int n_out, int row_blocks,
-                                             int block0, int nblocks, uint32_t sw_addr, Bar&& bar) {
+template <int NJ, int FMT, bool FUSE, int ABL, class XT, int PART, typename Bar>
+__device__ __forceinline__ void pc_produce_w_part(const uint8_t* __restrict__ w, int pt, int n0, int n_out, int row_blocks,
+                                                  int block0, int nblocks, uint32_t sw_addr, Bar&& bar) {
   constexpr int BN = NJ * 16;
   constexpr int kWUnits = 2 * NJ * 64;
   // thread -> (tile row, 16-byte half of every 32-byte chunk); with BN = 112 the last 32
   // threads mirror threads 0..31 (same loads, same LDS writes of the same values)
-  // (a 64-column tile needs only half of the producer threads: the others just keep the barriers)
-  constexpr bool kSpare = 4 * BN <= 256;
-  const bool widle = kSpare && pt >= 2 * BN;
-  const int wt = pt < 2 * BN ? pt : (kSpare ? pt % (2 * BN) : pt - 2 * BN);
+  const int wt = pt < 2 * BN ? pt : pt - 2 * BN;
   // the two halves of a row in adjacent lanes: a 64-lane load then touches 32 rows, not 64
   const int wr = wt >> 1, whalf = wt & 1;
   // clamped: rows past the end are never stored
@@ -591,13 +596,12 @@ __device__ __forceinline__ void pc_produce_w(const uint8_t* __restrict__ w, int 
   const uint8_t* wptr = w + (int64_t)row_blocks * WF::kUnitBytes * (int64_t)wrow + (int64_t)block0 * WF::kUnitBytes;
   const int wj = wr >> 4, wn = wr & 15;
   auto load_w = [&](WRaw& dst, int b) {
-    if (widle || (ABL & 16) != 0) return;
+    if ((ABL & 16) != 0) return;
     // past the end: a harmless re-read
     WF::load(dst, wptr + WF::kUnitBytes * (int64_t)min(b, nblocks - 1), whalf);
   };
   auto dequant_to_lds = [&](const WRaw& r, auto cc, int buf) {
-    if (widle) return;
-    pc_dequant_to_lds<NJ, FMT, ABL, decltype(cc)::value, XT>(r, buf, whalf, wj, wn, sw_addr);
+    pc_dequant_to_lds<NJ, FMT, ABL, decltype(cc)::value, XT, PART>(r, buf, whalf, wj, wn, sw_addr);
   };
   using I0 = std::integral_constant<int, 0>;
   using I1 = std::integral_constant<int, 1>;
@@ -628,6 +632,29 @@ __device__ __forceinline__ void pc_produce_w(const uint8_t* __restrict__ w, int 
     do_block(wa, wb, wc, b);
     if (b + 1 < nblocks) do_block(wb, wc, wa, b + 1);
     if (b + 2 < nblocks) do_block(wc, wa, wb, b + 2);
+  }
+}
+
+// Tiles of 64 columns have work for 128 threads of that kind, two wavefronts: a pair of threads shares it there, one makes the
+// weights of the first 32 k of a step, the other those of the last.  A SIMD starts a vector instruction of one wavefront every
+// five clocks at best, so the chain of the two producing wavefronts, some 90 (Q4_K) to 150 (Q6_K) instructions a step, was what a
+// step took: 5120 x 5120 Q6_K at 333 rows 53 -> 39 us, 4096 x 4096 Q4_K at 512 rows 34 -> 28, 4096 x 14336 Q6_K 100 -> 87.  Not Q8_0, whose
+// halves would both read the chunks with the scale and the middle of a block (2304 x 8192 at 400 rows 55 -> 70): half of its producers
+// keep the barriers only.
+template <int NJ, int FMT, bool FUSE, int ABL, class XT = bf16_tag, typename Bar>
+__device__ __forceinline__ void pc_produce_w(const uint8_t* __restrict__ w, int pt, int n0, int n_out, int row_blocks,
+                                             int block0, int nblocks, uint32_t sw_addr, Bar&& bar) {
+  if constexpr (4 * NJ * 16 <= 256 && WFmt<FMT>::kWholeKsub) {
+    if (pt < 2 * NJ * 16) {
+      pc_produce_w_part<NJ, FMT, FUSE, ABL, XT, 2>(w, pt, n0, n_out, row_blocks, block0, nblocks, sw_addr, bar);
+    } else {
+      for (int s = -1; s < 4 * nblocks; s++) bar();
+    }
+  } else if constexpr (4 * NJ * 16 <= 256) {
+    if (pt < 2 * NJ * 16) pc_produce_w_part<NJ, FMT, FUSE, ABL, XT, 0>(w, pt, n0, n_out, row_blocks, block0, nblocks, sw_addr, bar);
+    else pc_produce_w_part<NJ, FMT, FUSE, ABL, XT, 1>(w, pt - 2 * NJ * 16, n0, n_out, row_blocks, block0, nblocks, sw_addr, bar);
+  } else {
+    pc_produce_w_part<NJ, FMT, FUSE, ABL, XT, 2>(w, pt, n0, n_out, row_blocks, block0, nblocks, sw_addr, bar);
   }
 }
 

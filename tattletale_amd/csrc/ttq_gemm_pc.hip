@@ -28,61 +28,128 @@ static hipError_t launch_pc_tile(const uint8_t* wb, const uint16_t* x, void* y, 
   return launch_pc_grid<FMT, MB, NJ, FUSE>(wb, x, y, y_dtype, bias, bias_dtype, m, n_out, n_in, sp, s);
 }
 
-// Tile choice.  A workgroup owns 64*MB rows x 16*NJ columns (8*NJ outputs when fused); the grid
-// should fill the 256 CUs without a nearly empty last round.  Cost model: rounds of workgroups x
-// (64-k steps x time per step of the tile shape + a fixed cost per workgroup), both measured
-// (microseconds; 14336 x 4096 and x 8192 at 2048 rows).  Smaller tiles are cheaper per step --
-// down to the latency of the producers' load / dequantize / store / barrier chain, about 0.45 us
-// -- but dequantize every weight for fewer rows.
-struct PcTile { int mb, nj; float step_us; };
-static const PcTile kPcTiles[] = {{4, 7, 0.87f}, {4, 4, 0.68f}, {2, 7, 0.585f}, {2, 4, 0.55f}, {1, 7, 0.46f}, {1, 4, 0.52f}};
-constexpr float kPcFixedUs = 6.f;
+// Tile choice.  A workgroup owns 64 * mb rows x 16 * nj columns (8 * nj outputs when fused).
+struct PcTile { int mb, nj; };
+static const PcTile kPcTiles[] = {{4, 7}, {4, 4}, {2, 7}, {2, 4}, {1, 7}, {1, 4}};
+constexpr int kPcTileCount = 6;
+static const int kPcSplits[] = {1, 2, 4, 7, 8};
 
-// A grid that leaves most compute units idle (few columns x few rows: the attention output and down projections
-// at a few hundred rows) is also split along K, 2 / 4 / 7 / 8 ways while all copies still fit one round: the
-// length of a short round is the latency of its K loop.  What the meeting of the copies costs (measured, 1024 /
-// 4096 / 14336 columns x 4096 / 14336 inputs at 128 .. 1024 rows): a consumer stores its partial sums, counts,
-// and the last one loads the copies one after the other -- 2 + copies trips to the memory side (3 for two
-// copies), each the longer the more accumulators a lane holds -- and the partial sums cross the memory system
-// twice at about 4 TB/s.
-struct PcChoice { int tile, splits; float cost_us; };
-
-static float pc_split_us(const PcTile& t, int splits, int64_t padded_rows, int64_t padded_cols) {
-  const float trip = 0.9f + 0.06f * (float)(t.mb * t.nj);
-  const float trips = splits == 2 ? 3.f : 2.f + (float)splits;
-  return trips * trip + 2.f * (float)splits * (float)padded_rows * (float)padded_cols * 4.f / 4.0e6f;
-}
-
-static PcChoice pc_choose(int64_t m, int64_t n_out, int64_t n_in, bool fuse) {
-  static const int forced = dev_knob("TTQ_GEMM_TILE", -1);
-  static const int forced_splits = dev_knob("TTQ_GEMM_SPLITS", 0);   // A/B: 1 = never split, n = n ways where possible
-  static const int kSplits[] = {1, 2, 4, 7, 8};
+// Whether a call comes here at all: rounds of workgroups x (64-k steps x time per step of the tile + a fixed cost per workgroup).
+// The kernels that compete (few rows, decode) were weighed against these figures, and which calls may have their weights
+// rounded follows from them, so they stay when the kernels behind them get faster.
+struct PcRouteTile { int mb, nj; float step_us; };
+static const PcRouteTile kPcRouteTiles[] = {{4, 7, 0.87f}, {4, 4, 0.68f}, {2, 7, 0.585f}, {2, 4, 0.55f}, {1, 7, 0.46f}, {1, 4, 0.52f}};
+struct PcRoute { int tile, splits; float cost_us; };
+static PcRoute pc_route(int64_t m, int64_t n_out, int64_t n_in) {
   const int cus = device_num_cus();
   const int64_t blocks = n_in / 256;
-  PcChoice best{0, 1, 1e30f};
-  for (int pass = 0; pass < 2 && best.cost_us > 1e29f; pass++) {
-    for (int i = 0; i < (int)(sizeof(kPcTiles) / sizeof(kPcTiles[0])); i++) {
-      if (forced >= 0 && forced < (int)(sizeof(kPcTiles) / sizeof(kPcTiles[0])) && i != forced) continue;
-      const PcTile& t = kPcTiles[i];
-      const int64_t bo = fuse ? t.nj * 8 : t.nj * 16, bm = pc_bm(t.mb);
-      const int64_t nt = (n_out + bo - 1) / bo, mt = (m + bm - 1) / bm, tiles = nt * mt;
-      for (int sp : kSplits) {
-        if (pass == 0 && forced_splits > 0 && sp != forced_splits) continue;
-        if (pass == 1 && sp != 1) continue;
-        if (sp > 1 && (fuse || blocks % sp != 0 || blocks / sp < 2 || tiles * sp > cus || tiles * 4 > kPcMaxCounters)) continue;
-        const int64_t rounds = (tiles * sp + cus - 1) / cus;
-        const float cost = (float)rounds * ((float)(n_in / 64 / sp) * t.step_us + kPcFixedUs) +
-                           (sp > 1 ? pc_split_us(t, sp, mt * bm, nt * bo) : 0.f);
-        if (cost < best.cost_us * 0.999f) best = PcChoice{i, sp, cost};
+  PcRoute best{0, 1, 1e30f};
+  for (int i = 0; i < kPcTileCount; i++) {
+    const PcRouteTile& t = kPcRouteTiles[i];
+    const int64_t bm = pc_bm(t.mb), nt = (n_out + t.nj * 16 - 1) / (t.nj * 16), mt = (m + bm - 1) / bm, tiles = nt * mt;
+    for (int sp : kPcSplits) {
+      if (sp > 1 && (blocks % sp != 0 || blocks / sp < 2 || tiles * sp > cus || tiles * 4 > kPcMaxCounters)) continue;
+      const int64_t rounds = (tiles * sp + cus - 1) / cus;
+      float cost = (float)rounds * ((float)(n_in / 64 / sp) * t.step_us + 6.f);
+      if (sp > 1) {      // 2 + copies trips to the memory side (3 for two copies), the partial sums twice at 4 TB/s
+        const float trip = 0.9f + 0.06f * (float)(t.mb * t.nj);
+        cost += (sp == 2 ? 3.f : 2.f + (float)sp) * trip + 2.f * (float)sp * (float)(mt * bm) * (float)(nt * t.nj * 16) * 4.f / 4.0e6f;
       }
+      if (cost < best.cost_us * 0.999f) best = PcRoute{i, sp, cost};
     }
   }
   return best;
 }
 
-size_t gemm_pc_partials_bytes(int64_t m, int64_t n_out, int64_t n_in) {
+// What a launch takes, us, by format, by where the activations are read (row-major through LDS, or a packed copy) and by tile:
+//   rounds of workgroups * (64-k steps * (step + full * share of the compute units at work) + round) + launch
+//   + (split along K) trips0 + trips1 * copies + bytes of the partial sums, written and read, * traffic / 4 TB/s,
+// fitted to 150000 timed launches of 19000 layers: 768 .. 8192 wide models at 65 .. 4096 rows, and any 256 .. 120000 x 256 .. 14336 at 20 and
+// more, every tile, one to eight copies, both ways to the activations, 256 compute units; standard deviation 6 to 12 percent for tiles
+// of 128 and 64 rows, 9 to 17 for 256.  What these estimates choose is within one percent of the fastest launch of all (geometric mean)
+// and 9 percent below what the model above chooses, which has one time per step for all formats; its choice is kept where
+// the two are within five percent (slower than it by more than that: 1 percent of the layers, 2.3 without the margin).  A short
+// grid is split along K while all copies fit one round: the length of a short round is the latency of its K loop.
+struct PcCost { float step, full, round, launch, trips0, trips1, traffic; };
+static const PcCost kPcCosts[3][2][kPcTileCount] = {      // [format: Q8_0, Q4_K, Q6_K][packed][tile]
+    {  // Q8_0
+        {{0.663f, 0.201f, 6.98f, 4.21f, 3.17f, 7.70f, 0.57f}, {0.569f, 0.098f, 2.69f, 6.17f, 2.17f, 4.28f, 0.57f}, {0.497f, 0.111f, 4.56f, 4.79f, 1.97f, 1.14f, 0.58f},
+         {0.410f, 0.065f, 1.85f, 6.01f, 1.46f, 0.82f, 0.69f}, {0.474f, 0.056f, 3.26f, 4.88f, 0.95f, 0.80f, 0.89f}, {0.352f, 0.039f, 1.52f, 5.63f, 0.89f, 0.66f, 1.12f}},
+        {{0.617f, 0.184f, 11.29f, 2.55f, 2.79f, 1.84f, 0.51f}, {0.461f, 0.103f, 6.65f, 3.50f, 2.20f, 1.31f, 0.52f}, {0.511f, 0.105f, 3.53f, 6.88f, 1.85f, 1.08f, 0.48f},
+         {0.380f, 0.012f, 1.85f, 6.43f, 1.44f, 0.78f, 0.76f}, {0.473f, 0.055f, 2.42f, 6.14f, 1.16f, 0.74f, 0.72f}, {0.319f, 0.f, 1.29f, 6.32f, 1.02f, 0.57f, 1.45f}},
+    },
+    {  // Q4_K
+        {{0.567f, 0.200f, 6.74f, 4.18f, 2.38f, 7.64f, 0.59f}, {0.449f, 0.112f, 2.65f, 5.65f, 1.48f, 4.21f, 0.60f}, {0.400f, 0.110f, 2.59f, 6.27f, 1.22f, 0.98f, 0.75f},
+         {0.295f, 0.071f, 1.83f, 5.58f, 0.77f, 0.67f, 0.80f}, {0.356f, 0.061f, 1.99f, 5.80f, 0.74f, 0.69f, 0.85f}, {0.230f, 0.052f, 1.41f, 5.52f, 0.52f, 0.56f, 0.77f}},
+        {{0.461f, 0.222f, 10.20f, 3.11f, 1.49f, 1.95f, 0.66f}, {0.333f, 0.115f, 5.74f, 3.75f, 1.75f, 1.25f, 0.55f}, {0.374f, 0.060f, 2.44f, 7.43f, 1.14f, 1.03f, 0.75f},
+         {0.245f, 0.037f, 1.42f, 6.46f, 1.00f, 0.67f, 0.83f}, {0.343f, 0.f, 1.62f, 6.79f, 0.53f, 0.59f, 1.33f}, {0.205f, 0.f, 1.03f, 6.02f, 0.82f, 0.50f, 1.22f}},
+    },
+    {  // Q6_K
+        {{0.735f, 0.164f, 8.38f, 3.99f, 1.96f, 7.68f, 0.57f}, {0.567f, 0.091f, 3.53f, 6.07f, 0.99f, 4.18f, 0.54f}, {0.541f, 0.097f, 3.80f, 6.34f, 0.91f, 0.99f, 0.66f},
+         {0.400f, 0.068f, 2.53f, 5.76f, 0.68f, 0.62f, 0.74f}, {0.503f, 0.049f, 3.11f, 5.72f, 0.39f, 0.68f, 0.84f}, {0.336f, 0.047f, 2.06f, 5.55f, 0.20f, 0.51f, 1.00f}},
+        {{0.631f, 0.168f, 8.51f, 4.39f, 2.39f, 1.80f, 0.55f}, {0.440f, 0.095f, 5.06f, 4.67f, 1.75f, 1.12f, 0.56f}, {0.528f, 0.017f, 3.16f, 7.74f, 0.76f, 0.95f, 0.79f},
+         {0.357f, 0.012f, 2.07f, 6.59f, 0.79f, 0.64f, 0.85f}, {0.460f, 0.f, 2.25f, 7.47f, 0.67f, 0.64f, 0.94f}, {0.295f, 0.f, 1.71f, 6.32f, 0.47f, 0.50f, 1.21f}},
+    },
+};
+
+struct PcChoice { int tile, splits; bool packed; float cost_us; };
+
+// The pass that makes the packed copy: 2.5 us and its bytes, fp32 rows (a factor per row first) 5.5.
+static float pc_pack_us(int x_dtype, int64_t m, int64_t n_in) {
+  return x_dtype == kF32 ? 5.5f + (float)(m * n_in * 10) / 5.0e6f : 2.5f + (float)(m * n_in * 4) / 5.0e6f;
+}
+
+// The tile, the copies along K and the way to the activations of a launch.  Only bf16 activations can be read as they are, and the
+// fused gate||up form must (its epilogue does not fit beside the packed kernel's three steps of A fragments).
+static PcChoice pc_choose(int format, int x_dtype, int64_t m, int64_t n_out, int64_t n_in, bool fuse) {
+  static const int forced = dev_knob("TTQ_GEMM_TILE", -1);
+  static const int forced_splits = dev_knob("TTQ_GEMM_SPLITS", 0);   // A/B: 1 = never split, n = n ways where possible
+  static const int forced_packed = dev_knob("TTQ_GEMM_PACKED", -1);  // A/B: 0 never, 1 always
+  const int cus = device_num_cus();
+  const int64_t blocks = n_in / 256;
+  PcChoice best{0, 1, false, 1e30f}, before = best;
+  const PcRoute route = fuse ? PcRoute{-1, 1, 0.f} : pc_route(m, n_out, n_in);
+  const bool route_packed = x_dtype != kBF16 || (kPcTiles[route.tile < 0 ? 0 : route.tile].mb == 4 && route.cost_us >= 45.f);
+  for (int packed = fuse || x_dtype == kBF16 ? 0 : 1; packed <= (fuse ? 0 : 1); packed++) {
+    if (!fuse && x_dtype == kBF16 && forced_packed >= 0 && forced_packed != packed) continue;
+    const float pack = packed ? pc_pack_us(x_dtype, m, n_in) : 0.f;
+    for (int i = 0; i < kPcTileCount; i++) {
+      if (forced >= 0 && forced < kPcTileCount && i != forced) continue;
+      const PcTile& t = kPcTiles[i];
+      const PcCost& c = kPcCosts[format][packed][i];
+      const int64_t bo = fuse ? t.nj * 8 : t.nj * 16, bm = pc_bm(t.mb);
+      const int64_t nt = (n_out + bo - 1) / bo, mt = (m + bm - 1) / bm, tiles = nt * mt;
+      for (int sp : kPcSplits) {
+        if (forced_splits > 0 && sp != 1 && sp != forced_splits) continue;
+        if (sp > 1 && (fuse || blocks % sp != 0 || blocks / sp < 2 || tiles * sp > cus || tiles * 4 > kPcMaxCounters)) continue;
+        // (beyond four rounds the last one overlaps the others)
+        const float full = (float)(tiles * sp) / (float)cus;
+        const float rounds = full > 4.f ? full + 0.5f : (float)((tiles * sp + cus - 1) / cus);
+        const float step = c.step + c.full * (full < rounds ? full / rounds : 1.f);
+        float cost = pack + rounds * ((float)(n_in / 64 / sp) * step + c.round) + c.launch;
+        if (sp > 1)
+          cost += c.trips0 + c.trips1 * (float)(sp > 2 ? sp : 1) + c.traffic * 2.f * (float)sp * (float)(mt * bm) * (float)(nt * bo) / 1.0e6f;
+        if (i == route.tile && sp == route.splits && (packed != 0) == route_packed) before = PcChoice{i, sp, packed != 0, cost};
+        // (long launches of the K formats read a packed copy: the estimates are least sure of short rows, 20112 x 1024 Q4_K at 4079 rows
+        // 222 us without it and 208)
+        if (!fuse && !packed && forced_packed < 0 && format != kQ8_0 && cost >= 45.f) continue;
+        if (cost < best.cost_us * 0.999f || (forced_splits > 0 && sp == forced_splits && best.splits != sp))
+          best = PcChoice{i, sp, packed != 0, cost};
+      }
+    }
+  }
+  // (Q8_0, short rows of very many weight rows: the estimates' other weak place, 108544 x 256 at 712 rows 116 -> 165 us)
+  // (long launches one after the other run at the clock that the power limit leaves, where tiles that dequantize a weight for fewer
+  // products lose what they win alone: a block of 4096 / 14336 at 4096 rows with 64-column tiles in three of its layers 1860 us
+  // against 1830, each of those layers alone 2 to 5 percent faster)
+  const float margin = format == kQ8_0 && n_in <= 1024 && n_out > 16384 ? 0.f : (before.cost_us >= 100.f ? 0.9f : 0.95f);
+  return before.cost_us < 1e29f && forced < 0 && forced_splits == 0 && best.cost_us > margin * before.cost_us ? before : best;
+}
+
+// bytes of partial sums that a launch of this shape keeps in the workspace (0: not split along K)
+size_t gemm_pc_partials_bytes(int format, int x_dtype, int64_t m, int64_t n_out, int64_t n_in) {
   if (m <= 0 || n_out <= 0 || n_in < 256) return 0;
-  const PcChoice c = pc_choose(m, n_out, n_in, false);
+  const PcChoice c = pc_choose(format, x_dtype, m, n_out, n_in, false);
   if (c.splits <= 1) return 0;
   const PcTile& t = kPcTiles[c.tile];
   const int64_t nt = (n_out + t.nj * 16 - 1) / (t.nj * 16), mt = (m + pc_bm(t.mb) - 1) / pc_bm(t.mb);
@@ -92,26 +159,13 @@ size_t gemm_pc_partials_bytes(int64_t m, int64_t n_out, int64_t n_in) {
 // Rough time of the GEMM for this shape (microseconds), for callers that can also run the
 // operator as a few GEMV passes.  The Q6_K and Q8_0 producers are slower than the Q4_K one.
 float gemm_pc_estimate_us(int format, int64_t m, int64_t n_out, int64_t n_in) {
-  const float c = pc_choose(m, n_out, n_in, false).cost_us;
-  return c * (format == kQ8_0 ? 1.9f : (format == kQ6_K ? 1.4f : 1.f)) + 2.f;
+  return pc_route(m, n_out, n_in).cost_us * (format == kQ8_0 ? 1.9f : (format == kQ6_K ? 1.4f : 1.f)) + 2.f;
 }
 
-// Whether a launch for this shape is divided along K.
-bool gemm_pc_splits_k(int64_t m, int64_t n_out, int64_t n_in) { return pc_choose(m, n_out, n_in, false).splits > 1; }
+// Whether that model would divide a launch along K.
+bool gemm_pc_splits_k(int64_t m, int64_t n_out, int64_t n_in) { return pc_route(m, n_out, n_in).splits > 1; }
 
-// Launches of 256-row tiles read the activations from a copy in fragment order (ttq_gemm_pcd.h), made by one pass
-// over X into a workspace: with no X traffic through LDS their K loop is 6 % (64-column tiles) to 15 % (112-column
-// tiles) shorter, which pays for the pass (2.5 us + the bytes at about 7 TB/s, they come out of the caches) on every
-// shape measured from 50 us of GEMM on: 4096 x 14336 at 512 rows 90.4 -> 84.6 us, at 1024 rows 150.7 -> 142.2 us,
-// 5120 x 13824 at 512 rows 102.1 -> 94.2 us, 4096 x 4096 at 1024 rows 53.8 -> 51.6 us.  Tiles of 128 and 64 rows
-// move a half and a quarter of the activation bytes per step through LDS and gain nothing from the copy (-0.5 to
-// -6 us on seven shapes, split along K or not).
 constexpr int64_t kPackRows = 8192;         // rows packed (and multiplied) at a time
-static bool pc_use_packed(const PcChoice& c) {
-  static const int knob = dev_knob("TTQ_GEMM_PACKED", -1);      // A/B: 0 never, 1 always
-  if (knob >= 0) return knob != 0;
-  return kPcTiles[c.tile].mb == 4 && c.cost_us >= 45.f;
-}
 
 template <int FMT, bool FUSE>
 static hipError_t launch_pc_rows(const PcChoice& c, int tile_if_packed, const uint8_t* wb, const uint16_t* x, void* y,
@@ -128,16 +182,14 @@ static hipError_t launch_pc_rows(const PcChoice& c, int tile_if_packed, const ui
   }
 }
 
-// x in x_dtype: bf16 for the direct form; any type when the launch goes through the packed copy (the packing pass
+// x in x_dtype: any type when the launch goes through the packed copy (the packing pass
 // rounds to bf16, or -- keep_f16 -- leaves fp16 activations as they are for the fp16 form of the kernel).
 template <int FMT, bool FUSE>
 static hipError_t launch_pc_fmt(const uint8_t* wb, const void* x, int x_dtype, void* y, int y_dtype, const void* bias,
-                                int bias_dtype, int64_t m, int64_t n_out, int64_t n_in, bool force_packed, hipStream_t s,
+                                int bias_dtype, int64_t m, int64_t n_out, int64_t n_in, hipStream_t s,
                                 int f16_mode = 0) {      // 1: fp16 activations stay fp16; 2: fp32 activations as scaled fp16
-  const PcChoice whole = pc_choose(m, n_out, n_in, FUSE);
-  // (the fused gate||up form keeps the LDS-staged kernel: beside the packed kernel's three steps of A fragments its
-  // epilogue does not fit the registers, and a kernel that requests registers asynchronously must never spill them)
-  if (FUSE || (!force_packed && !pc_use_packed(whole)))
+  const PcChoice whole = pc_choose(FMT, x_dtype, m, n_out, n_in, FUSE);
+  if (!whole.packed)
     return launch_pc_rows<FMT, FUSE>(whole, -1, wb, static_cast<const uint16_t*>(x), y, y_dtype, bias, bias_dtype, m, n_out,
                                      n_in, s);
   const int64_t block_rows = m < kPackRows ? m : kPackRows;
@@ -157,7 +209,7 @@ static hipError_t launch_pc_fmt(const uint8_t* wb, const void* x, int x_dtype, v
       e = launch_gemm_pack_activations(static_cast<const char*>(x) + r0 * n_in * xsize, x_dtype, static_cast<uint16_t*>(ws),
                                        rows, n_in, s, f16_mode == 1);
     if (e != hipSuccess) return e;
-    const PcChoice c = rows == m ? whole : pc_choose(rows, n_out, n_in, FUSE);
+    PcChoice c = rows == m ? whole : pc_choose(FMT, x_dtype, rows, n_out, n_in, FUSE);      // (the copy is made: its tile alone counts)
     e = launch_pc_rows<FMT, FUSE>(c, c.tile, wb, static_cast<const uint16_t*>(ws), static_cast<char*>(y) + r0 * n_out * ysize,
                                   y_dtype, bias, bias_dtype, rows, n_out, n_in, s, f16_mode != 0, row_scale);
     if (e != hipSuccess) return e;
@@ -185,19 +237,18 @@ hipError_t launch_gemm_pc_x(int format, const void* w, const void* x, int x_dtyp
   if (m == 0 || n_out == 0) return hipSuccess;
   if (y_dtype != kBF16 && y_dtype != kF32 && y_dtype != kF16) return hipErrorInvalidValue;
   if (f16_native && x_dtype != kF16 && x_dtype != kF32) return hipErrorInvalidValue;
-  const PcChoice c = pc_choose(m, n_out, n_in, false);
-  const bool packed = x_dtype != kBF16 || pc_use_packed(c);
+  const PcChoice c = pc_choose(format, x_dtype, m, n_out, n_in, false);
+  const bool packed = c.packed;
   if (route_probe(f16_native ? (x_dtype == kF32 ? kRouteGemmPcF32ScaledF16 : kRouteGemmPcF16)
                              : (x_dtype != kBF16 ? kRouteGemmPcBf16Copy
                                                  : (c.splits > 1 ? (packed ? kRouteGemmPcPackedSplitK : kRouteGemmPcSplitK)
                                                                  : (packed ? kRouteGemmPcPacked : kRouteGemmPc)))))
     return hipSuccess;
   const uint8_t* wb = static_cast<const uint8_t*>(w);
-  const bool force = x_dtype != kBF16;
   switch (format) {
-    case kQ4_K: return launch_pc_fmt<kQ4_K, false>(wb, x, x_dtype, y, y_dtype, bias, bias_dtype, m, n_out, n_in, force, s, f16_native ? (x_dtype == kF32 ? 2 : 1) : 0);
-    case kQ6_K: return launch_pc_fmt<kQ6_K, false>(wb, x, x_dtype, y, y_dtype, bias, bias_dtype, m, n_out, n_in, force, s, f16_native ? (x_dtype == kF32 ? 2 : 1) : 0);
-    case kQ8_0: return launch_pc_fmt<kQ8_0, false>(wb, x, x_dtype, y, y_dtype, bias, bias_dtype, m, n_out, n_in, force, s, f16_native ? (x_dtype == kF32 ? 2 : 1) : 0);
+    case kQ4_K: return launch_pc_fmt<kQ4_K, false>(wb, x, x_dtype, y, y_dtype, bias, bias_dtype, m, n_out, n_in, s, f16_native ? (x_dtype == kF32 ? 2 : 1) : 0);
+    case kQ6_K: return launch_pc_fmt<kQ6_K, false>(wb, x, x_dtype, y, y_dtype, bias, bias_dtype, m, n_out, n_in, s, f16_native ? (x_dtype == kF32 ? 2 : 1) : 0);
+    case kQ8_0: return launch_pc_fmt<kQ8_0, false>(wb, x, x_dtype, y, y_dtype, bias, bias_dtype, m, n_out, n_in, s, f16_native ? (x_dtype == kF32 ? 2 : 1) : 0);
     default: return hipErrorInvalidValue;
   }
 }
@@ -209,10 +260,9 @@ hipError_t launch_gemm_pc(int format, const void* w, const uint16_t* x_bf16, voi
 }
 
 // bytes of the packed copy a launch of this shape takes from the workspace (0: it reads X itself)
-size_t gemm_pc_packed_bytes(int64_t m, int64_t n_out, int64_t n_in, int x_dtype) {
+size_t gemm_pc_packed_bytes(int format, int64_t m, int64_t n_out, int64_t n_in, int x_dtype) {
   if (m <= 0 || n_out <= 0 || n_in < 256) return 0;
-  const bool packed = x_dtype != kBF16 || pc_use_packed(pc_choose(m, n_out, n_in, false));
-  if (!packed) return 0;
+  if (!pc_choose(format, x_dtype, m, n_out, n_in, false).packed) return 0;
   const int64_t rows = m < kPackRows ? m : kPackRows;
   // (fp32 activations: room for a factor per row behind the copy, whichever way they are narrowed)
   return ((gemm_packed_activation_bytes(rows, n_in) + 255) & ~(size_t)255) + (x_dtype == kF32 ? (size_t)rows * 4 : 0);
@@ -226,7 +276,7 @@ hipError_t launch_gemm_pc_silu_mul(const void* w, const uint16_t* x_bf16, void* 
   if (m == 0 || n_ff == 0) return hipSuccess;
   if (y_dtype != kBF16 && y_dtype != kF32) return hipErrorInvalidValue;
   return launch_pc_fmt<kQ4_K, true>(static_cast<const uint8_t*>(w), x_bf16, kBF16, y, y_dtype, bias, bias_dtype, m, n_ff,
-                                    n_in, false, s);
+                                    n_in, s);
 }
 
 }  // namespace ttq

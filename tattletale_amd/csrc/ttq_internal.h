@@ -342,9 +342,9 @@ int64_t exl3_workspace_words();
 // of packed copy such a launch takes from the workspace
 hipError_t launch_gemm_pc_x(int format, const void* w, const void* x, int x_dtype, void* y, int y_dtype,
                             const void* bias, int bias_dtype, int64_t m, int64_t n_out, int64_t n_in, hipStream_t s, bool f16_native = false);
-size_t gemm_pc_packed_bytes(int64_t m, int64_t n_out, int64_t n_in, int x_dtype);
+size_t gemm_pc_packed_bytes(int format, int64_t m, int64_t n_out, int64_t n_in, int x_dtype);
 // exact size of the partial sums a split-K launch of the prefill GEMM takes for this shape (0: not split)
-size_t gemm_pc_partials_bytes(int64_t m, int64_t n_out, int64_t n_in);
+size_t gemm_pc_partials_bytes(int format, int x_dtype, int64_t m, int64_t n_out, int64_t n_in);
 // how often the trellis GEMV's last slice polls a missing word before it gives the row up; returns the old value
 int exl3_set_poll_limit(int limit);
 // n fp16 or fp32 values (n a multiple of 8) rounded to bf16
