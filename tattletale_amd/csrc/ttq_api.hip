@@ -488,7 +488,10 @@ int ttq_linear_forward(const ttq_qlinear* layer, const void* x, int x_dtype, int
     us_rounding = us_gemm < us_rounding ? us_gemm : us_rounding;
     const bool rounds = route == 2 || !newer || us_rounding < ttq::gemv_estimate_us(layer->format, x_dtype, m, n_out, n_in, false);
     const float us_gemv = ttq::gemv_estimate_us(layer->format, x_dtype, m, n_out, n_in);
-    if (rounds && us_gemm < 1e29f && us_gemm < us_few / few_margin() && (route == 2 || us_gemm < us_gemv || us_few < us_gemv))
+    // (between two kernels that round the weights the tiled one's fitted time has the last word)
+    const bool tiled = us_gemm < 1e29f && (us_gemm < us_few / few_margin() ||
+                                           ttq::gemm_pc_cost_us(layer->format, x_dtype, m, n_out, n_in) < us_few);
+    if (rounds && tiled && (route == 2 || us_gemm < us_gemv || us_few < us_gemv))
       return hip_status(ttq::launch_gemm_pc_x(layer->format, layer->qweight, x, x_dtype, y, y_dtype, layer->bias,
                                               layer->bias_dtype, m, n_out, n_in, s, true));
     if (rounds && us_few < 1e29f && (route == 2 || us_few < us_gemv)) {
@@ -537,12 +540,15 @@ int ttq_linear_forward(const ttq_qlinear* layer, const void* x, int x_dtype, int
     // same.  The small matrices, where the two agree to 3 us, stay with the kernel that takes any number of rows.)
     const bool integer_passes = (int64_t)n_out * n_in >= (int64_t)120 << 20 || ttq::gemv_short_first(layer->format, x_dtype, m, n_out, n_in);
     const float us_gemv = ttq::gemv_estimate_us(layer->format, x_dtype, m, n_out, n_in, integer_passes);
-    if (rounds && us_few / few_margin() < us_gemm && (route == 2 || us_few < us_gemv)) {
+    // (as for fp16)
+    const bool tiled = m > 64 && us_gemm < 1e29f && us_few < 1e29f &&
+                       ttq::gemm_pc_cost_us(layer->format, x_dtype, m, n_out, n_in) < us_few;
+    if (rounds && !tiled && us_few / few_margin() < us_gemm && (route == 2 || us_few < us_gemv)) {
       if (ttq::route_probe(ttq::kRouteGemmSkinnyF32ScaledF16)) return TTQ_OK;
       return hip_status(ttq::launch_gemm_skinny_f32(layer->format, layer->qweight, static_cast<const float*>(x), y, y_dtype,
                                                     layer->bias, layer->bias_dtype, m, n_out, n_in, s));
     }
-    if (rounds && us_gemm < 1e29f && (route == 2 || us_gemm < us_gemv))
+    if (rounds && us_gemm < 1e29f && (route == 2 || us_gemm < us_gemv || (tiled && us_few < us_gemv)))
       return hip_status(ttq::launch_gemm_pc_x(layer->format, layer->qweight, x, x_dtype, y, y_dtype, layer->bias,
                                               layer->bias_dtype, m, n_out, n_in, s, true));
   }

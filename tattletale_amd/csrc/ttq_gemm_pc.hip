@@ -162,6 +162,10 @@ float gemm_pc_estimate_us(int format, int64_t m, int64_t n_out, int64_t n_in) {
   return pc_route(m, n_out, n_in).cost_us * (format == kQ8_0 ? 1.9f : (format == kQ6_K ? 1.4f : 1.f)) + 2.f;
 }
 
+float gemm_pc_cost_us(int format, int x_dtype, int64_t m, int64_t n_out, int64_t n_in) {
+  return pc_choose(format, x_dtype, m, n_out, n_in, false).cost_us;
+}
+
 // Whether that model would divide a launch along K.
 bool gemm_pc_splits_k(int64_t m, int64_t n_out, int64_t n_in) { return pc_route(m, n_out, n_in).splits > 1; }
 

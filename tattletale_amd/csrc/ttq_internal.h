@@ -234,6 +234,8 @@ hipError_t launch_gemv_q4k_batch4(const void* w, const void* x, int x_dtype, voi
 // integer_kernels: with the kernels of ttq_gemv_tile.hip and the exact form of ttq_gemm_rows.hip among the decode kernels
 float gemv_estimate_us(int format, int x_dtype, int64_t m, int64_t n_out, int64_t n_in, bool integer_kernels = true);
 float gemm_pc_estimate_us(int format, int64_t m, int64_t n_out, int64_t n_in);
+// what the launch that it would choose takes, for callers that weigh it against another kernel with rounded weights
+float gemm_pc_cost_us(int format, int x_dtype, int64_t m, int64_t n_out, int64_t n_in);
 bool gemm_pc_splits_k(int64_t m, int64_t n_out, int64_t n_in);
 int gemv_q4k_batch_tokens(int64_t m, int64_t n_in);
 
