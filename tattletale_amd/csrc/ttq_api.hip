@@ -437,7 +437,7 @@ int ttq_linear_forward(const ttq_qlinear* layer, const void* x, int x_dtype, int
   // decode.
   // (fp16 outputs from bf16 activations: every GEMM kernel but the single-role one, which only more than 4 GiB of
   // activations reach, stores them)
-  const bool gemm_ok = x_dtype == TTQ_BF16 &&
+  const bool gemm_ok = x_dtype == TTQ_BF16 && m >= 5 &&
                        (y_dtype == TTQ_BF16 || y_dtype == TTQ_F32 ||
                         (y_dtype == TTQ_F16 && (ttq::gemm_skinny_supported(layer->format, m, n_out, n_in) ||
                                                 ttq::gemm_pc_supported(layer->format, m, n_out, n_in, 112)))) &&
@@ -454,7 +454,7 @@ int ttq_linear_forward(const ttq_qlinear* layer, const void* x, int x_dtype, int
   const bool streamed = m >= 2 && (layer->format == TTQ_Q4_K || layer->format == TTQ_Q6_K) &&
                         (ttq::gemm_rows_preferred(n_out) || few_us(m < 64 ? m : 64) > 1e29f);
   const bool newer = streamed || (layer->format == TTQ_Q6_K && (int64_t)n_out * n_in >= 6000000);
-  if (gemm_ok && m >= 5 && route != 1) {
+  if (gemm_ok && route != 1) {
     float us_rounding = 0.f;
     if (newer) {
       us_rounding = m <= 64 ? few_us(m) : 1e30f;
@@ -488,9 +488,10 @@ int ttq_linear_forward(const ttq_qlinear* layer, const void* x, int x_dtype, int
     us_rounding = us_gemm < us_rounding ? us_gemm : us_rounding;
     const bool rounds = route == 2 || !newer || us_rounding < ttq::gemv_estimate_us(layer->format, x_dtype, m, n_out, n_in, false);
     const float us_gemv = ttq::gemv_estimate_us(layer->format, x_dtype, m, n_out, n_in);
-    // (between two kernels that round the weights the tiled one's fitted time has the last word)
-    const bool tiled = us_gemm < 1e29f && (us_gemm < us_few / few_margin() ||
-                                           ttq::gemm_pc_cost_us(layer->format, x_dtype, m, n_out, n_in) < us_few);
+    // (a call that the few-row kernel would have, and so has its weights rounded either way, goes by the tiled one's fitted time)
+    const bool tiled = us_gemm < 1e29f &&
+                       (us_gemm < us_few / few_margin() ||
+                        (us_few < us_gemv && ttq::gemm_pc_cost_us(layer->format, x_dtype, m, n_out, n_in) < us_few));
     if (rounds && tiled && (route == 2 || us_gemm < us_gemv || us_few < us_gemv))
       return hip_status(ttq::launch_gemm_pc_x(layer->format, layer->qweight, x, x_dtype, y, y_dtype, layer->bias,
                                               layer->bias_dtype, m, n_out, n_in, s, true));
@@ -540,15 +541,16 @@ int ttq_linear_forward(const ttq_qlinear* layer, const void* x, int x_dtype, int
     // same.  The small matrices, where the two agree to 3 us, stay with the kernel that takes any number of rows.)
     const bool integer_passes = (int64_t)n_out * n_in >= (int64_t)120 << 20 || ttq::gemv_short_first(layer->format, x_dtype, m, n_out, n_in);
     const float us_gemv = ttq::gemv_estimate_us(layer->format, x_dtype, m, n_out, n_in, integer_passes);
-    // (as for fp16)
-    const bool tiled = m > 64 && us_gemm < 1e29f && us_few < 1e29f &&
+    // (as for fp16: only calls that the few-row kernel would have go by the fitted time)
+    const bool few = rounds && us_few / few_margin() < us_gemm && (route == 2 || us_few < us_gemv);
+    const bool tiled = few && m > 64 && us_gemm < 1e29f &&
                        ttq::gemm_pc_cost_us(layer->format, x_dtype, m, n_out, n_in) < us_few;
-    if (rounds && !tiled && us_few / few_margin() < us_gemm && (route == 2 || us_few < us_gemv)) {
+    if (few && !tiled) {
       if (ttq::route_probe(ttq::kRouteGemmSkinnyF32ScaledF16)) return TTQ_OK;
       return hip_status(ttq::launch_gemm_skinny_f32(layer->format, layer->qweight, static_cast<const float*>(x), y, y_dtype,
                                                     layer->bias, layer->bias_dtype, m, n_out, n_in, s));
     }
-    if (rounds && us_gemm < 1e29f && (route == 2 || us_gemm < us_gemv || (tiled && us_few < us_gemv)))
+    if (tiled || (rounds && us_gemm < 1e29f && (route == 2 || us_gemm < us_gemv)))
       return hip_status(ttq::launch_gemm_pc_x(layer->format, layer->qweight, x, x_dtype, y, y_dtype, layer->bias,
                                               layer->bias_dtype, m, n_out, n_in, s, true));
   }

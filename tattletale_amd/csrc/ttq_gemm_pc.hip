@@ -138,11 +138,12 @@ static PcChoice pc_choose(int format, int x_dtype, int64_t m, int64_t n_out, int
       }
     }
   }
-  // (Q8_0, short rows of very many weight rows: the estimates' other weak place, 108544 x 256 at 712 rows 116 -> 165 us)
+  // (short rows of very many weight rows: the estimates' other weak place, Q8_0 108544 x 256 at 712 rows 116 -> 165 us, Q6_K
+  // 43392 x 256 at 104 fp16 rows 15.4 -> 18.2, Q4_K 39552 x 512 at 92 16.6 -> 18.4: the model above decides)
   // (long launches one after the other run at the clock that the power limit leaves, where tiles that dequantize a weight for fewer
   // products lose what they win alone: a block of 4096 / 14336 at 4096 rows with 64-column tiles in three of its layers 1860 us
   // against 1830, each of those layers alone 2 to 5 percent faster)
-  const float margin = format == kQ8_0 && n_in <= 1024 && n_out > 16384 ? 0.f : (before.cost_us >= 100.f ? 0.9f : 0.95f);
+  const float margin = n_in <= (format == kQ8_0 ? 1024 : 512) && n_out > 16384 ? 0.f : (before.cost_us >= 100.f ? 0.9f : 0.95f);
   return before.cost_us < 1e29f && forced < 0 && forced_splits == 0 && best.cost_us > margin * before.cost_us ? before : best;
 }
 
@@ -162,8 +163,13 @@ float gemm_pc_estimate_us(int format, int64_t m, int64_t n_out, int64_t n_in) {
   return pc_route(m, n_out, n_in).cost_us * (format == kQ8_0 ? 1.9f : (format == kQ6_K ? 1.4f : 1.f)) + 2.f;
 }
 
+// The fitted time, for the choice against chunks of the few-row kernel.  It errs most for one or two short row tiles (of the
+// calls of 65 to 128 rows that it sent to tiles 20 in 326 were 5 to 30 percent slower than in chunks, over rows of more than 8192
+// values 6 in 45, by up to half), so the tiles have to be a tenth ahead there, Q8_0 (ten of fifteen that
+// were still slower) a quarter, and the long ones go by the model above alone.
 float gemm_pc_cost_us(int format, int x_dtype, int64_t m, int64_t n_out, int64_t n_in) {
-  return pc_choose(format, x_dtype, m, n_out, n_in, false).cost_us;
+  if (m <= 128 && n_in > 8192) return 1e30f;
+  return pc_choose(format, x_dtype, m, n_out, n_in, false).cost_us * (m <= 128 ? (format == kQ8_0 ? 1.25f : 1.1f) : 1.f);
 }
 
 // Whether that model would divide a launch along K.

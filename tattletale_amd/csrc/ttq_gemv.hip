@@ -567,17 +567,11 @@ hipError_t launch_gemv(int format, const void* w, const void* x, int x_dtype, vo
     TTQ_ROUTE(kRouteGemvQ6kStream, launch_gemv_q6k_stream(w, x, x_dtype, y, y_dtype, bias, bias_dtype, m, n_out, n_in, s));
   if (gemv_mfma_supported(format, x_dtype, n_out, n_in))
     TTQ_ROUTE(kRouteGemvQ4kMfma, launch_gemv_mfma(w, x, x_dtype, y, y_dtype, bias, bias_dtype, m, n_out, n_in, s));
-  // Q8_0 with few weights: the fp32 kernel (a wavefront per row, a row's activations in registers) has the shortest
-  // prologue; it re-reads the weights per activation row, so the more rows, the smaller the matrix it wins on.
-  // Measured against the matrix-core kernels: 1024x4096 3.9 / 4.8 / 6.3 us for 1 / 2 / 4 rows against 5.3 / 6.5 /
-  // 8.5, 2048x4096 5.0 / 6.6 / 10.3 against 5.6 / 6.9 / 8.8, 1024x14336 9.3 / 11.8 / 20.4 against 12.3 / 13.9 / 13.5.
-  // (Up to 2048 weight rows, two per wavefront: with short rows its lanes are mostly idle, and more rows of them
-  // are the matrix-core kernels' again -- 16384x256 9.2 us against 3.8.)
-  if (format == kQ8_0 && m <= 4 && n_out <= 2048) {
-    const float mb = (float)(n_out * (n_in / 32) * 34) * 1e-6f;
-    const float limit = n_in <= 4096 ? (m == 1 ? 12.f : (m == 2 ? 8.5f : 6.f)) : (m <= 2 ? 16.f : 0.f);
-    if (mb <= limit) TTQ_ROUTE(kRouteGemvGeneric, launch_generic_xy<FmtQ8_0>(w, x, x_dtype, y, y_dtype, bias, bias_dtype, m, n_out, n_in, s));
-  }
+  // Q8_0, long rows of few weights (up to 4096 values the kernel for matrices of a few MB has taken them already): the fp32 kernel (a
+  // wavefront per row, a row's activations in registers) has the shortest prologue; it re-reads the weights per activation row.
+  // Measured against the matrix-core kernels: 1024x14336 9.3 / 11.8 / 20.4 us for 1 / 2 / 4 rows against 12.3 / 13.9 / 13.5.
+  if (format == kQ8_0 && m <= 2 && n_out <= 2048 && (float)(n_out * (n_in / 32) * 34) * 1e-6f <= 16.f)
+    TTQ_ROUTE(kRouteGemvGeneric, launch_generic_xy<FmtQ8_0>(w, x, x_dtype, y, y_dtype, bias, bias_dtype, m, n_out, n_in, s));
   if (m == 1 && gemv_q8_stream_supported(format, x_dtype, n_out, n_in))
     TTQ_ROUTE(kRouteGemvQ8Stream, launch_gemv_q8_stream(w, x, x_dtype, y, y_dtype, bias, bias_dtype, m, n_out, n_in, s));
   if (gemv_q8_win_supported(format, n_out, n_in))

@@ -382,20 +382,20 @@ bool gemv_short_preferred(int format, int x_dtype, int64_t m, int64_t n_out, int
   if (n_out * n_in > 22000000 || disabled || !gemv_short_supported(format, m, n_out, n_in)) return false;
   const float e = short_mega(n_out, n_in);
   const bool f32 = x_dtype == kF32;
-  const bool one_wave = n_out <= 4 * device_num_cus();      // a workgroup of four rows to a compute unit
+  const auto one_wave = [n_out] { return n_out <= 4 * device_num_cus(); };      // a workgroup of four rows to a compute unit
   if (format == kQ8_0) {
     if (m == 1) return e <= (n_out <= 2048 ? 16.f : 9.5f) && !gemv_q8_stream_supported(format, x_dtype, n_out, n_in);
     return e <= (m <= 4 ? 12.f : 8.f);
   }
   if (format == kQ6_K) {
     if (m > 4) return f32 && e <= 8.f && n_in <= 4096;
-    if (m == 1) return (n_in <= 14336 || one_wave) && !gemv_q6k_stream_supported(format, x_dtype, n_out, n_in);
+    if (m == 1) return (n_in <= 14336 || one_wave()) && !gemv_q6k_stream_supported(format, x_dtype, n_out, n_in);
     if (f32) return e <= 12.f;
     return e <= (m > 2 ? 6.f : (n_out <= 2048 ? 4.5f : 8.f)) && !gemv_q6k_stream4_supported(format, x_dtype, m, n_out, n_in);
   }
   if (m == 1) {
     if (gemv_q4k_stream_supported(format, x_dtype, n_out, n_in) || gemv_q4k_slice_supported(format, x_dtype, n_out, n_in)) return false;
-    if (!gemv_mfma_supported(format, x_dtype, n_out, n_in)) return f32 || e <= 7.2f || one_wave;
+    if (!gemv_mfma_supported(format, x_dtype, n_out, n_in)) return f32 || e <= 7.2f || one_wave();
     return f32 ? e <= 4.2f && n_in <= 1024 : e <= 8.f;
   }
   if (m > 4) return f32 && e <= 6.f && n_in <= 4096;
