@@ -177,3 +177,10 @@ def test_workspace_size_query_and_argument_checks():
     assert L.ttq_linear_forward_ws(C.byref(q), None, BF16, 512, None, BF16, None, -1, None) == _lib.ERR_WORKSPACE
     assert L.ttq_linear_forward_ws(C.byref(q), None, BF16, 0, None, BF16, None, 0, None) == _lib.OK
     assert L.ttq_strerror(_lib.ERR_WORKSPACE) not in (b"unknown status", b"ok")
+
+
+def test_fitted_time_moves_no_exact_call():
+    """A long fp32 matrix of few rows decodes exactly (its estimate as tiles or few-row chunks is above the decode's), although
+    the tiled kernel's fitted time is below: the fitted time decides between kernels that round the weights only."""
+    assert route(Q4_K, 48, 14848, 170, F32, F32) == "gemv_generic"
+    assert route(Q4_K, 2816, 2816, 191, F32, F32) == "gemm_pc_f32_scaled_f16"
