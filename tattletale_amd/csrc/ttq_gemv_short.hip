@@ -252,7 +252,7 @@ gemv_short_kernel(const uint8_t* __restrict__ w, const XT* __restrict__ x, int n
   while (kw >= ks) { kw -= ks; group++; }
   const int p0 = lane & (G - 1), sub = lane / G;
   const int row0 = ((int)blockIdx.x * rg + group) * R, m0 = (int)blockIdx.y * M;
-  const int pieces = n_in / F::kW, p = kw * G + p0, at = p < pieces ? p : 0;     // (past the row's end: the first piece, times zero)
+  const int pieces = n_in / F::kW, p = kw * G + p0, at = p < pieces ? p : 0;     // (past the row's end: the first piece, its sums left out)
   const uint32_t rb = F::row_bytes(n_in);
   typename F::Raw raw[RW];
 #pragma unroll
@@ -269,14 +269,13 @@ gemv_short_kernel(const uint8_t* __restrict__ w, const XT* __restrict__ x, int n
 #pragma unroll
       for (int r = 0; r < RW; r++) F::weights(raw[r], p, W[r]);
     }
-    if (p >= pieces) {
-#pragma unroll
-      for (int i = 0; i < F::kW; i++) xv[i] = 0.f;
-    }
     float sx[F::kSums];
     F::sums(xv, sx);
 #pragma unroll
-    for (int r = 0; r < RW; r++) acc[j * RW + r] = F::dot(W[r], xv, sx);
+    for (int r = 0; r < RW; r++) {
+      const double t = F::dot(W[r], xv, sx);
+      acc[j * RW + r] = p < pieces ? t : 0.0;      // (not by zeros among the activations: that block's scale may be an infinity)
+    }
     if (j + 1 < M) {
 #pragma unroll
       for (int i = 0; i < F::kW; i++) xv[i] = next[i];

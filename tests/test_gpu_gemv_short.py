@@ -94,3 +94,36 @@ def test_non_finite_rows_stay_alone_and_large_values_are_exact(fmt, xk):
     z = torch.zeros_like(x)
     z[:, 513] = 2.0 ** 112
     assert torch.equal(lay.forward(z, out_dtype=torch.float32) + 0.0, (dense(lay)[:, 513] * 2.0 ** 112).float().expand(m, -1) + 0.0)
+
+
+def positive_rows(fmt, n_out, n_in):
+    """Packed rows whose weights are all above zero, and the byte range of a block's scale."""
+    blocks = n_out * (n_in // BLOCK[fmt])
+    one = torch.tensor([0.01], dtype=torch.float16).view(torch.uint8)
+    if fmt == F.Q8_0:
+        b = torch.full((blocks, 34), 3, dtype=torch.uint8)
+        b[:, :2] = one
+        return b, slice(0, 2)
+    if fmt == F.Q4_K:
+        b = torch.full((blocks, 144), 0x11, dtype=torch.uint8)       # scales and quants above zero, d_min zero
+        b[:, :2], b[:, 2:4] = one, 0
+        return b, slice(0, 2)
+    b = torch.full((blocks, 210), 0xFF, dtype=torch.uint8)           # q - 32 = 31
+    b[:, 192:208], b[:, 208:210] = 5, one
+    return b, slice(208, 210)
+
+
+@pytest.mark.parametrize("n_in", [256, 1024, 1280, 3072, 4352])
+@pytest.mark.parametrize("m", [1, 2, 3])
+@pytest.mark.parametrize("xk", ["f32", "bf16"])
+@pytest.mark.parametrize("fmt", list(BLOCK), ids=list(NAMES.values()))
+def test_infinite_block_scale_gives_infinity(fmt, xk, m, n_in):
+    """Lanes past the end of a row read its first block: its scale may be anything."""
+    n_out, row = 24, 5
+    b, scale = positive_rows(fmt, n_out, n_in)
+    b[row * (n_in // BLOCK[fmt]), scale] = torch.tensor([float("inf")], dtype=torch.float16).view(torch.uint8)
+    lay = QuantLinear.init(b.to(DEV).view(-1), fmt, n_in, n_out, precision=F.PRECISION_F32_SCALES)
+    x = torch.ones(m, n_in, device=DEV, dtype=DT[xk])
+    y = lay.forward(x, out_dtype=torch.float32)
+    assert torch.equal(torch.isposinf(y), torch.isposinf(x.double() @ dense(lay).T))
+    assert torch.isposinf(y[:, row]).all() and torch.isfinite(y).sum().item() == m * (n_out - 1)
