@@ -207,6 +207,15 @@ typedef enum {
   TTQ_ROUTE_EXL3_GEMV_TWO_LAUNCHES = 33
 } ttq_route_id;
 TTQ_API int ttq_route(const ttq_qlinear* layer, int64_t m, int x_dtype, int y_dtype);
+/* The same, and into `text` (`room` bytes, zero-terminated, cut where it does not fit) what exactly is
+ * launched: the family's name where it has one kernel; "gemv_short" for matrices of a few MB, whose calls
+ * belong to the families TTQ_ROUTE_GEMV_GENERIC (fp32 activations, Q8_0), _DOT2 and _DOT2_MULTI; and for the
+ * tiled GEMM its rows x columns of a tile, "k/<copies>" where K is divided and "packed" where the
+ * activations are copied in fragment order first, e.g. "gemm_pc 256x64 k/2 packed". */
+TTQ_API int ttq_route_detail(const ttq_qlinear* layer, int64_t m, int x_dtype, int y_dtype, char* text, int64_t room);
+/* The same for ttq_gemm_q4_k_silu_mul ("gemm_skinny_silu_mul" or "gemm_pc_silu_mul" and its tile, whose
+ * columns are gate and up outputs by turns). */
+TTQ_API int ttq_gemm_q4_k_silu_mul_detail(int64_t m, int64_t n_ff, int64_t n_in, char* text, int64_t room);
 TTQ_API const char* ttq_route_name(int route);
 
 /* ---- decode GEMV, one entry per block format (m rows of x, normally m == 1) -------- */

@@ -68,6 +68,8 @@ SIGNATURES = {
     "ttq_release_workspaces": (_i32, []),
     "ttq_route": (_i32, [C.POINTER(QLinearStruct), _i64, _i32, _i32]),
     "ttq_route_name": (C.c_char_p, [_i32]),
+    "ttq_route_detail": (_i32, [C.POINTER(QLinearStruct), _i64, _i32, _i32, C.c_char_p, _i64]),
+    "ttq_gemm_q4_k_silu_mul_detail": (_i32, [_i64, _i64, _i64, C.c_char_p, _i64]),
     "ttq_gemm_q4_k_ws": (_i32, [_vp, _vp, _vp, _i64, _i64, _i64, _vp, _i64, _vp]),
     "ttq_gemm_q6_k_ws": (_i32, [_vp, _vp, _vp, _i64, _i64, _i64, _vp, _i64, _vp]),
     "ttq_gemm_q8_0_ws": (_i32, [_vp, _vp, _vp, _i64, _i64, _i64, _vp, _i64, _vp]),

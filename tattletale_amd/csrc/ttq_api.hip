@@ -7,7 +7,10 @@
 #include "../../include/ttq.h"
 #include "ttq_internal.h"
 
+#include <stdarg.h>
+#include <stdio.h>
 #include <stdlib.h>
+#include <string.h>
 
 namespace ttq {
 
@@ -27,6 +30,18 @@ int device_num_cus() {
 }
 
 thread_local RouteProbe* t_route_probe = nullptr;
+
+void route_say(const char* format, ...) {
+  RouteProbe* p = t_route_probe;
+  if (!p || !p->text) return;
+  const size_t have = strlen(p->text);
+  if (have && have + 3 < p->room) strcat(p->text, "; ");
+  const size_t at = strlen(p->text);
+  va_list args;
+  va_start(args, format);
+  vsnprintf(p->text + at, p->room - at, format, args);
+  va_end(args);
+}
 
 hipError_t allow_large_lds(const void* kernel, LargeLds& state) {
   int dev = 0;
@@ -562,7 +577,7 @@ int ttq_linear_forward(const ttq_qlinear* layer, const void* x, int x_dtype, int
 }
 
 // ---- which kernel family ttq_linear_forward would launch
-int ttq_route(const ttq_qlinear* layer, int64_t m, int x_dtype, int y_dtype) {
+static int probe_forward(const ttq_qlinear* layer, int64_t m, int x_dtype, int y_dtype, ttq::RouteProbe& probe) {
   if (!layer) return TTQ_ERR_NULL;
   // the dispatch itself, with a probe bound to this thread (nothing is launched, allocated or dereferenced) and
   // stand-ins for the buffers
@@ -574,9 +589,31 @@ int ttq_route(const ttq_qlinear* layer, int64_t m, int x_dtype, int y_dtype) {
     probe_layer.svh = stand_in;
   }
   if (layer->bias) probe_layer.bias = stand_in;
-  ttq::RouteProbe probe{0};
   ttq::t_route_probe = &probe;
   const int rc = ttq_linear_forward(&probe_layer, stand_in, x_dtype, m, stand_in, y_dtype, nullptr);
+  ttq::t_route_probe = nullptr;
+  return rc != TTQ_OK ? rc : probe.route;
+}
+int ttq_route(const ttq_qlinear* layer, int64_t m, int x_dtype, int y_dtype) {
+  ttq::RouteProbe probe{0, nullptr, 0};
+  return probe_forward(layer, m, x_dtype, y_dtype, probe);
+}
+int ttq_route_detail(const ttq_qlinear* layer, int64_t m, int x_dtype, int y_dtype, char* text, int64_t room) {
+  if (!text || room <= 0) return TTQ_ERR_NULL;
+  text[0] = 0;
+  ttq::RouteProbe probe{0, text, (size_t)room};
+  const int r = probe_forward(layer, m, x_dtype, y_dtype, probe);
+  if (r >= 0 && !text[0]) snprintf(text, (size_t)room, "%s", ttq_route_name(r));
+  return r;
+}
+int ttq_gemm_q4_k_silu_mul_detail(int64_t m, int64_t n_ff, int64_t n_in, char* text, int64_t room) {
+  if (!text || room <= 0) return TTQ_ERR_NULL;
+  text[0] = 0;
+  alignas(16) static char stand_in[16];
+  ttq::RouteProbe probe{0, text, (size_t)room};
+  ttq::t_route_probe = &probe;
+  uint16_t* p = reinterpret_cast<uint16_t*>(stand_in);
+  const int rc = ttq_gemm_q4_k_silu_mul(stand_in, p, p, m, n_ff, n_in, nullptr);
   ttq::t_route_probe = nullptr;
   return rc != TTQ_OK ? rc : probe.route;
 }

@@ -2,6 +2,8 @@
 // tile choice, split along K and its workspace, and the launchers behind ttq_gemm_* / ttq_linear_forward.
 #include "ttq_gemm_pc.h"
 
+#include <stdio.h>
+
 namespace ttq {
 
 // x: the activations, or (tile_if_packed >= 0) their packed copy and the tile's index for launch_gemm_packed
@@ -192,6 +194,13 @@ static hipError_t launch_pc_rows(const PcChoice& c, int tile_if_packed, const ui
   }
 }
 
+static void say_pc(const char* kernel, const PcChoice& c) {
+  const PcTile& t = kPcTiles[c.tile];
+  char copies[16] = "";
+  if (c.splits > 1) snprintf(copies, sizeof copies, " k/%d", c.splits);
+  route_say("%s %dx%d%s%s", kernel, pc_bm(t.mb), t.nj * 16, copies, c.packed ? " packed" : "");
+}
+
 // x in x_dtype: any type when the launch goes through the packed copy (the packing pass
 // rounds to bf16, or -- keep_f16 -- leaves fp16 activations as they are for the fp16 form of the kernel).
 template <int FMT, bool FUSE>
@@ -252,8 +261,10 @@ hipError_t launch_gemm_pc_x(int format, const void* w, const void* x, int x_dtyp
   if (route_probe(f16_native ? (x_dtype == kF32 ? kRouteGemmPcF32ScaledF16 : kRouteGemmPcF16)
                              : (x_dtype != kBF16 ? kRouteGemmPcBf16Copy
                                                  : (c.splits > 1 ? (packed ? kRouteGemmPcPackedSplitK : kRouteGemmPcSplitK)
-                                                                 : (packed ? kRouteGemmPcPacked : kRouteGemmPc)))))
+                                                                 : (packed ? kRouteGemmPcPacked : kRouteGemmPc))))) {
+    say_pc("gemm_pc", c);
     return hipSuccess;
+  }
   const uint8_t* wb = static_cast<const uint8_t*>(w);
   switch (format) {
     case kQ4_K: return launch_pc_fmt<kQ4_K, false>(wb, x, x_dtype, y, y_dtype, bias, bias_dtype, m, n_out, n_in, s, f16_native ? (x_dtype == kF32 ? 2 : 1) : 0);
@@ -285,6 +296,10 @@ hipError_t launch_gemm_pc_silu_mul(const void* w, const uint16_t* x_bf16, void* 
                                    int bias_dtype, int64_t m, int64_t n_ff, int64_t n_in, hipStream_t s) {
   if (m == 0 || n_ff == 0) return hipSuccess;
   if (y_dtype != kBF16 && y_dtype != kF32) return hipErrorInvalidValue;
+  if (route_probe(kRouteGemmPc)) {
+    say_pc("gemm_pc_silu_mul", pc_choose(kQ4_K, kBF16, m, n_ff, n_in, true));
+    return hipSuccess;
+  }
   return launch_pc_fmt<kQ4_K, true>(static_cast<const uint8_t*>(w), x_bf16, kBF16, y, y_dtype, bias, bias_dtype, m, n_ff,
                                     n_in, s);
 }

@@ -667,6 +667,8 @@ hipError_t launch_gemm_skinny_silu_mul(const void* w, const uint16_t* x_bf16, vo
                                        int bias_dtype, int64_t m, int64_t n_ff, int64_t n_in, hipStream_t s) {
   if (m == 0 || n_ff == 0) return hipSuccess;
   if (y_dtype != kBF16 && y_dtype != kF32) return hipErrorInvalidValue;
+  route_say("gemm_skinny_silu_mul");
+  if (route_probe(kRouteGemmSkinny)) return hipSuccess;
   return launch_skinny_fmt<SkQ4K, bf16_tag, true>(kQ4_K, static_cast<const uint8_t*>(w), x_bf16, y, y_dtype, bias, bias_dtype, m,
                                         n_ff, n_in, s);
 }

@@ -506,6 +506,7 @@ bool gemv_short_first(int format, int x_dtype, int64_t m, int64_t n_out, int64_t
 hipError_t launch_gemv_short_routed(int format, const void* w, const void* x, int x_dtype, void* y, int y_dtype, const void* bias,
                                     int bias_dtype, int64_t m, int64_t n_out, int64_t n_in, hipStream_t s) {
   const int id = format == kQ8_0 || x_dtype == kF32 ? kRouteGemvGeneric : (m == 1 ? kRouteGemvDot2 : kRouteGemvDot2Multi);
+  if (t_route_probe) route_say("gemv_short");
   TTQ_ROUTE(id, launch_gemv_short(format, w, x, x_dtype, y, y_dtype, bias, bias_dtype, m, n_out, n_in, s));
 }
 

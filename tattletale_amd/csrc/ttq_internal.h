@@ -51,7 +51,7 @@ enum : int {
   kRouteExl3Gemm = 32,
   kRouteExl3GemvTwoLaunches = 33,
 };
-struct RouteProbe { int route; };
+struct RouteProbe { int route; char* text; size_t room; };      // text: what route_say adds goes here, if anywhere
 extern thread_local RouteProbe* t_route_probe;
 inline bool route_probe(int id) {
   RouteProbe* p = t_route_probe;
@@ -59,6 +59,8 @@ inline bool route_probe(int id) {
   if (p->route == 0) p->route = id;
   return true;
 }
+// what a dispatcher knows beyond the family: a kernel of its own, tiles and copies (joined by "; "); nothing unless a probe asks
+__attribute__((format(printf, 1, 2))) void route_say(const char* format, ...);
 #define TTQ_ROUTE(id, call)                      \
   do {                                           \
     if (::ttq::route_probe(id)) return hipSuccess; \

@@ -173,6 +173,15 @@ class QuantLinear:
             raise TtqError(int(r), "ttq_route")
         return _lib.lib().ttq_route_name(r).decode()
 
+    def route_detail(self, m: int, x_dtype: torch.dtype, out_dtype: Optional[torch.dtype] = None) -> str:
+        """What exactly that is: kernel, and for the tiled GEMM its tile, copies along K and way to the activations
+        (``ttq_route_detail``)."""
+        st, text = self._struct(), C.create_string_buffer(128)
+        r = _lib.lib().ttq_route_detail(C.byref(st), m, _code(x_dtype), _code(out_dtype or x_dtype), text, len(text))
+        if r < 0:
+            raise TtqError(int(r), "ttq_route_detail")
+        return text.value.decode()
+
     def forward(self, x: torch.Tensor, out_dtype: Optional[torch.dtype] = None,
                 workspace: Optional[torch.Tensor] = None) -> torch.Tensor:
         """x (..., in_features) -> (..., out_features)  (linear.nim:45-57).

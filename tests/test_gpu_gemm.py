@@ -56,12 +56,19 @@ def test_gemm_identity_activations_give_bf16_weights_exactly(n_in):
 # as 2 / 4 / 7 / 8 copies that split K and add their partial sums through a workspace.
 @pytest.mark.parametrize("fmt", [F.Q4_K, F.Q6_K, F.Q8_0])
 @pytest.mark.parametrize("m,n_out,n_in", [(512, 4096, 4096), (256, 1024, 4096), (300, 1000, 2048), (130, 2048, 14336),
-                                          (192, 4096 + 40, 3584), (300, 256, 6144), (300, 256, 5376)])
+                                          (192, 4096 + 40, 3584), (300, 256, 6144), (300, 256, 5376),
+                                          (200, 4096 + 64, 4096)])
 def test_gemm_split_along_k(fmt, m, n_out, n_in):
     """Against the float64 product; three calls in a row give the same bits (the copies of a tile are added in a
     fixed order, and the arrival counters are back at zero after every launch), also after a call with another
-    shape in between (the workspace grows).  On a 256-CU device the chooser takes two or four copies for the
-    first shapes, eight for 256 x 6144 and seven for 256 x 5376 (21 super-blocks)."""
+    shape in between (the workspace grows).  On a 256-CU device the chooser takes two copies for 1000 x 2048, 4160 x 4096
+    and, Q6_K and Q8_0, 4136 x 3584, four for 1024 x 4096 and 2048 x 14336, eight for 256 x 6144 and seven for
+    256 x 5376 (21 super-blocks), and one for 4096 x 4096 and Q4_K at 4136 x 3584, which are here as neighbours."""
+    copies = {(256, 1024, 4096): 4, (300, 1000, 2048): 2, (130, 2048, 14336): 4, (300, 256, 6144): 8, (300, 256, 5376): 7,
+              (200, 4160, 4096): 2, (192, 4136, 3584): 1 if fmt == F.Q4_K else 2, (512, 4096, 4096): 1}[m, n_out, n_in]
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        plan = QuantLinear(torch.empty(0, device=DEV), fmt, n_in, n_out).route_detail(m, torch.bfloat16)
+        assert (f" k/{copies}" in plan) if copies > 1 else " k/" not in plan
     w = Q.fill_normal(700 + m, 0, 0.02, n_out * n_in).reshape(n_out, n_in)
     p = Q.quantize(fmt, w)
     what = oracle.dequant(fmt, p, n_out, n_in)

@@ -53,6 +53,7 @@ def test_edges(fmt, n_out, n_in, xk):
     for m in rows(fmt, xk, n_in):
         family = "gemv_generic" if fmt == F.Q8_0 or xk == "f32" else ("gemv_dot2" if m == 1 else "gemv_dot2_multi")
         assert lay.route(m, DT[xk], torch.float32) == family
+        assert lay.route_detail(m, DT[xk], torch.float32) == "gemv_short"
         x = torch.randn(m, n_in, device=DEV, generator=gen).to(DT[xk])
         ref = x.double() @ wd.T + bias.double()
         y = lay.forward(x, out_dtype=torch.float32)
@@ -75,6 +76,9 @@ def test_more_wavefronts_than_two_rows_each(fmt, xk, m, n_out, n_in):
     ref = x.double() @ dense(lay).T
     y = lay.forward(x, out_dtype=torch.float32)
     bound = TOL if (fmt, n_out) != (F.Q4_K, 1536) else 2e-6     # (that one has the packed-dot kernel for 16-bit rows)
+    # (16-bit rows of 1536 x 5120 stay with the packed-dot kernels)
+    other = {(F.Q4_K, 1): "gemv_dot2", (F.Q6_K, 2): "gemv_dot2_multi"}.get((fmt, m)) if n_out == 1536 else None
+    assert lay.route_detail(m, DT[xk], torch.float32) == ("gemv_short" if other is None or xk == "f32" else other)
     assert ((y.double() - ref).norm(dim=-1) / ref.norm(dim=-1)).max().item() <= bound
 
 

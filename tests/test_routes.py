@@ -150,6 +150,43 @@ def test_route_is_a_pure_query():
     assert len({L.ttq_route(C.byref(st), 512, BF16, BF16) for _ in range(5)}) == 1
 
 
+def detail(fmt, n_out, n_in, m, x_dtype, y_dtype, precision=_lib.PRECISION_AUTO):
+    text = C.create_string_buffer(128)
+    st = QLinearStruct(format=fmt, n_out=n_out, n_in=n_in, precision=precision)
+    r = _lib.lib().ttq_route_detail(C.byref(st), m, x_dtype, y_dtype, text, len(text))
+    assert r == _lib.lib().ttq_route(C.byref(st), m, x_dtype, y_dtype) >= 0
+    return text.value.decode()
+
+
+def test_route_detail_names_the_kernel_and_the_tile():
+    """Calls of one family that go to different kernels, and the tiled GEMM's launches, told apart."""
+    assert detail(Q4_K, 14336, 4096, 1, BF16, F32) == "gemv_q4k_stream"         # a family of one kernel: its name
+    assert detail(Q4_K, 1024, 4096, 1, BF16, F32) == detail(Q8_0, 2048, 1024, 1, F32, F32) == "gemv_short"
+    assert detail(Q6_K, 2560, 2560, 3, F32, F32) == detail(Q6_K, 1024, 1024, 2, F16, F16) == "gemv_short"
+    assert detail(Q4_K, 16384, 53248, 1, BF16, F32) == "gemv_dot2"
+    assert detail(Q6_K, 1536, 4096, 4, BF16, BF16) == "gemv_dot2_multi"
+    assert detail(Q4_K, 14336, 4096, 512, BF16, BF16) == "gemm_pc 256x112 packed"
+    assert detail(Q4_K, 4096, 4096, 512, BF16, BF16) == "gemm_pc 128x64"
+    assert detail(Q4_K, 4096, 14336, 512, BF16, BF16) == "gemm_pc 256x64 k/2 packed"
+    assert detail(Q4_K, 14336, 4096, 0, BF16, BF16) == "none (empty call)"
+
+
+def test_route_detail_checks_its_arguments():
+    L, text = _lib.lib(), C.create_string_buffer(b"x" * 15, 16)
+    st = QLinearStruct(format=Q4_K, n_out=4096, n_in=14336)
+    assert L.ttq_route_detail(C.byref(st), 512, BF16, BF16, None, 16) == _lib.ERR_NULL
+    assert L.ttq_route_detail(C.byref(st), 512, BF16, BF16, text, 0) == _lib.ERR_NULL
+    assert L.ttq_route_detail(None, 512, BF16, BF16, text, 16) == _lib.ERR_NULL and text.value == b""
+    assert L.ttq_route_detail(C.byref(st), 512, BF16, BF16, text, 16) == _lib.ROUTE["gemm_pc_packed_split_k"]
+    assert text.value == b"gemm_pc 256x64 "                                     # cut, and zero-terminated
+    assert L.ttq_gemm_q4_k_silu_mul_detail(512, 14336, 4096, None, 16) == _lib.ERR_NULL
+    assert L.ttq_gemm_q4_k_silu_mul_detail(512, 14336, 100, text, 16) == _lib.ERR_SHAPE
+    big = C.create_string_buffer(64)
+    assert L.ttq_gemm_q4_k_silu_mul_detail(2048, 14336, 4096, big, 64) >= 0 and big.value == b"gemm_pc_silu_mul 256x112"
+    assert L.ttq_gemm_q4_k_silu_mul_detail(32, 3072, 1024, big, 64) >= 0 and big.value == b"gemm_skinny_silu_mul"
+    assert L.ttq_gemm_q4_k_silu_mul_detail(0, 3072, 1024, big, 64) == _lib.ROUTE["none"] and big.value == b""
+
+
 def test_workspace_size_query_and_argument_checks():
     L = _lib.lib()
     q = QLinearStruct(format=Q4_K, n_out=4096, n_in=14336)
