@@ -133,8 +133,9 @@ static PcChoice pc_choose(int format, int x_dtype, int64_t m, int64_t n_out, int
           cost += c.trips0 + c.trips1 * (float)(sp > 2 ? sp : 1) + c.traffic * 2.f * (float)sp * (float)(mt * bm) * (float)(nt * bo) / 1.0e6f;
         if (i == route.tile && sp == route.splits && (packed != 0) == route_packed) before = PcChoice{i, sp, packed != 0, cost};
         // (long launches of the K formats read a packed copy: the estimates are least sure of short rows, 20112 x 1024 Q4_K at 4079 rows
-        // 222 us without it and 208)
-        if (!fuse && !packed && forced_packed < 0 && format != kQ8_0 && cost >= 45.f) continue;
+        // 222 us without it and 208; and of Q8_0 beyond 4096 rows, but for few columns, where a packed block of 8192 rows leaves compute
+        // units idle: 5184 x 512 at 16871 rows 269 / 174, 9136 x 256 at 5868 102 / 90, but 512 x 4096 at 20000 0.6 to 0.9 of the time)
+        if (!fuse && !packed && forced_packed < 0 && cost >= 45.f && (format != kQ8_0 || (m > 4096 && n_out > 1024))) continue;
         if (cost < best.cost_us * 0.999f || (forced_splits > 0 && sp == forced_splits && best.splits != sp))
           best = PcChoice{i, sp, packed != 0, cost};
       }
@@ -145,7 +146,13 @@ static PcChoice pc_choose(int format, int x_dtype, int64_t m, int64_t n_out, int
   // (long launches one after the other run at the clock that the power limit leaves, where tiles that dequantize a weight for fewer
   // products lose what they win alone: a block of 4096 / 14336 at 4096 rows with 64-column tiles in three of its layers 1860 us
   // against 1830, each of those layers alone 2 to 5 percent faster)
-  const float margin = n_in <= (format == kQ8_0 ? 1024 : 512) && n_out > 16384 ? 0.f : (before.cost_us >= 100.f ? 0.9f : 0.95f);
+  // (beyond 4096 rows, which the fit has not seen, and for 256x112 tiles of Q4_K and Q8_0 from 2048 on, whose time it puts too high,
+  // 16-bit rows change over where the new choice is a fifth ahead: of 8200 such calls 11 percent were more than 5 percent slower than the
+  // earlier choice, by up to half, and 0.7 are; Q4_K 34944 x 1024 at 5993 rows 615 / 513 us, fp16 12288 x 1024 at 3905 161 / 133, Q8_0
+  // fp16 512 x 4096 at 6338 82 / 68)
+  float margin = n_in <= (format == kQ8_0 ? 1024 : 512) && n_out > 16384 ? 0.f : (before.cost_us >= 100.f ? 0.9f : 0.95f);
+  const bool unsure = m > 4096 || (m > 2048 && format != kQ6_K && before.tile == 0 && best.tile != 0);
+  if (unsure && x_dtype != kF32 && margin > 0.8f) margin = 0.8f;
   return before.cost_us < 1e29f && forced < 0 && forced_splits == 0 && best.cost_us > margin * before.cost_us ? before : best;
 }
 

@@ -171,6 +171,17 @@ def test_route_detail_names_the_kernel_and_the_tile():
     assert detail(Q4_K, 14336, 4096, 0, BF16, BF16) == "none (empty call)"
 
 
+def test_long_launches_keep_the_tile_that_was_measured_for_them():
+    """Beyond the rows that the fitted times have seen: Q8_0 with more than a few columns reads a packed copy, and another tile than the
+    earlier model's has to be a fifth ahead for 16-bit rows."""
+    for n_out, n_in, m in ((5184, 512, 16871), (9136, 256, 5868), (4096, 2048, 12000)):
+        assert route(Q8_0, n_out, n_in, m, BF16, BF16) == "gemm_pc_packed"
+    assert route(Q8_0, 512, 4096, 20000, BF16, BF16) == route(Q8_0, 256, 4096, 16384, BF16, BF16) == "gemm_pc"
+    assert detail(Q4_K, 34944, 1024, 5993, BF16, BF16) == detail(Q4_K, 2304, 1536, 3648, BF16, BF16) == "gemm_pc 256x112 packed"
+    assert detail(Q4_K, 12288, 1024, 3905, F16, F16) == "gemm_pc 256x112 packed"
+    assert detail(Q8_0, 512, 4096, 6338, F16, F16) == "gemm_pc 128x112 packed"
+
+
 def test_route_detail_checks_its_arguments():
     L, text = _lib.lib(), C.create_string_buffer(b"x" * 15, 16)
     st = QLinearStruct(format=Q4_K, n_out=4096, n_in=14336)
