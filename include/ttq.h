@@ -211,7 +211,8 @@ TTQ_API int ttq_route(const ttq_qlinear* layer, int64_t m, int x_dtype, int y_dt
  * launched: the family's name where it has one kernel; "gemv_short" for matrices of a few MB, whose calls
  * belong to the families TTQ_ROUTE_GEMV_GENERIC (fp32 activations, Q8_0), _DOT2 and _DOT2_MULTI; and for the
  * tiled GEMM its rows x columns of a tile, "k/<copies>" where K is divided and "packed" where the
- * activations are copied in fragment order first, e.g. "gemm_pc 256x64 k/2 packed". */
+ * activations are copied in fragment order first, e.g. "gemm_pc 256x64 k/2 packed" (more than 8192 packed
+ * rows: the launch of 8192 of them, then that of the rest). */
 TTQ_API int ttq_route_detail(const ttq_qlinear* layer, int64_t m, int x_dtype, int y_dtype, char* text, int64_t room);
 /* The same for ttq_gemm_q4_k_silu_mul ("gemm_skinny_silu_mul" or "gemm_pc_silu_mul" and its tile, whose
  * columns are gate and up outputs by turns). */

@@ -667,7 +667,7 @@ int64_t ttq_workspace_bytes(const ttq_qlinear* layer, int64_t m, int x_dtype) {
   if (m == 0 || layer->n_out == 0) return 0;
   const int64_t n_out = layer->n_out, n_in = layer->n_in;
   const int64_t header = (int64_t)ttq::caller_workspace_header_bytes();
-  constexpr int64_t kExl3Rows = 4096, kGemmRows = 8192;   // rows whose rotated / packed copy is in the workspace at a time
+  constexpr int64_t kExl3Rows = 4096;   // rows whose rotated copy is in the workspace at a time
   if (layer->format == TTQ_EXL3) {              // hand-off words; the rotated activations of the many-row form
     const int64_t block_rows = ((m < kExl3Rows ? m : kExl3Rows) + 15) / 16 * 16;   // whole blocks of 16 rows
     const int64_t partials = (int64_t)ttq::gemm_exl3_partials_bytes(m, n_out, n_in);
@@ -677,20 +677,15 @@ int64_t ttq_workspace_bytes(const ttq_qlinear* layer, int64_t m, int x_dtype) {
   // scaled fp16 copy)
   if (m < 5 && !(x_dtype == TTQ_F32 && m >= 2)) return 0;
   // the packed bf16 copy of the activations where the prefill GEMM wants one, then the partial sums of a launch
-  // split along K: the prefill GEMM's exact size for every row count it can be called with here, and the few-row
-  // kernel's bound (one 64 x 64 tile of sums per compute unit)
-  const int64_t block_rows = m < kGemmRows ? m : kGemmRows;
+  // split along K: the prefill GEMM's exact size, and the few-row kernel's bound (one 64 x 64 tile of sums per
+  // compute unit)
   // (fp16 activations beyond 64 rows may take the prefill GEMM over a packed fp16 copy; fp32 ones over a scaled
   // fp16 copy, or a bf16 copy where the layer allows it)
   const int copy_dtype = (x_dtype == TTQ_F16 && m > 64) || x_dtype == TTQ_F32 ? x_dtype : TTQ_BF16;
   int64_t scratch = ((int64_t)ttq::gemm_pc_packed_bytes(layer->format, m, n_out, n_in, copy_dtype) + 255) & ~(int64_t)255;
   int64_t partials = (int64_t)ttq::device_num_cus() * (16 * 4 * (16 * 4 + 1) * 4);
-  const int64_t rows[3] = {m, block_rows, m % kGemmRows};
-  for (int64_t r : rows) {
-    if (r <= 0) continue;
-    const int64_t p = (int64_t)ttq::gemm_pc_partials_bytes(layer->format, copy_dtype, r, n_out, n_in);
-    if (p > partials) partials = p;
-  }
+  const int64_t tiled = (int64_t)ttq::gemm_pc_partials_bytes(layer->format, copy_dtype, m, n_out, n_in);
+  if (tiled > partials) partials = tiled;
   return header + scratch + ((partials + 255) & ~(int64_t)255);
 }
 

@@ -102,8 +102,9 @@ static float pc_pack_us(int x_dtype, int64_t m, int64_t n_in) {
 }
 
 // The tile, the copies along K and the way to the activations of a launch.  Only bf16 activations can be read as they are, and the
-// fused gate||up form must (its epilogue does not fit beside the packed kernel's three steps of A fragments).
-static PcChoice pc_choose(int format, int x_dtype, int64_t m, int64_t n_out, int64_t n_in, bool fuse) {
+// fused gate||up form must (its epilogue does not fit beside the packed kernel's three steps of A fragments).  copied: the packed copy is
+// there already (a block of rows of a longer launch), so it is read and costs nothing.
+static PcChoice pc_choose(int format, int x_dtype, int64_t m, int64_t n_out, int64_t n_in, bool fuse, bool copied = false) {
   static const int forced = dev_knob("TTQ_GEMM_TILE", -1);
   static const int forced_splits = dev_knob("TTQ_GEMM_SPLITS", 0);   // A/B: 1 = never split, n = n ways where possible
   static const int forced_packed = dev_knob("TTQ_GEMM_PACKED", -1);  // A/B: 0 never, 1 always
@@ -111,10 +112,10 @@ static PcChoice pc_choose(int format, int x_dtype, int64_t m, int64_t n_out, int
   const int64_t blocks = n_in / 256;
   PcChoice best{0, 1, false, 1e30f}, before = best;
   const PcRoute route = fuse ? PcRoute{-1, 1, 0.f} : pc_route(m, n_out, n_in);
-  const bool route_packed = x_dtype != kBF16 || (kPcTiles[route.tile < 0 ? 0 : route.tile].mb == 4 && route.cost_us >= 45.f);
-  for (int packed = fuse || x_dtype == kBF16 ? 0 : 1; packed <= (fuse ? 0 : 1); packed++) {
-    if (!fuse && x_dtype == kBF16 && forced_packed >= 0 && forced_packed != packed) continue;
-    const float pack = packed ? pc_pack_us(x_dtype, m, n_in) : 0.f;
+  const bool route_packed = copied || x_dtype != kBF16 || (kPcTiles[route.tile < 0 ? 0 : route.tile].mb == 4 && route.cost_us >= 45.f);
+  for (int packed = fuse || (x_dtype == kBF16 && !copied) ? 0 : 1; packed <= (fuse ? 0 : 1); packed++) {
+    if (!fuse && !copied && x_dtype == kBF16 && forced_packed >= 0 && forced_packed != packed) continue;
+    const float pack = packed && !copied ? pc_pack_us(x_dtype, m, n_in) : 0.f;
     for (int i = 0; i < kPcTileCount; i++) {
       if (forced >= 0 && forced < kPcTileCount && i != forced) continue;
       const PcTile& t = kPcTiles[i];
@@ -156,14 +157,31 @@ static PcChoice pc_choose(int format, int x_dtype, int64_t m, int64_t n_out, int
   return before.cost_us < 1e29f && forced < 0 && forced_splits == 0 && best.cost_us > margin * before.cost_us ? before : best;
 }
 
-// bytes of partial sums that a launch of this shape keeps in the workspace (0: not split along K)
-size_t gemm_pc_partials_bytes(int format, int x_dtype, int64_t m, int64_t n_out, int64_t n_in) {
-  if (m <= 0 || n_out <= 0 || n_in < 256) return 0;
-  const PcChoice c = pc_choose(format, x_dtype, m, n_out, n_in, false);
+constexpr int64_t kPackRows = 8192;         // rows packed (and multiplied) at a time
+
+// the launch of `rows` of the m rows of a call that goes through the packed copy
+static PcChoice pc_choose_block(const PcChoice& whole, int64_t rows, int format, int x_dtype, int64_t m, int64_t n_out, int64_t n_in) {
+  return rows == m ? whole : pc_choose(format, x_dtype, rows, n_out, n_in, false, true);
+}
+
+static size_t pc_partials_bytes(const PcChoice& c, int64_t m, int64_t n_out) {
   if (c.splits <= 1) return 0;
   const PcTile& t = kPcTiles[c.tile];
   const int64_t nt = (n_out + t.nj * 16 - 1) / (t.nj * 16), mt = (m + pc_bm(t.mb) - 1) / pc_bm(t.mb);
   return (size_t)(nt * mt * 4) * (size_t)c.splits * (size_t)(t.mb * t.nj * 1024);
+}
+
+// bytes of partial sums that a call of this shape keeps in the workspace at a time (0: not split along K)
+size_t gemm_pc_partials_bytes(int format, int x_dtype, int64_t m, int64_t n_out, int64_t n_in) {
+  if (m <= 0 || n_out <= 0 || n_in < 256) return 0;
+  const PcChoice whole = pc_choose(format, x_dtype, m, n_out, n_in, false);
+  if (!whole.packed || m <= kPackRows) return pc_partials_bytes(whole, m, n_out);
+  size_t most = 0;
+  for (int64_t rows : {kPackRows, m % kPackRows}) {
+    const size_t bytes = rows ? pc_partials_bytes(pc_choose_block(whole, rows, format, x_dtype, m, n_out, n_in), rows, n_out) : 0;
+    most = bytes > most ? bytes : most;
+  }
+  return most;
 }
 
 // Rough time of the GEMM for this shape (microseconds), for callers that can also run the
@@ -183,8 +201,6 @@ float gemm_pc_cost_us(int format, int x_dtype, int64_t m, int64_t n_out, int64_t
 
 // Whether that model would divide a launch along K.
 bool gemm_pc_splits_k(int64_t m, int64_t n_out, int64_t n_in) { return pc_route(m, n_out, n_in).splits > 1; }
-
-constexpr int64_t kPackRows = 8192;         // rows packed (and multiplied) at a time
 
 template <int FMT, bool FUSE>
 static hipError_t launch_pc_rows(const PcChoice& c, int tile_if_packed, const uint8_t* wb, const uint16_t* x, void* y,
@@ -235,7 +251,7 @@ static hipError_t launch_pc_fmt(const uint8_t* wb, const void* x, int x_dtype, v
       e = launch_gemm_pack_activations(static_cast<const char*>(x) + r0 * n_in * xsize, x_dtype, static_cast<uint16_t*>(ws),
                                        rows, n_in, s, f16_mode == 1);
     if (e != hipSuccess) return e;
-    PcChoice c = rows == m ? whole : pc_choose(FMT, x_dtype, rows, n_out, n_in, FUSE);      // (the copy is made: its tile alone counts)
+    const PcChoice c = pc_choose_block(whole, rows, FMT, x_dtype, m, n_out, n_in);
     e = launch_pc_rows<FMT, FUSE>(c, c.tile, wb, static_cast<const uint16_t*>(ws), static_cast<char*>(y) + r0 * n_out * ysize,
                                   y_dtype, bias, bias_dtype, rows, n_out, n_in, s, f16_mode != 0, row_scale);
     if (e != hipSuccess) return e;
@@ -269,7 +285,8 @@ hipError_t launch_gemm_pc_x(int format, const void* w, const void* x, int x_dtyp
                              : (x_dtype != kBF16 ? kRouteGemmPcBf16Copy
                                                  : (c.splits > 1 ? (packed ? kRouteGemmPcPackedSplitK : kRouteGemmPcSplitK)
                                                                  : (packed ? kRouteGemmPcPacked : kRouteGemmPc))))) {
-    say_pc("gemm_pc", c);
+    say_pc("gemm_pc", packed ? pc_choose_block(c, m < kPackRows ? m : kPackRows, format, x_dtype, m, n_out, n_in) : c);
+    if (packed && m > kPackRows && m % kPackRows) say_pc("gemm_pc", pc_choose_block(c, m % kPackRows, format, x_dtype, m, n_out, n_in));
     return hipSuccess;
   }
   const uint8_t* wb = static_cast<const uint8_t*>(w);

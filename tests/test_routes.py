@@ -182,6 +182,16 @@ def test_long_launches_keep_the_tile_that_was_measured_for_them():
     assert detail(Q8_0, 512, 4096, 6338, F16, F16) == "gemm_pc 128x112 packed"
 
 
+@pytest.mark.parametrize("fmt,n_out,n_in,m", [(Q8_0, 8317, 3072, 25463), (Q8_0, 7773, 256, 18290), (Q4_K, 116, 7168, 13668), (Q4_K, 512, 14336, 8300),
+                                              (Q6_K, 258, 5376, 12071), (Q6_K, 9481, 512, 25813), (Q4_K, 3676, 256, 13139)])
+def test_blocks_of_a_packed_launch_are_chosen_among_packed_forms(fmt, n_out, n_in, m):
+    """More than 8192 rows are packed and multiplied a block at a time: a block's copy is there already, so its tile and copies along K
+    are those of the packed kernel's times alone, whatever type the copy was made from."""
+    plan = detail(fmt, n_out, n_in, m, BF16, BF16)
+    assert plan == detail(fmt, n_out, n_in, m, F16, F16)
+    assert [form.endswith(" packed") for form in plan.split("; ")] == [True, True]
+
+
 def test_route_detail_checks_its_arguments():
     L, text = _lib.lib(), C.create_string_buffer(b"x" * 15, 16)
     st = QLinearStruct(format=Q4_K, n_out=4096, n_in=14336)
