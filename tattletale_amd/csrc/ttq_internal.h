@@ -318,7 +318,7 @@ hipError_t launch_hadamard128(float* v, const uint16_t* pre, const uint16_t* pos
                               hipStream_t s);
 
 // Workspaces the library keeps per (slot, device, stream), grown on demand (ttq_workspace.hip).
-constexpr int kWsExl3Rotated = 0, kWsGemmPartials = 2, kWsGemmCounters = 3, kWsPackedActivations = 4;
+constexpr int kWsExl3Rotated = 0, kWsGemmPartials = 2, kWsGemmCounters = 3, kWsPackedActivations = 4, kWsSlots = 5;
 // zeroed: a newly allocated buffer is cleared (on the stream) before it is handed out
 hipError_t stream_workspace(int slot, hipStream_t s, size_t bytes, void** out, bool zeroed = false);
 // Frees every library-owned workspace (nothing that uses one may be in flight or captured).
@@ -335,10 +335,11 @@ class CallerWsScope {
   CallerWsScope& operator=(const CallerWsScope&) = delete;
   bool too_small() const;      // some request did not fit (the call then failed with hipErrorOutOfMemory)
  private:
-  alignas(8) unsigned char state_[40];
+  alignas(8) unsigned char state_[32 + 16 * kWsSlots];
 };
-// false: no caller workspace is bound.  true: *out / *err say where the region lies or that it does not fit.
-bool caller_workspace_region(int region, size_t bytes, void** out, hipError_t* err);
+// false: no caller workspace is bound.  true: *out / *err say where the region lies or that it does not fit.  slot: which kind of
+// scratch (kWs...) a request for kCwScratch is.
+bool caller_workspace_region(int region, size_t bytes, void** out, hipError_t* err, int slot = 0);
 // bytes in front of the scratch part of a caller-owned workspace (arrival counters, trellis hand-off words)
 size_t caller_workspace_header_bytes();
 int64_t exl3_workspace_words();

@@ -27,7 +27,12 @@ struct Owned { Buf cur; std::vector<void*> retired; };
 std::mutex g_mutex;
 std::unordered_map<uint64_t, Owned> g_bufs;
 
-struct CallerWs { uint8_t* base; size_t bytes, bump; bool too_small; };
+struct CallerWs {
+  uint8_t* base;
+  size_t bytes, bump;
+  bool too_small;
+  struct { size_t off, bytes; } scratch[kWsSlots];      // what the call has taken of each kind; bytes 0: nothing yet
+};
 thread_local CallerWs* t_caller = nullptr;
 
 constexpr size_t kCwCounterBytes = 64 * 1024;
@@ -45,12 +50,16 @@ CallerWsScope::CallerWsScope(void* ws, size_t bytes) {
   c->bytes = bytes;
   c->bump = caller_workspace_header_bytes();
   c->too_small = false;
+  for (auto& s : c->scratch) s = {0, 0};
   t_caller = c;
 }
 CallerWsScope::~CallerWsScope() { t_caller = nullptr; }
 bool CallerWsScope::too_small() const { return reinterpret_cast<const CallerWs*>(state_)->too_small; }
 
-bool caller_workspace_region(int region, size_t bytes, void** out, hipError_t* err) {
+// A call that runs in blocks of rows asks for its scratch once per launch.  The launches are on one stream, one after the
+// other, so they share a place, as they do in the library's own buffers: the size that ttq_workspace_bytes states is that of the
+// largest of them.  (What a later launch needs more is added where the place is the last one taken.)
+bool caller_workspace_region(int region, size_t bytes, void** out, hipError_t* err, int slot) {
   CallerWs* c = t_caller;
   if (!c) return false;
   size_t off = 0;
@@ -60,8 +69,14 @@ bool caller_workspace_region(int region, size_t bytes, void** out, hipError_t* e
     off = kCwCounterBytes;
     if (bytes > caller_workspace_header_bytes() - kCwCounterBytes) c->too_small = true;
   } else {
-    off = c->bump;
-    c->bump = off + round256(bytes);
+    auto& s = c->scratch[slot];
+    const size_t need = round256(bytes);
+    if (s.bytes < need || s.bytes == 0) {
+      if (s.bytes == 0 || s.off + s.bytes != c->bump) s.off = c->bump;
+      s.bytes = need;
+      c->bump = s.off + need;
+    }
+    off = s.off;
   }
   if (!c->base || off + bytes > c->bytes) c->too_small = true;
   *out = c->too_small ? nullptr : c->base + off;
@@ -71,7 +86,7 @@ bool caller_workspace_region(int region, size_t bytes, void** out, hipError_t* e
 
 hipError_t stream_workspace(int slot, hipStream_t s, size_t bytes, void** out, bool zeroed) {
   hipError_t e = hipSuccess;
-  if (caller_workspace_region(slot == kWsGemmCounters ? kCwCounters : kCwScratch, bytes, out, &e)) return e;
+  if (caller_workspace_region(slot == kWsGemmCounters ? kCwCounters : kCwScratch, bytes, out, &e, slot)) return e;
   int dev = 0;
   e = hipGetDevice(&dev);
   if (e != hipSuccess) return e;

@@ -156,6 +156,21 @@ def test_fp16_gemm_with_a_caller_workspace(m, n_out, n_in, xk):
     assert e.value.status == F.ERR_WORKSPACE
 
 
+@pytest.mark.parametrize("xk", ["bf16", "f16"])
+@pytest.mark.parametrize("m,n_out,n_in,last", [(13668, 116, 7168, "k/4"), (8300, 512, 14336, "k/8")])
+def test_blocks_of_a_packed_launch_with_a_caller_workspace(m, n_out, n_in, last, xk):
+    """More than 8192 rows, the last block of them divided along K: a workspace of the size asked for holds the copy and the sums."""
+    layer = QuantLinear.init(packed_to_dev(random_blocks(F.Q4_K, n_out * (n_in // 256), seed=m)), F.Q4_K, n_in, n_out)
+    x = (torch.randn(m, n_in, device=DEV, generator=torch.Generator(DEV).manual_seed(m)) * 0.05).to({"bf16": torch.bfloat16, "f16": torch.float16}[xk])
+    assert f" {last} packed" in layer.route_detail(m, x.dtype).split("; ")[1]
+    y = layer.forward(x, workspace=zeros_ws(layer.workspace_bytes(m, x.dtype)), out_dtype=torch.float32)
+    assert torch.equal(y, layer.forward(x, out_dtype=torch.float32))
+    w = QL.dequantize(F.Q4_K, layer.qweight, n_out, n_in).to(x.dtype)          # as the kernel rounds them
+    for rows in (slice(0, 300), slice(m - 300, m)):
+        ref = x[rows].double() @ w.double().T
+        assert ((y[rows] - ref).norm() / ref.norm()).item() <= 1e-5
+
+
 @pytest.mark.parametrize("m", [16, 80])
 def test_few_fp32_rows_with_a_caller_workspace(m):
     """fp32 activations of a few rows: the scaled fp16 copy and its row factors (and the partial sums of a launch
