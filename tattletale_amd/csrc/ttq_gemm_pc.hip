@@ -190,13 +190,20 @@ float gemm_pc_estimate_us(int format, int64_t m, int64_t n_out, int64_t n_in) {
   return pc_route(m, n_out, n_in).cost_us * (format == kQ8_0 ? 1.9f : (format == kQ6_K ? 1.4f : 1.f)) + 2.f;
 }
 
-// The fitted time, for the choice against chunks of the few-row kernel.  It errs most for one or two short row tiles (of the
-// calls of 65 to 128 rows that it sent to tiles 20 in 326 were 5 to 30 percent slower than in chunks, over rows of more than 8192
-// values 6 in 45, by up to half), so the tiles have to be a tenth ahead there, Q8_0 (ten of fifteen that
-// were still slower) a quarter, and the long ones go by the model above alone.
+// The fitted time, for the choice against chunks of the few-row kernel.  It errs most for one or two short row tiles, so up to 128 rows
+// the tiles have to be a tenth ahead, Q8_0 a quarter, and long rows of weights go by the model above alone.  Where it still sent calls to tiles
+// that were more than 3 percent slower there than in chunks (of 10600 timed calls that it had moved), the model above decides too:
+//   Q6_K, 65 to 128 rows, more than 4096 outputs and values: two thirds of them (fp16 5440 x 6400 at 68 rows 39 us in chunks, 55 in tiles)
+//   Q6_K, 129 to 184 rows, a full tile and the rest of the next: over rows of more than 6144 values, up to 144 rows of 4096, a fifth to a
+//     half (bf16 192 x 6400 at 141 39 / 50)
+//   Q8_0, 97 to 128 rows, 1025 to 4096 outputs, more than 2048 values, if not a third ahead: a sixth to a half (fp16 2608 x 6400 at 122 35 / 43)
+// (altogether 9.0 percent were slower, 0.7 are; the mean over all of them is 0.848 of the time in chunks, 0.844 before.)
 float gemm_pc_cost_us(int format, int x_dtype, int64_t m, int64_t n_out, int64_t n_in) {
   if (m <= 128 && n_in > 8192) return 1e30f;
-  return pc_choose(format, x_dtype, m, n_out, n_in, false).cost_us * (m <= 128 ? (format == kQ8_0 ? 1.25f : 1.1f) : 1.f);
+  if (format == kQ6_K && (m <= 128 ? n_out > 4096 && n_in > 4096 : m <= 184 && n_in > (m <= 144 ? 4096 : 6144))) return 1e30f;
+  const bool q8_gap = format == kQ8_0 && m > 96 && n_out > 1024 && n_out <= 4096 && n_in > 2048;
+  const float margin = m > 128 ? 1.f : (q8_gap ? 1.35f : (format == kQ8_0 ? 1.25f : 1.1f));
+  return pc_choose(format, x_dtype, m, n_out, n_in, false).cost_us * margin;
 }
 
 // Whether that model would divide a launch along K.

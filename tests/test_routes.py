@@ -171,6 +171,15 @@ def test_route_detail_names_the_kernel_and_the_tile():
     assert detail(Q4_K, 14336, 4096, 0, BF16, BF16) == "none (empty call)"
 
 
+def test_calls_that_are_faster_in_chunks_of_64_rows_stay_there():
+    """65 to 184 rows where the tiled kernel's fitted time is too low, and neighbours that do go to tiles."""
+    for fmt, n_out, n_in, m, xd, chunks in ((Q6_K, 5440, 6400, 68, F16, True), (Q6_K, 192, 6400, 141, BF16, True), (Q6_K, 864, 9984, 139, BF16, True),
+                                            (Q6_K, 4112, 6400, 79, F32, True), (Q8_0, 2608, 6400, 122, F16, True), (Q6_K, 1408, 2560, 102, BF16, False),
+                                            (Q6_K, 1008, 7168, 77, BF16, False), (Q8_0, 928, 5376, 72, BF16, False), (Q8_0, 1424, 2048, 160, BF16, False)):
+        want = "gemm_skinny_f32_scaled_f16" if xd == F32 else "gemm_skinny_chunked"
+        assert (route(fmt, n_out, n_in, m, xd, xd) == want) is chunks, (fmt, n_out, n_in, m)
+
+
 def test_long_launches_keep_the_tile_that_was_measured_for_them():
     """Beyond the rows that the fitted times have seen: Q8_0 with more than a few columns reads a packed copy, and another tile than the
     earlier model's has to be a fifth ahead for 16-bit rows."""
