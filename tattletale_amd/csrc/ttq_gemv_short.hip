@@ -375,7 +375,8 @@ float gemv_short_estimate_us(int format, int x_dtype, int64_t m, int64_t n_out, 
 //     624 x 3584 (2.5) at two 3.8 / 4.0, 1024 x 4096 at four 5.0 / 5.0.  Q6_K: packed dots 1216 x 4096 (5) at two 4.7 / 4.9, 1712 x 5120
 //     (8.8) at four 9.0 / 10.8; tiles 2560 x 2560 at two 6.1 / 5.0, 7008 x 1024 (7.2) at four 5.7 / 6.2.  fp32 Q4_K 2048 x 2048
 //     at two rows 3.8 / 4.2, 2560 x 2560 6.7 / 5.1.  Q8_0: 1536 x 6912 (11) at two / four 11.6 / 8.9, 13.9 / 12.8.
-//   five to eight: Q8_0 2560 x 2560 fp32 19.9 / 11.5, 1536 x 6912 14.1 / 20.
+//   five to eight: Q8_0 2560 x 2560 fp32 19.9 / 11.5, 1536 x 6912 14.1 / 20; the windows on long fp32 rows, 1289 x 5632 (E = 7.9) at eight
+//     12.6 / 13.6, 1536 x 4608 (7.9) at seven 12.0 / 12.9; E of 6.5 to 7 0.93 of their time in the mean, 7 to 7.5 0.96, 7.5 to 8 0.99.
 bool gemv_short_preferred(int format, int x_dtype, int64_t m, int64_t n_out, int64_t n_in) {
   static const int disabled = dev_knob("TTQ_NO_SHORT", 0);
   if (n_out * n_in > 22000000 || disabled || !gemv_short_supported(format, m, n_out, n_in)) return false;
@@ -384,7 +385,8 @@ bool gemv_short_preferred(int format, int x_dtype, int64_t m, int64_t n_out, int
   const auto one_wave = [n_out] { return n_out <= 4 * device_num_cus(); };      // a workgroup of four rows to a compute unit
   if (format == kQ8_0) {
     if (m == 1) return e <= (n_out <= 2048 ? 16.f : 9.5f) && !gemv_q8_stream_supported(format, x_dtype, n_out, n_in);
-    return e <= (m <= 4 ? 12.f : 8.f);
+    if (m <= 4) return e <= 12.f;
+    return e <= (f32 && n_in > 3072 && gemv_q8_win_supported(format, n_out, n_in) ? 7.2f : 8.f);
   }
   if (format == kQ6_K) {
     if (m > 4) return f32 && e <= 8.f && n_in <= 4096;

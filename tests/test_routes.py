@@ -180,6 +180,15 @@ def test_calls_that_are_faster_in_chunks_of_64_rows_stay_there():
         assert (route(fmt, n_out, n_in, m, xd, xd) == want) is chunks, (fmt, n_out, n_in, m)
 
 
+def test_long_fp32_rows_of_q8_0_at_five_to_eight_rows():
+    """The windowed kernel is the faster one from some 7 million weights (rows rounded up to 1024 values) on; bf16 rows are not concerned."""
+    exact = _lib.PRECISION_F32_SCALES
+    for n_out, n_in, m in ((1289, 5632, 8), (1536, 4608, 7), (1281, 5376, 5)):
+        assert detail(Q8_0, n_out, n_in, m, F32, F32, exact) == "gemv_q8_win"
+        assert detail(Q8_0, n_out, n_in, m, BF16, F32, exact) == "gemv_short"
+    assert detail(Q8_0, 1100, 5632, 8, F32, F32, exact) == detail(Q8_0, 2560, 2560, 8, F32, F32, exact) == "gemv_short"
+
+
 def test_long_launches_keep_the_tile_that_was_measured_for_them():
     """Beyond the rows that the fitted times have seen: Q8_0 with more than a few columns reads a packed copy, and another tile than the
     earlier model's has to be a fifth ahead for 16-bit rows."""
