@@ -356,7 +356,11 @@ bool gemv_short_supported(int format, int64_t m, int64_t n_out, int64_t n_in) {
   return m >= 1 && m <= 8 && n_in <= (m > 1 ? 8192 : 16384) && n_out <= (1 << 20);
 }
 
-// The time of a call, us, within a fifth of 0.5 to 12 million weights.
+// The time of a call, us.  Of 15981 timed calls 0.74 to 1.19 of it in nine of ten, 0.66 to 1.31 in 49 of 50: too low for small matrices, whose
+// launch is most of it, for Q8_0 with 16-bit rows and for rows of many wavefronts (Q4_K 1152 x 10240 5.2 for 7.1, Q6_K 1712 x 5120 at four
+// rows 7.9 for 10.8), too high for 8 million weights and more of the K formats.  It decides between this kernel and the few-row kernel for fp32
+// calls of two to eight rows: of 545 timed calls that this took from the few-row kernel one got more than 3 percent slower (1712 x 5376 Q6_K at
+// four rows 10.6 / 11.1), 17 of them between 8 and 12 million weights.
 float gemv_short_estimate_us(int format, int x_dtype, int64_t m, int64_t n_out, int64_t n_in) {
   const float row = format == kQ8_0 && x_dtype != kF32 ? 0.08f : (x_dtype == kF32 ? 0.15f : 0.13f);
   return 2.6f + short_mega(n_out, n_in) * (0.09f + row * (float)m * (m > 1 && m % 2 ? 1.1f : 1.f));
@@ -395,9 +399,11 @@ bool gemv_short_preferred(int format, int x_dtype, int64_t m, int64_t n_out, int
     return e <= (m > 2 ? 6.f : (n_out <= 2048 ? 4.5f : 8.f)) && !gemv_q6k_stream4_supported(format, x_dtype, m, n_out, n_in);
   }
   if (m == 1) {
+    // (sizes first: what asks for the device costs a launch on the host 0.1 us)
+    const bool mfma = gemv_mfma_supported(format, x_dtype, n_out, n_in);
+    if (mfma && !(f32 ? e <= 4.2f && n_in <= 1024 : e <= 8.f)) return false;
     if (gemv_q4k_stream_supported(format, x_dtype, n_out, n_in) || gemv_q4k_slice_supported(format, x_dtype, n_out, n_in)) return false;
-    if (!gemv_mfma_supported(format, x_dtype, n_out, n_in)) return f32 || e <= 7.2f || one_wave();
-    return f32 ? e <= 4.2f && n_in <= 1024 : e <= 8.f;
+    return mfma || f32 || e <= 7.2f || one_wave();
   }
   if (m > 4) return f32 && e <= 6.f && n_in <= 4096;
   if (f32) return e <= 8.f && (m > 2 || n_in % 2048 != 0 || !gemv_mfma_supported(format, x_dtype, n_out, n_in));
