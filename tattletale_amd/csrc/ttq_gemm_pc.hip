@@ -68,10 +68,12 @@ static PcRoute pc_route(int64_t m, int64_t n_out, int64_t n_in) {
 //   + (split along K) trips0 + trips1 * copies + bytes of the partial sums, written and read, * traffic / 4 TB/s,
 // fitted to 150000 timed launches of 19000 layers: 768 .. 8192 wide models at 65 .. 4096 rows, and any 256 .. 120000 x 256 .. 14336 at 20 and
 // more, every tile, one to eight copies, both ways to the activations, 256 compute units; standard deviation 6 to 12 percent for tiles
-// of 128 and 64 rows, 9 to 17 for 256.  What these estimates choose is within one percent of the fastest launch of all (geometric mean)
-// and 9 percent below what the model above chooses, which has one time per step for all formats; its choice is kept where
-// the two are within five percent (slower than it by more than that: 1 percent of the layers, 2.3 without the margin).  A short
-// grid is split along K while all copies fit one round: the length of a short round is the latency of its K loop.
+// of 128 and 64 rows, 9 to 17 for 256 (profiles/gemm_tile_times.md has the fit and what it leaves over).  What these estimates choose is
+// 1 to 4 percent above the fastest launch of all (geometric means, per format and type) and 5 to 10 percent below what the model above
+// chooses, which has one time per step for all formats; its choice is kept where the two are within five percent (slower than it by more
+// than that: 0.1 to 1.6 percent of the layers).  A short grid is split along K while all copies fit one round: the length of a short round is
+// the latency of its K loop.  The fused gate||up form goes by the row-major times of Q4_K, although its tiles have half the outputs and an
+// epilogue of their own: over 1384 random layers its choice is 0.6 to 1.5 percent above the fastest tile, the model above 2.7 to 4.2.
 struct PcCost { float step, full, round, launch, trips0, trips1, traffic; };
 static const PcCost kPcCosts[3][2][kPcTileCount] = {      // [format: Q8_0, Q4_K, Q6_K][packed][tile]
     {  // Q8_0

@@ -4,7 +4,7 @@
 // Caller-owned (the ttq_*_ws entry points): the caller's buffer is bound to the calling thread for the duration of
 // one call and every request is served from it; nothing is allocated, so the call can be captured into a HIP graph
 // the first time it runs.  Layout: [0, 64 KiB) arrival counters, then the trellis hand-off words with their control
-// words, then the scratch of the call, handed out front to back.  The first two regions rely on what earlier calls
+// words, then the scratch of the call, one place for each kind of it, front to back.  The first two regions rely on what earlier calls
 // left there (counters back at zero, a generation count): the caller clears the buffer once, before its first use.
 //
 // Library-owned (the entry points without a workspace argument): one buffer per (slot, device, stream) -- launches

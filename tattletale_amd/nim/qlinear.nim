@@ -167,7 +167,7 @@ proc forward*(self: QuantLinear, x: TorchTensor, workspace = none(TorchTensor)):
 # projection, silu_and_mul (workspace/transformers/src/kernels/activations.nim:14-38), down.
 
 const kTtqErrUnsupported = -6
-const kFusedGemmMinRows = 2048   # from it on gate and up reach silu in fp32 (error 2.9e-3 against 3.9e-3), at 6 to 11 % more
+const kFusedGemmMinRows = 2048   # from it on gate and up reach silu in fp32 (error 2.9e-3 against 3.9e-3), at 3 to 8 % more
                                  # time on layers of 3584 values and more; below it the separate launches, which are faster
 const kFusedFewRowsMin = 17     # 17..64 rows: the few-row kernel with silu_and_mul in its epilogue
 const kFusedFewRowsMax = 64

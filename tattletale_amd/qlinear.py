@@ -502,9 +502,10 @@ class QuantGatedMLP:
     # arithmetic 2.9e-3 against 3.9e-3), and the (rows, 2 * intermediate) tensor is never made (235 MB at 4096 rows of
     # 28672).  On wide layers that costs time, because the epilogue's exponentials and reciprocals are quarter rate and
     # this GEMM reads its activations through LDS where the plain one reads a packed copy.  Fused / separate, us:
-    # 28672 x 4096 442 / 414 at 2048 rows, 885 / 823 at 4096, 1818 / 1670 at 8192; 27648 x 5120 and 37888 x 3584 6 to 11 %
-    # in the same direction; 6144 x 1024 43.8 / 47.6 and 77.8 / 77.9.  Fewer rows take the separate launches (28672 x 4096
-    # 125 / 118 at 512 rows, 416 / 371 at 1792): prompts of those lengths keep the faster form.
+    # 28672 x 4096 466 / 441 at 2048 rows, 910 / 865 at 4096, 1820 / 1748 at 8192; 27648 x 5120 563 / 524 and 1100 / 1030,
+    # 37888 x 3584 558 / 523 and 1098 / 1042, 16384 x 2048 168 / 161 and 321 / 310; 6144 x 1024 39.8 / 50.0 and 83.6 / 85.9.
+    # Fewer rows take the separate launches (28672 x 4096 131 / 123 at 512 rows, 432 / 404 at 1792): prompts of those lengths
+    # keep the faster form.
     FUSED_GEMM_MIN_ROWS = 2048
     # 17 to 64 rows: the same entry point runs the few-row kernel with the activation in its epilogue, one launch and one
     # (rows, 2 * intermediate) round trip less, and the same fp32 sums.  It is faster where the separate GEMM would be the
