@@ -554,7 +554,7 @@ int ttq_linear_forward(const ttq_qlinear* layer, const void* x, int x_dtype, int
     // (the integer kernel takes two rows of Q6_K to a pass: us of it / of the few-row kernel 14336 x 4096 18.1 / 21.1, 28672 x 4096
     // 27.0 / 28.9, 32000 x 5120 33.8 / 34.5, 43008 x 4096 38.2 / 36.4, 128256 x 4096 106 / 92 -- and of four rows twice that / the
     // same.  The small matrices, where the two agree to 3 us, stay with the kernel that takes any number of rows.)
-    const bool integer_passes = (int64_t)n_out * n_in >= (int64_t)120 << 20 || ttq::gemv_short_first(layer->format, x_dtype, m, n_out, n_in);
+    const bool integer_passes = (int64_t)n_out * n_in >= (int64_t)120 << 20 || ttq::gemv_short_first(layer->format, x_dtype, y_dtype, m, n_out, n_in);
     const float us_gemv = ttq::gemv_estimate_us(layer->format, x_dtype, m, n_out, n_in, integer_passes);
     // (as for fp16: only calls that the few-row kernel would have go by the fitted time)
     const bool few = rounds && us_few / few_margin() < us_gemm && (route == 2 || us_few < us_gemv);
@@ -569,7 +569,7 @@ int ttq_linear_forward(const ttq_qlinear* layer, const void* x, int x_dtype, int
       return hip_status(ttq::launch_gemm_pc_x(layer->format, layer->qweight, x, x_dtype, y, y_dtype, layer->bias,
                                               layer->bias_dtype, m, n_out, n_in, s, true));
   }
-  if (block_fmt && ttq::gemv_short_first(layer->format, x_dtype, m, n_out, n_in))
+  if (block_fmt && ttq::gemv_short_first(layer->format, x_dtype, y_dtype, m, n_out, n_in))
     return hip_status(ttq::launch_gemv_short_routed(layer->format, layer->qweight, x, x_dtype, y, y_dtype, layer->bias,
                                                     layer->bias_dtype, m, n_out, n_in, s));
   return hip_status(launch_gemv_any_m(layer->format, layer->qweight, x, x_dtype, y, y_dtype, layer->bias,

@@ -495,8 +495,8 @@ static ManyRows many_rows(int format, int x_dtype, int64_t m, int64_t n_out, int
 
 // Small matrices take the kernel that reads everything at once, but for calls of Q6_K that the tile kernel has: one or two
 // fp32 rows, and any of 8 million weights and more.
-bool gemv_short_first(int format, int x_dtype, int64_t m, int64_t n_out, int64_t n_in) {
-  if (!gemv_short_preferred(format, x_dtype, m, n_out, n_in)) return false;
+bool gemv_short_first(int format, int x_dtype, int y_dtype, int64_t m, int64_t n_out, int64_t n_in) {
+  if (!gemv_short_preferred(format, x_dtype, y_dtype, m, n_out, n_in)) return false;
   const bool large = n_out * n_in >= 8000000;
   if (format != kQ6_K || !(large || (x_dtype == kF32 && m <= 2))) return true;
   return !gemv_tile_preferred(format, x_dtype, m, n_out, n_in) && !(large && many_rows(format, x_dtype, m, n_out, n_in) != ManyRows::kOther);
@@ -524,7 +524,7 @@ hipError_t launch_gemv(int format, const void* w, const void* x, int x_dtype, vo
   }
   // (16-bit rows of Q4_K: the operator alone, calls of the GEMV itself with one row and with several stay within
   // 2e-6 of each other there, as the kernels below do)
-  if (!(format == kQ4_K && x_dtype != kF32) && gemv_short_first(format, x_dtype, m, n_out, n_in))
+  if (!(format == kQ4_K && x_dtype != kF32) && gemv_short_first(format, x_dtype, y_dtype, m, n_out, n_in))
     return launch_gemv_short_routed(format, w, x, x_dtype, y, y_dtype, bias, bias_dtype, m, n_out, n_in, s);
   const ManyRows many = many_rows(format, x_dtype, m, n_out, n_in);
   if (many != ManyRows::kOther) {
@@ -601,7 +601,7 @@ float gemv_estimate_us(int format, int x_dtype, int64_t m, int64_t n_out, int64_
   if (integer_kernels) {
     // (never more than the estimate without it: no call that decoded is moved to rounded weights by the better guess; five rows of 16 bits
     // and more keep the rounding kernels that they have, 2432 x 1024 Q8_0 fp16 at six rows 4.4 there and 4.9)
-    if ((x_dtype == kF32 || m <= 4) && gemv_short_first(format, x_dtype, m, n_out, n_in)) {
+    if ((x_dtype == kF32 || m <= 4) && gemv_short_first(format, x_dtype, x_dtype, m, n_out, n_in)) {
       const float us = gemv_short_estimate_us(format, x_dtype, m, n_out, n_in), old = gemv_estimate_us(format, x_dtype, m, n_out, n_in, false);
       return us < old ? us : old;
     }

@@ -367,7 +367,7 @@ float gemv_short_estimate_us(int format, int x_dtype, int64_t m, int64_t n_out, 
 }
 
 // Whether it is the faster one; the kernels that would run otherwise are asked for in the order of launch_gemv.  E: millions of
-// weights, rows rounded up to 1024 values.  us, the other kernel / this one:
+// weights, rows rounded up to 1024 values.  us, the other kernel / this one, 16-bit rows with 16-bit outputs unless it says otherwise:
 //   one row.  Q8_0, the stream (16 rows to a compute unit, whole rounds): 4096 x 2048 4.5 / 4.6, so not there; the windows, from 2048 rows
 //     of weights on, 3072 x 2304 (E = 9.4) 6.4 / 4.9, 9504 x 256 (9.7) 4.1 / 4.3, 5520 x 2048 (11) 5.8 / 6.2; else 1024 x 14336 (15) 10.6 / 6.5.
 //     Q4_K, the stream: 4096 x 2048 3.1 / 3.8; the int8 kernel, from 2048 rows of weights on, 16-bit 5120 x 1280 (10) 4.4 / 4.0,
@@ -375,13 +375,17 @@ float gemv_short_estimate_us(int format, int x_dtype, int64_t m, int64_t n_out, 
 //     packed dots, 1024 x 14336 6.4 / 5.2, a wave of workgroups; 1152 x 10240 (12) 5.6 / 7.1, two; the generic kernel 1536 x 6912 8.1 / 5.4.
 //     Q6_K, the stream: 4096 x 2048 4.0 / 4.4; packed dots 10240 x 1280 10.2 / 6.4, 1536 x 6912 6.5 / 5.5, 1152 x 14848 8.9 / 9.4; generic
 //     kernel 3072 x 2304 6.7 / 4.7.
+//     fp32 outputs of 16-bit rows cost the packed dots 0.8 less than 16-bit ones and this kernel nothing: Q4_K bf16 1536 x 4096 (6.3) 3.5 / 3.7,
+//     1024 x 4096 3.4 / 3.4, so from E = 3.3 on, rows of 2049 to 4096 values, they keep the dots.  fp16 rows do not, although 1 to 11 percent
+//     slower: their sums with the quants as 1024 + q are 5e-6 to 9e-6 from 64 bits, here 0.5e-7; nor Q8_0 8300 x 256 and more (4.1 / 4.3): the windows
+//     read 16-bit rows as fixed point (2e-5).
 //   two to four rows.  Q4_K 16-bit, the four-row int8 kernel: 2560 x 2560 (7.9) at two / four rows 6.5 / 5.0, 6.5 / 7.0; packed dots
-//     624 x 3584 (2.5) at two 3.8 / 4.0, 1024 x 4096 at four 5.0 / 5.0.  Q6_K: packed dots 1216 x 4096 (5) at two 4.7 / 4.9, 1712 x 5120
-//     (8.8) at four 9.0 / 10.8; tiles 2560 x 2560 at two 6.1 / 5.0, 7008 x 1024 (7.2) at four 5.7 / 6.2.  fp32 Q4_K 2048 x 2048
+//     624 x 3584 (2.5) at two 3.8 / 4.0, 1024 x 4096 at four 5.0 / 5.0, 1145 x 2816 (3.5) with 16-bit outputs 5.2 / 5.4.  Q6_K: packed dots
+//     1216 x 4096 (5) at two 4.7 / 4.9, 1312 x 2560 (4) 4.3 / 4.6 (1025 to 2048 rows of 2049 to 4096 values), 1712 x 5120 (8.8) at four 9.0 / 10.8; tiles 2560 x 2560 at two 6.1 / 5.0, 7008 x 1024 (7.2) at four 5.7 / 6.2.  fp32 Q4_K 2048 x 2048
 //     at two rows 3.8 / 4.2, 2560 x 2560 6.7 / 5.1.  Q8_0: 1536 x 6912 (11) at two / four 11.6 / 8.9, 13.9 / 12.8.
 //   five to eight: Q8_0 2560 x 2560 fp32 19.9 / 11.5, 1536 x 6912 14.1 / 20; the windows on long fp32 rows, 1289 x 5632 (E = 7.9) at eight
 //     12.6 / 13.6, 1536 x 4608 (7.9) at seven 12.0 / 12.9; E of 6.5 to 7 0.93 of their time in the mean, 7 to 7.5 0.96, 7.5 to 8 0.99.
-bool gemv_short_preferred(int format, int x_dtype, int64_t m, int64_t n_out, int64_t n_in) {
+bool gemv_short_preferred(int format, int x_dtype, int y_dtype, int64_t m, int64_t n_out, int64_t n_in) {
   static const int disabled = dev_knob("TTQ_NO_SHORT", 0);
   if (n_out * n_in > 22000000 || disabled || !gemv_short_supported(format, m, n_out, n_in)) return false;
   const float e = short_mega(n_out, n_in);
@@ -396,6 +400,7 @@ bool gemv_short_preferred(int format, int x_dtype, int64_t m, int64_t n_out, int
     if (m > 4) return f32 && e <= 8.f && n_in <= 4096;
     if (m == 1) return (n_in <= 14336 || one_wave()) && !gemv_q6k_stream_supported(format, x_dtype, n_out, n_in);
     if (f32) return e <= 12.f;
+    if (m == 2 && n_out > 1024 && n_out <= 2048 && n_in > 2048 && n_in <= 4096) return false;
     return e <= (m > 2 ? 6.f : (n_out <= 2048 ? 4.5f : 8.f)) && !gemv_q6k_stream4_supported(format, x_dtype, m, n_out, n_in);
   }
   if (m == 1) {
@@ -403,13 +408,14 @@ bool gemv_short_preferred(int format, int x_dtype, int64_t m, int64_t n_out, int
     const bool mfma = gemv_mfma_supported(format, x_dtype, n_out, n_in);
     if (mfma && !(f32 ? e <= 4.2f && n_in <= 1024 : e <= 8.f)) return false;
     if (gemv_q4k_stream_supported(format, x_dtype, n_out, n_in) || gemv_q4k_slice_supported(format, x_dtype, n_out, n_in)) return false;
+    if (!mfma && x_dtype == kBF16 && y_dtype == kF32 && n_in > 2048 && n_in <= 4096 && e > 3.3f) return false;
     return mfma || f32 || e <= 7.2f || one_wave();
   }
   if (m > 4) return f32 && e <= 6.f && n_in <= 4096;
   if (f32) return e <= 8.f && (m > 2 || n_in % 2048 != 0 || !gemv_mfma_supported(format, x_dtype, n_out, n_in));
   if (gemv_q4k_stream4_supported(format, x_dtype, m, n_out, n_in)) return false;
   if (gemv_q4k_batch4_supported(format, x_dtype, m, n_out, n_in)) return e <= (m == 2 ? 8.f : 5.f);
-  return e <= (m == 2 ? 2.f : 4.f);
+  return e <= (m == 2 ? 2.f : (m == 4 && y_dtype != kF32 && n_in > 2048 && n_in <= 3072 ? 3.1f : 4.f));
 }
 
 hipError_t launch_gemv_short(int format, const void* w, const void* x, int x_dtype, void* y, int y_dtype, const void* bias,

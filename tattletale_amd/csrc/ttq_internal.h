@@ -112,8 +112,8 @@ hipError_t launch_gemv_dot2(int format, const void* w, const void* x, int x_dtyp
 
 // Matrices of a few MB, up to eight activation rows, everything straight into registers (ttq_gemv_short.hip).
 bool gemv_short_supported(int format, int64_t m, int64_t n_out, int64_t n_in);
-bool gemv_short_preferred(int format, int x_dtype, int64_t m, int64_t n_out, int64_t n_in);
-bool gemv_short_first(int format, int x_dtype, int64_t m, int64_t n_out, int64_t n_in);      // (ttq_gemv.hip: among all decode kernels)
+bool gemv_short_preferred(int format, int x_dtype, int y_dtype, int64_t m, int64_t n_out, int64_t n_in);
+bool gemv_short_first(int format, int x_dtype, int y_dtype, int64_t m, int64_t n_out, int64_t n_in);      // (ttq_gemv.hip: among all decode kernels)
 float gemv_short_estimate_us(int format, int x_dtype, int64_t m, int64_t n_out, int64_t n_in);
 hipError_t launch_gemv_short(int format, const void* w, const void* x, int x_dtype, void* y, int y_dtype, const void* bias,
                              int bias_dtype, int64_t m, int64_t n_out, int64_t n_in, hipStream_t s);

@@ -161,7 +161,7 @@ def detail(fmt, n_out, n_in, m, x_dtype, y_dtype, precision=_lib.PRECISION_AUTO)
 def test_route_detail_names_the_kernel_and_the_tile():
     """Calls of one family that go to different kernels, and the tiled GEMM's launches, told apart."""
     assert detail(Q4_K, 14336, 4096, 1, BF16, F32) == "gemv_q4k_stream"         # a family of one kernel: its name
-    assert detail(Q4_K, 1024, 4096, 1, BF16, F32) == detail(Q8_0, 2048, 1024, 1, F32, F32) == "gemv_short"
+    assert detail(Q4_K, 1024, 4096, 1, BF16, BF16) == detail(Q8_0, 2048, 1024, 1, F32, F32) == "gemv_short"
     assert detail(Q6_K, 2560, 2560, 3, F32, F32) == detail(Q6_K, 1024, 1024, 2, F16, F16) == "gemv_short"
     assert detail(Q4_K, 16384, 53248, 1, BF16, F32) == "gemv_dot2"
     assert detail(Q6_K, 1536, 4096, 4, BF16, BF16) == "gemv_dot2_multi"
@@ -187,6 +187,18 @@ def test_long_fp32_rows_of_q8_0_at_five_to_eight_rows():
         assert detail(Q8_0, n_out, n_in, m, F32, F32, exact) == "gemv_q8_win"
         assert detail(Q8_0, n_out, n_in, m, BF16, F32, exact) == "gemv_short"
     assert detail(Q8_0, 1100, 5632, 8, F32, F32, exact) == detail(Q8_0, 2560, 2560, 8, F32, F32, exact) == "gemv_short"
+
+
+def test_matrices_that_the_packed_dots_are_faster_on_stay_with_them():
+    """bf16 rows with fp32 outputs, whose stores cost the packed dots less; two rows of Q6_K with more than 1024 outputs."""
+    for n_out, n_in in ((1536, 4096), (1999, 2560), (1200, 3584)):
+        assert detail(Q4_K, n_out, n_in, 1, BF16, F32) == "gemv_dot2"
+        assert detail(Q4_K, n_out, n_in, 1, BF16, BF16) == detail(Q4_K, n_out, n_in, 1, F16, F32) == "gemv_short"
+    assert detail(Q4_K, 800, 4096, 1, BF16, F32) == detail(Q4_K, 1536, 2048, 1, BF16, F32) == "gemv_short"
+    for n_out, n_in in ((1312, 2560), (1090, 4096)):
+        assert detail(Q6_K, n_out, n_in, 2, F16, F16) == detail(Q6_K, n_out, n_in, 2, BF16, F32) == "gemv_dot2_multi"
+    assert detail(Q6_K, 1000, 2560, 2, F16, F16) == detail(Q6_K, 1312, 2048, 2, F16, F16) == "gemv_short"
+    assert detail(Q4_K, 1145, 2816, 4, F16, F16) == "gemv_dot2_multi" and detail(Q4_K, 1145, 2816, 4, F16, F32) == "gemv_short"
 
 
 def test_long_launches_keep_the_tile_that_was_measured_for_them():
