@@ -210,6 +210,8 @@ def test_long_launches_keep_the_tile_that_was_measured_for_them():
     assert detail(Q4_K, 34944, 1024, 5993, BF16, BF16) == detail(Q4_K, 2304, 1536, 3648, BF16, BF16) == "gemm_pc 256x112 packed"
     assert detail(Q4_K, 12288, 1024, 3905, F16, F16) == "gemm_pc 256x112 packed"
     assert detail(Q8_0, 512, 4096, 6338, F16, F16) == "gemm_pc 128x112 packed"
+    # and the shortest: two copies along K are kept against one of smaller tiles
+    assert detail(Q4_K, 14048, 8192, 62, BF16, BF16) == "gemm_pc 64x112 k/2"
 
 
 @pytest.mark.parametrize("fmt,n_out,n_in,m", [(Q8_0, 8317, 3072, 25463), (Q8_0, 7773, 256, 18290), (Q4_K, 116, 7168, 13668), (Q4_K, 512, 14336, 8300),
